@@ -60,91 +60,143 @@ void prof_end(dndsmi_ctx *c) {
 // kernels
 // ========================================================================
 
-// Boundary correction of a Wall_Euler / Wall_NoSlip face w to its cell's
-// sweep (DNDS_FV_VR.hpp:1577-1657), from the cell's coefficients xi and mean
-// ui: corr = relax A^-1 sum_g w_g |n_g| D0^T W0^2 (uBV - u_i).  ADD adds the
-// correction to corr (xi may then be corr itself: xi is read in full before
-// corr is written); otherwise it is stored there.
-template <bool ADD>
-__device__ inline void wall_correction(int32_t w, int32_t bc, const double *xi, const double ui[4],
-                                       const double *__restrict__ wall_ainv, const double *__restrict__ wall_d0,
-                                       const double *__restrict__ wall_nrm, const double *__restrict__ wall_w0,
-                                       int64_t ldw, double relax, const GasParams &gp, double t, int32_t *errw,
-                                       double *corr) {
-    double BCc[36];
-    for (int k = 0; k < 36; k++)
-        BCc[k] = 0.0;
-    const double w0 = wall_w0[w];
-    for (int g = 0; g < 3; g++) {
-        const double gw = g == 1 ? kLine3W1 : kLine3W0;
-        const double nx = wall_nrm[(2 * g) * ldw + w], ny = wall_nrm[(2 * g + 1) * ldw + w];
-        double uBL[4];
-        for (int v = 0; v < 4; v++) {
-            double acc = 0;
-            for (int c = 0; c < 9; c++)
-                acc += wall_d0[(g * 9 + c) * ldw + w] * xi[c + 9 * v];
-            uBL[v] = acc;
-        }
-        for (int v = 0; v < 4; v++)
-            uBL[v] += ui[v];
-        double n0, n1;
-        stable_normalized(nx, ny, n0, n1);
-        double uBV[4];
-        if (bc == BC_WALL_EULER) {
-            for (int v = 0; v < 4; v++)
-                uBV[v] = uBL[v];
-            const double dd = n0 * uBV[1] + n1 * uBV[2];
-            uBV[1] = uBL[1] - n0 * dd;
-            uBV[2] = uBL[2] - n1 * dd;
-        } else if (!boundary_value(gp, uBL, n0, n1, 0.0, 0.0, t, bc, uBV)) {
-            atomicOr(errw, ERRBIT_NONPOSITIVE);
-            for (int v = 0; v < 4; v++)
-                uBV[v] = uBL[v];
-        }
-        const double nl = sqrt(nx * nx + ny * ny);
-        for (int r = 0; r < 9; r++)
-            for (int v = 0; v < 4; v++) {
-                double inc = wall_d0[(g * 9 + r) * ldw + w] * w0 * w0 * (uBV[v] - ui[v]);
-                inc *= nl;
-                BCc[r + 9 * v] += inc * gw;
-            }
-    }
-    for (int r = 0; r < 9; r++)
-        for (int v = 0; v < 4; v++) {
-            double acc = 0;
-            for (int c = 0; c < 9; c++)
-                acc += wall_ainv[(r * 9 + c) * ldw + w] * BCc[c + 9 * v];
-            if (ADD)
-                corr[r + 9 * v] += relax * acc;
-            else
-                corr[r + 9 * v] = relax * acc;
-        }
+// ---- reconstruction sweeps: four lanes per cell --------------------------
+//
+// A sweep is bound by its stream of A^-1 B (720 B per cell and face, read
+// once) and by the latency of the gathers beside it.  Four neighbouring lanes
+// (a quad) own one cell, lane v of the quad variable v, so a wave covers 16
+// cells: a lane keeps 9 coefficients instead of 36, which leaves registers
+// for the loads of several slots in flight.  Each lane loads a quarter of the
+// cell's A^-1 B (one contiguous KiB per wave and load) and the quad passes
+// the entries around with DPP moves, so no byte is loaded twice.  Every sum
+// runs in the order of a one-lane-per-cell sweep.
+
+// `a` of lane Q of the quad, in all four lanes
+template <int Q>
+__device__ __forceinline__ int quad_bcast32(int a) {
+    return __builtin_amdgcn_mov_dpp(a, Q * 0x55, 0xf, 0xf, true);
+}
+template <int Q>
+__device__ __forceinline__ double quad_bcast(double a) {
+    const uint64_t w = __builtin_bit_cast(uint64_t, a);
+    const uint32_t lo = uint32_t(quad_bcast32<Q>(int(uint32_t(w))));
+    const uint32_t hi = uint32_t(quad_bcast32<Q>(int(uint32_t(w >> 32))));
+    return __builtin_bit_cast(double, uint64_t(lo) | uint64_t(hi) << 32);
+}
+template <int Q>
+__device__ __forceinline__ float quad_bcast(float a) {
+    return __builtin_bit_cast(float, quad_bcast32<Q>(__builtin_bit_cast(int, a)));
+}
+template <typename T>
+__device__ __forceinline__ T quad_get(T a, int q) { // q: a constant after unrolling
+    return q == 0 ? quad_bcast<0>(a) : q == 1 ? quad_bcast<1>(a) : q == 2 ? quad_bcast<2>(a) : quad_bcast<3>(a);
 }
 
-// The Jacobi sweep's wall corrections, computed before the sweep from the
-// current iterate; the sweep adds each in the face's slot, which keeps the
-// reference's accumulation order.
-__global__ __launch_bounds__(kBlock) void k_wall_corr(int32_t nw, int64_t ldc, const int32_t *__restrict__ wcell,
-                                                      const int32_t *__restrict__ wbc,
-                                                      const double *__restrict__ wall_ainv,
-                                                      const double *__restrict__ wall_d0,
-                                                      const double *__restrict__ wall_nrm,
-                                                      const double *__restrict__ wall_w0, int64_t ldw,
-                                                      const double *__restrict__ u, const double *__restrict__ x,
-                                                      double relax, GasParams gp, double t,
-                                                      double *__restrict__ corr, int32_t *errw) {
-    const int32_t w = blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= nw)
-        return;
-    const int32_t i = wcell[w];
-    double xi[36], ui[4], cw[36];
-    for (int k = 0; k < 36; k++)
-        xi[k] = x[k * ldc + i];
-    for (int v = 0; v < 4; v++)
-        ui[v] = u[4 * int64_t(i) + v];
-    wall_correction<false>(w, wbc[w], xi, ui, wall_ainv, wall_d0, wall_nrm, wall_w0, ldw, relax, gp, t, errw, cw);
-    for (int k = 0; k < 36; k++)
-        corr[k * ldw + w] = cw[k];
+// the neighbouring lane's `a` (lanes 2 k and 2 k + 1 exchange)
+__device__ __forceinline__ double pair_swap(double a) {
+    const uint64_t w = __builtin_bit_cast(uint64_t, a);
+    const uint32_t lo = uint32_t(__builtin_amdgcn_mov_dpp(int(uint32_t(w)), 0xb1, 0xf, 0xf, true));
+    const uint32_t hi = uint32_t(__builtin_amdgcn_mov_dpp(int(uint32_t(w >> 32)), 0xb1, 0xf, 0xf, true));
+    return __builtin_bit_cast(double, uint64_t(lo) | uint64_t(hi) << 32);
+}
+
+// A lane's part of the A^-1 B, A^-1 b of one cell and slot (ab_vec's layout)
+struct AbPart {
+    dbl2 w[kAbVecs / 4], last;
+    __device__ __forceinline__ void load(const double *__restrict__ M, int s, int32_t i, int64_t ldc, int v) {
+        // a wave holds one group of 16 cells: a scalar base
+        const int32_t g = __builtin_amdgcn_readfirstlane(i);
+        const dbl2 *p = reinterpret_cast<const dbl2 *>(M) + ab_group(s, g, ldc, kAbVecs);
+        const uint32_t cl = i & 15;
+#pragma unroll
+        for (int k = 0; k < kAbVecs / 4; k++)
+            w[k] = __builtin_nontemporal_load(p + 64 * k + (4 * cl + v));
+        last = __builtin_nontemporal_load(p + 16 * (kAbVecs - 1) + cl);
+    }
+    // entry d = 10 r + c: A^-1 B (c < 9) or A^-1 b (c = 9) of row r
+    __device__ __forceinline__ double get(int d) const {
+        const int p = d / 2;
+        if (p == kAbVecs - 1)
+            return d % 2 ? last.y : last.x;
+        return quad_get(d % 2 ? w[p / 4].y : w[p / 4].x, p % 4);
+    }
+};
+
+// nw[r] += relax ((M xj)_r + du (bmul b_r)), rows in turn
+__device__ __forceinline__ void ab_apply(const AbPart &ab, const double xj[9], double du, double bmul, double relax,
+                                         double nw[9]) {
+#pragma unroll
+    for (int r = 0; r < 9; r++) {
+        double tt = 0.0;
+#pragma unroll
+        for (int c = 0; c < 9; c++)
+            tt += ab.get(10 * r + c) * xj[c];
+        const double b = bmul * ab.get(10 * r + 9);
+        nw[r] += relax * (tt + du * b);
+    }
+}
+
+// Boundary correction of Wall_Euler / Wall_NoSlip face w to its cell's sweep
+// (DNDS_FV_VR.hpp:1577-1657), from the cell's coefficients xi and mean ui of
+// this lane's variable v: out = relax A^-1 sum_g w_g |n_g| D0^T W0^2 (uBV -
+// u_i).  The four lanes of the cell's quad call it together.
+__device__ __forceinline__ void wall_correction(int32_t w, int32_t bc, const double xi[9], double ui, int v,
+                                                const WallFaces &wf, double relax, int32_t *errw, double out[9]) {
+    double BCc[9];
+#pragma unroll
+    for (int r = 0; r < 9; r++)
+        BCc[r] = 0.0;
+    const double w0 = wf.w0[w];
+#pragma unroll 1
+    for (int g = 0; g < 3; g++) {
+        const double gw = g == 1 ? kLine3W1 : kLine3W0;
+        const double nx = wf.nrm[(2 * g) * wf.ld + w], ny = wf.nrm[(2 * g + 1) * wf.ld + w];
+        double d0[9];
+#pragma unroll
+        for (int c = 0; c < 9; c++)
+            d0[c] = wf.d0[(g * 9 + c) * wf.ld + w];
+        double uB = 0;
+#pragma unroll
+        for (int c = 0; c < 9; c++)
+            uB += d0[c] * xi[c];
+        uB += ui;
+        double n0, n1;
+        stable_normalized(nx, ny, n0, n1);
+        const double rho = quad_bcast<0>(uB), m0 = quad_bcast<1>(uB), m1 = quad_bcast<2>(uB);
+        double uBV = uB;
+        if (bc == BC_WALL_EULER) {
+            const double dd = n0 * m0 + n1 * m1;
+            if (v == 1)
+                uBV = uB - n0 * dd;
+            else if (v == 2)
+                uBV = uB - n1 * dd;
+        } else if (!(rho > 0)) {
+            atomicOr(errw, ERRBIT_NONPOSITIVE);
+        } else if (v == 1 || v == 2) {
+            uBV *= -1;
+        }
+        const double nl = sqrt(nx * nx + ny * ny);
+#pragma unroll
+        for (int r = 0; r < 9; r++) {
+            double inc = d0[r] * w0 * w0 * (uBV - ui);
+            inc *= nl;
+            BCc[r] += inc * gw;
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 9; r++) {
+        double acc = 0;
+#pragma unroll
+        for (int c = 0; c < 9; c++)
+            acc += wf.ainv[(r * 9 + c) * wf.ld + w] * BCc[c];
+        out[r] = relax * acc;
+    }
+}
+
+// where the wave's group of 16 cells starts in a REC array; lane l's variable
+// of its cell lies l further on, coefficient c 256 c further on
+__device__ __forceinline__ int64_t rec_group(int32_t i) {
+    return rec(__builtin_amdgcn_readfirstlane(i) & ~15, 0, 0);
 }
 
 // One SOR pass over cells of one colour (SOR_Instead,
@@ -154,304 +206,242 @@ __global__ __launch_bounds__(kBlock) void k_wall_corr(int32_t nw, int64_t ldc, c
 // order.  As in the reference, every term is added to the cell's own
 // coefficients: the far-field product M x_i and the Wall_Euler / Wall_NoSlip
 // corrections take the partial sum after (1 - w) scaling and the faces before
-// them (the product is formed from a copy, then added).
+// them.
 //
 // The cells are the device range [base, base + n): with SOR_Instead the
-// device numbering is colour-major.  SELF: the cells may have far-field,
-// Wall_Euler or Wall_NoSlip faces, the terms that read the cell's own partial
-// sum; the numbering puts those cells after the colour's others, so that the
-// others (all but the boundary layer) run without the registers of the copy
-// and of the wall correction.  x and xo are the
-// same array: the new coefficients go out through xo so that the compiler
-// does not keep the 36 addresses of the first reads live until the stores.
-template <int NF, bool SELF>
-__global__ __launch_bounds__(kBlock) void k_sor(int32_t n, int32_t base, int64_t ldc, const int32_t *__restrict__ nbr,
-                                                const int32_t *__restrict__ sbc, const int32_t *__restrict__ wall_idx,
-                                                const double *__restrict__ M, const double *__restrict__ bv,
-                                                const double *__restrict__ u, const double *x, double *xo,
-                                                double relax, const double *__restrict__ wall_ainv,
-                                                const double *__restrict__ wall_d0,
-                                                const double *__restrict__ wall_nrm,
-                                                const double *__restrict__ wall_w0, int64_t ldw, GasParams gp,
-                                                double t, int32_t *errw) {
-    const int32_t tid = xcd_block() * blockDim.x + threadIdx.x;
-    if (tid >= n)
+// device numbering is colour-major.  x and xo are the same array.
+template <int NF>
+__global__ __launch_bounds__(kBlock, 2) void k_sor(int32_t n, int32_t base, int64_t ldc,
+                                                   const int32_t *__restrict__ nbr, const int32_t *__restrict__ sbc,
+                                                   const int32_t *__restrict__ wall_idx,
+                                                   const double *__restrict__ M, const double *__restrict__ u,
+                                                   const double *x, double *xo, double relax, WallFaces wf,
+                                                   int32_t *errw) {
+    const int32_t t = xcd_block() * blockDim.x + threadIdx.x, v = t & 3;
+    // whole groups of 16 cells from the one that holds `base`
+    const int32_t i = (base & ~15) + (t >> 2);
+    if (i < base || i >= base + n)
         return;
-    const int32_t i = base + tid;
-    double nw[36];
+    const uint32_t lane = threadIdx.x & 63;
+    int32_t jn[NF];
 #pragma unroll
-    for (int k = 0; k < 36; k++)
-        nw[k] = (1 - relax) * x[k * ldc + i];
-    double ui[4];
+    for (int s = 0; s < NF; s++)
+        jn[s] = nbr[s * ldc + i];
+    const double ui = u[4 * int64_t(i) + v];
+    double nw[9];
 #pragma unroll
-    for (int v = 0; v < 4; v++)
-        ui[v] = u[4 * int64_t(i) + v];
-#pragma unroll 1
+    for (int r = 0; r < 9; r++)
+        nw[r] = (1 - relax) * (x + rec_group(i))[256 * r + lane];
+#pragma unroll
     for (int s = 0; s < NF; s++) {
-        const int32_t j = nbr[s * ldc + i];
+        const int32_t j = jn[s];
         if (j == -2)
             continue;
-        const double *bs = bv + int64_t(s) * 9 * ldc + i;
-        double xj[36], du[4], bmul = 1.0;
+        AbPart ab;
+        ab.load(M, s, i, ldc, v);
         if (j >= 0) {
+            double xj[9];
 #pragma unroll
-            for (int v = 0; v < 4; v++)
-                du[v] = u[4 * int64_t(j) + v] - ui[v];
-#pragma unroll
-            for (int k = 0; k < 36; k++)
-                xj[k] = x[k * ldc + j];
-        } else {
-            const int32_t bc = sbc[s * ldc + i];
-            if (bc == BC_WALL) {
-#pragma unroll
-                for (int r = 0; r < 9; r++) {
-                    const double b = bs[r * ldc];
-#pragma unroll
-                    for (int v = 0; v < 4; v++)
-                        nw[r + 9 * v] += relax * ((0.0 - ui[v]) * b);
-                }
-                continue;
-            }
-            if (!SELF) { // not in this launch's lists
-                atomicOr(errw, ERRBIT_BC);
-                continue;
-            }
-            if (bc == BC_WALL_EULER || bc == BC_WALL_NOSLIP) {
-                wall_correction<true>(wall_idx[s * ldc + i], bc, nw, ui, wall_ainv, wall_d0, wall_nrm, wall_w0, ldw,
-                                      relax, gp, t, errw, nw);
-                continue;
-            }
-            if (!is_far(bc)) {
-                atomicOr(errw, ERRBIT_BC);
-                continue;
-            }
-            // far field: M_if times the partial sum, no mean-value term
-#pragma unroll
-            for (int v = 0; v < 4; v++)
-                du[v] = 0.0;
-#pragma unroll
-            for (int k = 0; k < 36; k++)
-                xj[k] = nw[k];
-            bmul = 0.0;
+            for (int c = 0; c < 9; c++)
+                xj[c] = x[rec(j, c, v)];
+            ab_apply(ab, xj, u[4 * int64_t(j) + v] - ui, 1.0, relax, nw);
+            continue;
         }
-        const dbl2 *Ms = reinterpret_cast<const dbl2 *>(M) + m_vec_index(s, 0, i, ldc, kMPairs);
-        dbl2 mp = {0.0, 0.0};
-        double tt[4] = {0, 0, 0, 0};
+        const int32_t bc = sbc[s * ldc + i];
+        if (bc == BC_WALL) {
 #pragma unroll
-        for (int e = 0; e < 81; e++) {
-            const int r = e / 9, c = e % 9;
-            if (e % 2 == 0)
-                mp = __builtin_nontemporal_load(Ms + (e / 2) * 64);
-            const double m = e % 2 == 0 ? mp.x : mp.y;
-            if (c == 0)
-                tt[0] = tt[1] = tt[2] = tt[3] = 0.0;
+            for (int r = 0; r < 9; r++)
+                nw[r] += relax * ((0.0 - ui) * ab.get(10 * r + 9));
+        } else if (bc == BC_WALL_EULER || bc == BC_WALL_NOSLIP) {
+            double cw[9];
+            wall_correction(wall_idx[s * ldc + i], bc, nw, ui, v, wf, relax, errw, cw);
 #pragma unroll
-            for (int v = 0; v < 4; v++)
-                tt[v] += m * xj[c + 9 * v];
-            if (c == 8) {
-                const double b = bmul * __builtin_nontemporal_load(bs + r * ldc);
+            for (int r = 0; r < 9; r++)
+                nw[r] += cw[r];
+        } else if (is_far(bc)) {
+            // M_if times the partial sum, no mean-value term
+            double own[9];
 #pragma unroll
-                for (int v = 0; v < 4; v++)
-                    nw[r + 9 * v] += relax * (tt[v] + du[v] * b);
-            }
+            for (int c = 0; c < 9; c++)
+                own[c] = nw[c];
+            ab_apply(ab, own, 0.0, 0.0, relax, nw);
+        } else {
+            atomicOr(errw, ERRBIT_BC);
         }
     }
 #pragma unroll
-    for (int k = 0; k < 36; k++)
-        __builtin_nontemporal_store(nw[k], &xo[k * ldc + i]);
+    for (int r = 0; r < 9; r++)
+        __builtin_nontemporal_store(nw[r], xo + rec_group(i) + (256 * r + lane));
 }
 
 // One block-Jacobi VR sweep, SOR off (ReconstructionJacobiStep,
 // DNDS_FV_VR.hpp:1495-1682): new_i = (1-w) x_i + w sum_f [M_if x_j + b_if (u_j - u_i)^T]
 // in cell2face order, with the reference's boundary variants: far field
 // couples the cell to itself (M_if x_i), a Wall face adds b_if (0 - u_i)^T,
-// Wall_Euler / Wall_NoSlip faces add the correction of k_wall_corr.
+// Wall_Euler / Wall_NoSlip faces add their correction from the old iterate.
 //
 // RESID (the FP64 step of the mixed-precision sweeps): instead of the new
-// iterate, writes the increment r = J(x) - x rounded to FP32 into r32 and d32
-// (the start of the FP32 correction sweeps, k_delta32).
-template <int NF, bool RESID = false>
-__global__ __launch_bounds__(kBlock) void k_jacobi(int32_t nc, int64_t ldc, const int32_t *__restrict__ nbr,
-                                                   const int32_t *__restrict__ sbc,
-                                                   const int32_t *__restrict__ wall_idx,
-                                                   const double *__restrict__ M, const double *__restrict__ bv,
-                                                   const double *__restrict__ u, const double *__restrict__ x,
-                                                   double *__restrict__ xn, double relax,
-                                                   const double *__restrict__ corr, int64_t ldw, int32_t *errw,
-                                                   float *__restrict__ r32 = nullptr,
-                                                   float *__restrict__ d32 = nullptr) {
-    const int32_t i = xcd_block() * blockDim.x + threadIdx.x;
+// iterate, writes the increment r = J(x) - x rounded to FP32 into r32 (also the
+// start of the FP32 correction sweeps, k_delta32).
+template <int NF, bool RESID>
+__global__ __launch_bounds__(kBlock, 2) void k_jacobi(int32_t nc, int64_t ldc, const int32_t *__restrict__ nbr,
+                                                      const int32_t *__restrict__ sbc,
+                                                      const int32_t *__restrict__ wall_idx,
+                                                      const double *__restrict__ M, const double *__restrict__ u,
+                                                      const double *__restrict__ x, double *__restrict__ xn,
+                                                      double relax, WallFaces wf, double *corr, int32_t *errw,
+                                                      float *__restrict__ r32) {
+    const int32_t t = xcd_block() * blockDim.x + threadIdx.x, i = t >> 2, v = t & 3;
     if (i >= nc)
         return;
-    double nw[36];
+    const uint32_t lane = threadIdx.x & 63;
+    const double *xo = x + rec_group(i);
+    int32_t jn[NF], least = 0;
 #pragma unroll
-    for (int k = 0; k < 36; k++)
-        nw[k] = (1 - relax) * x[k * ldc + i];
-    double ui[4];
-#pragma unroll
-    for (int v = 0; v < 4; v++)
-        ui[v] = u[4 * int64_t(i) + v];
-#pragma unroll 1
     for (int s = 0; s < NF; s++) {
-        int32_t j = nbr[s * ldc + i];
-        if (j == -2)
+        jn[s] = nbr[s * ldc + i];
+        least = min(least, jn[s] == -2 ? 0 : jn[s]);
+    }
+    const double ui = u[4 * int64_t(i) + v];
+    // wall corrections first (stored, and read back in their slot), before
+    // the loads in flight take the registers
+    if (least < 0) {
+#pragma unroll 1
+        for (int s = 0; s < NF; s++) {
+            const int32_t w = wall_idx[s * ldc + i];
+            if (w < 0)
+                continue;
+            double own[9], cw[9];
+#pragma unroll
+            for (int r = 0; r < 9; r++)
+                own[r] = xo[256 * r + lane];
+            wall_correction(w, sbc[s * ldc + i], own, ui, v, wf, relax, errw, cw);
+#pragma unroll
+            for (int r = 0; r < 9; r++)
+                corr[kRec * int64_t(w) + 9 * v + r] = cw[r];
+        }
+    }
+    double nw[9];
+#pragma unroll
+    for (int r = 0; r < 9; r++)
+        nw[r] = (1 - relax) * xo[256 * r + lane];
+#pragma unroll
+    for (int s = 0; s < NF; s++) {
+        if (s == 3 && jn[s] == -2)
             continue;
-        const double *bs = bv + int64_t(s) * 9 * ldc + i;
-        double bmul = 1.0;
-        if (j < 0) {
-            const int32_t bc = sbc[s * ldc + i];
-            if (bc == BC_WALL) {
+        AbPart ab;
+        ab.load(M, s, i, ldc, v);
+        const int32_t j = jn[s] < 0 ? i : jn[s];
+        const double uj = u[4 * int64_t(j) + v];
+        double xj[9];
 #pragma unroll
-                for (int r = 0; r < 9; r++) {
-                    const double b = bs[r * ldc];
+        for (int c = 0; c < 9; c++)
+            xj[c] = x[rec(j, c, v)];
+        const int32_t bc = jn[s] < 0 ? sbc[s * ldc + i] : BC_INNER;
+        if (jn[s] >= 0 || is_far(bc)) {
+            // far field: M_if x_i (gathered from i), no mean-value term
+            const double bmul = jn[s] < 0 ? 0.0 : 1.0;
+            ab_apply(ab, xj, bmul * (uj - ui), bmul, relax, nw);
+        } else if (bc == BC_WALL) {
 #pragma unroll
-                    for (int v = 0; v < 4; v++)
-                        nw[r + 9 * v] += relax * ((0.0 - ui[v]) * b);
-                }
-                continue;
-            }
-            if (bc == BC_WALL_EULER || bc == BC_WALL_NOSLIP) {
-                const int64_t w = wall_idx[s * ldc + i];
+            for (int r = 0; r < 9; r++)
+                nw[r] += relax * ((0.0 - ui) * ab.get(10 * r + 9));
+        } else if (bc == BC_WALL_EULER || bc == BC_WALL_NOSLIP) {
+            const int64_t w = wall_idx[s * ldc + i];
 #pragma unroll
-                for (int k = 0; k < 36; k++)
-                    nw[k] += corr[k * ldw + w];
-                continue;
-            }
-            if (!is_far(bc)) {
-                atomicOr(errw, ERRBIT_BC);
-                continue;
-            }
-            j = i; // far field: M_if x_i, no mean-value term
-            bmul = 0.0;
-        }
-        // A^-1 B entries e = 9 r + c, two per 16-byte load (entry 81 pads)
-        const dbl2 *Ms = reinterpret_cast<const dbl2 *>(M) + m_vec_index(s, 0, i, ldc, kMPairs);
-        double du[4];
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-            du[v] = bmul * (u[4 * int64_t(j) + v] - ui[v]);
-        double xj[36];
-#pragma unroll
-        for (int k = 0; k < 36; k++)
-            xj[k] = x[k * ldc + j];
-        dbl2 mp = {0.0, 0.0};
-        double tt[4] = {0, 0, 0, 0};
-#pragma unroll
-        for (int e = 0; e < 81; e++) {
-            const int r = e / 9, c = e % 9;
-            if (e % 2 == 0)
-                mp = __builtin_nontemporal_load(Ms + (e / 2) * 64);
-            const double m = e % 2 == 0 ? mp.x : mp.y;
-            if (c == 0)
-                tt[0] = tt[1] = tt[2] = tt[3] = 0.0;
-#pragma unroll
-            for (int v = 0; v < 4; v++)
-                tt[v] += m * xj[c + 9 * v];
-            if (c == 8) {
-                const double b = bmul * __builtin_nontemporal_load(bs + r * ldc);
-#pragma unroll
-                for (int v = 0; v < 4; v++)
-                    nw[r + 9 * v] += relax * (tt[v] + du[v] * b);
-            }
+            for (int r = 0; r < 9; r++)
+                nw[r] += corr[kRec * w + 9 * v + r];
+        } else {
+            atomicOr(errw, ERRBIT_BC);
         }
     }
-    // the new iterate streams out with non-temporal stores: written once
-    // and read by the next launch, it would only displace the neighbours'
-    // reconstructions that this sweep still gathers (4 % faster on the 2.1M
-    // triangles, 2 % on the 6.3M mixed cells)
-    if (RESID) {
+    // the new iterate streams out with non-temporal stores: written once and
+    // read by the next launch, it would only displace the neighbours'
+    // reconstructions that this sweep still gathers
 #pragma unroll
-        for (int k = 0; k < 36; k++) {
-            const float r = float(nw[k] - x[k * ldc + i]);
-            __builtin_nontemporal_store(r, &r32[k * ldc + i]);
-            __builtin_nontemporal_store(r, &d32[k * ldc + i]);
-        }
-        return;
+    for (int r = 0; r < 9; r++) {
+        if (RESID) {
+            const float d = float(nw[r] - xo[256 * r + lane]);
+            __builtin_nontemporal_store(d, r32 + rec_group(i) + (256 * r + lane));
+        } else
+            __builtin_nontemporal_store(nw[r], xn + rec_group(i) + (256 * r + lane));
     }
-#pragma unroll
-    for (int k = 0; k < 36; k++)
-        __builtin_nontemporal_store(nw[k], &xn[k * ldc + i]);
 }
 
 // Read-bandwidth probe of the sweep's dominant stream: every cell streams its
-// slots' A^-1 B pairs exactly as k_jacobi does (16-byte non-temporal loads,
+// slots' A^-1 B, A^-1 b exactly as k_jacobi does (16-byte non-temporal loads,
 // the same slots skipped) with none of the sweep's gathers, and writes one
-// double.  Its rate is the ceiling of the sweep's streaming part.
+// double per lane.  Its rate is the ceiling of the sweep's streaming part.
 template <int NF>
 __global__ __launch_bounds__(kBlock) void k_read_probe(int32_t nc, int64_t ldc, const int32_t *__restrict__ nbr,
                                                        const double *__restrict__ M, double *__restrict__ out) {
-    const int32_t i = xcd_block() * blockDim.x + threadIdx.x;
+    const int32_t t = xcd_block() * blockDim.x + threadIdx.x, i = t >> 2, v = t & 3;
     if (i >= nc)
         return;
-    double a0 = 0.0, a1 = 0.0;
-#pragma unroll 1
+    double a = 0.0;
+#pragma unroll
     for (int s = 0; s < NF; s++) {
         if (nbr[s * ldc + i] == -2)
             continue;
-        const dbl2 *Ms = reinterpret_cast<const dbl2 *>(M) + m_vec_index(s, 0, i, ldc, kMPairs);
+        AbPart ab;
+        ab.load(M, s, i, ldc, v);
 #pragma unroll
-        for (int e = 0; e < kMPairs; e++) {
-            const dbl2 m = __builtin_nontemporal_load(Ms + e * 64);
-            a0 += m.x, a1 += m.y;
-        }
+        for (int k = 0; k < kAbVecs / 4; k++)
+            a += ab.w[k].x + ab.w[k].y;
+        a += v == 0 ? ab.last.x + ab.last.y : 0.0;
     }
-    out[i] = a0 + a1;
+    out[4 * int64_t(i) + v] = a;
 }
 
-// Linear part of the Wall_Euler / Wall_NoSlip correction (k_wall_corr) for a
-// correction d of the reconstruction: the wall state is the reconstructed
-// value D d with the normal momentum removed (Wall_Euler) or the momentum
-// reversed (Wall_NoSlip), both linear, and the cell mean drops out.
-__global__ __launch_bounds__(kBlock) void k_wall_corr_lin(int32_t nw, int64_t ldc, const int32_t *__restrict__ wcell,
-                                                          const int32_t *__restrict__ wbc,
-                                                          const double *__restrict__ wall_ainv,
-                                                          const double *__restrict__ wall_d0,
-                                                          const double *__restrict__ wall_nrm,
-                                                          const double *__restrict__ wall_w0, int64_t ldw,
-                                                          const float *__restrict__ d, float relax,
-                                                          float *__restrict__ corr) {
-    const int32_t w = blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= nw)
-        return;
-    const int32_t i = wcell[w];
-    const int32_t bc = wbc[w];
-    float di[36], BCc[36];
-    for (int k = 0; k < 36; k++)
-        di[k] = d[k * ldc + i], BCc[k] = 0.f;
-    const float w0 = float(wall_w0[w]);
+// Linear part of the Wall_Euler / Wall_NoSlip correction (wall_correction)
+// for a correction d of the reconstruction: the wall state is the
+// reconstructed value D d with the normal momentum removed (Wall_Euler) or
+// the momentum reversed (Wall_NoSlip), both linear, and the cell mean drops
+// out.  di: this lane's variable; the cell's quad calls it together.
+__device__ __forceinline__ void wall_correction_lin(int32_t w, int32_t bc, const float di[9], int v,
+                                                    const WallFaces &wf, float relax, float out[9]) {
+    float BCc[9];
+#pragma unroll
+    for (int r = 0; r < 9; r++)
+        BCc[r] = 0.f;
+    const float w0 = float(wf.w0[w]);
+#pragma unroll 1
     for (int g = 0; g < 3; g++) {
         const float gw = float(g == 1 ? kLine3W1 : kLine3W0);
-        const double nx = wall_nrm[(2 * g) * ldw + w], ny = wall_nrm[(2 * g + 1) * ldw + w];
-        float uBL[4];
-        for (int v = 0; v < 4; v++) {
-            float acc = 0.f;
-            for (int c = 0; c < 9; c++)
-                acc = fmaf(float(wall_d0[(g * 9 + c) * ldw + w]), di[c + 9 * v], acc);
-            uBL[v] = acc;
-        }
+        const double nx = wf.nrm[(2 * g) * wf.ld + w], ny = wf.nrm[(2 * g + 1) * wf.ld + w];
+        float d0[9], uB = 0.f;
+#pragma unroll
+        for (int c = 0; c < 9; c++)
+            d0[c] = float(wf.d0[(g * 9 + c) * wf.ld + w]);
+#pragma unroll
+        for (int c = 0; c < 9; c++)
+            uB = fmaf(d0[c], di[c], uB);
         double n0, n1;
         stable_normalized(nx, ny, n0, n1);
-        float uBV[4] = {uBL[0], uBL[1], uBL[2], uBL[3]};
+        const float m0 = quad_bcast<1>(uB), m1 = quad_bcast<2>(uB);
+        float uBV = uB;
         if (bc == BC_WALL_EULER) {
-            const float dd = float(n0) * uBL[1] + float(n1) * uBL[2];
-            uBV[1] = uBL[1] - float(n0) * dd;
-            uBV[2] = uBL[2] - float(n1) * dd;
-        } else {
-            uBV[1] = -uBL[1];
-            uBV[2] = -uBL[2];
+            const float dd = float(n0) * m0 + float(n1) * m1;
+            if (v == 1)
+                uBV = uB - float(n0) * dd;
+            else if (v == 2)
+                uBV = uB - float(n1) * dd;
+        } else if (v == 1 || v == 2) {
+            uBV = -uB;
         }
         const float nl = float(sqrt(nx * nx + ny * ny));
+#pragma unroll
         for (int r = 0; r < 9; r++)
-            for (int v = 0; v < 4; v++)
-                BCc[r + 9 * v] += float(wall_d0[(g * 9 + r) * ldw + w]) * w0 * w0 * uBV[v] * nl * gw;
+            BCc[r] += d0[r] * w0 * w0 * uBV * nl * gw;
     }
-    for (int r = 0; r < 9; r++)
-        for (int v = 0; v < 4; v++) {
-            float acc = 0.f;
-            for (int c = 0; c < 9; c++)
-                acc = fmaf(float(wall_ainv[(r * 9 + c) * ldw + w]), BCc[c + 9 * v], acc);
-            corr[(r + 9 * v) * ldw + w] = relax * acc;
-        }
+#pragma unroll
+    for (int r = 0; r < 9; r++) {
+        float acc = 0.f;
+#pragma unroll
+        for (int c = 0; c < 9; c++)
+            acc = fmaf(float(wf.ainv[(r * 9 + c) * wf.ld + w]), BCc[c], acc);
+        out[r] = relax * acc;
+    }
 }
 
 // FP32 correction sweep of the mixed-precision reconstruction.  The Jacobi
@@ -462,97 +452,107 @@ __global__ __launch_bounds__(kBlock) void k_wall_corr_lin(int32_t nw, int64_t ld
 // after one FP64 step reproduce n FP64 sweeps, with FP32 rounding confined
 // to the correction d (iterative refinement).  M is read as FP32.  LAST adds
 // the correction to the FP64 iterate in place.  Wall_Euler / Wall_NoSlip
-// faces contribute the linear part of their boundary correction, computed
-// from d by k_wall_corr_lin (the wall state is linear in the reconstructed
-// value there).
+// faces contribute the linear part of their boundary correction (the wall
+// state is linear in the reconstructed value there).  Four lanes per cell, as
+// in k_jacobi.
 template <int NF, bool LAST>
-__global__ __launch_bounds__(kBlock) void k_delta32(int32_t nc, int64_t ldc, const int32_t *__restrict__ nbr,
-                                                    const int32_t *__restrict__ sbc, const float *__restrict__ M32,
-                                                    const float *__restrict__ r32, const float *__restrict__ din,
-                                                    float *__restrict__ dout, float relax,
-                                                    double *__restrict__ x, const int32_t *__restrict__ wall_idx,
-                                                    const float *__restrict__ wcorr, int64_t ldw) {
-    const int32_t i = xcd_block() * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(kBlock, 2) void k_delta32(int32_t nc, int64_t ldc, const int32_t *__restrict__ nbr,
+                                                       const int32_t *__restrict__ sbc,
+                                                       const int32_t *__restrict__ wall_idx,
+                                                       const float *__restrict__ M32, const float *__restrict__ r32,
+                                                       const float *__restrict__ din, float *__restrict__ dout,
+                                                       float relax, double *__restrict__ x, WallFaces wf) {
+    const int32_t t = xcd_block() * blockDim.x + threadIdx.x, i = t >> 2, v = t & 3;
     if (i >= nc)
         return;
-    float nw[36];
+    int32_t jn[NF];
 #pragma unroll
-    for (int k = 0; k < 36; k++)
-        nw[k] = (1.0f - relax) * din[k * ldc + i];
-#pragma unroll 1
+    for (int s = 0; s < NF; s++)
+        jn[s] = nbr[s * ldc + i];
+    const uint32_t lane = threadIdx.x & 63;
+    constexpr int kW = kAb32Vecs / 4;
+    flt4 w[NF][kW], last[NF];
+    float dj[NF][9], own[9], res[9], nw[9];
+#pragma unroll
     for (int s = 0; s < NF; s++) {
-        int32_t j = nbr[s * ldc + i];
+        if (s == 3 && jn[s] == -2)
+            continue;
+        const int32_t g = __builtin_amdgcn_readfirstlane(i);
+        const flt4 *p = reinterpret_cast<const flt4 *>(M32) + ab_group(s, g, ldc, kAb32Vecs);
+        const uint32_t cl = i & 15;
+#pragma unroll
+        for (int k = 0; k < kW; k++)
+            w[s][k] = __builtin_nontemporal_load(p + 64 * k + (4 * cl + v));
+        last[s] = __builtin_nontemporal_load(p + 16 * (kAb32Vecs - 1) + cl);
+    }
+#pragma unroll
+    for (int r = 0; r < 9; r++) {
+        own[r] = (din + rec_group(i))[256 * r + lane];
+        res[r] = (r32 + rec_group(i))[256 * r + lane];
+    }
+#pragma unroll
+    for (int s = 0; s < NF; s++) {
+        const int32_t j = jn[s] < 0 ? i : jn[s];
+        if (s == 3 && jn[s] == -2)
+            continue;
+#pragma unroll
+        for (int c = 0; c < 9; c++)
+            dj[s][c] = din[rec(j, c, v)];
+    }
+#pragma unroll
+    for (int r = 0; r < 9; r++)
+        nw[r] = (1.0f - relax) * own[r];
+#pragma unroll
+    for (int s = 0; s < NF; s++) {
+        const int32_t j = jn[s];
         if (j == -2)
             continue;
-        if (j < 0) {
-            const int32_t bc = sbc[s * ldc + i];
-            if (bc == BC_WALL) // constant term: in r only
-                continue;
-            if (bc == BC_WALL_EULER || bc == BC_WALL_NOSLIP) {
-                const int64_t w = wall_idx[s * ldc + i];
+        const int32_t bc = j < 0 ? sbc[s * ldc + i] : 0;
+        if (j >= 0 || !(bc == BC_WALL || bc == BC_WALL_EULER || bc == BC_WALL_NOSLIP)) { // far field: d_i
 #pragma unroll
-                for (int k = 0; k < 36; k++)
-                    nw[k] += wcorr[k * ldw + w];
-                continue;
+            for (int r = 0; r < 9; r++) {
+                float tt = 0.f;
+#pragma unroll
+                for (int c = 0; c < 9; c++) {
+                    const int e = 9 * r + c, p = e / 4;
+                    const float m = p == kAb32Vecs - 1 ? last[s][e % 4]
+                                                       : quad_get(float(w[s][p < 20 ? p / 4 : 0][e % 4]), p % 4);
+                    tt = fmaf(m, dj[s][c], tt);
+                }
+                nw[r] = fmaf(relax, tt, nw[r]);
             }
-            j = i; // far field
-        }
-        // FP32 A^-1 B entries, four per 16-byte load (81..83 pad)
-        const flt4 *Ms = reinterpret_cast<const flt4 *>(M32) + m_vec_index(s, 0, i, ldc, kMQuads);
-        float dj[36];
+        } else if (bc != BC_WALL) { // (a Wall face's constant term is in r only)
+            float cw[9];
+            wall_correction_lin(wall_idx[s * ldc + i], bc, own, v, wf, relax, cw);
 #pragma unroll
-        for (int k = 0; k < 36; k++)
-            dj[k] = din[k * ldc + j];
-        flt4 mq = {0.f, 0.f, 0.f, 0.f};
-        float tt[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int e = 0; e < 81; e++) {
-            const int r = e / 9, c = e % 9;
-            if (e % 4 == 0)
-                mq = __builtin_nontemporal_load(Ms + (e / 4) * 64);
-            const float m = mq[e % 4];
-            if (c == 0)
-                tt[0] = tt[1] = tt[2] = tt[3] = 0.f;
-#pragma unroll
-            for (int v = 0; v < 4; v++)
-                tt[v] = fmaf(m, dj[c + 9 * v], tt[v]);
-            if (c == 8)
-#pragma unroll
-                for (int v = 0; v < 4; v++)
-                    nw[r + 9 * v] = fmaf(relax, tt[v], nw[r + 9 * v]);
+            for (int r = 0; r < 9; r++)
+                nw[r] += cw[r];
         }
     }
 #pragma unroll
-    for (int k = 0; k < 36; k++) {
-        const float d = nw[k] + r32[k * ldc + i];
+    for (int r = 0; r < 9; r++) {
+        const float d = nw[r] + res[r];
         if (LAST)
-            x[k * ldc + i] += double(d);
+            (x + rec_group(i))[256 * r + lane] += double(d);
         else
-            __builtin_nontemporal_store(d, &dout[k * ldc + i]); // streamed, as in k_jacobi
+            __builtin_nontemporal_store(d, dout + rec_group(i) + (256 * r + lane)); // streamed, as in k_jacobi
     }
 }
 
-// A^-1 B from FP64 pairs to FP32 quads (both in the m_vec_index layout)
+// A^-1 B in FP32, one thread per 16-byte vector of the FP32 stream
 __global__ __launch_bounds__(kBlock) void k_m_to_f32(int32_t nfmax, int64_t ldc, const double *__restrict__ M,
                                                      float *__restrict__ M32) {
     const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= int64_t(nfmax) * kMQuads * ldc)
+    if (t >= int64_t(nfmax) * kAb32Vecs * ldc)
         return;
     const int64_t i = t % ldc, sq = t / ldc;
-    const int s = int(sq / kMQuads), q = int(sq % kMQuads);
-    const int64_t o = m_vec_index(s, q, i, ldc, kMQuads) * 4;
+    const int s = int(sq / kAb32Vecs), q = int(sq % kAb32Vecs);
+    const int64_t o = ab_vec(s, q, i, ldc, kAb32Vecs) * 4;
 #pragma unroll
     for (int w = 0; w < 4; w++) {
-        const int k = 4 * q + w;
-        M32[o + w] = k < 81 ? float(M[m_vec_index(s, k / 2, i, ldc, kMPairs) * 2 + k % 2]) : 0.f;
+        const int k = 4 * q + w, d = 10 * (k / 9) + k % 9;
+        M32[o + w] = k < 81 ? float(M[ab_vec(s, d / 2, i, ldc, kAbVecs) * 2 + d % 2]) : 0.f;
     }
-}
-
-__global__ __launch_bounds__(kBlock) void k_to_f32(int64_t n, const double *__restrict__ src,
-                                                   float *__restrict__ dst) {
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < n)
-        dst[i] = float(src[i]);
 }
 
 // EvaluateDt face loop (DNDS_FV_EulerEvaluator.cpp:25-137): lambdaFace and
@@ -686,7 +686,7 @@ __global__ __launch_bounds__(kBlock) void k_fill_from(int32_t n, const double *_
 // push to 3e200 (:356-395, USE_DISABLE_DIST_GRP_FIX_AT_WALL), and fluxFace's
 // viscous flux (DNDS_FV_EulerEvaluator.hpp:397-430, 574-577).
 template <bool BOUNDARY, bool MIXED = false, bool STRAIGHT = false, bool VIS = false>
-__global__ __launch_bounds__(kBlock, VIS && !BOUNDARY ? 2 : 1) void k_rhs_face(int32_t n, int64_t ldf, int64_t ldc,
+__global__ __launch_bounds__(kBlock, VIS && !BOUNDARY ? 2 : 1) void k_rhs_face(int32_t n, int64_t ldf, int nfmax,
                                                      const int32_t *__restrict__ list,
                                                      const int32_t *__restrict__ f2c,
                                                      const int32_t *__restrict__ fbc, const double *__restrict__ fxy,
@@ -725,7 +725,7 @@ __global__ __launch_bounds__(kBlock, VIS && !BOUNDARY ? 2 : 1) void k_rhs_face(i
 #pragma unroll
         for (int v = 0; v < 4; v++)
             incL[g][v] = 0.0, incR[g][v] = 0.0;
-    const dbl2 *xy = reinterpret_cast<const dbl2 *>(fxy) + f;
+    const dbl2 *xy = reinterpret_cast<const dbl2 *>(fxy) + blk64(f, 6);
 #pragma unroll 1
     for (int sd = 0; sd < (BOUNDARY ? 1 : 2); sd++) {
         const int32_t cell = sd ? R : L;
@@ -734,7 +734,7 @@ __global__ __launch_bounds__(kBlock, VIS && !BOUNDARY ? 2 : 1) void k_rhs_face(i
         double pX[3][4], pY[3][4];
 #pragma unroll
         for (int g = 0; g < 3; g++) {
-            const dbl2 q = __builtin_nontemporal_load(xy + (sd * 3 + g) * ldf);
+            const dbl2 q = __builtin_nontemporal_load(xy + 64 * (sd * 3 + g));
             int_powers(q.x, pX[g]);
             int_powers(q.y, pY[g]);
         }
@@ -747,11 +747,10 @@ __global__ __launch_bounds__(kBlock, VIS && !BOUNDARY ? 2 : 1) void k_rhs_face(i
                 inc[g][v] = 0.0, acc[g][v] = 0.f;
 #pragma unroll
         for (int c = 0; c < 9; c++) {
-            const double m = cmom[c * ldc + cell];
-            double xc[4];
-#pragma unroll
-            for (int v = 0; v < 4; v++)
-                xc[v] = xs[(c + 9 * v) * ldc + cell];
+            const double m = cmom[blk64(cell, 9) + 64 * c];
+            const dbl2 *xq = reinterpret_cast<const dbl2 *>(xs + rec(cell, c, 0));
+            const dbl2 xa = xq[0], xb = xq[1];
+            const double xc[4] = {xa.x, xa.y, xb.x, xb.y};
 #pragma unroll
             for (int g = 0; g < 3; g++) {
                 const double d = pX[g][kBX[c + 1]] * pY[g][kBY[c + 1]] - m;
@@ -797,7 +796,7 @@ __global__ __launch_bounds__(kBlock, VIS && !BOUNDARY ? 2 : 1) void k_rhs_face(i
     for (int g = 0; g < 3; g++) {
         double ULxy[4], URxy[4], URm[4];
         if (!STRAIGHT || g == 0) {
-            const double nx = fn[(2 * g) * ldf + f], ny = fn[(2 * g + 1) * ldf + f];
+            const double nx = fn[blk64(f, 6) + 64 * (2 * g)], ny = fn[blk64(f, 6) + 64 * (2 * g + 1)];
             normalized(nx, ny, n0, n1);
             nl = sqrt(nx * nx + ny * ny);
         }
@@ -820,7 +819,7 @@ __global__ __launch_bounds__(kBlock, VIS && !BOUNDARY ? 2 : 1) void k_rhs_face(i
             // the gradients of both sides at this point, formed here rather
             // than kept for all three points
             auto grad_at = [&](int32_t cell, int sd, double G[2][4]) {
-                const dbl2 q = xy[(sd * 3 + g) * ldf];
+                const dbl2 q = xy[64 * (sd * 3 + g)];
                 double px[4], py[4];
                 int_powers(q.x, px);
                 int_powers(q.y, py);
@@ -836,10 +835,9 @@ __global__ __launch_bounds__(kBlock, VIS && !BOUNDARY ? 2 : 1) void k_rhs_face(i
 #pragma unroll
                 for (int c = 0; c < 9; c++) {
                     const int bx = kBX[c + 1], by = kBY[c + 1];
-                    double xc[4];
-#pragma unroll
-                    for (int v = 0; v < 4; v++)
-                        xc[v] = xs[(c + 9 * v) * ldc + cell];
+                    const dbl2 *xq = reinterpret_cast<const dbl2 *>(xs + rec(cell, c, 0));
+                    const dbl2 xa = xq[0], xb = xq[1];
+                    const double xc[4] = {xa.x, xa.y, xb.x, xb.y};
                     if (bx > 0) {
                         const double dx = double(bx) * px[bx - 1] * py[by] * isx;
 #pragma unroll
@@ -902,25 +900,30 @@ __global__ __launch_bounds__(kBlock, VIS && !BOUNDARY ? 2 : 1) void k_rhs_face(i
     // the cell applies them (negation is exact, so the cell's sums are
     // unchanged bit for bit)
     const int32_t pos = fpos[f];
-    const int64_t oL = int64_t(pos & 15) * 8 * ldc + L, oR = int64_t(pos >> 4) * 8 * ldc + R;
+    const int64_t oL = quad64(L, 2 * nfmax, 2 * (pos & 15)), oR = quad64(R, 2 * nfmax, 2 * (pos >> 4));
     if (MIXED) {
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-            fslot32[oL + v * ldc] = float(acc[v]), fslot32[oL + (4 + v) * ldc] = -float(acc[4 + v]);
-        if (!BOUNDARY)
-#pragma unroll
-            for (int v = 0; v < 4; v++)
-                fslot32[oR + v * ldc] = -float(acc[v]), fslot32[oR + (4 + v) * ldc] = float(acc[8 + v]);
+        auto put = [&](int64_t o, float a, float b, float c, float d) {
+            *reinterpret_cast<flt4 *>(fslot32 + o) = flt4{a, b, c, d};
+        };
+        put(oL, float(acc[0]), float(acc[1]), float(acc[2]), float(acc[3]));
+        put(oL + 256, -float(acc[4]), -float(acc[5]), -float(acc[6]), -float(acc[7]));
+        if (!BOUNDARY) {
+            put(oR, -float(acc[0]), -float(acc[1]), -float(acc[2]), -float(acc[3]));
+            put(oR + 256, float(acc[8]), float(acc[9]), float(acc[10]), float(acc[11]));
+        }
         return;
     }
     // plain stores (with non-temporal ones this kernel ran 19 % slower)
-#pragma unroll
-    for (int v = 0; v < 4; v++)
-        fslot[oL + v * ldc] = acc[v], fslot[oL + (4 + v) * ldc] = -acc[4 + v];
-    if (!BOUNDARY)
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-            fslot[oR + v * ldc] = -acc[v], fslot[oR + (4 + v) * ldc] = acc[8 + v];
+    auto put = [&](int64_t o, double a, double b, double c, double d) {
+        dbl2 *p = reinterpret_cast<dbl2 *>(fslot + o);
+        p[0] = dbl2{a, b}, p[1] = dbl2{c, d};
+    };
+    put(oL, acc[0], acc[1], acc[2], acc[3]);
+    put(oL + 256, -acc[4], -acc[5], -acc[6], -acc[7]);
+    if (!BOUNDARY) {
+        put(oR, -acc[0], -acc[1], -acc[2], -acc[3]);
+        put(oR + 256, acc[8], acc[9], acc[10], acc[11]);
+    }
 }
 
 // EvaluateRHS scatter as a per-cell gather in ascending face order
@@ -953,10 +956,10 @@ __global__ __launch_bounds__(kBlock) void k_rhs_cell(int32_t nc, int64_t ldc, co
             break;
 #pragma unroll
         for (int v = 0; v < 4; v++)
-            r[v] += fslot[(s * 8 + v) * ldc + i] / V;
+            r[v] += fslot[quad64(i, 2 * NF, 2 * s) + v] / V;
 #pragma unroll
         for (int v = 0; v < 4; v++)
-            r[v] += fslot[(s * 8 + 4 + v) * ldc + i] / V;
+            r[v] += fslot[quad64(i, 2 * NF, 2 * s + 1) + v] / V;
     }
     bool finite = true;
 #pragma unroll
@@ -992,7 +995,12 @@ __global__ __launch_bounds__(kBlock) void k_rhs_cell(int32_t nc, int64_t ldc, co
 // LINE_3 point with the LINE_1 weight 2, for both adjacent cells.  As in the
 // reference, a cell evaluates the face's side-0 basis with its own
 // coefficients and the side-1 basis with its neighbour's.
-__global__ __launch_bounds__(kBlock) void k_wbap_face(int32_t nf, int64_t ldf, int64_t ldc,
+//
+// Two lanes per face, one per side: each evaluates its side's basis (the
+// divisions, which bound this kernel), applies it to both cells'
+// coefficients, and finishes its own cell's terms; the coefficients and the
+// products that the other side needs change lanes with DPP moves.
+__global__ __launch_bounds__(kBlock) void k_wbap_face(int32_t nf, int64_t ldf, int nfmax,
                                                       const int32_t *__restrict__ f2c,
                                                       const double *__restrict__ fxy, const double *__restrict__ cmom,
                                                       const double *__restrict__ cscale,
@@ -1000,56 +1008,51 @@ __global__ __launch_bounds__(kBlock) void k_wbap_face(int32_t nf, int64_t ldf, i
                                                       const double *__restrict__ fn, const double *__restrict__ u,
                                                       const double *__restrict__ x, double tang_weight, int twd_norm,
                                                       const uint8_t *__restrict__ wpos, double *__restrict__ wslot) {
-    const int32_t f = xcd_block() * blockDim.x + threadIdx.x;
+    const int32_t t = xcd_block() * blockDim.x + threadIdx.x, f = t >> 1;
+    const bool sd = t & 1;
     if (f >= nf)
         return;
     const int32_t L = f2c[f], R = f2c[ldf + f];
     if (R < 0)
         return;
-    // The DiBj blocks of both sides at point 0 (side 0: cell L's basis,
-    // side 1: cell R's), evaluated from the point's scaled coordinates and
-    // the cells' scales and moments; zero entries are skipped (adding them
-    // would not change any sum).  Cell side cs sees its own coefficients on
-    // the side-0 basis and the neighbour's on the side-1 basis.  The rows are
-    // taken in the functional's groups {0}, {1, 2}, {3, 4, 5}, {6..9}: one
-    // pass over the coefficients per group, whose terms then join the
-    // indicator sums in their order.
-    const dbl2 *xy = reinterpret_cast<const dbl2 *>(fxy) + f;
-    const dbl2 q0 = __builtin_nontemporal_load(xy), q1 = __builtin_nontemporal_load(xy + 3 * ldf);
-    const dbl2 *sc = reinterpret_cast<const dbl2 *>(cscale);
-    const dbl2 s0 = sc[L], s1 = sc[R];
-    double pX0[4], pY0[4], pX1[4], pY1[4], sX0[4], sY0[4], sX1[4], sY1[4];
-    int_powers(q0.x, pX0), int_powers(q0.y, pY0), int_powers(q1.x, pX1), int_powers(q1.y, pY1);
-    int_powers(s0.x, sX0), int_powers(s0.y, sY0), int_powers(s1.x, sX1), int_powers(s1.y, sY1);
+    const int32_t cell = sd ? R : L;
+    // the cell's rho and E, coefficients and mean, and the other side's
+    double xs[9][2], xt[9][2];
+#pragma unroll
+    for (int c = 0; c < 9; c++)
+        xs[c][0] = x[rec(cell, c, 0)], xs[c][1] = x[rec(cell, c, 3)];
+    const double us[2] = {u[4 * int64_t(cell)], u[4 * int64_t(cell) + 3]};
+    // the DiBj block of this side at point 0, evaluated from the point's
+    // scaled coordinates and the cell's scales and moments; zero entries are
+    // skipped (adding them would not change any sum).  The rows are taken in
+    // the functional's groups {0}, {1, 2}, {3, 4, 5}, {6..9}, whose terms then
+    // join the indicator sums in their order.
+    const dbl2 p0 = __builtin_nontemporal_load(reinterpret_cast<const dbl2 *>(fxy) + blk64(f, 6) + (sd ? 64 * 3 : 0));
+    const dbl2 sc = reinterpret_cast<const dbl2 *>(cscale)[cell];
+    double pX[4], pY[4], sX[4], sY[4];
+    int_powers(p0.x, pX), int_powers(p0.y, pY), int_powers(sc.x, sX), int_powers(sc.y, sY);
     double W[10];
 #pragma unroll
     for (int k = 0; k < 10; k++)
-        W[k] = fw[k * ldf + f];
-    const double gx = fn[f], gy = fn[ldf + f];
+        W[k] = fw[blk64(f, 10) + 64 * k];
+    const double gx = fn[blk64(f, 6)], gy = fn[blk64(f, 6) + 64];
     const FFParams P = ff_params(W, gx, gy, tang_weight, twd_norm);
     const double nl = sqrt(gx * gx + gy * gy);
-    const double uL[2] = {u[4 * int64_t(L)], u[4 * int64_t(L) + 3]};
-    const double uR[2] = {u[4 * int64_t(R)], u[4 * int64_t(R) + 3]};
-    double sums[2][2][2]; // [cell side][rho, E][IJI, ISI]
 #pragma unroll
-    for (int k = 0; k < 8; k++)
-        (&sums[0][0][0])[k] = 0.0;
+    for (int c = 0; c < 9; c++)
+        xt[c][0] = pair_swap(xs[c][0]), xt[c][1] = pair_swap(xs[c][1]);
+    const double ut[2] = {pair_swap(us[0]), pair_swap(us[1])};
+    double sums[2][2] = {{0.0, 0.0}, {0.0, 0.0}}; // [rho, E][IJI, ISI]
     auto pass = [&](auto group) {
         constexpr int G = decltype(group)::value;
         constexpr int r0 = G == 0 ? 0 : G == 1 ? 1 : G == 2 ? 3 : 6, nr = G == 0 ? 1 : G == 1 ? 2 : G == 2 ? 3 : 4;
-        // each pass reloads the coefficients (cache hits) rather than keeping
-        // all of them in registers across the passes
-        __asm__ volatile("" ::: "memory");
-        // b[0]: side-0 basis x L, b[1]: side-0 x R, b[2]: side-1 x R, b[3]: side-1 x L
-        double b[4][nr][2];
+        double bs[nr][2], bt[nr][2]; // this side's basis times its own and the other cell's coefficients
 #pragma unroll
-        for (int k = 0; k < 4 * nr * 2; k++)
-            (&b[0][0][0])[k] = 0.0;
+        for (int k = 0; k < nr * 2; k++)
+            (&bs[0][0])[k] = 0.0, (&bt[0][0])[k] = 0.0;
 #pragma unroll
         for (int c = 0; c < 9; c++) {
-            const double xL[2] = {x[c * ldc + L], x[(c + 27) * ldc + L]};
-            const double xR[2] = {x[c * ldc + R], x[(c + 27) * ldc + R]};
-            const double m0 = G == 0 ? cmom[c * ldc + L] : 0.0, m1 = G == 0 ? cmom[c * ldc + R] : 0.0;
+            const double m = G == 0 ? cmom[blk64(cell, 9) + 64 * c] : 0.0;
 #pragma unroll
             for (int rr = 0; rr < nr; rr++) {
                 const int r = r0 + rr;
@@ -1057,64 +1060,55 @@ __global__ __launch_bounds__(kBlock) void k_wbap_face(int32_t nf, int64_t ldf, i
                 if (coef == 0)
                     continue;
                 const int ex = kBX[c + 1] - kBX[r], ey = kBY[c + 1] - kBY[r];
-                double d0 = double(coef) * pX0[ex] * pY0[ey] * 1.0;
-                double d1 = double(coef) * pX1[ex] * pY1[ey] * 1.0;
-                if (r == 0) {
-                    d0 -= m0, d1 -= m1;
-                } else {
-                    d0 = d0 / (sX0[kBX[r]] * sY0[kBY[r]] * 1.0);
-                    d1 = d1 / (sX1[kBX[r]] * sY1[kBY[r]] * 1.0);
-                }
+                double d = double(coef) * pX[ex] * pY[ey] * 1.0;
+                if (r == 0)
+                    d -= m;
+                else
+                    d = d / (sX[kBX[r]] * sY[kBY[r]] * 1.0);
 #pragma unroll
                 for (int q = 0; q < 2; q++) {
-                    b[0][rr][q] += d0 * xL[q];
-                    b[1][rr][q] += d0 * xR[q];
-                    b[2][rr][q] += d1 * xR[q];
-                    b[3][rr][q] += d1 * xL[q];
+                    bs[rr][q] += d * xs[c][q];
+                    bt[rr][q] += d * xt[c][q];
                 }
             }
         }
 #pragma unroll
-        for (int cs = 0; cs < 2; cs++)
+        for (int q = 0; q < 2; q++) {
+            double val[nr], jmp[nr];
 #pragma unroll
-            for (int q = 0; q < 2; q++) {
-                double val[nr], jmp[nr];
-#pragma unroll
-                for (int rr = 0; rr < nr; rr++) {
-                    double vl = b[cs == 0 ? 0 : 1][rr][q], vr = b[cs == 0 ? 2 : 3][rr][q];
-                    if (r0 + rr == 0) {
-                        vl += cs == 0 ? uL[q] : uR[q];
-                        vr += cs == 0 ? uR[q] : uL[q];
-                    }
-                    val[rr] = (vl + vr) * 0.5;
-                    jmp[rr] = (vl - vr) * 0.5;
+            for (int rr = 0; rr < nr; rr++) {
+                // cell L: side 0 with its own, side 1 with R's own; cell R:
+                // side 0 with R's, side 1 with L's coefficients
+                const double other = pair_swap(sd ? bs[rr][q] : bt[rr][q]);
+                double vl = sd ? other : bs[rr][q], vr = sd ? bt[rr][q] : other;
+                if (r0 + rr == 0) {
+                    vl += us[q];
+                    vr += ut[q];
                 }
-                ff_group<G>(P, jmp, sums[cs][q][0]);
-                ff_group<G>(P, val, sums[cs][q][1]);
+                val[rr] = (vl + vr) * 0.5;
+                jmp[rr] = (vl - vr) * 0.5;
             }
+            ff_group<G>(P, jmp, sums[q][0]);
+            ff_group<G>(P, val, sums[q][1]);
+        }
     };
     pass(std::integral_constant<int, 0>{});
     pass(std::integral_constant<int, 1>{});
     pass(std::integral_constant<int, 2>{});
     pass(std::integral_constant<int, 3>{});
+    double out[4];
 #pragma unroll
-    for (int cs = 0; cs < 2; cs++) {
-        double out[4];
-#pragma unroll
-        for (int q = 0; q < 2; q++) {
-            double a = sums[cs][q][0], b = sums[cs][q][1];
-            a *= nl, b *= nl;
-            out[2 * q] = a * 2.0;
-            out[2 * q + 1] = b * 2.0;
-        }
-        // into the cell's own slot of this face, [slot][4][cell], so that the
-        // indicator reads its terms as a coalesced stream
-        const int32_t cell = cs ? R : L;
-        const int slot = cs ? (wpos[f] >> 4) : (wpos[f] & 15);
-#pragma unroll
-        for (int k = 0; k < 4; k++)
-            wslot[(int64_t(slot) * 4 + k) * ldc + cell] = out[k];
+    for (int q = 0; q < 2; q++) {
+        double a = sums[q][0], b = sums[q][1];
+        a *= nl, b *= nl;
+        out[2 * q] = a * 2.0;
+        out[2 * q + 1] = b * 2.0;
     }
+    // into the cell's own slot of this face, so that the indicator reads its
+    // terms as a coalesced stream
+    const int slot = sd ? (wpos[f] >> 4) : (wpos[f] & 15);
+    dbl2 *to = reinterpret_cast<dbl2 *>(wslot + quad64(cell, nfmax, slot));
+    to[0] = dbl2{out[0], out[1]}, to[1] = dbl2{out[2], out[3]};
 }
 
 // WBAP V3 smoothness indicator: sum over the cell's faces in cell2face order
@@ -1139,7 +1133,7 @@ __global__ __launch_bounds__(kBlock) void k_wbap_ind(int32_t nc, int64_t ldc, co
                 continue;
 #pragma unroll
             for (int k = 0; k < 4; k++)
-                sum[k] += wslot[(int64_t(s) * 4 + k) * ldc + i];
+                sum[k] += wslot[quad64(i, NF, s) + k];
         }
         const double si0 = sum[0] / (sum[1] + kVerySmallReal);
         const double si1 = sum[2] / (sum[3] + kVerySmallReal);
@@ -1150,8 +1144,11 @@ __global__ __launch_bounds__(kBlock) void k_wbap_ind(int32_t nc, int64_t ldc, co
             limf[i] = uint8_t(lim);
         else if (!lim) {
 #pragma unroll
-            for (int k = 0; k < 36; k++)
-                xo[k * ldc + i] = x[k * ldc + i];
+            for (int c = 0; c < 9; c++) {
+                const dbl2 *from = reinterpret_cast<const dbl2 *>(x + rec(i, c, 0));
+                dbl2 *to = reinterpret_cast<dbl2 *>(xo + rec(i, c, 0));
+                to[0] = from[0], to[1] = from[1];
+            }
         }
     }
     const uint64_t mask = __ballot(lim);
@@ -1201,7 +1198,7 @@ __global__ __launch_bounds__(kBlock) void k_wbap_lim(int64_t ldc, int64_t ldf, c
         for (int r = 0; r < kMaxR; r++)
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                u0[r][v] = r < nr ? x[((ls + r) + 9 * v) * ldc + i] : 0.0;
+                u0[r][v] = r < nr ? x[rec(i, ls + r, v)] : 0.0;
                 up[r][v] = 0.0, down[r][v] = 0.0;
             }
 #pragma unroll 1
@@ -1213,8 +1210,8 @@ __global__ __launch_bounds__(kBlock) void k_wbap_lim(int64_t ldc, int64_t ldf, c
             const int side = f2c[f] == i ? 0 : 1;
             double un0, un1;
             stable_normalized(fnc[f], fnc[ldf + f], un0, un1);
-            const double *ms = msec + int64_t(81 * side) * ldf + f;
-            const double *msO = msec + int64_t(81 * (1 - side)) * ldf + f;
+            const double *ms = msec + blk64(f, 162) + 64 * (81 * side);
+            const double *msO = msec + blk64(f, 162) + 64 * (81 * (1 - side));
             double oIn[kMaxR][4];
 #pragma unroll
             for (int r = 0; r < kMaxR; r++)
@@ -1229,21 +1226,21 @@ __global__ __launch_bounds__(kBlock) void k_wbap_lim(int64_t ldc, int64_t ldf, c
                 if (c <= le) {
 #pragma unroll
                     for (int v = 0; v < 4; v++)
-                        uoo[v] = x[(c + 9 * v) * ldc + j];
+                        uoo[v] = x[rec(j, c, v)];
                 } else {
 #pragma unroll
                     for (int v = 0; v < 4; v++) {
                         double acc = 0;
 #pragma unroll
                         for (int cc = le + 1; cc < 9; cc++)
-                            acc += msO[(9 * c + cc) * ldf] * uF[((s * 7 + (cc - 2)) * 4 + v) * ldc + i];
+                            acc += msO[64 * (9 * c + cc)] * uF[quad64(i, 7 * NF, s * 7 + (cc - 2)) + v];
                         uoo[v] = acc;
                     }
                 }
 #pragma unroll
                 for (int r = 0; r < kMaxR; r++)
                     if (r < nr) {
-                        const double m = ms[(9 * (ls + r) + c) * ldf];
+                        const double m = ms[64 * (9 * (ls + r) + c)];
 #pragma unroll
                         for (int v = 0; v < 4; v++)
                             oIn[r][v] += m * uoo[v];
@@ -1288,7 +1285,7 @@ __global__ __launch_bounds__(kBlock) void k_wbap_lim(int64_t ldc, int64_t ldf, c
                     for (int b = 0; b < 4; b++)
                         xv += MR[4 * a + b] * out[b];
                     if (ls + r >= 2)
-                        uF[((s * 7 + (ls + r - 2)) * 4 + a) * ldc + i] = xv;
+                        uF[quad64(i, 7 * NF, s * 7 + (ls + r - 2)) + a] = xv;
                     // FWBAP_L2_Multiway accumulation, neighbours in cell2face order
                     const double ti = u0[r][a] / (fabs(xv) + eps4) * sgn(xv);
                     down[r][a] += (ti * ti) * (ti * ti);
@@ -1301,7 +1298,7 @@ __global__ __launch_bounds__(kBlock) void k_wbap_lim(int64_t ldc, int64_t ldf, c
             if (r < nr)
 #pragma unroll
                 for (int v = 0; v < 4; v++)
-                    xo[((ls + r) + 9 * v) * ldc + i] = u0[r][v] * (up[r][v] + nStd) / (down[r][v] + nStd);
+                    xo[rec(i, ls + r, v)] = u0[r][v] * (up[r][v] + nStd) / (down[r][v] + nStd);
     }
     if (!ok)
         atomicOr(errw, ERRBIT_NONPOSITIVE);
@@ -1344,7 +1341,7 @@ __global__ __launch_bounds__(kBlock) void k_wbap_lim_v2(int64_t ldc, int64_t ldf
     for (int r = 0; r < nr; r++)
 #pragma unroll
         for (int v = 0; v < 4; v++) {
-            uC[r][v] = x[((ls + r) + 9 * v) * ldc + i];
+            uC[r][v] = x[rec(i, ls + r, v)];
             first[r][v] = 0.0, up[r][v] = 0.0, down[r][v] = 0.0;
         }
     bool ok = true;
@@ -1358,7 +1355,7 @@ __global__ __launch_bounds__(kBlock) void k_wbap_lim_v2(int64_t ldc, int64_t ldf
         const int side = f2c[f] == i ? 0 : 1;
         double un0, un1;
         stable_normalized(fnc[f], fnc[ldf + f], un0, un1);
-        const double *ms = msec + int64_t(81 * side) * ldf + f;
+        const double *ms = msec + blk64(f, 162) + 64 * (81 * side);
         // the neighbour's rows above le: limited (xo) or, with limf, as given (x)
         const double *above = (limf && !limf[j]) ? x : xo;
         double oIn[nr][4];
@@ -1373,10 +1370,10 @@ __global__ __launch_bounds__(kBlock) void k_wbap_lim_v2(int64_t ldc, int64_t ldf
             double uj[4];
 #pragma unroll
             for (int v = 0; v < 4; v++)
-                uj[v] = src[(c + 9 * v) * ldc + j];
+                uj[v] = src[rec(j, c, v)];
 #pragma unroll
             for (int r = 0; r < nr; r++) {
-                const double m = ms[(9 * (ls + r) + c) * ldf];
+                const double m = ms[64 * (9 * (ls + r) + c)];
 #pragma unroll
                 for (int v = 0; v < 4; v++)
                     oIn[r][v] += m * uj[v];
@@ -1433,7 +1430,7 @@ __global__ __launch_bounds__(kBlock) void k_wbap_lim_v2(int64_t ldc, int64_t ldf
     for (int r = 0; r < nr; r++)
 #pragma unroll
         for (int v = 0; v < 4; v++)
-            xo[((ls + r) + 9 * v) * ldc + i] =
+            xo[rec(i, ls + r, v)] =
                 nOther ? first[r][v] * (up[r][v] + 1.0) / (down[r][v] + 1.0) : uC[r][v];
     if (!ok)
         atomicOr(errw, ERRBIT_NONPOSITIVE);
@@ -1652,7 +1649,7 @@ extern "C" int dndsmi_ctx_create(const dndsmi_mesh_view *mesh, const dndsmi_vr_v
         std::vector<int32_t> nbr(size_t(nfmax) * ldc, -2), sbc(size_t(nfmax) * ldc, 0), sface(size_t(nfmax) * ldc, -1);
         std::vector<int32_t> gat(size_t(nfmax) * ldc, -1), widx(size_t(nfmax) * ldc, -1);
         std::vector<uint8_t> wpos(ldf, 0);
-        std::vector<double> M(size_t(nfmax) * kMPairs * 2 * ldc, 0.0), bv(size_t(nfmax) * 9 * ldc, 0.0), vol(ldc, 1.0);
+        std::vector<double> M(size_t(nfmax) * kAbVecs * 2 * ldc, 0.0), vol(ldc, 1.0);
         std::vector<double> cmom(9 * size_t(ldc), 0.0), cscale(2 * size_t(ldc), 1.0);
         std::vector<int64_t> wall_cell, wall_face, wall_c2f;
         for (int64_t i = 0; i < nc; i++) {
@@ -1661,7 +1658,7 @@ extern "C" int dndsmi_ctx_create(const dndsmi_mesh_view *mesh, const dndsmi_vr_v
             const int64_t ci = c2d[i]; // device column of mesh cell i
             vol[ci] = vr->volume[i];
             for (int k = 0; k < 9; k++)
-                cmom[k * ldc + ci] = vr->base_moment[10 * i + 1 + k];
+                cmom[blk64(ci, 9) + 64 * k] = vr->base_moment[10 * i + 1 + k];
             cscale[2 * ci] = vr->cell_scale[2 * i], cscale[2 * ci + 1] = vr->cell_scale[2 * i + 1];
             std::vector<std::pair<int64_t, int>> order;
             for (int s = 0; s < n; s++) {
@@ -1674,10 +1671,10 @@ extern "C" int dndsmi_ctx_create(const dndsmi_mesh_view *mesh, const dndsmi_vr_v
                 sface[s * ldc + ci] = f2d[f];
                 if (j != DNDSMI_NO_CELL)
                     wpos[f2d[f]] |= uint8_t(s << (4 * side));
-                for (int k = 0; k < 81; k++)
-                    M[size_t(m_vec_index(s, k / 2, ci, ldc, kMPairs)) * 2 + k % 2] = vr->ainv_b[81 * (b0 + s) + k];
-                for (int k = 0; k < 9; k++)
-                    bv[(size_t(s) * 9 + k) * ldc + ci] = vr->ainv_bvec[9 * (b0 + s) + k];
+                for (int d = 0; d < 90; d++)
+                    M[size_t(ab_vec(s, d / 2, ci, ldc, kAbVecs)) * 2 + d % 2] =
+                        d % 10 < 9 ? vr->ainv_b[81 * (b0 + s) + 9 * (d / 10) + d % 10]
+                                   : vr->ainv_bvec[9 * (b0 + s) + d / 10];
                 order.push_back({f, side});
                 if (j == DNDSMI_NO_CELL &&
                     (mesh->face_bc[f] == DNDSMI_BC_WALL_EULER || mesh->face_bc[f] == DNDSMI_BC_WALL_NOSLIP)) {
@@ -1714,11 +1711,9 @@ extern "C" int dndsmi_ctx_create(const dndsmi_mesh_view *mesh, const dndsmi_vr_v
         }
         DNDSMI_TRY(c->alloc(c->wall_idx, nfmax * ldc));
         DNDSMI_TRY(c->upload(c->wall_idx, widx));
-        DNDSMI_TRY(c->alloc(c->M, int64_t(nfmax) * kMPairs * 2 * ldc));
+        DNDSMI_TRY(c->alloc(c->M, int64_t(nfmax) * kAbVecs * 2 * ldc));
         DNDSMI_TRY(c->upload(c->M, M));
         M.clear(), M.shrink_to_fit();
-        DNDSMI_TRY(c->alloc(c->bv, int64_t(nfmax) * 9 * ldc));
-        DNDSMI_TRY(c->upload(c->bv, bv));
         DNDSMI_TRY(c->alloc(c->vol, ldc));
         DNDSMI_TRY(c->upload(c->vol, vol));
         DNDSMI_TRY(c->alloc(c->cmom, 9 * ldc));
@@ -1757,7 +1752,7 @@ extern "C" int dndsmi_ctx_create(const dndsmi_mesh_view *mesh, const dndsmi_vr_v
             DNDSMI_TRY(c->upload(c->wall_cell, wc));
             DNDSMI_TRY(c->alloc(c->wall_bc, c->n_wall));
             DNDSMI_TRY(c->upload(c->wall_bc, wb));
-            DNDSMI_TRY(c->alloc(c->wall_corr, 36 * c->n_wall));
+            DNDSMI_TRY(c->alloc(c->wall_corr, kRec * c->n_wall));
             c->n_wall_faces = nw;
         }
         // ---- face streams
@@ -1774,9 +1769,10 @@ extern "C" int dndsmi_ctx_create(const dndsmi_mesh_view *mesh, const dndsmi_vr_v
             for (int g = 0; g < 3; g++) // rows [side][g] of (X, Y) pairs
                 for (int sd = 0; sd < 2; sd++)
                     for (int k = 0; k < 2; k++)
-                        fxy[(size_t(sd * 3 + g) * ldf + f) * 2 + k] = vr->face_gauss_xy[12 * fo + 4 * g + 2 * sd + k];
+                        fxy[(blk64(f, 6) + 64 * (sd * 3 + g)) * 2 + k] =
+                            vr->face_gauss_xy[12 * fo + 4 * g + 2 * sd + k];
             for (int k = 0; k < 6; k++)
-                fn[k * ldf + f] = vr->face_norm[6 * fo + k];
+                fn[blk64(f, 6) + 64 * k] = vr->face_norm[6 * fo + k];
             for (int k = 2; k < 6; k++)
                 straight &= std::memcmp(&vr->face_norm[6 * fo + k], &vr->face_norm[6 * fo + k % 2], 8) == 0;
             fnc[f] = vr->face_norm_center[2 * fo], fnc[ldf + f] = vr->face_norm_center[2 * fo + 1];
@@ -1819,13 +1815,13 @@ extern "C" int dndsmi_ctx_create(const dndsmi_mesh_view *mesh, const dndsmi_vr_v
             buf.assign(162 * size_t(ldf), 0.0);
             for (int64_t f = 0; f < nf; f++)
                 for (int k = 0; k < 162; k++)
-                    buf[k * ldf + f2d[f]] = vr->matrix_secondary[162 * f + k];
+                    buf[blk64(f2d[f], 162) + 64 * k] = vr->matrix_secondary[162 * f + k];
             DNDSMI_TRY(c->alloc(c->msec, 162 * ldf));
             DNDSMI_TRY(c->upload(c->msec, buf));
             buf.assign(10 * size_t(ldf), 0.0);
             for (int64_t f = 0; f < nf; f++)
                 for (int k = 0; k < 10; k++)
-                    buf[k * ldf + f2d[f]] = vr->face_weight[10 * f + k];
+                    buf[blk64(f2d[f], 10) + 64 * k] = vr->face_weight[10 * f + k];
             DNDSMI_TRY(c->alloc(c->fw, 10 * ldf));
             DNDSMI_TRY(c->upload(c->fw, buf));
             DNDSMI_TRY(c->alloc(c->wslot, int64_t(nfmax) * 4 * ldc));
@@ -1976,7 +1972,7 @@ extern "C" int dndsmi_array_upload(dndsmi_array *a, const double *host) {
         std::vector<double> buf(36 * size_t(ldc), 0.0);
         for (int64_t i = 0; i < nc; i++)
             for (int k = 0; k < 36; k++)
-                buf[k * ldc + c2d[i]] = host[36 * i + k];
+                buf[rec(c2d[i], k % 9, k / 9)] = host[36 * i + k];
         return c->upload(a->d, buf);
     }
     const int w = a->kind == DNDSMI_ARRAY_DOF ? 4 : 1;
@@ -2000,7 +1996,7 @@ extern "C" int dndsmi_array_download(const dndsmi_array *a, double *host) {
         DNDSMI_TRY(c->hip(hipStreamSynchronize(c->stream), "hipStreamSynchronize"));
         for (int64_t i = 0; i < nc; i++)
             for (int k = 0; k < 36; k++)
-                host[36 * i + k] = buf[k * ldc + c->c2d[i]];
+                host[36 * i + k] = buf[rec(c->c2d[i], k % 9, k / 9)];
         return DNDSMI_OK;
     }
     const int w = a->kind == DNDSMI_ARRAY_DOF ? 4 : 1;
@@ -2031,6 +2027,10 @@ extern "C" int dndsmi_array_set_constant(dndsmi_array *a, double value) {
 
 namespace dndsmi_host {
 
+// Workgroup size of a sweep over `lanes` lanes.  Waves are independent; small
+// sweeps take one wave per workgroup, so that their waves spread over all CUs.
+int sweep_block(int64_t lanes) { return lanes < 300000 ? 64 : kBlock; }
+
 // SOR_Instead: colour by colour in place on x (forward; with
 // SOR_InverseScanning then backward, DNDS_FV_VR.hpp:1493-1502)
 int launch_sor(dndsmi_ctx *c, const double *u, double *x, double t) {
@@ -2038,24 +2038,19 @@ int launch_sor(dndsmi_ctx *c, const double *u, double *x, double t) {
     for (int pass = 0; pass < passes; pass++)
         for (int32_t kk = 0; kk < c->n_colour; kk++) {
             const int32_t col = pass == 0 ? kk : c->n_colour - 1 - kk;
-            for (int w = 0; w < 2; w++) {
-                const int64_t b = w ? c->sor_wall[col] : c->sor_start[col];
-                const int64_t n = (w ? c->sor_start[col + 1] : c->sor_wall[col]) - b;
-                if (n == 0)
-                    continue;
-                auto kern = c->nfmax == 3 ? (w ? k_sor<3, true> : k_sor<3, false>)
-                                          : (w ? k_sor<4, true> : k_sor<4, false>);
-                // the boundary cells are a few thousand: one wave per
-                // workgroup spreads them over as many CUs as there are waves
-                const int block = w ? 64 : kBlock;
-                prof_begin(c, DNDSMI_K_JACOBI);
-                hipLaunchKernelGGL(kern, dim3(unsigned((n + block - 1) / block)), dim3(block), 0, c->stream,
-                                   int32_t(n), int32_t(b),
-                                   c->ldc, c->nbr, c->sbc, c->wall_idx, c->M, c->bv, u, x, x, c->relax,
-                                   c->wall_ainv, c->wall_d0, c->wall_nrm, c->wall_w0, c->n_wall, c->gas, t, c->errw);
-                prof_end(c);
-                DNDSMI_TRY(c->launch_check("k_sor"));
-            }
+            // whole groups of 16 cells around the colour's range
+            const int64_t b = c->sor_start[col], n = c->sor_start[col + 1] - b;
+            if (n == 0)
+                continue;
+            const int64_t lanes = 4 * ((b & 15) + n);
+            const int block = sweep_block(lanes);
+            auto kern = c->nfmax == 3 ? k_sor<3> : k_sor<4>;
+            prof_begin(c, DNDSMI_K_JACOBI);
+            hipLaunchKernelGGL(kern, dim3(grid_for(lanes, block)), dim3(block), 0,
+                               c->stream, int32_t(n), int32_t(b), c->ldc, c->nbr, c->sbc, c->wall_idx, c->M, u, x, x,
+                               c->relax, c->wall_faces(), c->errw);
+            prof_end(c);
+            DNDSMI_TRY(c->launch_check("k_sor"));
         }
     return DNDSMI_OK;
 }
@@ -2075,22 +2070,13 @@ int launch_jacobi(dndsmi_ctx *c, const double *u, const double *x, double *xn, d
                           "copy uRec"));
         return launch_sor(c, u, xn, t);
     }
-    const int nc = int(c->nc);
-    if (c->n_wall_faces > 0) {
-        prof_begin(c, DNDSMI_K_WALL_CORR);
-        hipLaunchKernelGGL(k_wall_corr, dim3(grid_for(c->n_wall_faces)), dim3(kBlock), 0, c->stream,
-                           int32_t(c->n_wall_faces), c->ldc, c->wall_cell, c->wall_bc, c->wall_ainv, c->wall_d0,
-                           c->wall_nrm, c->wall_w0, c->n_wall, u, x, c->relax, c->gas, t, c->wall_corr, c->errw);
-        prof_end(c);
-        DNDSMI_TRY(c->launch_check("k_wall_corr"));
-    }
+    const int64_t lanes = 4 * c->nc;
+    const int block = sweep_block(lanes);
     prof_begin(c, DNDSMI_K_JACOBI);
-    if (c->nfmax == 3)
-        hipLaunchKernelGGL(k_jacobi<3>, dim3(grid_for(nc)), dim3(kBlock), 0, c->stream, nc, c->ldc, c->nbr, c->sbc,
-                           c->wall_idx, c->M, c->bv, u, x, xn, c->relax, c->wall_corr, c->n_wall, c->errw);
-    else
-        hipLaunchKernelGGL(k_jacobi<4>, dim3(grid_for(nc)), dim3(kBlock), 0, c->stream, nc, c->ldc, c->nbr, c->sbc,
-                           c->wall_idx, c->M, c->bv, u, x, xn, c->relax, c->wall_corr, c->n_wall, c->errw);
+    auto kern = c->nfmax == 3 ? k_jacobi<3, false> : k_jacobi<4, false>;
+    hipLaunchKernelGGL(kern, dim3(grid_for(lanes, block)), dim3(block), 0, c->stream, int32_t(c->nc),
+                       c->ldc, c->nbr, c->sbc, c->wall_idx, c->M, u, x, xn, c->relax, c->wall_faces(), c->wall_corr,
+                       c->errw, nullptr);
     prof_end(c);
     return c->launch_check("k_jacobi");
 }
@@ -2121,12 +2107,12 @@ int launch_rhs(dndsmi_ctx *c, const double *u, const double *x, double t, double
     if (c->gas.mu > 0) {
         hipLaunchKernelGGL((c->straight_faces ? k_rhs_face<false, false, true, true>
                                               : k_rhs_face<false, false, false, true>),
-                           dim3(grid_for(nf)), dim3(kBlock), 0, c->stream, nf, c->ldf, c->ldc, c->bfaces, c->f2c,
+                           dim3(grid_for(nf)), dim3(kBlock), 0, c->stream, nf, c->ldf, c->nfmax, c->bfaces, c->f2c,
                            c->fbc, c->fxy, c->cmom, c->fn, c->fctr, c->dlambda_face, u, x, c->gas, t, c->fpos,
                            c->fslot, c->errw, nullptr, c->cscale, c->vol, c->farea, xalt, limf);
     } else {
         hipLaunchKernelGGL((c->straight_faces ? k_rhs_face<false, false, true> : k_rhs_face<false, false, false>),
-                           dim3(grid_for(nf)), dim3(kBlock), 0, c->stream, nf, c->ldf, c->ldc, c->bfaces, c->f2c,
+                           dim3(grid_for(nf)), dim3(kBlock), 0, c->stream, nf, c->ldf, c->nfmax, c->bfaces, c->f2c,
                            c->fbc, c->fxy, c->cmom, c->fn, c->fctr, c->dlambda_face, u, x, c->gas, t, c->fpos,
                            c->fslot, c->errw, nullptr, nullptr, nullptr, nullptr, xalt, limf);
     }
@@ -2135,12 +2121,12 @@ int launch_rhs(dndsmi_ctx *c, const double *u, const double *x, double t, double
         prof_begin(c, DNDSMI_K_RHS_BFACE);
         if (c->gas.mu > 0)
             hipLaunchKernelGGL((k_rhs_face<true, false, false, true>), dim3(grid_for(c->n_bface)), dim3(kBlock), 0,
-                               c->stream, int32_t(c->n_bface), c->ldf, c->ldc, c->bfaces, c->f2c, c->fbc, c->fxy,
+                               c->stream, int32_t(c->n_bface), c->ldf, c->nfmax, c->bfaces, c->f2c, c->fbc, c->fxy,
                                c->cmom, c->fn, c->fctr, c->dlambda_face, u, x, c->gas, t, c->fpos, c->fslot, c->errw,
                                nullptr, c->cscale, c->vol, c->farea, xalt, limf);
         else
             hipLaunchKernelGGL(k_rhs_face<true>, dim3(grid_for(c->n_bface)), dim3(kBlock), 0, c->stream,
-                               int32_t(c->n_bface), c->ldf, c->ldc, c->bfaces, c->f2c, c->fbc, c->fxy, c->cmom, c->fn,
+                               int32_t(c->n_bface), c->ldf, c->nfmax, c->bfaces, c->f2c, c->fbc, c->fxy, c->cmom, c->fn,
                                c->fctr, c->dlambda_face, u, x, c->gas, t, c->fpos, c->fslot, c->errw, nullptr,
                                nullptr, nullptr, nullptr, xalt, limf);
         prof_end(c);
@@ -2166,8 +2152,8 @@ int launch_wbap(dndsmi_ctx *c, const double *u, const double *x, double *xo, dou
     const int nc = int(c->nc), nf = int(c->nf);
     const double eps4 = std::pow(1e-200, 1.0 / 4); // verySmallReal_pDiP, DNDS_FV_Limiters.hpp:345
     prof_begin(c, DNDSMI_K_WBAP_FACE);
-    hipLaunchKernelGGL(k_wbap_face, dim3(grid_for(nf)), dim3(kBlock), 0, c->stream, nf, c->ldf, c->ldc, c->f2c,
-                       c->fxy, c->cmom, c->cscale, c->fw, c->fn, u, x, c->tang_weight, c->twd_norm, c->wpos,
+    hipLaunchKernelGGL(k_wbap_face, dim3(grid_for(2 * int64_t(nf))), dim3(kBlock), 0, c->stream, nf, c->ldf,
+                       c->nfmax, c->f2c, c->fxy, c->cmom, c->cscale, c->fw, c->fn, u, x, c->tang_weight, c->twd_norm, c->wpos,
                        c->wslot);
     prof_end(c);
     hipLaunchKernelGGL(k_zero_int2, dim3(1), dim3(64), 0, c->stream, c->lim_count);
@@ -2217,73 +2203,43 @@ int launch_wbap(dndsmi_ctx *c, const double *u, const double *x, double *xo, dou
 int ensure_mixed(dndsmi_ctx *c) {
     if (c->M32)
         return DNDSMI_OK;
-    const int64_t nm = int64_t(c->nfmax) * kMQuads * 4 * c->ldc;
+    const int64_t nm = int64_t(c->nfmax) * kAb32Vecs * 4 * c->ldc;
     DNDSMI_TRY(c->alloc(c->M32, nm));
     DNDSMI_TRY(c->alloc(c->r32, 36 * c->ldc));
     DNDSMI_TRY(c->alloc(c->dA32, 36 * c->ldc));
     DNDSMI_TRY(c->alloc(c->dB32, 36 * c->ldc));
     DNDSMI_TRY(c->alloc(c->fslot32, int64_t(c->nfmax) * 8 * c->ldc));
-    DNDSMI_TRY(c->alloc(c->wcorr32, 36 * c->n_wall));
     hipLaunchKernelGGL(k_m_to_f32, dim3(grid_for(nm / 4)), dim3(kBlock), 0, c->stream, int32_t(c->nfmax), c->ldc,
                        c->M, c->M32);
-    DNDSMI_TRY(c->launch_check("k_to_f32"));
+    DNDSMI_TRY(c->launch_check("k_m_to_f32"));
     return c->hip(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
 }
 
 // one FP64 step that yields r = J(x) - x, then n - 1 FP32 correction sweeps,
 // the last adding the correction to x in place
 int launch_jacobi_mixed(dndsmi_ctx *c, const double *u, double *x, int n_sweeps, double t) {
-    const int nc = int(c->nc);
-    if (c->n_wall_faces > 0) {
-        hipLaunchKernelGGL(k_wall_corr, dim3(grid_for(c->n_wall_faces)), dim3(kBlock), 0, c->stream,
-                           int32_t(c->n_wall_faces), c->ldc, c->wall_cell, c->wall_bc, c->wall_ainv, c->wall_d0,
-                           c->wall_nrm, c->wall_w0, c->n_wall, u, x, c->relax, c->gas, t, c->wall_corr, c->errw);
-        DNDSMI_TRY(c->launch_check("k_wall_corr"));
-    }
+    const int64_t lanes = 4 * c->nc;
+    const int block = sweep_block(lanes), nc = int(c->nc);
+    const dim3 grid(grid_for(lanes, block));
     prof_begin(c, DNDSMI_K_JACOBI);
-    if (c->nfmax == 3)
-        hipLaunchKernelGGL((k_jacobi<3, true>), dim3(grid_for(nc)), dim3(kBlock), 0, c->stream, nc, c->ldc, c->nbr,
-                           c->sbc, c->wall_idx, c->M, c->bv, u, x, nullptr, c->relax, c->wall_corr, c->n_wall,
-                           c->errw, c->r32, c->dA32);
-    else
-        hipLaunchKernelGGL((k_jacobi<4, true>), dim3(grid_for(nc)), dim3(kBlock), 0, c->stream, nc, c->ldc, c->nbr,
-                           c->sbc, c->wall_idx, c->M, c->bv, u, x, nullptr, c->relax, c->wall_corr, c->n_wall,
-                           c->errw, c->r32, c->dA32);
+    auto first = c->nfmax == 3 ? k_jacobi<3, true> : k_jacobi<4, true>;
+    hipLaunchKernelGGL(first, grid, dim3(block), 0, c->stream, nc,
+                       c->ldc, c->nbr, c->sbc, c->wall_idx, c->M, u, x, nullptr, c->relax, c->wall_faces(),
+                       c->wall_corr, c->errw, c->r32);
     prof_end(c);
     DNDSMI_TRY(c->launch_check("k_jacobi (residual)"));
-    float *din = c->dA32, *dout = c->dB32;
-    const float w = float(c->relax);
+    // d_0 = r: the first correction sweep reads r itself
+    float *din = c->r32, *dout = c->dA32, *next = c->dB32;
     for (int k = 1; k < n_sweeps; k++) {
-        const bool last = k == n_sweeps - 1;
-        if (c->n_wall_faces > 0) {
-            hipLaunchKernelGGL(k_wall_corr_lin, dim3(grid_for(c->n_wall_faces)), dim3(kBlock), 0, c->stream,
-                               int32_t(c->n_wall_faces), c->ldc, c->wall_cell, c->wall_bc, c->wall_ainv, c->wall_d0,
-                               c->wall_nrm, c->wall_w0, c->n_wall, din, w, c->wcorr32);
-            DNDSMI_TRY(c->launch_check("k_wall_corr_lin"));
-        }
+        auto kern = k == n_sweeps - 1 ? (c->nfmax == 3 ? k_delta32<3, true> : k_delta32<4, true>)
+                                      : (c->nfmax == 3 ? k_delta32<3, false> : k_delta32<4, false>);
         prof_begin(c, DNDSMI_K_DELTA32);
-        if (c->nfmax == 3) {
-            if (last)
-                hipLaunchKernelGGL((k_delta32<3, true>), dim3(grid_for(nc)), dim3(kBlock), 0, c->stream, nc, c->ldc,
-                                   c->nbr, c->sbc, c->M32, c->r32, din, nullptr, w, x, c->wall_idx, c->wcorr32,
-                                   c->n_wall);
-            else
-                hipLaunchKernelGGL((k_delta32<3, false>), dim3(grid_for(nc)), dim3(kBlock), 0, c->stream, nc,
-                                   c->ldc, c->nbr, c->sbc, c->M32, c->r32, din, dout, w, nullptr, c->wall_idx,
-                                   c->wcorr32, c->n_wall);
-        } else {
-            if (last)
-                hipLaunchKernelGGL((k_delta32<4, true>), dim3(grid_for(nc)), dim3(kBlock), 0, c->stream, nc, c->ldc,
-                                   c->nbr, c->sbc, c->M32, c->r32, din, nullptr, w, x, c->wall_idx, c->wcorr32,
-                                   c->n_wall);
-            else
-                hipLaunchKernelGGL((k_delta32<4, false>), dim3(grid_for(nc)), dim3(kBlock), 0, c->stream, nc,
-                                   c->ldc, c->nbr, c->sbc, c->M32, c->r32, din, dout, w, nullptr, c->wall_idx,
-                                   c->wcorr32, c->n_wall);
-        }
+        hipLaunchKernelGGL(kern, grid, dim3(block), 0, c->stream, nc, c->ldc, c->nbr, c->sbc, c->wall_idx, c->M32,
+                           c->r32, din, dout, float(c->relax), x, c->wall_faces());
         prof_end(c);
         DNDSMI_TRY(c->launch_check("k_delta32"));
-        std::swap(din, dout);
+        din = dout;
+        std::swap(dout, next);
     }
     return DNDSMI_OK;
 }
@@ -2293,13 +2249,13 @@ int launch_rhs_mixed(dndsmi_ctx *c, const double *u, const double *x, double t, 
     const int nc = int(c->nc), nf = int(c->nf);
     prof_begin(c, DNDSMI_K_RHS_FACE32);
     hipLaunchKernelGGL((c->straight_faces ? k_rhs_face<false, true, true> : k_rhs_face<false, true, false>),
-                       dim3(grid_for(nf)), dim3(kBlock), 0, c->stream, nf, c->ldf, c->ldc, c->bfaces, c->f2c, c->fbc,
+                       dim3(grid_for(nf)), dim3(kBlock), 0, c->stream, nf, c->ldf, c->nfmax, c->bfaces, c->f2c, c->fbc,
                        c->fxy, c->cmom, c->fn, c->fctr, c->dlambda_face, u, x, c->gas, t, c->fpos, nullptr, c->errw,
                        c->fslot32, nullptr, nullptr, nullptr, xalt, limf);
     prof_end(c);
     if (c->n_bface > 0)
         hipLaunchKernelGGL((k_rhs_face<true, true>), dim3(grid_for(c->n_bface)), dim3(kBlock), 0, c->stream,
-                           int32_t(c->n_bface), c->ldf, c->ldc, c->bfaces, c->f2c, c->fbc, c->fxy, c->cmom, c->fn,
+                           int32_t(c->n_bface), c->ldf, c->nfmax, c->bfaces, c->f2c, c->fbc, c->fxy, c->cmom, c->fn,
                            c->fctr, c->dlambda_face, u, x, c->gas, t, c->fpos, nullptr, c->errw, c->fslot32,
                            nullptr, nullptr, nullptr, xalt, limf);
     prof_begin(c, DNDSMI_K_RHS_CELL32);
@@ -2536,15 +2492,11 @@ extern "C" int dndsmi_read_probe(dndsmi_ctx *c, int32_t reps) {
     if (!c || reps < 1)
         return DNDSMI_ERR_INVALID_ARGUMENT;
     if (!c->probe_out)
-        DNDSMI_TRY(c->alloc(c->probe_out, c->ldc));
+        DNDSMI_TRY(c->alloc(c->probe_out, 4 * c->ldc));
     for (int k = 0; k < reps; k++) {
         prof_begin(c, DNDSMI_K_READ_PROBE);
-        if (c->nfmax == 3)
-            hipLaunchKernelGGL(k_read_probe<3>, dim3(grid_for(c->nc)), dim3(kBlock), 0, c->stream, int32_t(c->nc),
-                               c->ldc, c->nbr, c->M, c->probe_out);
-        else
-            hipLaunchKernelGGL(k_read_probe<4>, dim3(grid_for(c->nc)), dim3(kBlock), 0, c->stream, int32_t(c->nc),
-                               c->ldc, c->nbr, c->M, c->probe_out);
+        hipLaunchKernelGGL((c->nfmax == 3 ? k_read_probe<3> : k_read_probe<4>), dim3(grid_for(4 * c->nc)),
+                           dim3(kBlock), 0, c->stream, int32_t(c->nc), c->ldc, c->nbr, c->M, c->probe_out);
         prof_end(c);
         DNDSMI_TRY(c->launch_check("k_read_probe"));
     }
@@ -2627,8 +2579,8 @@ extern "C" int64_t dndsmi_kernel_bytes(const dndsmi_ctx *c, int32_t kernel) {
         return nif * (8 + 1 + 96 + (c->straight_faces ? 16 : 48) + 8 + 64) + nc * (36 * 8 + 32 + 72);
     case DNDSMI_K_RHS_CELL32: // 8 FP32 terms per slot, volume, x read+write, xLast (+ last-slot index)
         return c2f * 32 + nc * (8 + 32 * 3 + (c->nfmax == 4 ? 4 : 0));
-    case DNDSMI_K_READ_PROBE: // the sweep's A^-1 B pairs (41 x 16 B per slot) and slot index, one double out
-        return c2f * (kMPairs * 16 + 4) + nc * 8;
+    case DNDSMI_K_READ_PROBE: // the sweep's A^-1 B, A^-1 b (45 x 16 B per slot) and slot index, four doubles out
+        return c2f * (kAbVecs * 16 + 4) + nc * 32;
     default:
         return 0;
     }

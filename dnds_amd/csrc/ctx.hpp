@@ -56,8 +56,7 @@ struct dndsmi_ctx {
     int32_t *sbc = nullptr;    // [nfmax][ldc] boundary kind of the slot's face
     int32_t *sface = nullptr;  // [nfmax][ldc] face index of the slot
     int32_t *gat = nullptr;    // [nfmax][ldc] (face << 1 | side) sorted by face, -1 = none
-    double *M = nullptr;       // [nfmax][41][ldc][2] A^-1 B entry pairs
-    double *bv = nullptr;      // [nfmax*9][ldc]
+    double *M = nullptr;       // A^-1 B and A^-1 b, 45 pairs per cell and slot (ab_vec)
     double *vol = nullptr;     // [ldc]
     int32_t *wall_idx = nullptr; // [nfmax][ldc] index into the wall-face arrays, -1 = none
     int64_t n_wall = 0;
@@ -67,15 +66,16 @@ struct dndsmi_ctx {
     double *wall_w0 = nullptr;   // [n_wall]
     int32_t *wall_cell = nullptr; // [n_wall]
     int32_t *wall_bc = nullptr;   // [n_wall]
-    double *wall_corr = nullptr;  // [36][n_wall]
+    double *wall_corr = nullptr;  // [n_wall][36] the running sweep's wall corrections
     int64_t n_wall_faces = 0;     // real count (n_wall >= 1 for allocation)
     // face side
     int32_t *f2c = nullptr;    // [2][ldf]
     int32_t *fbc = nullptr;    // [ldf]
-    double *fxy = nullptr;     // [6][ldf][2] (X, Y) of LINE_3 point g seen from side s, row 3 s + g
-    double *cmom = nullptr;    // [9][ldc] base moments 1..9 of the cell
+    // face and cell data in blocks of 64 (blk64, quad64; elements in brackets)
+    double *fxy = nullptr;     // [6] pairs (X, Y) of LINE_3 point g seen from side s, pair 3 s + g
+    double *cmom = nullptr;    // [9] base moments 1..9 of the cell
     double *cscale = nullptr;  // [ldc][2] (sx, sy) of the cell's scaled monomials
-    double *fn = nullptr;      // [6][ldf] normals at the LINE_3 points
+    double *fn = nullptr;      // [6] normals at the LINE_3 points
     double *fnc = nullptr;     // [2][ldf] normal at the face centre
     double *farea = nullptr;   // [ldf]
     double *fctr = nullptr;    // [2][ldf]
@@ -83,13 +83,13 @@ struct dndsmi_ctx {
     int64_t n_bface = 0;
     // WBAP data (present when the setup carries limiter data)
     bool has_limiter = false;
-    double *fw = nullptr;      // [10][ldf] face weights
-    double *msec = nullptr;    // [162][ldf] matrixSecondary (R2L, L2R)
-    double *wslot = nullptr;   // [nfmax][4][ldc] indicator terms of the cell's faces, cell2face slot order
+    double *fw = nullptr;      // [10] face weights
+    double *msec = nullptr;    // [162] matrixSecondary (R2L, L2R)
+    double *wslot = nullptr;   // [nfmax] quads: indicator terms of the cell's faces, cell2face slot order
     uint8_t *wpos = nullptr;   // [ldf] the face's cell2face slot in cell L (low 4 bits) and in cell R (high)
-    double *uF = nullptr;      // [nfmax*28][ldc] WBAP per-cell face scratch
+    double *uF = nullptr;      // [nfmax * 7] quads: WBAP per-cell face scratch
     double *ind = nullptr;     // [ldc] indicator when the caller passes none
-    double *xlim = nullptr;    // [36][ldc] limited reconstruction inside SSP-RK3 steps (limited cells only)
+    double *xlim = nullptr;    // REC layout: limited reconstruction inside SSP-RK3 steps (limited cells only)
     uint8_t *limf = nullptr;   // [ldc] 1 where the steps' limiter wrote the cell into xlim
     bool wbap_full_copy = true; // the last WBAP launch copied the unlimited cells (byte model)
     int32_t *lim_list = nullptr;  // [ldc] cells to limit
@@ -103,7 +103,7 @@ struct dndsmi_ctx {
     double *lambda_face = nullptr;
     double *dlambda_face = nullptr;
     // face fluxes integrated over the face, stored at the slot of each side's
-    // cell: [nfmax][8][ldc], per slot F then the side's flux-balance term,
+    // cell: [2 nfmax] quads, per slot F then the side's flux-balance term,
     // signed as the cell adds them (side 0: F, -FLfix; side 1: -F, FRfix)
     double *fslot = nullptr;
     uint8_t *fpos = nullptr;   // [ldf] slot of the face in cell L (low 4 bits) and in cell R (high 4 bits)
@@ -139,10 +139,9 @@ struct dndsmi_ctx {
     double *sc_n0 = nullptr, *sc_n1 = nullptr, *sc_area = nullptr, *sc_vol = nullptr;
     // mixed precision (allocated on first use): FP32 copy of A^-1 B, FP32
     // correction vectors, FP32 face fluxes
-    float *M32 = nullptr;             // [nfmax][21][ldc][4]
-    float *r32 = nullptr, *dA32 = nullptr, *dB32 = nullptr; // [36][ldc]
-    float *fslot32 = nullptr;         // [nfmax][8][ldc]
-    float *wcorr32 = nullptr;         // [36][n_wall] linear wall correction of a correction sweep
+    float *M32 = nullptr;             // A^-1 B, 21 vectors per cell and slot (ab_vec)
+    float *r32 = nullptr, *dA32 = nullptr, *dB32 = nullptr; // REC layout
+    float *fslot32 = nullptr;         // [2 nfmax] quads
     // implicit dual-time scratch (allocated on first use)
     double *imp_rhs = nullptr;        // [ldc][4]
     double *imp_xinc = nullptr;       // [ldc][4]
@@ -153,7 +152,7 @@ struct dndsmi_ctx {
     // the learned warm start inside the mixed-precision step
     // (dndsmi_ssprk3_set_warm_start): the previous stage's cell means and
     // their change [ldc][4], the plain shadow run of a check window
-    // ([ldc][4], [36][ldc]) and its reduction partials (all first use)
+    // ([ldc][4], REC layout) and its reduction partials (all first use)
     struct dndsmi_warmstart *step_ws = nullptr;
     double *ws_uprev = nullptr, *ws_du = nullptr;
     double *ws_sh_u = nullptr, *ws_sh_x = nullptr, *ws_part = nullptr;
@@ -202,6 +201,7 @@ struct dndsmi_ctx {
             return rc;
         return hip(hipStreamSynchronize(stream), "hipStreamSynchronize");
     }
+    dndsmi_dev::WallFaces wall_faces() const { return {wall_ainv, wall_d0, wall_nrm, wall_w0, n_wall}; }
     int launch_check(const char *what) { return hip(hipGetLastError(), what); }
 };
 

@@ -1,14 +1,10 @@
 // gfx950 device code of the FP64 hot path.
 //
-// Layouts (all device arrays padded to ld = n rounded up to 64):
-//   DOF arrays   u[cell][4]             (AoS, 32 B per cell)
-//   REC arrays   x[k][cell], k = r + 9 v (SoA: lane-contiguous per element)
-//   A^-1 B       M[slot][e/2][cell][e%2], e = r*9 + c (pairs of doubles)
-//   A^-1 b       bv[(slot*9 + r)][cell]
-//   face rows    d0[(g*18 + side*9 + c)][face]
-// One thread owns one cell (sweep, gather) or one face (fluxes); the cell
-// gathers visit a cell's faces in ascending face index, which reproduces the
-// reference's face-loop scatter order without atomics.
+// Layouts: all device arrays are padded to ld = n rounded up to 64; DOF arrays
+// are u[cell][4], the others in blocks of 64 cells or faces (below).
+// The sweeps run four lanes per cell; the cell gathers visit a cell's faces in
+// ascending face index, which reproduces the reference's face-loop scatter
+// order without atomics.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -46,20 +42,47 @@ __device__ __forceinline__ int32_t xcd_block() {
     return x * base + (x < extra ? x : extra) + q;
 }
 
-// 16-byte vectors for streaming loads of the A^-1 B blocks: 81 entries per
-// slot stored as 41 FP64 pairs (FP64 path) or 21 FP32 quads (mixed path)
+// 16-byte vectors for streaming loads
 typedef double dbl2 __attribute__((ext_vector_type(2)));
 typedef float flt4 __attribute__((ext_vector_type(4)));
-constexpr int kMPairs = 41, kMQuads = 21;
 
-// Layout of the A^-1 B stream: per slot, blocks of 64 consecutive cells,
-// and within a block the 16-byte vectors (pair e or quad q) of all 64 cells
-// contiguous, vector after vector.  A wavefront (64 cells) then reads one
-// contiguous 41 KiB (FP64) or 21 KiB (FP32) run per slot instead of 41 or 21
-// runs of 1 KiB spread over the whole array.  ldc is a multiple of 64.
-__host__ __device__ __forceinline__ int64_t m_vec_index(int s, int e, int64_t i, int64_t ldc, int nvec) {
-    return ((int64_t(s) * (ldc >> 6) + (i >> 6)) * nvec + e) * 64 + (i & 63);
+// Layouts.  Arrays with several values per cell or face are stored in blocks
+// of 64 consecutive items, so that what a wave or a workgroup reads lies
+// together: whole planes [element][item] put a cell's elements megabytes
+// apart, on as many pages and often on the same memory channels.
+//
+// blk64: within a block element after element, each as the 64 items' values
+// in a row; element k lies at blk64(i, n) + 64 k (n elements per item).
+__host__ __device__ __forceinline__ int64_t blk64(int64_t i, int n) { return (i >> 6) * (64 * int64_t(n)) + (i & 63); }
+// quad64: the same with quads of four variables (32 bytes) as elements;
+// variable v of quad e lies at quad64(i, n, e) + v.
+__host__ __device__ __forceinline__ int64_t quad64(int64_t i, int n, int e) {
+    return (i >> 6) * (256 * int64_t(n)) + 256 * e + 4 * (i & 63);
 }
+// REC arrays: the 9 coefficients of the 4 variables
+constexpr int kRec = 36;
+__host__ __device__ __forceinline__ int64_t rec(int64_t i, int r, int v) { return quad64(i, 9, r) + v; }
+
+// The stream of A^-1 B and A^-1 b: per slot and group of 16 cells, the
+// 16-byte vectors of the cells in the order in which a wave of four lanes per
+// cell loads them: vectors 4 k .. 4 k + 3 of all 16 cells (one vector per
+// lane, 1 KiB), k in turn, then the last vector of each cell (read by the
+// cell's four lanes together).  FP64: rows of 10 doubles, the 9 entries of
+// A^-1 B and the row's A^-1 b, 45 vectors; FP32 (mixed path): the 81 entries
+// of A^-1 B, 21 vectors (three pads).  ldc is a multiple of 64.
+constexpr int kAbVecs = 45, kAb32Vecs = 21;
+__host__ __device__ __forceinline__ int64_t ab_group(int s, int64_t i, int64_t ldc, int nvec) {
+    return (int64_t(s) * (ldc >> 4) + (i >> 4)) * (16 * nvec);
+}
+__host__ __device__ __forceinline__ int64_t ab_vec(int s, int e, int64_t i, int64_t ldc, int nvec) {
+    return ab_group(s, i, ldc, nvec) + (e == nvec - 1 ? 16 * e + (i & 15) : (e >> 2) * 64 + 4 * (i & 15) + (e & 3));
+}
+
+// the Wall_Euler / Wall_NoSlip faces' data, [element][ld]
+struct WallFaces {
+    const double *ainv, *d0, *nrm, *w0; // 81, 27, 6, 1 elements
+    int64_t ld;
+};
 
 struct GasParams {
     double gamma;

@@ -422,7 +422,7 @@ __global__ __launch_bounds__(256) void k_features(int32_t nc, int64_t ldc, const
         X[i0 * kIn + e] = tile[e / kIn][e % kIn];
 }
 
-// targets: converged rec coefficients x [k][ldc] (k = r + 9 v) divided by
+// targets: converged rec coefficients x (k = r + 9 v) divided by
 // s_v, rows of 36 formed in LDS and written contiguously
 __global__ __launch_bounds__(256) void k_targets(int32_t nc, int64_t ldc, const double *__restrict__ x,
                                                  const float *__restrict__ S, float *__restrict__ T) {
@@ -432,7 +432,7 @@ __global__ __launch_bounds__(256) void k_targets(int32_t nc, int64_t ldc, const 
     if (i < nc) {
 #pragma unroll
         for (int k = 0; k < kOut; k++)
-            tile[threadIdx.x][k] = float(x[k * ldc + i] / double(S[4 * int64_t(i) + k / 9]));
+            tile[threadIdx.x][k] = float(x[rec(i, k % 9, k / 9)] / double(S[4 * int64_t(i) + k / 9]));
     }
     __syncthreads();
     const int64_t nrow = min(int64_t(256), int64_t(nc) - i0);
@@ -459,9 +459,9 @@ __global__ __launch_bounds__(256) void k_unscale(int32_t nc, int64_t ldc, const 
     for (int k = 0; k < kOut; k++) {
         const double v = double(tile[threadIdx.x][k]) * double(S[4 * int64_t(i) + k / 9]);
         if (ADD)
-            x[k * ldc + i] += v;
+            x[rec(i, k % 9, k / 9)] += v;
         else
-            x[k * ldc + i] = v;
+            x[rec(i, k % 9, k / 9)] = v;
     }
 }
 
@@ -516,7 +516,7 @@ __global__ __launch_bounds__(256) void k_rec_diff2(int32_t nc, int64_t ldc, cons
     double s = 0.0;
     if (i < nc)
         for (int k = 0; k < 36; k++) {
-            const double d = a[k * ldc + i] - b[k * ldc + i];
+            const double d = a[rec(i, k % 9, k / 9)] - b[rec(i, k % 9, k / 9)];
             s += d * d;
         }
     red[threadIdx.x] = s;

@@ -549,7 +549,7 @@ int dndsmi_reconstruct_to_tolerance(dndsmi_ctx *ctx, const dndsmi_array *u, dnds
 /* Kernels of the hot path, for per-kernel timing and byte counts. */
 enum {
     DNDSMI_K_JACOBI = 0,     /* Jacobi sweep                                 */
-    DNDSMI_K_WALL_CORR = 1,  /* Wall_Euler / Wall_NoSlip correction of a sweep */
+    DNDSMI_K_WALL_CORR = 1,  /* no launches: the sweeps correct their wall cells themselves */
     DNDSMI_K_DT_FACE = 2,    /* EvaluateDt, face part                         */
     DNDSMI_K_DT_CELL = 3,    /* EvaluateDt, cell part + block minima          */
     DNDSMI_K_RHS_FACE = 4,   /* EvaluateRHS, inner-face fluxes                */
