@@ -1164,144 +1164,201 @@ __global__ __launch_bounds__(kBlock) void k_wbap_ind(int32_t nc, int64_t ldc, co
         list[base + __popcll(mask & ((1ull << lane) - 1))] = i;
 }
 
+// ---- WBAP limiting: sixteen lanes per limited cell -----------------------
+//
+// The limited cells are few (a shock's neighbourhood), so what counts is how
+// long one cell takes: with one lane per cell the face loop's chain of index
+// loads, products, eigenvectors and divisions ran once per neighbour, at one
+// wave per SIMD.  A row of 16 lanes now owns a cell, quad s of the row the
+// neighbour in slot s, lane v of the quad variable v: the neighbours' terms
+// are formed side by side and then combined in slot order by the row's first
+// quad.  The secondary matrices are stored face by face ([face][side][82]):
+// what a cell reads of them is contiguous.
+//
+// Measured against one lane per cell, a Mach-3 shock on 24 727 mixed cells:
+// V2 (three launches) 138 -> 23 us, V3 349 -> 13; on 393 734 cells 201 -> 35
+// and 487 -> 22.  With every cell limited (262 088 triangles) V2 keeps its
+// time (536, 525 us) and V3 goes from 1577 to 430.
+
+// `a` of the lane 4 q further on in the row
+template <typename T>
+__device__ __forceinline__ T row_ahead(T a, int q) { // q: a constant after unrolling
+    auto get = [&](uint32_t w) -> uint32_t {
+        return q == 0   ? w
+               : q == 1 ? uint32_t(__builtin_amdgcn_mov_dpp(int(w), 0x104, 0xf, 0xf, true))
+               : q == 2 ? uint32_t(__builtin_amdgcn_mov_dpp(int(w), 0x108, 0xf, 0xf, true))
+                        : uint32_t(__builtin_amdgcn_mov_dpp(int(w), 0x10c, 0xf, 0xf, true));
+    };
+    if constexpr (sizeof(T) == 4) {
+        return __builtin_bit_cast(T, get(__builtin_bit_cast(uint32_t, a)));
+    } else {
+        const uint64_t w = __builtin_bit_cast(uint64_t, a);
+        return __builtin_bit_cast(T, uint64_t(get(uint32_t(w))) | uint64_t(get(uint32_t(w >> 32))) << 32);
+    }
+}
+
+// entries 2 P0 .. 2 P1 + 1 of a secondary matrix, a quarter per lane
+constexpr int kSecEntries = 82; // 81 and a pad, per face and side
+constexpr unsigned kLimBlocks = 8192; // workgroups that walk the list (131 072 cells at once)
+template <int P0, int P1>
+struct SecPart {
+    static constexpr int N = (P1 - P0) / 4 + 1;
+    dbl2 w[N];
+    __device__ __forceinline__ void load(const double *__restrict__ m, int v) {
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+            w[k] = dbl2{0.0, 0.0};
+            if (P0 + 4 * k + v <= P1)
+                w[k] = reinterpret_cast<const dbl2 *>(m)[P0 + 4 * k + v];
+        }
+    }
+    __device__ __forceinline__ double get(int e) const {
+        const int p = e / 2 - P0;
+        return quad_get(e % 2 ? w[p / 4].y : w[p / 4].x, p % 4);
+    }
+};
+
+// row v of a 4 x 4 matrix
+__device__ __forceinline__ void matrix_row(const double M[16], int v, double row[4]) {
+#pragma unroll
+    for (int b = 0; b < 4; b++)
+        row[b] = v == 0 ? M[b] : v == 1 ? M[4 + b] : v == 2 ? M[8 + b] : M[12 + b];
+}
+
+// a lane's row of the face's eigenvector matrices for neighbour j of cell i
+// through face f, and the side of i
+__device__ __forceinline__ bool face_char_rows(double gamma, const double *__restrict__ u, int32_t i, int32_t j,
+                                               int32_t f, int side, int64_t ldf, const double *__restrict__ fnc, int v,
+                                               double ml[4], double mr[4]) {
+    double un0, un1;
+    stable_normalized(fnc[f], fnc[ldf + f], un0, un1);
+    const double *uLp = u + 4 * int64_t(side ? j : i), *uRp = u + 4 * int64_t(side ? i : j);
+    double UL[4], UR[4], ML[16], MR[16];
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        UL[k] = uLp[k], UR[k] = uRp[k];
+    const bool ok = char_matrices(gamma, UL, UR, un0, un1, ML, MR);
+    matrix_row(ML, v, ml);
+    matrix_row(MR, v, mr);
+    return ok;
+}
+
+// sum over the quad's lanes b of row[b] a_b, in order
+__device__ __forceinline__ double quad_dot(const double row[4], double a) {
+    double p = 0;
+#pragma unroll
+    for (int b = 0; b < 4; b++)
+        p += row[b] * quad_get(a, b);
+    return p;
+}
+
 // WBAP V3 per-order characteristic limiting of the listed cells
-// (DNDS_FV_VR.hpp:2152-2317).  Reads x, writes xo.  uF is per-cell scratch
-// holding the limited face values of rows 2..8 of the orders already done.
+// (DNDS_FV_VR.hpp:2152-2317).  Reads x, writes xo.  uF: the limited face
+// values of rows 2..8 of the orders already done.
 template <int NF>
-__global__ __launch_bounds__(kBlock) void k_wbap_lim(int64_t ldc, int64_t ldf, const int32_t *__restrict__ count,
-                                                     const int32_t *__restrict__ list,
-                                                     const int32_t *__restrict__ nbr,
-                                                     const int32_t *__restrict__ sface,
-                                                     const int32_t *__restrict__ f2c,
-                                                     const double *__restrict__ fnc,
-                                                     const double *__restrict__ msec, const double *__restrict__ u,
-                                                     const double *__restrict__ x, double *__restrict__ xo,
-                                                     double *__restrict__ uF, double gamma, double nStd, double eps4,
-                                                     int32_t *errw) {
-    const int32_t tid = blockIdx.x * blockDim.x + threadIdx.x;
-    if (tid >= count[0])
-        return;
-    const int32_t i = list[tid];
-    double ui[4];
+__global__ __launch_bounds__(kBlock, 2) void k_wbap_lim(int64_t ldc, int64_t ldf, const int32_t *__restrict__ count,
+                                                        const int32_t *__restrict__ list,
+                                                        const int32_t *__restrict__ nbr,
+                                                        const int32_t *__restrict__ sface,
+                                                        const int32_t *__restrict__ f2c,
+                                                        const double *__restrict__ fnc,
+                                                        const double *__restrict__ msec, const double *__restrict__ u,
+                                                        const double *__restrict__ x, double *__restrict__ xo,
+                                                        double gamma, double nStd, double eps4, int32_t *errw) {
+    const int s = (threadIdx.x >> 2) & 3, v = threadIdx.x & 3;
+    const int32_t n = count[0];
+    for (int32_t q = blockIdx.x * (kBlock / 16) + (threadIdx.x >> 4); q < n; q += gridDim.x * (kBlock / 16)) {
+        const int32_t i = list[q];
+        const int32_t j = s < NF ? nbr[s * ldc + i] : -1;
+        const bool valid = j >= 0;
+        double own[9], xj[9], uF[7], ml[4], mr[4];
+        SecPart<0, 40> ms, msO;
 #pragma unroll
-    for (int v = 0; v < 4; v++)
-        ui[v] = u[4 * int64_t(i) + v];
-    bool ok = true;
-#pragma unroll
-    for (int order = 3; order >= 1; order--) {
-        const int ls = order == 3 ? 5 : (order == 2 ? 2 : 0);
-        const int le = order == 3 ? 8 : (order == 2 ? 4 : 1);
-        constexpr int kMaxR = 4;
-        const int nr = le - ls + 1;
-        double u0[kMaxR][4], up[kMaxR][4], down[kMaxR][4];
-#pragma unroll
-        for (int r = 0; r < kMaxR; r++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                u0[r][v] = r < nr ? x[rec(i, ls + r, v)] : 0.0;
-                up[r][v] = 0.0, down[r][v] = 0.0;
-            }
-#pragma unroll 1
-        for (int s = 0; s < NF; s++) {
-            const int32_t j = nbr[s * ldc + i];
-            if (j < 0)
-                continue;
+        for (int r = 0; r < 9; r++)
+            own[r] = x[rec(i, r, v)];
+        if (valid) {
             const int32_t f = sface[s * ldc + i];
             const int side = f2c[f] == i ? 0 : 1;
-            double un0, un1;
-            stable_normalized(fnc[f], fnc[ldf + f], un0, un1);
-            const double *ms = msec + blk64(f, 162) + 64 * (81 * side);
-            const double *msO = msec + blk64(f, 162) + 64 * (81 * (1 - side));
-            double oIn[kMaxR][4];
+            const double *m = msec + 2 * kSecEntries * int64_t(f);
+            ms.load(m + kSecEntries * side, v);
+            msO.load(m + kSecEntries * (1 - side), v);
+#pragma unroll
+            for (int c = 0; c < 9; c++)
+                xj[c] = x[rec(j, c, v)];
+            if (!face_char_rows(gamma, u, i, j, f, side, ldf, fnc, v, ml, mr))
+                atomicOr(errw, ERRBIT_NONPOSITIVE);
+        }
+#pragma unroll
+        for (int order = 3; order >= 1; order--) {
+            const int ls = order == 3 ? 5 : (order == 2 ? 2 : 0);
+            const int le = order == 3 ? 8 : (order == 2 ? 4 : 1);
+            constexpr int kMaxR = 4;
+            const int nr = le - ls + 1;
+            double up[kMaxR], down[kMaxR]; // this neighbour's terms
 #pragma unroll
             for (int r = 0; r < kMaxR; r++)
-#pragma unroll
-                for (int v = 0; v < 4; v++)
-                    oIn[r][v] = 0.0;
-            // uOtherOther rows: the neighbour's coefficients up to le, above le
-            // the limited face values of the higher orders mapped to its basis
-#pragma unroll
-            for (int c = 0; c < 9; c++) {
-                double uoo[4];
-                if (c <= le) {
-#pragma unroll
-                    for (int v = 0; v < 4; v++)
-                        uoo[v] = x[rec(j, c, v)];
-                } else {
-#pragma unroll
-                    for (int v = 0; v < 4; v++) {
-                        double acc = 0;
-#pragma unroll
-                        for (int cc = le + 1; cc < 9; cc++)
-                            acc += msO[64 * (9 * c + cc)] * uF[quad64(i, 7 * NF, s * 7 + (cc - 2)) + v];
-                        uoo[v] = acc;
-                    }
-                }
+                up[r] = down[r] = 0.0;
+            if (valid) {
+                double oIn[kMaxR];
 #pragma unroll
                 for (int r = 0; r < kMaxR; r++)
-                    if (r < nr) {
-                        const double m = ms[64 * (9 * (ls + r) + c)];
+                    oIn[r] = 0.0;
+                // uOtherOther rows: the neighbour's coefficients up to le, above
+                // le the limited face values of the higher orders mapped to its
+                // basis
 #pragma unroll
-                        for (int v = 0; v < 4; v++)
-                            oIn[r][v] += m * uoo[v];
+                for (int c = 0; c < 9; c++) {
+                    double uoo = xj[c];
+                    if (c > le) {
+                        uoo = 0;
+#pragma unroll
+                        for (int cc = 0; cc < 9; cc++)
+                            if (cc > le)
+                                uoo += msO.get(9 * c + cc) * uF[cc - 2];
                     }
-            }
-            const double *uLp = side ? u + 4 * int64_t(j) : ui;
-            const double *uRp = side ? ui : u + 4 * int64_t(j);
-            double UL[4], UR[4];
 #pragma unroll
-            for (int v = 0; v < 4; v++)
-                UL[v] = uLp[v], UR[v] = uRp[v];
-            double ML[16], MR[16];
-            ok &= char_matrices(gamma, UL, UR, un0, un1, ML, MR);
+                    for (int r = 0; r < kMaxR; r++)
+                        if (r < nr)
+                            oIn[r] += ms.get(9 * (ls + r) + c) * uoo;
+                }
+#pragma unroll
+                for (int r = 0; r < kMaxR; r++) {
+                    if (r >= nr)
+                        continue;
+                    const double u0 = own[ls + r];
+                    const double oC = quad_dot(ml, oIn[r]), tC = quad_dot(ml, u0);
+                    // FWBAP_L2_Biway(uThisIn, uOtherIn, 1)
+                    const double frac = tC / (fabs(oC) + 1e-12) * sgn(oC);
+                    const double th1 = frac * frac * frac;
+                    const double th2 = (frac * frac) * (frac * frac);
+                    const double xv = quad_dot(mr, tC * (1.0 + th1) / (1.0 + th2));
+                    if (ls + r >= 2)
+                        uF[ls + r - 2] = xv;
+                    // FWBAP_L2_Multiway's terms
+                    const double ti = u0 / (fabs(xv) + eps4) * sgn(xv);
+                    down[r] = (ti * ti) * (ti * ti);
+                    up[r] = ti * ti * ti;
+                }
+            }
+            // the neighbours in cell2face order, in the row's first quad
 #pragma unroll
             for (int r = 0; r < kMaxR; r++) {
                 if (r >= nr)
                     continue;
-                double oC[4], tC[4], out[4];
+                double sd = 0.0, su = 0.0;
 #pragma unroll
-                for (int a = 0; a < 4; a++) {
-                    double p = 0, q = 0;
-#pragma unroll
-                    for (int b = 0; b < 4; b++) {
-                        p += ML[4 * a + b] * oIn[r][b];
-                        q += ML[4 * a + b] * u0[r][b];
+                for (int t = 0; t < NF; t++) {
+                    const double d = row_ahead(down[r], t), p = row_ahead(up[r], t);
+                    if (row_ahead(int(valid), t)) {
+                        sd += d;
+                        su += p;
                     }
-                    oC[a] = p, tC[a] = q;
                 }
-                // FWBAP_L2_Biway(uThisIn, uOtherIn, 1)
-#pragma unroll
-                for (int a = 0; a < 4; a++) {
-                    const double u1 = tC[a], u2 = oC[a];
-                    const double frac = u1 / (fabs(u2) + 1e-12) * sgn(u2);
-                    const double th1 = frac * frac * frac;
-                    const double th2 = (frac * frac) * (frac * frac);
-                    out[a] = u1 * (1.0 + th1) / (1.0 + th2);
-                }
-#pragma unroll
-                for (int a = 0; a < 4; a++) {
-                    double xv = 0;
-#pragma unroll
-                    for (int b = 0; b < 4; b++)
-                        xv += MR[4 * a + b] * out[b];
-                    if (ls + r >= 2)
-                        uF[quad64(i, 7 * NF, s * 7 + (ls + r - 2)) + a] = xv;
-                    // FWBAP_L2_Multiway accumulation, neighbours in cell2face order
-                    const double ti = u0[r][a] / (fabs(xv) + eps4) * sgn(xv);
-                    down[r][a] += (ti * ti) * (ti * ti);
-                    up[r][a] += ti * ti * ti;
-                }
+                if (s == 0)
+                    xo[rec(i, ls + r, v)] = own[ls + r] * (su + nStd) / (sd + nStd);
             }
         }
-#pragma unroll
-        for (int r = 0; r < kMaxR; r++)
-            if (r < nr)
-#pragma unroll
-                for (int v = 0; v < 4; v++)
-                    xo[rec(i, ls + r, v)] = u0[r][v] * (up[r][v] + nStd) / (down[r][v] + nStd);
     }
-    if (!ok)
-        atomicOr(errw, ERRBIT_NONPOSITIVE);
 }
 
 // WBAP V2 limiting of the listed cells for one order (DNDS_FV_VR.hpp:1843-2040,
@@ -1314,126 +1371,83 @@ __global__ __launch_bounds__(kBlock) void k_wbap_lim(int64_t ldc, int64_t ldf, c
 // what another writes.  FWBAP_L2_Biway with n = nStd per neighbour, then
 // FWBAP_L2_Multiway centred on the first neighbour's result with n1 = 1.
 template <int NF, int ORDER>
-__global__ __launch_bounds__(kBlock) void k_wbap_lim_v2(int64_t ldc, int64_t ldf, const int32_t *__restrict__ count,
-                                                        const int32_t *__restrict__ list,
-                                                        const int32_t *__restrict__ nbr,
-                                                        const int32_t *__restrict__ sface,
-                                                        const int32_t *__restrict__ f2c,
-                                                        const double *__restrict__ fnc,
-                                                        const double *__restrict__ msec,
-                                                        const double *__restrict__ u, const double *__restrict__ x,
-                                                        double *__restrict__ xo, double gamma, double nStd,
-                                                        double eps4, int32_t *errw,
-                                                        const uint8_t *__restrict__ limf) {
+__global__ __launch_bounds__(kBlock, 3) void k_wbap_lim_v2(int64_t ldc, int64_t ldf, const int32_t *__restrict__ count,
+                                                           const int32_t *__restrict__ list,
+                                                           const int32_t *__restrict__ nbr,
+                                                           const int32_t *__restrict__ sface,
+                                                           const int32_t *__restrict__ f2c,
+                                                           const double *__restrict__ fnc,
+                                                           const double *__restrict__ msec,
+                                                           const double *__restrict__ u, const double *__restrict__ x,
+                                                           double *__restrict__ xo, double gamma, double nStd,
+                                                           double eps4, int32_t *errw,
+                                                           const uint8_t *__restrict__ limf) {
     constexpr int ls = ORDER == 3 ? 5 : (ORDER == 2 ? 2 : 0);
     constexpr int le = ORDER == 3 ? 8 : (ORDER == 2 ? 4 : 1);
     constexpr int nr = le - ls + 1;
-    const int32_t tid = blockIdx.x * blockDim.x + threadIdx.x;
-    if (tid >= count[0])
-        return;
-    const int32_t i = list[tid];
-    double ui[4];
-#pragma unroll
-    for (int v = 0; v < 4; v++)
-        ui[v] = u[4 * int64_t(i) + v];
-    double uC[nr][4], first[nr][4], up[nr][4], down[nr][4];
-#pragma unroll
-    for (int r = 0; r < nr; r++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            uC[r][v] = x[rec(i, ls + r, v)];
-            first[r][v] = 0.0, up[r][v] = 0.0, down[r][v] = 0.0;
-        }
-    bool ok = true;
-    int nOther = 0;
-#pragma unroll 1
-    for (int s = 0; s < NF; s++) {
-        const int32_t j = nbr[s * ldc + i];
-        if (j < 0)
-            continue;
-        const int32_t f = sface[s * ldc + i];
-        const int side = f2c[f] == i ? 0 : 1;
-        double un0, un1;
-        stable_normalized(fnc[f], fnc[ldf + f], un0, un1);
-        const double *ms = msec + blk64(f, 162) + 64 * (81 * side);
-        // the neighbour's rows above le: limited (xo) or, with limf, as given (x)
-        const double *above = (limf && !limf[j]) ? x : xo;
-        double oIn[nr][4];
-#pragma unroll
-        for (int r = 0; r < nr; r++)
-#pragma unroll
-            for (int v = 0; v < 4; v++)
-                oIn[r][v] = 0.0;
-#pragma unroll
-        for (int c = 0; c < 9; c++) {
-            const double *src = c <= le ? x : above;
-            double uj[4];
-#pragma unroll
-            for (int v = 0; v < 4; v++)
-                uj[v] = src[rec(j, c, v)];
-#pragma unroll
-            for (int r = 0; r < nr; r++) {
-                const double m = ms[64 * (9 * (ls + r) + c)];
-#pragma unroll
-                for (int v = 0; v < 4; v++)
-                    oIn[r][v] += m * uj[v];
-            }
-        }
-        const double *uLp = side ? u + 4 * int64_t(j) : ui;
-        const double *uRp = side ? ui : u + 4 * int64_t(j);
-        double UL[4], UR[4];
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-            UL[v] = uLp[v], UR[v] = uRp[v];
-        double ML[16], MR[16];
-        ok &= char_matrices(gamma, UL, UR, un0, un1, ML, MR);
+    const int s = (threadIdx.x >> 2) & 3, v = threadIdx.x & 3;
+    const int32_t n = count[0];
+    for (int32_t q = blockIdx.x * (kBlock / 16) + (threadIdx.x >> 4); q < n; q += gridDim.x * (kBlock / 16)) {
+        const int32_t i = list[q];
+        const int32_t j = s < NF ? nbr[s * ldc + i] : -1;
+        const bool valid = j >= 0;
+        double uC[nr], xv[nr];
 #pragma unroll
         for (int r = 0; r < nr; r++) {
-            double oC[4], tC[4], out[4];
+            uC[r] = x[rec(i, ls + r, v)];
+            xv[r] = 0.0;
+        }
+        if (valid) {
+            const int32_t f = sface[s * ldc + i];
+            const int side = f2c[f] == i ? 0 : 1;
+            SecPart<9 * ls / 2, (9 * le + 8) / 2> ms;
+            ms.load(msec + kSecEntries * (2 * int64_t(f) + side), v);
+            // the neighbour's rows above le: limited (xo) or, with limf, as given (x)
+            const double *above = (limf && !limf[j]) ? x : xo;
+            double uj[9];
 #pragma unroll
-            for (int a = 0; a < 4; a++) {
-                double p = 0, q = 0;
+            for (int c = 0; c < 9; c++)
+                uj[c] = (c <= le ? x : above)[rec(j, c, v)];
+            double ml[4], mr[4];
+            if (!face_char_rows(gamma, u, i, j, f, side, ldf, fnc, v, ml, mr))
+                atomicOr(errw, ERRBIT_NONPOSITIVE);
 #pragma unroll
-                for (int b = 0; b < 4; b++) {
-                    p += ML[4 * a + b] * oIn[r][b];
-                    q += ML[4 * a + b] * uC[r][b];
-                }
-                oC[a] = p, tC[a] = q;
-            }
-            // FWBAP_L2_Biway(uThisIn, uOtherIn, nStd)
+            for (int r = 0; r < nr; r++) {
+                double oIn = 0.0;
 #pragma unroll
-            for (int a = 0; a < 4; a++) {
-                const double u1 = tC[a], u2 = oC[a];
-                const double frac = u1 / (fabs(u2) + 1e-12) * sgn(u2);
+                for (int c = 0; c < 9; c++)
+                    oIn += ms.get(9 * (ls + r) + c) * uj[c];
+                const double oC = quad_dot(ml, oIn), tC = quad_dot(ml, uC[r]);
+                // FWBAP_L2_Biway(uThisIn, uOtherIn, nStd)
+                const double frac = tC / (fabs(oC) + 1e-12) * sgn(oC);
                 const double th1 = frac * frac * frac;
                 const double th2 = (frac * frac) * (frac * frac);
-                out[a] = u1 * (nStd + th1) / (nStd + th2);
-            }
-#pragma unroll
-            for (int a = 0; a < 4; a++) {
-                double xv = 0;
-#pragma unroll
-                for (int b = 0; b < 4; b++)
-                    xv += MR[4 * a + b] * out[b];
-                if (nOther == 0) {
-                    first[r][a] = xv;
-                } else {
-                    const double ti = first[r][a] / (fabs(xv) + eps4) * sgn(xv);
-                    down[r][a] += (ti * ti) * (ti * ti);
-                    up[r][a] += ti * ti * ti;
-                }
+                xv[r] = quad_dot(mr, tC * (nStd + th1) / (nStd + th2));
             }
         }
-        nOther++;
+        // the neighbours in cell2face order, in the row's first quad
+#pragma unroll
+        for (int r = 0; r < nr; r++) {
+            double first = 0.0, up = 0.0, down = 0.0;
+            bool any = false;
+#pragma unroll
+            for (int t = 0; t < NF; t++) {
+                const double a = row_ahead(xv[r], t);
+                if (!row_ahead(int(valid), t))
+                    continue;
+                if (!any) {
+                    first = a;
+                } else {
+                    const double ti = first / (fabs(a) + eps4) * sgn(a);
+                    down += (ti * ti) * (ti * ti);
+                    up += ti * ti * ti;
+                }
+                any = true;
+            }
+            if (s == 0)
+                xo[rec(i, ls + r, v)] = any ? first * (up + 1.0) / (down + 1.0) : uC[r];
+        }
     }
-#pragma unroll
-    for (int r = 0; r < nr; r++)
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-            xo[rec(i, ls + r, v)] =
-                nOther ? first[r][v] * (up[r][v] + 1.0) / (down[r][v] + 1.0) : uC[r][v];
-    if (!ok)
-        atomicOr(errw, ERRBIT_NONPOSITIVE);
 }
 
 __global__ void k_zero_int2(int32_t *p) {
@@ -1563,10 +1577,10 @@ extern "C" int dndsmi_ctx_create(const dndsmi_mesh_view *mesh, const dndsmi_vr_v
         //
         // With SOR_Instead the numbering is colour-major instead: each colour
         // is a contiguous range (its cells in mesh order), so that a colour's
-        // pass streams whole lines of the A^-1 B pairs and coefficients; in
+        // pass streams whole lines of the A^-1 B stream and the coefficients; in
         // each colour the cells with terms on their own partial sum (far
-        // field, Wall_Euler, Wall_NoSlip) come last and take their own kernel
-        // variant.  The windows of 64 then start at each range's start.
+        // field, Wall_Euler, Wall_NoSlip) come last, so that their longer
+        // waves are few.  The windows of 64 then start at each range's start.
         //
         // Colouring (multicolour LU-SGS and SOR): each cell takes the
         // smallest colour that no lower-numbered neighbour holds.
@@ -1610,9 +1624,8 @@ extern "C" int dndsmi_ctx_create(const dndsmi_mesh_view *mesh, const dndsmi_vr_v
                 for (int64_t i = 0; i < nc; i++)
                     seq[fill[2 * col[i] + self[size_t(i)]]++] = i;
                 c->sor_start.assign(size_t(ncol) + 1, nc);
-                c->sor_wall.assign(size_t(ncol), nc);
                 for (int32_t k = 0; k < ncol; k++)
-                    c->sor_start[k] = cnt[2 * k], c->sor_wall[k] = cnt[2 * k + 1];
+                    c->sor_start[k] = cnt[2 * k];
             } else {
                 for (int64_t i = 0; i < nc; i++)
                     seq[i] = i;
@@ -1812,11 +1825,11 @@ extern "C" int dndsmi_ctx_create(const dndsmi_mesh_view *mesh, const dndsmi_vr_v
         if (vr->matrix_secondary) {
             c->has_limiter = true;
             std::vector<double> buf;
-            buf.assign(162 * size_t(ldf), 0.0);
+            buf.assign(2 * kSecEntries * size_t(ldf), 0.0);
             for (int64_t f = 0; f < nf; f++)
                 for (int k = 0; k < 162; k++)
-                    buf[blk64(f2d[f], 162) + 64 * k] = vr->matrix_secondary[162 * f + k];
-            DNDSMI_TRY(c->alloc(c->msec, 162 * ldf));
+                    buf[kSecEntries * (2 * size_t(f2d[f]) + k / 81) + k % 81] = vr->matrix_secondary[162 * f + k];
+            DNDSMI_TRY(c->alloc(c->msec, 2 * kSecEntries * ldf));
             DNDSMI_TRY(c->upload(c->msec, buf));
             buf.assign(10 * size_t(ldf), 0.0);
             for (int64_t f = 0; f < nf; f++)
@@ -1825,7 +1838,6 @@ extern "C" int dndsmi_ctx_create(const dndsmi_mesh_view *mesh, const dndsmi_vr_v
             DNDSMI_TRY(c->alloc(c->fw, 10 * ldf));
             DNDSMI_TRY(c->upload(c->fw, buf));
             DNDSMI_TRY(c->alloc(c->wslot, int64_t(nfmax) * 4 * ldc));
-            DNDSMI_TRY(c->alloc(c->uF, int64_t(nfmax) * 28 * ldc));
             DNDSMI_TRY(c->alloc(c->ind, ldc));
             DNDSMI_TRY(c->alloc(c->xlim, 36 * ldc));
             DNDSMI_TRY(c->alloc(c->limf, ldc));
@@ -2168,33 +2180,23 @@ int launch_wbap(dndsmi_ctx *c, const double *u, const double *x, double *xo, dou
                            full_copy ? nullptr : c->limf);
     prof_end(c);
     prof_begin(c, DNDSMI_K_WBAP_LIM);
+    // rows of 16 lanes walk the list, whose length only the device knows
+    const dim3 grid(std::min(grid_for(16 * int64_t(nc)), kLimBlocks));
     if (procedure == 1) {
-        if (c->nfmax == 3)
-            hipLaunchKernelGGL(k_wbap_lim<3>, dim3(grid_for(nc)), dim3(kBlock), 0, c->stream, c->ldc, c->ldf,
-                               c->lim_count, c->lim_list, c->nbr, c->sface, c->f2c, c->fnc, c->msec, u, x, xo, c->uF,
-                               c->gas.gamma, c->wbap_nstd, eps4, c->errw);
-        else
-            hipLaunchKernelGGL(k_wbap_lim<4>, dim3(grid_for(nc)), dim3(kBlock), 0, c->stream, c->ldc, c->ldf,
-                               c->lim_count, c->lim_list, c->nbr, c->sface, c->f2c, c->fnc, c->msec, u, x, xo, c->uF,
-                               c->gas.gamma, c->wbap_nstd, eps4, c->errw);
+        hipLaunchKernelGGL((c->nfmax == 3 ? k_wbap_lim<3> : k_wbap_lim<4>), grid, dim3(kBlock), 0, c->stream, c->ldc,
+                           c->ldf, c->lim_count, c->lim_list, c->nbr, c->sface, c->f2c, c->fnc, c->msec, u, x, xo,
+                           c->gas.gamma, c->wbap_nstd, eps4, c->errw);
     } else {
         // orders 3, 2, 1 in stream order: each launch reads the rows the
         // previous ones wrote
-        auto order = [&](auto nf_c, auto order_c) {
-            constexpr int NF = decltype(nf_c)::value, O = decltype(order_c)::value;
-            hipLaunchKernelGGL((k_wbap_lim_v2<NF, O>), dim3(grid_for(nc)), dim3(kBlock), 0, c->stream, c->ldc,
-                               c->ldf, c->lim_count, c->lim_list, c->nbr, c->sface, c->f2c, c->fnc, c->msec, u, x,
-                               xo, c->gas.gamma, c->wbap_nstd, eps4, c->errw, full_copy ? nullptr : c->limf);
+        auto order = [&](auto kern) {
+            hipLaunchKernelGGL(kern, grid, dim3(kBlock), 0, c->stream, c->ldc, c->ldf, c->lim_count, c->lim_list,
+                               c->nbr, c->sface, c->f2c, c->fnc, c->msec, u, x, xo, c->gas.gamma, c->wbap_nstd, eps4,
+                               c->errw, full_copy ? nullptr : c->limf);
         };
-        using I3 = std::integral_constant<int, 3>;
-        using I4 = std::integral_constant<int, 4>;
-        using O3 = std::integral_constant<int, 3>;
-        using O2 = std::integral_constant<int, 2>;
-        using O1 = std::integral_constant<int, 1>;
-        if (c->nfmax == 3)
-            order(I3{}, O3{}), order(I3{}, O2{}), order(I3{}, O1{});
-        else
-            order(I4{}, O3{}), order(I4{}, O2{}), order(I4{}, O1{});
+        order(c->nfmax == 3 ? k_wbap_lim_v2<3, 3> : k_wbap_lim_v2<4, 3>);
+        order(c->nfmax == 3 ? k_wbap_lim_v2<3, 2> : k_wbap_lim_v2<4, 2>);
+        order(c->nfmax == 3 ? k_wbap_lim_v2<3, 1> : k_wbap_lim_v2<4, 1>);
     }
     prof_end(c);
     return c->launch_check("wbap kernels");

@@ -40,9 +40,8 @@ struct dndsmi_ctx {
     // the multicolour scan (col_cells), forward (then backward)
     bool sor = false, sor_inverse = false;
     // SOR_Instead (colour-major device numbering): colour k holds the device
-    // cells [sor_start[k], sor_start[k + 1]), those with a far-field,
-    // Wall_Euler or Wall_NoSlip face from sor_wall[k] on
-    std::vector<int64_t> sor_start, sor_wall;
+    // cells [sor_start[k], sor_start[k + 1])
+    std::vector<int64_t> sor_start;
     int64_t bytes = 0;
     std::vector<void *> allocs;
     // live arrays and other objects bound to this context, detached when it
@@ -84,10 +83,9 @@ struct dndsmi_ctx {
     // WBAP data (present when the setup carries limiter data)
     bool has_limiter = false;
     double *fw = nullptr;      // [10] face weights
-    double *msec = nullptr;    // [162] matrixSecondary (R2L, L2R)
+    double *msec = nullptr;    // [face][R2L, L2R][82] matrixSecondary
     double *wslot = nullptr;   // [nfmax] quads: indicator terms of the cell's faces, cell2face slot order
     uint8_t *wpos = nullptr;   // [ldf] the face's cell2face slot in cell L (low 4 bits) and in cell R (high)
-    double *uF = nullptr;      // [nfmax * 7] quads: WBAP per-cell face scratch
     double *ind = nullptr;     // [ldc] indicator when the caller passes none
     double *xlim = nullptr;    // REC layout: limited reconstruction inside SSP-RK3 steps (limited cells only)
     uint8_t *limf = nullptr;   // [ldc] 1 where the steps' limiter wrote the cell into xlim

@@ -1,0 +1,73 @@
+"""The lane groups of the sweeps (four lanes per cell, 16 cells per wave) and
+of the limiter (16 lanes per cell) at their edges, against the oracle: cell
+counts around a group, a wave and a workgroup's worth of cells, the counts
+where the workgroup size changes, and more limited cells than the limiter's
+grid holds at once.  All of it is FP64 in the oracle's operation order, so the
+tolerance is that of the other FP64 parity tests."""
+import numpy as np
+import pytest
+
+from conftest import rel_err
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-12
+
+
+def _case(kind, nx, ny, sor=0, limiter=0, seed=3):
+    from dnds_amd import _capi as A
+    from dnds_amd.host import RIEMANN_VR_SETTING, CompactFacedMeshSerialRW, VRFiniteVolume2D, vr_setting
+    bcs = (A.BC_FARFIELD, A.BC_WALL_NOSLIP, A.BC_WALL_EULER, A.BC_WALL)
+    mesh = CompactFacedMeshSerialRW.generate(kind, nx, ny, 0.0, 1.0, 0.0, ny / nx, jitter=0.2, seed=seed, bc=bcs)
+    vfv = VRFiniteVolume2D(mesh, vr_setting(**dict(RIEMANN_VR_SETTING, far_weight=1.0, jacobi_relax=0.9),
+                                            build_limiter_data=limiter, sor_instead=sor))
+    vfv.Initialization(8)
+    return mesh, vfv
+
+
+def _state(n, seed):
+    rng = np.random.default_rng(seed)
+    rho, vx, vy, p = 1 + 0.3 * rng.random(n), 0.4 * rng.random(n), -0.3 * rng.random(n), 1 + 0.2 * rng.random(n)
+    u = np.stack([rho, rho * vx, rho * vy, p / 0.4 + 0.5 * rho * (vx * vx + vy * vy)], 1)
+    return u, 1e-2 * rng.standard_normal((n, 36))
+
+
+def _oracle(mesh, vfv, far):
+    import oracle
+    st = vfv.setting
+    return oracle.Oracle(mesh.arrays(), vfv.arrays(), riemann_solver=2, far_field=far, jacobi_relax=st.jacobi_relax,
+                         tang_weight=st.tang_weight, tang_weight_direction=st.tang_weight_direction,
+                         wbap_smooth_indicator_scale=st.wbap_smooth_indicator_scale)
+
+
+FAR = (1.1, 0.3, -0.1, 2.8)
+
+
+@pytest.mark.parametrize("kind,nx,ny", [(0, 1, 1), (1, 3, 5), (1, 4, 4), (1, 17, 1), (0, 4, 8), (1, 5, 13), (2, 9, 11),
+                                        (1, 273, 274), (1, 274, 274), (2, 224, 224)])
+def test_sweep_at_group_and_workgroup_edges(kind, nx, ny):
+    from dnds_amd.host import EulerEvaluator
+    mesh, vfv = _case(kind, nx, ny)
+    ev = EulerEvaluator(mesh, vfv, riemannSolverType="HLLC", farFieldStaticValue=FAR)
+    u, x = _state(mesh.n_cell, 5)
+    du, dx, dn = ev.BuildMean().upload(u), vfv.BuildRec().upload(x), vfv.BuildRec()
+    vfv.ReconstructionJacobiStep(du, dx, dn, 0.0)
+    ref = _oracle(mesh, vfv, FAR).jacobi_step(u, x)
+    assert rel_err(dn.download(), ref) <= TOL
+    assert rel_err(dx.download(), ref) <= TOL
+    ev.device.sync()
+
+
+@pytest.mark.parametrize("procedure", [2, 3])
+def test_more_limited_cells_than_the_grid_holds(procedure):
+    from dnds_amd.host import EulerEvaluator
+    mesh, vfv = _case(2, 304, 304, limiter=1)  # about 138 000 cells, 131 072 at once
+    assert mesh.n_cell > 131072
+    ev = EulerEvaluator(mesh, vfv, riemannSolverType="HLLC", farFieldStaticValue=FAR)
+    u, x = _state(mesh.n_cell, 6)
+    du, dx, dn = ev.BuildMean().upload(u), vfv.BuildRec().upload(x), vfv.BuildRec()
+    limit = vfv.ReconstructionWBAPLimitFacialV3 if procedure == 3 else vfv.ReconstructionWBAPLimitFacialV2
+    limit(du, dx, dn, ifAll=True)
+    orc = _oracle(mesh, vfv, FAR)
+    ref, _ = (orc.wbap_v3 if procedure == 3 else orc.wbap_v2)(u, x, if_all=True)
+    assert rel_err(dn.download(), ref) <= TOL
