@@ -136,35 +136,55 @@ __device__ __forceinline__ void ab_apply(const AbPart &ab, const double xj[9], d
     }
 }
 
-// Boundary correction of Wall_Euler / Wall_NoSlip face w to its cell's sweep
+// doubles 2 P0 .. 2 P1 + 1 of a contiguous run, a quarter per lane of the quad
+template <int P0, int P1>
+struct QuadPart {
+    static constexpr int N = (P1 - P0) / 4 + 1;
+    dbl2 w[N];
+    __device__ __forceinline__ void load(const double *__restrict__ m, int v) {
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+            w[k] = dbl2{0.0, 0.0};
+            if (P0 + 4 * k + v <= P1)
+                w[k] = reinterpret_cast<const dbl2 *>(m)[P0 + 4 * k + v];
+        }
+    }
+    __device__ __forceinline__ double get(int e) const {
+        const int p = e / 2 - P0;
+        return quad_get(e % 2 ? w[p / 4].y : w[p / 4].x, p % 4);
+    }
+};
+
+// Boundary correction of a Wall_Euler / Wall_NoSlip face to its cell's sweep
 // (DNDS_FV_VR.hpp:1577-1657), from the cell's coefficients xi and mean ui of
 // this lane's variable v: out = relax A^-1 sum_g w_g |n_g| D0^T W0^2 (uBV -
 // u_i).  The four lanes of the cell's quad call it together.
-__device__ __forceinline__ void wall_correction(int32_t w, int32_t bc, const double xi[9], double ui, int v,
-                                                const WallFaces &wf, double relax, int32_t *errw, double out[9]) {
+__device__ __forceinline__ void wall_correction(int32_t slot, const double xi[9], double ui, int v,
+                                                const double *__restrict__ walls, double relax, int32_t *errw,
+                                                double out[9]) {
+    const double *wd = walls + kWallEntries * int64_t(wall_of(slot));
+    QuadPart<0, 40> ainv;
+    QuadPart<0, 13> d0;
+    d0.load(wd + kWallD0, v);
     double BCc[9];
 #pragma unroll
     for (int r = 0; r < 9; r++)
         BCc[r] = 0.0;
-    const double w0 = wf.w0[w];
-#pragma unroll 1
+    const double w0 = wd[kWallW0];
+#pragma unroll
     for (int g = 0; g < 3; g++) {
         const double gw = g == 1 ? kLine3W1 : kLine3W0;
-        const double nx = wf.nrm[(2 * g) * wf.ld + w], ny = wf.nrm[(2 * g + 1) * wf.ld + w];
-        double d0[9];
-#pragma unroll
-        for (int c = 0; c < 9; c++)
-            d0[c] = wf.d0[(g * 9 + c) * wf.ld + w];
+        const double nx = wd[kWallNrm + 2 * g], ny = wd[kWallNrm + 2 * g + 1];
         double uB = 0;
 #pragma unroll
         for (int c = 0; c < 9; c++)
-            uB += d0[c] * xi[c];
+            uB += d0.get(9 * g + c) * xi[c];
         uB += ui;
         double n0, n1;
         stable_normalized(nx, ny, n0, n1);
         const double rho = quad_bcast<0>(uB), m0 = quad_bcast<1>(uB), m1 = quad_bcast<2>(uB);
         double uBV = uB;
-        if (bc == BC_WALL_EULER) {
+        if (!wall_noslip(slot)) {
             const double dd = n0 * m0 + n1 * m1;
             if (v == 1)
                 uBV = uB - n0 * dd;
@@ -178,17 +198,18 @@ __device__ __forceinline__ void wall_correction(int32_t w, int32_t bc, const dou
         const double nl = sqrt(nx * nx + ny * ny);
 #pragma unroll
         for (int r = 0; r < 9; r++) {
-            double inc = d0[r] * w0 * w0 * (uBV - ui);
+            double inc = d0.get(9 * g + r) * w0 * w0 * (uBV - ui);
             inc *= nl;
             BCc[r] += inc * gw;
         }
     }
+    ainv.load(wd, v);
 #pragma unroll
     for (int r = 0; r < 9; r++) {
         double acc = 0;
 #pragma unroll
         for (int c = 0; c < 9; c++)
-            acc += wf.ainv[(r * 9 + c) * wf.ld + w] * BCc[c];
+            acc += ainv.get(9 * r + c) * BCc[c];
         out[r] = relax * acc;
     }
 }
@@ -211,11 +232,10 @@ __device__ __forceinline__ int64_t rec_group(int32_t i) {
 // The cells are the device range [base, base + n): with SOR_Instead the
 // device numbering is colour-major.  x and xo are the same array.
 template <int NF>
-__global__ __launch_bounds__(kBlock, 2) void k_sor(int32_t n, int32_t base, int64_t ldc,
+__global__ __launch_bounds__(kBlock, 3) void k_sor(int32_t n, int32_t base, int64_t ldc,
                                                    const int32_t *__restrict__ nbr, const int32_t *__restrict__ sbc,
-                                                   const int32_t *__restrict__ wall_idx,
                                                    const double *__restrict__ M, const double *__restrict__ u,
-                                                   const double *x, double *xo, double relax, WallFaces wf,
+                                                   const double *x, double *xo, double relax, const double *__restrict__ walls,
                                                    int32_t *errw) {
     const int32_t t = xcd_block() * blockDim.x + threadIdx.x, v = t & 3;
     // whole groups of 16 cells from the one that holds `base`
@@ -247,17 +267,19 @@ __global__ __launch_bounds__(kBlock, 2) void k_sor(int32_t n, int32_t base, int6
             ab_apply(ab, xj, u[4 * int64_t(j) + v] - ui, 1.0, relax, nw);
             continue;
         }
+        if (is_wall_slot(j)) {
+            double cw[9];
+            wall_correction(j, nw, ui, v, walls, relax, errw, cw);
+#pragma unroll
+            for (int r = 0; r < 9; r++)
+                nw[r] += cw[r];
+            continue;
+        }
         const int32_t bc = sbc[s * ldc + i];
         if (bc == BC_WALL) {
 #pragma unroll
             for (int r = 0; r < 9; r++)
                 nw[r] += relax * ((0.0 - ui) * ab.get(10 * r + 9));
-        } else if (bc == BC_WALL_EULER || bc == BC_WALL_NOSLIP) {
-            double cw[9];
-            wall_correction(wall_idx[s * ldc + i], bc, nw, ui, v, wf, relax, errw, cw);
-#pragma unroll
-            for (int r = 0; r < 9; r++)
-                nw[r] += cw[r];
         } else if (is_far(bc)) {
             // M_if times the partial sum, no mean-value term
             double own[9];
@@ -283,61 +305,80 @@ __global__ __launch_bounds__(kBlock, 2) void k_sor(int32_t n, int32_t base, int6
 // RESID (the FP64 step of the mixed-precision sweeps): instead of the new
 // iterate, writes the increment r = J(x) - x rounded to FP32 into r32 (also the
 // start of the FP32 correction sweeps, k_delta32).
-template <int NF, bool RESID>
-__global__ __launch_bounds__(kBlock, 2) void k_jacobi(int32_t nc, int64_t ldc, const int32_t *__restrict__ nbr,
+template <int NF, bool RESID, bool TILE>
+__global__ __launch_bounds__(TILE ? kBlock : 64, 3) void k_jacobi(int32_t nc, int64_t ldc, const int32_t *__restrict__ nbr,
                                                       const int32_t *__restrict__ sbc,
-                                                      const int32_t *__restrict__ wall_idx,
                                                       const double *__restrict__ M, const double *__restrict__ u,
                                                       const double *__restrict__ x, double *__restrict__ xn,
-                                                      double relax, WallFaces wf, double *corr, int32_t *errw,
+                                                      double relax, const double *__restrict__ walls, double *corr, int32_t *errw,
                                                       float *__restrict__ r32) {
-    const int32_t t = xcd_block() * blockDim.x + threadIdx.x, i = t >> 2, v = t & 3;
-    if (i >= nc)
+    __shared__ double tile[TILE ? 9 : 1][TILE ? kBlock : 1];
+    const int32_t t = xcd_block() * blockDim.x + threadIdx.x, v = t & 3;
+    const bool live = (t >> 2) < nc;
+    if (!TILE && !live)
         return;
+    const int32_t i = live ? t >> 2 : nc - 1;
     const uint32_t lane = threadIdx.x & 63;
-    const double *xo = x + rec_group(i);
-    int32_t jn[NF], least = 0;
+    const double *xo = x + rec((t >> 2) & ~15, 0, 0);
+    int32_t jn[NF];
+    bool wall = false;
 #pragma unroll
     for (int s = 0; s < NF; s++) {
         jn[s] = nbr[s * ldc + i];
-        least = min(least, jn[s] == -2 ? 0 : jn[s]);
+        wall |= is_wall_slot(jn[s]);
     }
     const double ui = u[4 * int64_t(i) + v];
     // wall corrections first (stored, and read back in their slot), before
     // the loads in flight take the registers
-    if (least < 0) {
+    if (live && wall) {
 #pragma unroll 1
         for (int s = 0; s < NF; s++) {
-            const int32_t w = wall_idx[s * ldc + i];
-            if (w < 0)
+            const int32_t j = s == 0 ? jn[0] : s == 1 ? jn[1] : s == 2 ? jn[2] : jn[NF - 1];
+            if (!is_wall_slot(j))
                 continue;
             double own[9], cw[9];
 #pragma unroll
             for (int r = 0; r < 9; r++)
                 own[r] = xo[256 * r + lane];
-            wall_correction(w, sbc[s * ldc + i], own, ui, v, wf, relax, errw, cw);
+            wall_correction(j, own, ui, v, walls, relax, errw, cw);
 #pragma unroll
             for (int r = 0; r < 9; r++)
-                corr[kRec * int64_t(w) + 9 * v + r] = cw[r];
+                corr[kRec * int64_t(wall_of(j)) + 9 * v + r] = cw[r];
         }
     }
     double nw[9];
 #pragma unroll
-    for (int r = 0; r < 9; r++)
-        nw[r] = (1 - relax) * xo[256 * r + lane];
+    for (int r = 0; r < 9; r++) {
+        nw[r] = xo[256 * r + lane];
+        if (TILE)
+            tile[r][threadIdx.x] = nw[r];
+        nw[r] = (1 - relax) * nw[r];
+    }
+    AbPart ab;
+    ab.load(M, 0, i, ldc, v);
+    if (TILE)
+        __syncthreads();
+    const int32_t i0 = (t - int32_t(threadIdx.x)) >> 2;
 #pragma unroll
     for (int s = 0; s < NF; s++) {
         if (s == 3 && jn[s] == -2)
             continue;
-        AbPart ab;
-        ab.load(M, s, i, ldc, v);
+        if (s > 0)
+            ab.load(M, s, i, ldc, v);
         const int32_t j = jn[s] < 0 ? i : jn[s];
         const double uj = u[4 * int64_t(j) + v];
         double xj[9];
+        const uint32_t jl = uint32_t(j - i0);
+        if (TILE && jl < kBlock / 4) {
 #pragma unroll
-        for (int c = 0; c < 9; c++)
-            xj[c] = x[rec(j, c, v)];
-        const int32_t bc = jn[s] < 0 ? sbc[s * ldc + i] : BC_INNER;
+            for (int c = 0; c < 9; c++)
+                xj[c] = tile[c][4 * jl + v];
+        } else {
+#pragma unroll
+            for (int c = 0; c < 9; c++)
+                xj[c] = x[rec(j, c, v)];
+        }
+        const int32_t bc = jn[s] == -1 ? sbc[s * ldc + i] : BC_INNER;
         if (jn[s] >= 0 || is_far(bc)) {
             // far field: M_if x_i (gathered from i), no mean-value term
             const double bmul = jn[s] < 0 ? 0.0 : 1.0;
@@ -346,15 +387,16 @@ __global__ __launch_bounds__(kBlock, 2) void k_jacobi(int32_t nc, int64_t ldc, c
 #pragma unroll
             for (int r = 0; r < 9; r++)
                 nw[r] += relax * ((0.0 - ui) * ab.get(10 * r + 9));
-        } else if (bc == BC_WALL_EULER || bc == BC_WALL_NOSLIP) {
-            const int64_t w = wall_idx[s * ldc + i];
+        } else if (is_wall_slot(jn[s])) {
 #pragma unroll
             for (int r = 0; r < 9; r++)
-                nw[r] += corr[kRec * w + 9 * v + r];
+                nw[r] += corr[kRec * int64_t(wall_of(jn[s])) + 9 * v + r];
         } else {
             atomicOr(errw, ERRBIT_BC);
         }
     }
+    if (TILE && !live)
+        return;
     // the new iterate streams out with non-temporal stores: written once and
     // read by the next launch, it would only displace the neighbours'
     // reconstructions that this sweep still gathers
@@ -398,29 +440,30 @@ __global__ __launch_bounds__(kBlock) void k_read_probe(int32_t nc, int64_t ldc, 
 // reconstructed value D d with the normal momentum removed (Wall_Euler) or
 // the momentum reversed (Wall_NoSlip), both linear, and the cell mean drops
 // out.  di: this lane's variable; the cell's quad calls it together.
-__device__ __forceinline__ void wall_correction_lin(int32_t w, int32_t bc, const float di[9], int v,
-                                                    const WallFaces &wf, float relax, float out[9]) {
+__device__ __forceinline__ void wall_correction_lin(int32_t slot, const float di[9], int v,
+                                                    const double *__restrict__ walls, float relax, float out[9]) {
+    const double *wd = walls + kWallEntries * int64_t(wall_of(slot));
+    QuadPart<0, 40> ainv;
+    QuadPart<0, 13> d0;
+    d0.load(wd + kWallD0, v);
     float BCc[9];
 #pragma unroll
     for (int r = 0; r < 9; r++)
         BCc[r] = 0.f;
-    const float w0 = float(wf.w0[w]);
-#pragma unroll 1
+    const float w0 = float(wd[kWallW0]);
+#pragma unroll
     for (int g = 0; g < 3; g++) {
         const float gw = float(g == 1 ? kLine3W1 : kLine3W0);
-        const double nx = wf.nrm[(2 * g) * wf.ld + w], ny = wf.nrm[(2 * g + 1) * wf.ld + w];
-        float d0[9], uB = 0.f;
+        const double nx = wd[kWallNrm + 2 * g], ny = wd[kWallNrm + 2 * g + 1];
+        float uB = 0.f;
 #pragma unroll
         for (int c = 0; c < 9; c++)
-            d0[c] = float(wf.d0[(g * 9 + c) * wf.ld + w]);
-#pragma unroll
-        for (int c = 0; c < 9; c++)
-            uB = fmaf(d0[c], di[c], uB);
+            uB = fmaf(float(d0.get(9 * g + c)), di[c], uB);
         double n0, n1;
         stable_normalized(nx, ny, n0, n1);
         const float m0 = quad_bcast<1>(uB), m1 = quad_bcast<2>(uB);
         float uBV = uB;
-        if (bc == BC_WALL_EULER) {
+        if (!wall_noslip(slot)) {
             const float dd = float(n0) * m0 + float(n1) * m1;
             if (v == 1)
                 uBV = uB - float(n0) * dd;
@@ -432,14 +475,15 @@ __device__ __forceinline__ void wall_correction_lin(int32_t w, int32_t bc, const
         const float nl = float(sqrt(nx * nx + ny * ny));
 #pragma unroll
         for (int r = 0; r < 9; r++)
-            BCc[r] += d0[r] * w0 * w0 * uBV * nl * gw;
+            BCc[r] += float(d0.get(9 * g + r)) * w0 * w0 * uBV * nl * gw;
     }
+    ainv.load(wd, v);
 #pragma unroll
     for (int r = 0; r < 9; r++) {
         float acc = 0.f;
 #pragma unroll
         for (int c = 0; c < 9; c++)
-            acc = fmaf(float(wf.ainv[(r * 9 + c) * wf.ld + w]), BCc[c], acc);
+            acc = fmaf(float(ainv.get(9 * r + c)), BCc[c], acc);
         out[r] = relax * acc;
     }
 }
@@ -456,23 +500,46 @@ __device__ __forceinline__ void wall_correction_lin(int32_t w, int32_t bc, const
 // state is linear in the reconstructed value there).  Four lanes per cell, as
 // in k_jacobi.
 template <int NF, bool LAST>
-__global__ __launch_bounds__(kBlock, 2) void k_delta32(int32_t nc, int64_t ldc, const int32_t *__restrict__ nbr,
+__global__ __launch_bounds__(kBlock, 4) void k_delta32(int32_t nc, int64_t ldc, const int32_t *__restrict__ nbr,
                                                        const int32_t *__restrict__ sbc,
-                                                       const int32_t *__restrict__ wall_idx,
                                                        const float *__restrict__ M32, const float *__restrict__ r32,
                                                        const float *__restrict__ din, float *__restrict__ dout,
-                                                       float relax, double *__restrict__ x, WallFaces wf) {
+                                                       float relax, double *__restrict__ x, const double *__restrict__ walls,
+                                                       float *corr) {
     const int32_t t = xcd_block() * blockDim.x + threadIdx.x, i = t >> 2, v = t & 3;
     if (i >= nc)
         return;
-    int32_t jn[NF];
-#pragma unroll
-    for (int s = 0; s < NF; s++)
-        jn[s] = nbr[s * ldc + i];
     const uint32_t lane = threadIdx.x & 63;
+    const float *xo = din + rec_group(i);
+    int32_t jn[NF];
+    bool wall = false;
+#pragma unroll
+    for (int s = 0; s < NF; s++) {
+        jn[s] = nbr[s * ldc + i];
+        wall |= is_wall_slot(jn[s]);
+    }
+    // wall corrections first, as in k_jacobi
+    if (wall) {
+#pragma unroll 1
+        for (int s = 0; s < NF; s++) {
+            const int32_t j = s == 0 ? jn[0] : s == 1 ? jn[1] : s == 2 ? jn[2] : jn[NF - 1];
+            if (!is_wall_slot(j))
+                continue;
+            float own[9], cw[9];
+#pragma unroll
+            for (int r = 0; r < 9; r++)
+                own[r] = xo[256 * r + lane];
+            wall_correction_lin(j, own, v, walls, relax, cw);
+#pragma unroll
+            for (int r = 0; r < 9; r++)
+                corr[kRec * int64_t(wall_of(j)) + 9 * v + r] = cw[r];
+        }
+    }
+    float nw[9];
+#pragma unroll
+    for (int r = 0; r < 9; r++)
+        nw[r] = (1.0f - relax) * xo[256 * r + lane];
     constexpr int kW = kAb32Vecs / 4;
-    flt4 w[NF][kW], last[NF];
-    float dj[NF][9], own[9], res[9], nw[9];
 #pragma unroll
     for (int s = 0; s < NF; s++) {
         if (s == 3 && jn[s] == -2)
@@ -480,58 +547,39 @@ __global__ __launch_bounds__(kBlock, 2) void k_delta32(int32_t nc, int64_t ldc, 
         const int32_t g = __builtin_amdgcn_readfirstlane(i);
         const flt4 *p = reinterpret_cast<const flt4 *>(M32) + ab_group(s, g, ldc, kAb32Vecs);
         const uint32_t cl = i & 15;
+        flt4 w[kW];
 #pragma unroll
         for (int k = 0; k < kW; k++)
-            w[s][k] = __builtin_nontemporal_load(p + 64 * k + (4 * cl + v));
-        last[s] = __builtin_nontemporal_load(p + 16 * (kAb32Vecs - 1) + cl);
-    }
-#pragma unroll
-    for (int r = 0; r < 9; r++) {
-        own[r] = (din + rec_group(i))[256 * r + lane];
-        res[r] = (r32 + rec_group(i))[256 * r + lane];
-    }
-#pragma unroll
-    for (int s = 0; s < NF; s++) {
+            w[k] = __builtin_nontemporal_load(p + 64 * k + (4 * cl + v));
+        const flt4 last = __builtin_nontemporal_load(p + 16 * (kAb32Vecs - 1) + cl);
         const int32_t j = jn[s] < 0 ? i : jn[s];
-        if (s == 3 && jn[s] == -2)
-            continue;
+        float dj[9];
 #pragma unroll
         for (int c = 0; c < 9; c++)
-            dj[s][c] = din[rec(j, c, v)];
-    }
+            dj[c] = din[rec(j, c, v)];
+        const int32_t bc = jn[s] == -1 ? sbc[s * ldc + i] : BC_INNER;
+        if (is_wall_slot(jn[s])) {
 #pragma unroll
-    for (int r = 0; r < 9; r++)
-        nw[r] = (1.0f - relax) * own[r];
-#pragma unroll
-    for (int s = 0; s < NF; s++) {
-        const int32_t j = jn[s];
-        if (j == -2)
-            continue;
-        const int32_t bc = j < 0 ? sbc[s * ldc + i] : 0;
-        if (j >= 0 || !(bc == BC_WALL || bc == BC_WALL_EULER || bc == BC_WALL_NOSLIP)) { // far field: d_i
+            for (int r = 0; r < 9; r++)
+                nw[r] += corr[kRec * int64_t(wall_of(jn[s])) + 9 * v + r];
+        } else if (bc != BC_WALL) { // far field: d_i; a Wall face's constant term is in r only
 #pragma unroll
             for (int r = 0; r < 9; r++) {
                 float tt = 0.f;
 #pragma unroll
                 for (int c = 0; c < 9; c++) {
-                    const int e = 9 * r + c, p = e / 4;
-                    const float m = p == kAb32Vecs - 1 ? last[s][e % 4]
-                                                       : quad_get(float(w[s][p < 20 ? p / 4 : 0][e % 4]), p % 4);
-                    tt = fmaf(m, dj[s][c], tt);
+                    const int e = 9 * r + c, k = e / 4;
+                    const float m = k == kAb32Vecs - 1 ? last[e % 4]
+                                                       : quad_get(float(w[k < 20 ? k / 4 : 0][e % 4]), k % 4);
+                    tt = fmaf(m, dj[c], tt);
                 }
                 nw[r] = fmaf(relax, tt, nw[r]);
             }
-        } else if (bc != BC_WALL) { // (a Wall face's constant term is in r only)
-            float cw[9];
-            wall_correction_lin(wall_idx[s * ldc + i], bc, own, v, wf, relax, cw);
-#pragma unroll
-            for (int r = 0; r < 9; r++)
-                nw[r] += cw[r];
         }
     }
 #pragma unroll
     for (int r = 0; r < 9; r++) {
-        const float d = nw[r] + res[r];
+        const float d = nw[r] + (r32 + rec_group(i))[256 * r + lane];
         if (LAST)
             (x + rec_group(i))[256 * r + lane] += double(d);
         else
@@ -1197,26 +1245,8 @@ __device__ __forceinline__ T row_ahead(T a, int q) { // q: a constant after unro
     }
 }
 
-// entries 2 P0 .. 2 P1 + 1 of a secondary matrix, a quarter per lane
 constexpr int kSecEntries = 82; // 81 and a pad, per face and side
 constexpr unsigned kLimBlocks = 8192; // workgroups that walk the list (131 072 cells at once)
-template <int P0, int P1>
-struct SecPart {
-    static constexpr int N = (P1 - P0) / 4 + 1;
-    dbl2 w[N];
-    __device__ __forceinline__ void load(const double *__restrict__ m, int v) {
-#pragma unroll
-        for (int k = 0; k < N; k++) {
-            w[k] = dbl2{0.0, 0.0};
-            if (P0 + 4 * k + v <= P1)
-                w[k] = reinterpret_cast<const dbl2 *>(m)[P0 + 4 * k + v];
-        }
-    }
-    __device__ __forceinline__ double get(int e) const {
-        const int p = e / 2 - P0;
-        return quad_get(e % 2 ? w[p / 4].y : w[p / 4].x, p % 4);
-    }
-};
 
 // row v of a 4 x 4 matrix
 __device__ __forceinline__ void matrix_row(const double M[16], int v, double row[4]) {
@@ -1272,7 +1302,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_wbap_lim(int64_t ldc, int64_t ldf
         const int32_t j = s < NF ? nbr[s * ldc + i] : -1;
         const bool valid = j >= 0;
         double own[9], xj[9], uF[7], ml[4], mr[4];
-        SecPart<0, 40> ms, msO;
+        QuadPart<0, 40> ms, msO;
 #pragma unroll
         for (int r = 0; r < 9; r++)
             own[r] = x[rec(i, r, v)];
@@ -1400,7 +1430,7 @@ __global__ __launch_bounds__(kBlock, 3) void k_wbap_lim_v2(int64_t ldc, int64_t 
         if (valid) {
             const int32_t f = sface[s * ldc + i];
             const int side = f2c[f] == i ? 0 : 1;
-            SecPart<9 * ls / 2, (9 * le + 8) / 2> ms;
+            QuadPart<9 * ls / 2, (9 * le + 8) / 2> ms;
             ms.load(msec + kSecEntries * (2 * int64_t(f) + side), v);
             // the neighbour's rows above le: limited (xo) or, with limf, as given (x)
             const double *above = (limf && !limf[j]) ? x : xo;
@@ -1660,7 +1690,7 @@ extern "C" int dndsmi_ctx_create(const dndsmi_mesh_view *mesh, const dndsmi_vr_v
         }
         // ---- cell streams
         std::vector<int32_t> nbr(size_t(nfmax) * ldc, -2), sbc(size_t(nfmax) * ldc, 0), sface(size_t(nfmax) * ldc, -1);
-        std::vector<int32_t> gat(size_t(nfmax) * ldc, -1), widx(size_t(nfmax) * ldc, -1);
+        std::vector<int32_t> gat(size_t(nfmax) * ldc, -1);
         std::vector<uint8_t> wpos(ldf, 0);
         std::vector<double> M(size_t(nfmax) * kAbVecs * 2 * ldc, 0.0), vol(ldc, 1.0);
         std::vector<double> cmom(9 * size_t(ldc), 0.0), cscale(2 * size_t(ldc), 1.0);
@@ -1691,7 +1721,7 @@ extern "C" int dndsmi_ctx_create(const dndsmi_mesh_view *mesh, const dndsmi_vr_v
                 order.push_back({f, side});
                 if (j == DNDSMI_NO_CELL &&
                     (mesh->face_bc[f] == DNDSMI_BC_WALL_EULER || mesh->face_bc[f] == DNDSMI_BC_WALL_NOSLIP)) {
-                    widx[s * ldc + ci] = int32_t(wall_cell.size());
+                    nbr[s * ldc + ci] = wall_slot(int32_t(wall_cell.size()), mesh->face_bc[f]);
                     wall_cell.push_back(i), wall_face.push_back(f), wall_c2f.push_back(b0 + s);
                 }
             }
@@ -1722,8 +1752,6 @@ extern "C" int dndsmi_ctx_create(const dndsmi_mesh_view *mesh, const dndsmi_vr_v
             DNDSMI_TRY(c->alloc(c->fpos, ldf));
             DNDSMI_TRY(c->upload(c->fpos, fpos));
         }
-        DNDSMI_TRY(c->alloc(c->wall_idx, nfmax * ldc));
-        DNDSMI_TRY(c->upload(c->wall_idx, widx));
         DNDSMI_TRY(c->alloc(c->M, int64_t(nfmax) * kAbVecs * 2 * ldc));
         DNDSMI_TRY(c->upload(c->M, M));
         M.clear(), M.shrink_to_fit();
@@ -1737,34 +1765,18 @@ extern "C" int dndsmi_ctx_create(const dndsmi_mesh_view *mesh, const dndsmi_vr_v
         const int64_t nw = int64_t(wall_cell.size());
         c->n_wall = std::max<int64_t>(nw, 1);
         {
-            std::vector<double> wa(81 * size_t(c->n_wall), 0.0), wd(27 * size_t(c->n_wall), 0.0),
-                wn(6 * size_t(c->n_wall), 0.0), w0(size_t(c->n_wall), 0.0);
+            std::vector<double> wd(kWallEntries * size_t(c->n_wall), 0.0);
             for (int64_t w = 0; w < nw; w++) {
                 const int64_t i = wall_cell[w], f = wall_face[w];
-                for (int k = 0; k < 81; k++)
-                    wa[k * c->n_wall + w] = vr->ainv[81 * i + k];
+                double *p = &wd[kWallEntries * size_t(w)];
+                std::copy_n(vr->ainv + 81 * i, 81, p);
                 for (int g = 0; g < 3; g++)
-                    for (int k = 0; k < 9; k++)
-                        wd[(g * 9 + k) * c->n_wall + w] = vr->face_d0[54 * f + 18 * g + k];
-                for (int k = 0; k < 6; k++)
-                    wn[k * c->n_wall + w] = vr->face_norm[6 * f + k];
-                w0[w] = vr->face_weight[10 * f];
+                    std::copy_n(vr->face_d0 + 54 * f + 18 * g, 9, p + kWallD0 + 9 * g);
+                std::copy_n(vr->face_norm + 6 * f, 6, p + kWallNrm);
+                p[kWallW0] = vr->face_weight[10 * f];
             }
-            DNDSMI_TRY(c->alloc(c->wall_ainv, 81 * c->n_wall));
-            DNDSMI_TRY(c->upload(c->wall_ainv, wa));
-            DNDSMI_TRY(c->alloc(c->wall_d0, 27 * c->n_wall));
-            DNDSMI_TRY(c->upload(c->wall_d0, wd));
-            DNDSMI_TRY(c->alloc(c->wall_nrm, 6 * c->n_wall));
-            DNDSMI_TRY(c->upload(c->wall_nrm, wn));
-            DNDSMI_TRY(c->alloc(c->wall_w0, c->n_wall));
-            DNDSMI_TRY(c->upload(c->wall_w0, w0));
-            std::vector<int32_t> wc(size_t(c->n_wall), 0), wb(size_t(c->n_wall), 0);
-            for (int64_t w = 0; w < nw; w++)
-                wc[w] = c2d[wall_cell[w]], wb[w] = mesh->face_bc[wall_face[w]];
-            DNDSMI_TRY(c->alloc(c->wall_cell, c->n_wall));
-            DNDSMI_TRY(c->upload(c->wall_cell, wc));
-            DNDSMI_TRY(c->alloc(c->wall_bc, c->n_wall));
-            DNDSMI_TRY(c->upload(c->wall_bc, wb));
+            DNDSMI_TRY(c->alloc(c->walls, kWallEntries * c->n_wall));
+            DNDSMI_TRY(c->upload(c->walls, wd));
             DNDSMI_TRY(c->alloc(c->wall_corr, kRec * c->n_wall));
             c->n_wall_faces = nw;
         }
@@ -2059,8 +2071,8 @@ int launch_sor(dndsmi_ctx *c, const double *u, double *x, double t) {
             auto kern = c->nfmax == 3 ? k_sor<3> : k_sor<4>;
             prof_begin(c, DNDSMI_K_JACOBI);
             hipLaunchKernelGGL(kern, dim3(grid_for(lanes, block)), dim3(block), 0,
-                               c->stream, int32_t(n), int32_t(b), c->ldc, c->nbr, c->sbc, c->wall_idx, c->M, u, x, x,
-                               c->relax, c->wall_faces(), c->errw);
+                               c->stream, int32_t(n), int32_t(b), c->ldc, c->nbr, c->sbc, c->M, u, x, x,
+                               c->relax, c->walls, c->errw);
             prof_end(c);
             DNDSMI_TRY(c->launch_check("k_sor"));
         }
@@ -2085,9 +2097,10 @@ int launch_jacobi(dndsmi_ctx *c, const double *u, const double *x, double *xn, d
     const int64_t lanes = 4 * c->nc;
     const int block = sweep_block(lanes);
     prof_begin(c, DNDSMI_K_JACOBI);
-    auto kern = c->nfmax == 3 ? k_jacobi<3, false> : k_jacobi<4, false>;
+    auto kern = block == 64 ? (c->nfmax == 3 ? k_jacobi<3, false, false> : k_jacobi<4, false, false>)
+                            : (c->nfmax == 3 ? k_jacobi<3, false, true> : k_jacobi<4, false, true>);
     hipLaunchKernelGGL(kern, dim3(grid_for(lanes, block)), dim3(block), 0, c->stream, int32_t(c->nc),
-                       c->ldc, c->nbr, c->sbc, c->wall_idx, c->M, u, x, xn, c->relax, c->wall_faces(), c->wall_corr,
+                       c->ldc, c->nbr, c->sbc, c->M, u, x, xn, c->relax, c->walls, c->wall_corr,
                        c->errw, nullptr);
     prof_end(c);
     return c->launch_check("k_jacobi");
@@ -2211,6 +2224,7 @@ int ensure_mixed(dndsmi_ctx *c) {
     DNDSMI_TRY(c->alloc(c->dA32, 36 * c->ldc));
     DNDSMI_TRY(c->alloc(c->dB32, 36 * c->ldc));
     DNDSMI_TRY(c->alloc(c->fslot32, int64_t(c->nfmax) * 8 * c->ldc));
+    DNDSMI_TRY(c->alloc(c->wcorr32, kRec * c->n_wall));
     hipLaunchKernelGGL(k_m_to_f32, dim3(grid_for(nm / 4)), dim3(kBlock), 0, c->stream, int32_t(c->nfmax), c->ldc,
                        c->M, c->M32);
     DNDSMI_TRY(c->launch_check("k_m_to_f32"));
@@ -2224,9 +2238,10 @@ int launch_jacobi_mixed(dndsmi_ctx *c, const double *u, double *x, int n_sweeps,
     const int block = sweep_block(lanes), nc = int(c->nc);
     const dim3 grid(grid_for(lanes, block));
     prof_begin(c, DNDSMI_K_JACOBI);
-    auto first = c->nfmax == 3 ? k_jacobi<3, true> : k_jacobi<4, true>;
+    auto first = block == 64 ? (c->nfmax == 3 ? k_jacobi<3, true, false> : k_jacobi<4, true, false>)
+                             : (c->nfmax == 3 ? k_jacobi<3, true, true> : k_jacobi<4, true, true>);
     hipLaunchKernelGGL(first, grid, dim3(block), 0, c->stream, nc,
-                       c->ldc, c->nbr, c->sbc, c->wall_idx, c->M, u, x, nullptr, c->relax, c->wall_faces(),
+                       c->ldc, c->nbr, c->sbc, c->M, u, x, nullptr, c->relax, c->walls,
                        c->wall_corr, c->errw, c->r32);
     prof_end(c);
     DNDSMI_TRY(c->launch_check("k_jacobi (residual)"));
@@ -2236,8 +2251,9 @@ int launch_jacobi_mixed(dndsmi_ctx *c, const double *u, double *x, int n_sweeps,
         auto kern = k == n_sweeps - 1 ? (c->nfmax == 3 ? k_delta32<3, true> : k_delta32<4, true>)
                                       : (c->nfmax == 3 ? k_delta32<3, false> : k_delta32<4, false>);
         prof_begin(c, DNDSMI_K_DELTA32);
-        hipLaunchKernelGGL(kern, grid, dim3(block), 0, c->stream, nc, c->ldc, c->nbr, c->sbc, c->wall_idx, c->M32,
-                           c->r32, din, dout, float(c->relax), x, c->wall_faces());
+        hipLaunchKernelGGL(kern, grid, dim3(block), 0, c->stream, nc, c->ldc, c->nbr, c->sbc, c->M32,
+                           c->r32, din, dout, float(c->relax), x, c->walls,
+                           c->wcorr32);
         prof_end(c);
         DNDSMI_TRY(c->launch_check("k_delta32"));
         din = dout;

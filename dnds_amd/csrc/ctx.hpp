@@ -51,20 +51,14 @@ struct dndsmi_ctx {
     std::unordered_set<struct dndsmi_bdf *> bdfs;
 
     // cell side
-    int32_t *nbr = nullptr;    // [nfmax][ldc] neighbour cell, -1 = boundary slot, -2 = absent slot
+    int32_t *nbr = nullptr;    // [nfmax][ldc] neighbour cell, -1 = boundary slot, -2 = absent slot, wall_slot() = wall
     int32_t *sbc = nullptr;    // [nfmax][ldc] boundary kind of the slot's face
     int32_t *sface = nullptr;  // [nfmax][ldc] face index of the slot
     int32_t *gat = nullptr;    // [nfmax][ldc] (face << 1 | side) sorted by face, -1 = none
     double *M = nullptr;       // A^-1 B and A^-1 b, 45 pairs per cell and slot (ab_vec)
     double *vol = nullptr;     // [ldc]
-    int32_t *wall_idx = nullptr; // [nfmax][ldc] index into the wall-face arrays, -1 = none
     int64_t n_wall = 0;
-    double *wall_ainv = nullptr; // [81][n_wall]
-    double *wall_d0 = nullptr;   // [27][n_wall]
-    double *wall_nrm = nullptr;  // [6][n_wall]
-    double *wall_w0 = nullptr;   // [n_wall]
-    int32_t *wall_cell = nullptr; // [n_wall]
-    int32_t *wall_bc = nullptr;   // [n_wall]
+    double *walls = nullptr;      // [n_wall][kWallEntries]
     double *wall_corr = nullptr;  // [n_wall][36] the running sweep's wall corrections
     int64_t n_wall_faces = 0;     // real count (n_wall >= 1 for allocation)
     // face side
@@ -139,6 +133,7 @@ struct dndsmi_ctx {
     // correction vectors, FP32 face fluxes
     float *M32 = nullptr;             // A^-1 B, 21 vectors per cell and slot (ab_vec)
     float *r32 = nullptr, *dA32 = nullptr, *dB32 = nullptr; // REC layout
+    float *wcorr32 = nullptr;         // [n_wall][36] a correction sweep's wall corrections
     float *fslot32 = nullptr;         // [2 nfmax] quads
     // implicit dual-time scratch (allocated on first use)
     double *imp_rhs = nullptr;        // [ldc][4]
@@ -199,7 +194,6 @@ struct dndsmi_ctx {
             return rc;
         return hip(hipStreamSynchronize(stream), "hipStreamSynchronize");
     }
-    dndsmi_dev::WallFaces wall_faces() const { return {wall_ainv, wall_d0, wall_nrm, wall_w0, n_wall}; }
     int launch_check(const char *what) { return hip(hipGetLastError(), what); }
 };
 

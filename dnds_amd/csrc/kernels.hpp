@@ -78,11 +78,17 @@ __host__ __device__ __forceinline__ int64_t ab_vec(int s, int e, int64_t i, int6
     return ab_group(s, i, ldc, nvec) + (e == nvec - 1 ? 16 * e + (i & 15) : (e >> 2) * 64 + 4 * (i & 15) + (e & 3));
 }
 
-// the Wall_Euler / Wall_NoSlip faces' data, [element][ld]
-struct WallFaces {
-    const double *ainv, *d0, *nrm, *w0; // 81, 27, 6, 1 elements
-    int64_t ld;
-};
+// A Wall_Euler / Wall_NoSlip face's data for its cell's sweeps, one run per
+// face: A^-1 of the cell (81), D0 at the three points (27), their normals (6)
+// and the face weight.  The slot of such a face holds, in place of a neighbour,
+// the code wall_slot(its number, its kind) <= -3.
+constexpr int kWallD0 = 82, kWallNrm = 110, kWallW0 = 116, kWallEntries = 118;
+__host__ __device__ __forceinline__ int32_t wall_slot(int32_t w, int32_t bc) {
+    return -3 - (2 * w + (bc == BC_WALL_NOSLIP ? 1 : 0));
+}
+__device__ __forceinline__ bool is_wall_slot(int32_t j) { return j <= -3; }
+__device__ __forceinline__ int32_t wall_of(int32_t j) { return (-3 - j) >> 1; }
+__device__ __forceinline__ bool wall_noslip(int32_t j) { return (-3 - j) & 1; }
 
 struct GasParams {
     double gamma;
