@@ -100,18 +100,41 @@ __device__ __forceinline__ double pair_swap(double a) {
     return __builtin_bit_cast(double, uint64_t(lo) | uint64_t(hi) << 32);
 }
 
+// 16-byte loads from one group of the stream through a buffer descriptor,
+// whose cache policy is part of the instruction (with plain and non-temporal
+// pointer loads on two sides of a branch, the compiler makes one plain load)
+struct ab_stream {
+    __amdgpu_buffer_rsrc_t rs;
+    __device__ __forceinline__ ab_stream(const void *p, int bytes)
+        : rs(__builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, bytes, 0x00020000)) {}
+    template <typename T, bool NT>
+    __device__ __forceinline__ T get(uint32_t off, int soff) const {
+        return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b128(rs, off, soff, NT ? 2 : 0));
+    }
+};
+
 // A lane's part of the A^-1 B, A^-1 b of one cell and slot (ab_vec's layout)
 struct AbPart {
     dbl2 w[kAbVecs / 4], last;
-    __device__ __forceinline__ void load(const double *__restrict__ M, int s, int32_t i, int64_t ldc, int v) {
+    // groups with (i / 64) mod 64 below `keep` are read with ordinary loads
+    __device__ __forceinline__ void load(const double *__restrict__ M, int s, int32_t i, int64_t ldc, int v,
+                                         int32_t keep) {
         // a wave holds one group of 16 cells: a scalar base
         const int32_t g = __builtin_amdgcn_readfirstlane(i);
-        const dbl2 *p = reinterpret_cast<const dbl2 *>(M) + ab_group(s, g, ldc, kAbVecs);
+        const double *p = M + 2 * ab_group(s, g, ldc, kAbVecs);
         const uint32_t cl = i & 15;
+        const ab_stream rs(p, 256 * kAbVecs);
+        if (((g >> 6) & 63) < keep) {
 #pragma unroll
-        for (int k = 0; k < kAbVecs / 4; k++)
-            w[k] = __builtin_nontemporal_load(p + 64 * k + (4 * cl + v));
-        last = __builtin_nontemporal_load(p + 16 * (kAbVecs - 1) + cl);
+            for (int k = 0; k < kAbVecs / 4; k++)
+                w[k] = rs.get<dbl2, false>((4 * cl + v) * 16, 1024 * k);
+            last = rs.get<dbl2, false>(cl * 16, 256 * (kAbVecs - 1));
+        } else {
+#pragma unroll
+            for (int k = 0; k < kAbVecs / 4; k++)
+                w[k] = rs.get<dbl2, true>((4 * cl + v) * 16, 1024 * k);
+            last = rs.get<dbl2, true>(cl * 16, 256 * (kAbVecs - 1));
+        }
     }
     // entry d = 10 r + c: A^-1 B (c < 9) or A^-1 b (c = 9) of row r
     __device__ __forceinline__ double get(int d) const {
@@ -235,8 +258,8 @@ template <int NF>
 __global__ __launch_bounds__(kBlock, 3) void k_sor(int32_t n, int32_t base, int64_t ldc,
                                                    const int32_t *__restrict__ nbr, const int32_t *__restrict__ sbc,
                                                    const double *__restrict__ M, const double *__restrict__ u,
-                                                   const double *x, double *xo, double relax, const double *__restrict__ walls,
-                                                   int32_t *errw) {
+                                                   const double *x, double *xo, double relax,
+                                                   const double *__restrict__ walls, int32_t *errw, int32_t keep) {
     const int32_t t = xcd_block() * blockDim.x + threadIdx.x, v = t & 3;
     // whole groups of 16 cells from the one that holds `base`
     const int32_t i = (base & ~15) + (t >> 2);
@@ -258,7 +281,7 @@ __global__ __launch_bounds__(kBlock, 3) void k_sor(int32_t n, int32_t base, int6
         if (j == -2)
             continue;
         AbPart ab;
-        ab.load(M, s, i, ldc, v);
+        ab.load(M, s, i, ldc, v, keep);
         if (j >= 0) {
             double xj[9];
 #pragma unroll
@@ -310,8 +333,8 @@ __global__ __launch_bounds__(TILE ? kBlock : 64, 3) void k_jacobi(int32_t nc, in
                                                       const int32_t *__restrict__ sbc,
                                                       const double *__restrict__ M, const double *__restrict__ u,
                                                       const double *__restrict__ x, double *__restrict__ xn,
-                                                      double relax, const double *__restrict__ walls, double *corr, int32_t *errw,
-                                                      float *__restrict__ r32) {
+                                                      double relax, const double *__restrict__ walls, double *corr,
+                                                      int32_t *errw, float *__restrict__ r32, int32_t keep) {
     __shared__ double tile[TILE ? 9 : 1][TILE ? kBlock : 1];
     const int32_t t = xcd_block() * blockDim.x + threadIdx.x, v = t & 3;
     const bool live = (t >> 2) < nc;
@@ -355,7 +378,7 @@ __global__ __launch_bounds__(TILE ? kBlock : 64, 3) void k_jacobi(int32_t nc, in
         nw[r] = (1 - relax) * nw[r];
     }
     AbPart ab;
-    ab.load(M, 0, i, ldc, v);
+    ab.load(M, 0, i, ldc, v, keep);
     if (TILE)
         __syncthreads();
     const int32_t i0 = (t - int32_t(threadIdx.x)) >> 2;
@@ -364,7 +387,7 @@ __global__ __launch_bounds__(TILE ? kBlock : 64, 3) void k_jacobi(int32_t nc, in
         if (s == 3 && jn[s] == -2)
             continue;
         if (s > 0)
-            ab.load(M, s, i, ldc, v);
+            ab.load(M, s, i, ldc, v, keep);
         const int32_t j = jn[s] < 0 ? i : jn[s];
         const double uj = u[4 * int64_t(j) + v];
         double xj[9];
@@ -426,7 +449,7 @@ __global__ __launch_bounds__(kBlock) void k_read_probe(int32_t nc, int64_t ldc, 
         if (nbr[s * ldc + i] == -2)
             continue;
         AbPart ab;
-        ab.load(M, s, i, ldc, v);
+        ab.load(M, s, i, ldc, v, 0);
 #pragma unroll
         for (int k = 0; k < kAbVecs / 4; k++)
             a += ab.w[k].x + ab.w[k].y;
@@ -505,7 +528,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_delta32(int32_t nc, int64_t ldc, 
                                                        const float *__restrict__ M32, const float *__restrict__ r32,
                                                        const float *__restrict__ din, float *__restrict__ dout,
                                                        float relax, double *__restrict__ x, const double *__restrict__ walls,
-                                                       float *corr) {
+                                                       float *corr, int32_t keep) {
     const int32_t t = xcd_block() * blockDim.x + threadIdx.x, i = t >> 2, v = t & 3;
     if (i >= nc)
         return;
@@ -545,13 +568,20 @@ __global__ __launch_bounds__(kBlock, 4) void k_delta32(int32_t nc, int64_t ldc, 
         if (s == 3 && jn[s] == -2)
             continue;
         const int32_t g = __builtin_amdgcn_readfirstlane(i);
-        const flt4 *p = reinterpret_cast<const flt4 *>(M32) + ab_group(s, g, ldc, kAb32Vecs);
+        const ab_stream rs(M32 + 4 * ab_group(s, g, ldc, kAb32Vecs), 256 * kAb32Vecs);
         const uint32_t cl = i & 15;
-        flt4 w[kW];
+        flt4 w[kW], last;
+        if (((g >> 6) & 63) < keep) {
 #pragma unroll
-        for (int k = 0; k < kW; k++)
-            w[k] = __builtin_nontemporal_load(p + 64 * k + (4 * cl + v));
-        const flt4 last = __builtin_nontemporal_load(p + 16 * (kAb32Vecs - 1) + cl);
+            for (int k = 0; k < kW; k++)
+                w[k] = rs.get<flt4, false>((4 * cl + v) * 16, 1024 * k);
+            last = rs.get<flt4, false>(cl * 16, 256 * (kAb32Vecs - 1));
+        } else {
+#pragma unroll
+            for (int k = 0; k < kW; k++)
+                w[k] = rs.get<flt4, true>((4 * cl + v) * 16, 1024 * k);
+            last = rs.get<flt4, true>(cl * 16, 256 * (kAb32Vecs - 1));
+        }
         const int32_t j = jn[s] < 0 ? i : jn[s];
         float dj[9];
 #pragma unroll
@@ -2051,6 +2081,28 @@ extern "C" int dndsmi_array_set_constant(dndsmi_array *a, double value) {
 
 namespace dndsmi_host {
 
+// How many of every 64 blocks of the A^-1 B stream (`vecs` 16-byte vectors per
+// cell and face) a sweep reads with ordinary loads.  The Infinity Cache (256
+// MB) then still holds those at the next sweep, while the others, loaded
+// non-temporally, pass it by; a stream read by ordinary loads throughout
+// evicts itself once it is larger.  112 MB is what stays; small streams stay
+// as a whole, and beyond `largest` bytes the rest of the traffic wins.
+// Jacobi sweeps, us, none / 112 MB / all kept: 97 k triangles 52.7 / 49.4 /
+// 46.2 (209 MB), 131 k 69.5 / 60.4 / 73.4 (283 MB), 218 k 105 / 93 / 116 (470),
+// 320 k 152 / 143 / 168 (691), 405 k 200 / 194 / 215 (874), 524 k 255 / 254 / 274
+// (1132), 1.0 M mixed cells 571 / 573 (2400).  FP32 sweeps: 264 k 76.6 / 69 / 87
+// (265 MB), 524 k 147 / 142 / 163 (528), 980 k 268 / 276 / 289 (987).
+int32_t keep_share(const dndsmi_ctx *c, int vecs, int64_t largest) {
+    const int64_t stream = (2 * c->nf - c->n_bface) * 16 * vecs;
+    constexpr int64_t kKept = 112000000;
+    if (stream > largest)
+        return 0;
+    return stream <= kKept * 3 / 2 ? 64 : int32_t(kKept * 64 / stream);
+}
+constexpr int64_t kKeepLargest = 900000000, kKeepLargest32 = 600000000;
+// the FP64 sweep of a mixed-precision stage shares the cache with the FP32 ones
+constexpr int64_t kKeepLargestMixed = 450000000;
+
 // Workgroup size of a sweep over `lanes` lanes.  Waves are independent; small
 // sweeps take one wave per workgroup, so that their waves spread over all CUs.
 int sweep_block(int64_t lanes) { return lanes < 300000 ? 64 : kBlock; }
@@ -2072,7 +2124,7 @@ int launch_sor(dndsmi_ctx *c, const double *u, double *x, double t) {
             prof_begin(c, DNDSMI_K_JACOBI);
             hipLaunchKernelGGL(kern, dim3(grid_for(lanes, block)), dim3(block), 0,
                                c->stream, int32_t(n), int32_t(b), c->ldc, c->nbr, c->sbc, c->M, u, x, x,
-                               c->relax, c->walls, c->errw);
+                               c->relax, c->walls, c->errw, keep_share(c, kAbVecs, kKeepLargest));
             prof_end(c);
             DNDSMI_TRY(c->launch_check("k_sor"));
         }
@@ -2101,7 +2153,7 @@ int launch_jacobi(dndsmi_ctx *c, const double *u, const double *x, double *xn, d
                             : (c->nfmax == 3 ? k_jacobi<3, false, true> : k_jacobi<4, false, true>);
     hipLaunchKernelGGL(kern, dim3(grid_for(lanes, block)), dim3(block), 0, c->stream, int32_t(c->nc),
                        c->ldc, c->nbr, c->sbc, c->M, u, x, xn, c->relax, c->walls, c->wall_corr,
-                       c->errw, nullptr);
+                       c->errw, nullptr, keep_share(c, kAbVecs, kKeepLargest));
     prof_end(c);
     return c->launch_check("k_jacobi");
 }
@@ -2242,9 +2294,11 @@ int launch_jacobi_mixed(dndsmi_ctx *c, const double *u, double *x, int n_sweeps,
                              : (c->nfmax == 3 ? k_jacobi<3, true, true> : k_jacobi<4, true, true>);
     hipLaunchKernelGGL(first, grid, dim3(block), 0, c->stream, nc,
                        c->ldc, c->nbr, c->sbc, c->M, u, x, nullptr, c->relax, c->walls,
-                       c->wall_corr, c->errw, c->r32);
+                       c->wall_corr, c->errw, c->r32,
+                       keep_share(c, kAbVecs, kKeepLargestMixed));
     prof_end(c);
     DNDSMI_TRY(c->launch_check("k_jacobi (residual)"));
+    const int32_t keep = keep_share(c, kAb32Vecs, kKeepLargest32);
     // d_0 = r: the first correction sweep reads r itself
     float *din = c->r32, *dout = c->dA32, *next = c->dB32;
     for (int k = 1; k < n_sweeps; k++) {
@@ -2253,7 +2307,7 @@ int launch_jacobi_mixed(dndsmi_ctx *c, const double *u, double *x, int n_sweeps,
         prof_begin(c, DNDSMI_K_DELTA32);
         hipLaunchKernelGGL(kern, grid, dim3(block), 0, c->stream, nc, c->ldc, c->nbr, c->sbc, c->M32,
                            c->r32, din, dout, float(c->relax), x, c->walls,
-                           c->wcorr32);
+                           c->wcorr32, keep);
         prof_end(c);
         DNDSMI_TRY(c->launch_check("k_delta32"));
         din = dout;
