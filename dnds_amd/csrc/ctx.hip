@@ -214,7 +214,7 @@ __device__ __forceinline__ void wall_correction(int32_t slot, const double xi[9]
             else if (v == 2)
                 uBV = uB - n1 * dd;
         } else if (!(rho > 0)) {
-            atomicOr(errw, ERRBIT_NONPOSITIVE);
+            raise_error(errw, ERR_NONPOSITIVE);
         } else if (v == 1 || v == 2) {
             uBV *= -1;
         }
@@ -311,7 +311,7 @@ __global__ __launch_bounds__(kBlock, 3) void k_sor(int32_t n, int32_t base, int6
                 own[c] = nw[c];
             ab_apply(ab, own, 0.0, 0.0, relax, nw);
         } else {
-            atomicOr(errw, ERRBIT_BC);
+            raise_error(errw, ERR_BC);
         }
     }
 #pragma unroll
@@ -415,7 +415,7 @@ __global__ __launch_bounds__(TILE ? kBlock : 64, 3) void k_jacobi(int32_t nc, in
             for (int r = 0; r < 9; r++)
                 nw[r] += corr[kRec * int64_t(wall_of(jn[s])) + 9 * v + r];
         } else {
-            atomicOr(errw, ERRBIT_BC);
+            raise_error(errw, ERR_BC);
         }
     }
     if (TILE && !live)
@@ -666,7 +666,7 @@ __global__ __launch_bounds__(kBlock) void k_dt_face(int32_t nf, int64_t ldf, con
         ideal_gas_thermal(UR[3], UR[0], vR0 * vR0 + vR1 * vR1, gamma, pR, asqrR, HR);
     }
     if (!(uMean[0] > 0))
-        atomicOr(errw, ERRBIT_NONPOSITIVE);
+        raise_error(errw, ERR_NONPOSITIVE);
     const double veloNMean = 0.5 * ((vL0 + vR0) * n0 + (vL1 + vR1) * n1);
     const double pMean = (pL + pR) * 0.5;
     const double aMean = sqrt(gamma * pMean / uMean[0]);
@@ -716,7 +716,7 @@ __global__ __launch_bounds__(kBlock) void k_dt_cell(int32_t nc, int64_t ldc, con
 }
 
 __global__ __launch_bounds__(kBlock) void k_min_final(int32_t n, const double *__restrict__ part,
-                                                      double *__restrict__ out, int32_t *errw) {
+                                                      double *__restrict__ out, double *host_out, int32_t *errw) {
     __shared__ double red[kBlock];
     double d = 3e200;
     for (int32_t k = threadIdx.x; k < n; k += kBlock)
@@ -730,8 +730,9 @@ __global__ __launch_bounds__(kBlock) void k_min_final(int32_t n, const double *_
     }
     if (threadIdx.x == 0) {
         out[0] = red[0];
+        *host_out = red[0];
         if (!isfinite(red[0]))
-            atomicOr(errw, ERRBIT_NAN);
+            raise_error(errw, ERR_NAN);
     }
 }
 
@@ -973,7 +974,7 @@ __global__ __launch_bounds__(kBlock, VIS && !BOUNDARY ? 2 : 1) void k_rhs_face(i
         }
     }
     if (!ok)
-        atomicOr(errw, ERRBIT_NONPOSITIVE);
+        raise_error(errw, ERR_NONPOSITIVE);
     // each side's two terms go to its cell's slot for this face, signed as
     // the cell applies them (negation is exact, so the cell's sums are
     // unchanged bit for bit)
@@ -1044,7 +1045,7 @@ __global__ __launch_bounds__(kBlock) void k_rhs_cell(int32_t nc, int64_t ldc, co
     for (int v = 0; v < 4; v++)
         finite &= isfinite(r[v]);
     if (!finite)
-        atomicOr(errw, ERRBIT_NAN);
+        raise_error(errw, ERR_NAN);
     if (stage == 0) {
 #pragma unroll
         for (int v = 0; v < 4; v++)
@@ -1346,7 +1347,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_wbap_lim(int64_t ldc, int64_t ldf
             for (int c = 0; c < 9; c++)
                 xj[c] = x[rec(j, c, v)];
             if (!face_char_rows(gamma, u, i, j, f, side, ldf, fnc, v, ml, mr))
-                atomicOr(errw, ERRBIT_NONPOSITIVE);
+                raise_error(errw, ERR_NONPOSITIVE);
         }
 #pragma unroll
         for (int order = 3; order >= 1; order--) {
@@ -1470,7 +1471,7 @@ __global__ __launch_bounds__(kBlock, 3) void k_wbap_lim_v2(int64_t ldc, int64_t 
                 uj[c] = (c <= le ? x : above)[rec(j, c, v)];
             double ml[4], mr[4];
             if (!face_char_rows(gamma, u, i, j, f, side, ldf, fnc, v, ml, mr))
-                atomicOr(errw, ERRBIT_NONPOSITIVE);
+                raise_error(errw, ERR_NONPOSITIVE);
 #pragma unroll
             for (int r = 0; r < nr; r++) {
                 double oIn = 0.0;
@@ -1521,11 +1522,6 @@ __global__ __launch_bounds__(kBlock) void k_set(int64_t n, double *__restrict__ 
         p[i] = v;
 }
 
-__global__ __launch_bounds__(kBlock) void k_zero_int(int32_t *p) {
-    if (threadIdx.x == 0 && blockIdx.x == 0)
-        p[0] = 0;
-}
-
 // ========================================================================
 // host side
 // ========================================================================
@@ -1533,17 +1529,18 @@ __global__ __launch_bounds__(kBlock) void k_zero_int(int32_t *p) {
 namespace dndsmi_host {
 
 int check_errw(dndsmi_ctx *c) {
-    int32_t h = 0;
-    DNDSMI_TRY(c->hip(hipMemcpyAsync(&h, c->errw, sizeof(h), hipMemcpyDeviceToHost, c->stream), "hipMemcpyAsync"));
     DNDSMI_TRY(c->hip(hipStreamSynchronize(c->stream), "hipStreamSynchronize"));
-    if (h == 0)
+    volatile int32_t *e = c->host->err;
+    const bool nonpositive = e[ERR_NONPOSITIVE], nan = e[ERR_NAN], bc = e[ERR_BC];
+    if (!nonpositive && !nan && !bc)
         return DNDSMI_OK;
-    hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, c->stream, c->errw);
-    if (h & ERRBIT_NONPOSITIVE) {
+    for (int k = 0; k < ERR_KINDS; k++)
+        e[k] = 0;
+    if (nonpositive) {
         c->err = "non-positive density or sound speed in a flux or boundary state";
         return DNDSMI_ERR_NONPOSITIVE_STATE;
     }
-    if (h & ERRBIT_NAN) {
+    if (nan) {
         c->err = "non-finite value in the right-hand side or time step";
         return DNDSMI_ERR_NAN;
     }
@@ -1913,10 +1910,11 @@ extern "C" int dndsmi_ctx_create(const dndsmi_mesh_view *mesh, const dndsmi_vr_v
         DNDSMI_TRY(c->alloc(c->fslot, int64_t(nfmax) * 8 * ldc));
         DNDSMI_TRY(c->alloc(c->dt_part, int64_t(grid_for(nc)) + 1));
         DNDSMI_TRY(c->alloc(c->dt_min, 1));
-        DNDSMI_TRY(c->alloc(c->errw, 1));
+        DNDSMI_TRY(c->hip(hipHostMalloc(&c->host, sizeof(HostWords), hipHostMallocCoherent), "hipHostMalloc"));
+        std::memset(static_cast<void *>(c->host), 0, sizeof(HostWords));
+        c->errw = c->host->err;
         DNDSMI_TRY(c->alloc(c->xlast, 4 * ldc));
         DNDSMI_TRY(c->alloc(c->dt_tmp, ldc));
-        hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, c->stream, c->errw);
         hipLaunchKernelGGL(k_set, dim3(grid_for(ldf)), dim3(kBlock), 0, c->stream, ldf, c->dlambda_face, 0.0);
         DNDSMI_TRY(c->launch_check("init kernels"));
         DNDSMI_TRY(c->hip(hipStreamSynchronize(c->stream), "hipStreamSynchronize"));
@@ -1953,6 +1951,8 @@ extern "C" void dndsmi_ctx_destroy(dndsmi_ctx *c) {
     c->bdfs.clear();
     for (void *p : c->allocs)
         (void)hipFree(p);
+    if (c->host)
+        (void)hipHostFree(c->host);
     for (hipEvent_t e : c->ev_pool)
         (void)hipEventDestroy(e);
     if (c->own_stream && c->stream)
@@ -1970,7 +1970,6 @@ extern "C" int dndsmi_last_error(const dndsmi_ctx *c, char *buf, size_t n) {
 extern "C" int dndsmi_sync(dndsmi_ctx *c) {
     if (!c)
         return DNDSMI_ERR_INVALID_ARGUMENT;
-    DNDSMI_TRY(c->hip(hipStreamSynchronize(c->stream), "hipStreamSynchronize"));
     return check_errw(c);
 }
 
@@ -2173,7 +2172,8 @@ int launch_dt(dndsmi_ctx *c, const double *u, double cfl, double max_dt, double 
         hipLaunchKernelGGL(k_dt_cell<4>, dim3(g), dim3(kBlock), 0, c->stream, nc, c->ldc, c->gat, c->lambda_face,
                            c->farea, c->vol, cfl, max_dt, dt_out, c->dt_part);
     prof_end(c);
-    hipLaunchKernelGGL(k_min_final, dim3(1), dim3(kBlock), 0, c->stream, int32_t(g), c->dt_part, c->dt_min, c->errw);
+    hipLaunchKernelGGL(k_min_final, dim3(1), dim3(kBlock), 0, c->stream, int32_t(g), c->dt_part, c->dt_min,
+                       &c->host->dt_min, c->errw);
     return c->launch_check("dt kernels");
 }
 
@@ -2418,9 +2418,9 @@ extern "C" int dndsmi_evaluate_dt(dndsmi_ctx *c, dndsmi_array *dt, const dndsmi_
         DNDSMI_TRY(c->launch_check("k_fill_from"));
     }
     if (dtMinall) {
-        DNDSMI_TRY(c->hip(hipMemcpyAsync(dtMinall, c->dt_min, sizeof(double), hipMemcpyDeviceToHost, c->stream),
-                          "hipMemcpyAsync"));
-        DNDSMI_TRY(check_errw(c));
+        const int rc = check_errw(c);
+        *dtMinall = c->host->dt_min;
+        return rc;
     }
     return DNDSMI_OK;
 }
@@ -2446,10 +2446,8 @@ extern "C" int dndsmi_ssprk3_step(dndsmi_ctx *c, dndsmi_array *u, dndsmi_array *
     // fdt: EvaluateDt; the stage update reads dt_i (local) or the device minimum
     DNDSMI_TRY(launch_dt(c, u->d, CFL, MaxDt, c->dt_tmp));
     // the global minimum sets the stage times (one host read per step)
-    double dtmin = 0;
-    DNDSMI_TRY(c->hip(hipMemcpyAsync(&dtmin, c->dt_min, sizeof(double), hipMemcpyDeviceToHost, c->stream),
-                      "hipMemcpyAsync"));
     DNDSMI_TRY(check_errw(c));
+    const double dtmin = c->host->dt_min;
     if (dt_out)
         *dt_out = dtmin;
     const double Coef[3] = {1.0, 0.25, 2.0 / 3.0};
@@ -2530,10 +2528,8 @@ extern "C" int dndsmi_ssprk3_step_mixed(dndsmi_ctx *c, dndsmi_array *u, dndsmi_a
     }
     // the step's dt: from the plain run's state in a window, used by both runs
     DNDSMI_TRY(launch_dt(c, window ? c->ws_sh_u : u->d, CFL, MaxDt, c->dt_tmp));
-    double dtmin = 0;
-    DNDSMI_TRY(c->hip(hipMemcpyAsync(&dtmin, c->dt_min, sizeof(double), hipMemcpyDeviceToHost, c->stream),
-                      "hipMemcpyAsync"));
     DNDSMI_TRY(check_errw(c));
+    const double dtmin = c->host->dt_min;
     if (dt_out)
         *dt_out = dtmin;
     if (!window) {

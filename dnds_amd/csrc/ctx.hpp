@@ -102,7 +102,8 @@ struct dndsmi_ctx {
     bool straight_faces = false; // every face's normal is bitwise the same at its three LINE_3 points
     double *dt_part = nullptr; // [grid] partial minima
     double *dt_min = nullptr;  // [1]
-    int32_t *errw = nullptr;   // [1] error bits
+    dndsmi_dev::HostWords *host = nullptr; // pinned host memory that the kernels write
+    int32_t *errw = nullptr;   // host->err
     double *xlast = nullptr;   // [ldc][4] SSP-RK3 / dual-time xLast
     double *dt_tmp = nullptr;  // [ldc]
     // multicolour LU-SGS: greedy colouring in cell order, cells of a colour
@@ -216,7 +217,8 @@ namespace dndsmi_host {
 // profiling brackets around one launch (no-ops unless profiling is on)
 void prof_begin(dndsmi_ctx *c, int id);
 void prof_end(dndsmi_ctx *c);
-// reads and clears the device error word; a status for the first bit set
+// waits for the stream, reads and clears the error words; a status for the first
+// one set
 int check_errw(dndsmi_ctx *c);
 // the learned warm start inside the mixed-precision step (warmstart.hip):
 // before a stage's sweeps, the change of the means since the previous stage

@@ -19,8 +19,21 @@ enum : int32_t {
     BC_INNER = -1, BC_WALL = 1, BC_FARFIELD = 2, BC_WALL_EULER = 3, BC_WALL_NOSLIP = 4,
     BC_DMRFAR = -2, BC_RTFAR = -3, BC_IVFAR = -4, BC_2DRIEMANNFAR = -5
 };
-// bits of the device error word
-enum : int32_t { ERRBIT_NONPOSITIVE = 1, ERRBIT_NAN = 2, ERRBIT_BC = 4 };
+// What the host reads back in the middle of a step lies in pinned host memory
+// that the kernels write themselves (fine-grained, so a finished kernel's
+// stores are there): after a wait for the stream it is read in place.  With
+// copies of a few bytes to pageable memory the wait for an idle stream took 21
+// us, and 0.5 now.
+enum : int32_t { ERR_NONPOSITIVE = 0, ERR_NAN = 1, ERR_BC = 2, ERR_KINDS = 3 };
+constexpr int kMaxKrylov = 32;
+struct HostWords {
+    int32_t err[4]; // one word per kind of error, set by the kernels
+    double dt_min, res[4], beta;
+    double h[(kMaxKrylov + 1) * kMaxKrylov], y[kMaxKrylov];
+};
+__device__ __forceinline__ void raise_error(int32_t *err, int32_t kind) {
+    __hip_atomic_store(err + kind, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 __device__ inline bool is_far(int32_t bc) {
     return bc == BC_FARFIELD || bc == BC_DMRFAR || bc == BC_RTFAR || bc == BC_IVFAR || bc == BC_2DRIEMANNFAR;

@@ -160,7 +160,6 @@ __global__ __launch_bounds__(kBlock) void k_lusgs_matvec(int32_t nc, int64_t ldc
 // ------------------------------------------------------- GMRES vectors ----
 // Per-block partial sums of nq dot products w . V_q (V_q = V + q ldv), each
 // cell's 4 products summed in order, then a fixed tree over the block.
-constexpr int kMaxDots = 33;
 __global__ __launch_bounds__(kBlock) void k_gm_dots(int32_t nc, int32_t nq, const double *__restrict__ w,
                                                     const double *__restrict__ V, int64_t ldv,
                                                     double *__restrict__ part) {
@@ -191,9 +190,10 @@ __global__ __launch_bounds__(kBlock) void k_gm_dots(int32_t nc, int32_t nq, cons
 }
 
 // folds the partials of each dot product in a fixed order; out[q * ostride]
-// = the sum, or its square root (norms)
+// = the sum, or its square root (norms), in host_out too
 __global__ __launch_bounds__(64) void k_gm_dots_final(int32_t nblk, int32_t nq, const double *__restrict__ part,
-                                                      int32_t take_sqrt, double *__restrict__ out, int32_t ostride) {
+                                                      int32_t take_sqrt, double *__restrict__ out, int32_t ostride,
+                                                      double *host_out) {
     const int lane = threadIdx.x;
     for (int32_t q = 0; q < nq; q++) {
         double a = 0.0;
@@ -201,8 +201,11 @@ __global__ __launch_bounds__(64) void k_gm_dots_final(int32_t nblk, int32_t nq, 
             a += part[int64_t(q) * nblk + b];
         for (int off = 32; off > 0; off >>= 1)
             a += __shfl_down(a, off, 64);
-        if (lane == 0)
-            out[q * ostride] = take_sqrt ? sqrt(a) : a;
+        if (lane == 0) {
+            const double d = take_sqrt ? sqrt(a) : a;
+            out[q * ostride] = d;
+            host_out[q * ostride] = d;
+        }
     }
 }
 
@@ -297,7 +300,7 @@ __global__ __launch_bounds__(kBlock) void k_lusgs_sweep(int32_t n, int32_t b, in
         uIncNew[4 * int64_t(i) + v] = o;
     }
     if (!finite)
-        atomicOr(errw, ERRBIT_NAN);
+        raise_error(errw, ERR_NAN);
 }
 
 // Dual-time right-hand side of ImplicitEulerDualTimeStep::Step
@@ -363,7 +366,7 @@ __global__ __launch_bounds__(kBlock) void k_residual(int32_t nc, const double *_
 
 // one wavefront per variable folds the block partials in a fixed order
 __global__ __launch_bounds__(kBlock) void k_residual_final(int32_t nblk, int32_t P, const double *__restrict__ part,
-                                                           double *__restrict__ res) {
+                                                           double *__restrict__ res, double *host_res) {
     const int v = threadIdx.x / 64, lane = threadIdx.x % 64;
     if (v >= 4)
         return;
@@ -374,8 +377,10 @@ __global__ __launch_bounds__(kBlock) void k_residual_final(int32_t nblk, int32_t
         const double o = __shfl_down(a, off, 64);
         a = P >= 3 ? fmax(a, o) : a + o;
     }
-    if (lane == 0)
+    if (lane == 0) {
         res[v] = a;
+        host_res[v] = a;
+    }
 }
 
 // fdtau's division by alphaDiag (DNDS_FV_EulerSolver.hpp:846-847)
@@ -598,10 +603,10 @@ int gmres_solve(dndsmi_ctx *c, double alpha, const double *b, const double *u, d
         DNDSMI_TRY(launch_lusgs_sweep<true>(c, alpha, in, u, out, out));
         return launch_lusgs_sweep<false>(c, alpha, in, u, out, out);
     };
-    auto dots = [&](const double *w, const double *Vq, int nq, int take_sqrt, double *out, int ostride) -> int {
+    auto dots = [&](const double *w, const double *Vq, int nq, int take_sqrt, double *out, int ostride, double *host) -> int {
         hipLaunchKernelGGL(k_gm_dots, dim3(gc), dim3(kBlock), 0, c->stream, nc, nq, w, Vq, ldv, c->gm_part);
         hipLaunchKernelGGL(k_gm_dots_final, dim3(1), dim3(64), 0, c->stream, int32_t(gc), nq, c->gm_part, take_sqrt,
-                           out, ostride);
+                           out, ostride, host);
         return c->launch_check("GMRES dot products");
     };
     DNDSMI_TRY(FML(b, MLb));
@@ -610,10 +615,9 @@ int gmres_solve(dndsmi_ctx *c, double alpha, const double *b, const double *u, d
         DNDSMI_TRY(launch_lusgs_matvec(c, alpha, u, x, Vt));
         DNDSMI_TRY(FML(Vt, V));
         hipLaunchKernelGGL(k_gm_axpy, dim3(gn), dim3(kBlock), 0, c->stream, n, V, MLb, -1.0);
-        DNDSMI_TRY(dots(V, V, 1, 1, c->gm_y, 1));
-        double beta = 0.0;
-        DNDSMI_TRY(c->hip(hipMemcpyAsync(&beta, c->gm_y, sizeof(double), hipMemcpyDeviceToHost, c->stream), "copy"));
+        DNDSMI_TRY(dots(V, V, 1, 1, c->gm_y, 1, &c->host->beta));
         DNDSMI_TRY(c->hip(hipStreamSynchronize(c->stream), "hipStreamSynchronize"));
+        const double beta = c->host->beta;
         if (std::fabs(beta) < 1e-200 || iRestart == c->n_gmres_iter)
             break;
         hipLaunchKernelGGL(k_gm_scale, dim3(gn), dim3(kBlock), 0, c->stream, n, V, -1.0 / beta, nullptr);
@@ -621,27 +625,26 @@ int gmres_solve(dndsmi_ctx *c, double alpha, const double *b, const double *u, d
             double *Vj = V + int64_t(j) * ldv, *Vn = Vj + ldv;
             DNDSMI_TRY(launch_lusgs_matvec(c, alpha, u, Vj, Vt));
             DNDSMI_TRY(FML(Vt, Vn));
-            DNDSMI_TRY(dots(Vn, V, j + 1, 0, c->gm_h + j, k)); // h(i, j), i <= j
+            DNDSMI_TRY(dots(Vn, V, j + 1, 0, c->gm_h + j, k, c->host->h + j)); // h(i, j), i <= j
             hipLaunchKernelGGL(k_gm_combine, dim3(gn), dim3(kBlock), 0, c->stream, n, j + 1, Vn, V, ldv, c->gm_h + j,
                                k, 1);
-            DNDSMI_TRY(dots(Vn, Vn, 1, 1, c->gm_h + int64_t(j + 1) * k + j, 1)); // h(j + 1, j)
+            const int64_t sub = int64_t(j + 1) * k + j; // h(j + 1, j)
+            DNDSMI_TRY(dots(Vn, Vn, 1, 1, c->gm_h + sub, 1, c->host->h + sub));
             hipLaunchKernelGGL(k_gm_scale, dim3(gn), dim3(kBlock), 0, c->stream, n, Vn, 0.0,
-                               c->gm_h + int64_t(j + 1) * k + j);
+                               c->gm_h + sub);
             DNDSMI_TRY(c->launch_check("GMRES Arnoldi"));
         }
-        DNDSMI_TRY(c->hip(hipMemcpyAsync(H.data(), c->gm_h, sizeof(double) * H.size(), hipMemcpyDeviceToHost,
-                                         c->stream),
-                          "copy"));
         DNDSMI_TRY(c->hip(hipStreamSynchronize(c->stream), "hipStreamSynchronize"));
+        std::copy_n(c->host->h, H.size(), H.begin());
         for (int i = 0; i <= k; i++) // below the subdiagonal: zero (never written on the device)
             for (int j = 0; j < i - 1; j++)
                 H[size_t(i) * k + j] = 0.0;
         const std::vector<double> y = hessenberg_lsq_householder(H, k, beta);
-        DNDSMI_TRY(c->hip(hipMemcpyAsync(c->gm_y, y.data(), sizeof(double) * size_t(k), hipMemcpyHostToDevice,
+        std::copy_n(y.begin(), k, c->host->y); // free again: the next wait comes before the next y
+        DNDSMI_TRY(c->hip(hipMemcpyAsync(c->gm_y, c->host->y, sizeof(double) * size_t(k), hipMemcpyHostToDevice,
                                          c->stream),
                           "copy"));
         hipLaunchKernelGGL(k_gm_combine, dim3(gn), dim3(kBlock), 0, c->stream, n, k, x, V, ldv, c->gm_y, 1, 0);
-        DNDSMI_TRY(c->hip(hipStreamSynchronize(c->stream), "hipStreamSynchronize")); // y lives on the host stack
         DNDSMI_TRY(c->launch_check("GMRES update"));
     }
     return DNDSMI_OK;
@@ -669,11 +672,11 @@ int residual(dndsmi_ctx *c, const double *r, double *x, int32_t P, int32_t vol_w
     const unsigned g = grid_for(c->nc);
     hipLaunchKernelGGL(k_residual, dim3(g), dim3(kBlock), 0, c->stream, int32_t(c->nc), r, x, c->vol, P, vol_wise,
                        part);
-    hipLaunchKernelGGL(k_residual_final, dim3(1), dim3(kBlock), 0, c->stream, int32_t(g), P, part, res_dev);
+    hipLaunchKernelGGL(k_residual_final, dim3(1), dim3(kBlock), 0, c->stream, int32_t(g), P, part, res_dev,
+                       c->host->res);
     DNDSMI_TRY(c->launch_check("residual kernels"));
-    double h[4];
-    DNDSMI_TRY(c->hip(hipMemcpyAsync(h, res_dev, sizeof(h), hipMemcpyDeviceToHost, c->stream), "hipMemcpyAsync"));
     DNDSMI_TRY(check_errw(c));
+    const double *h = c->host->res;
     for (int v = 0; v < 4; v++)
         res_host[v] = P >= 3 ? h[v] : (P == 2 ? std::sqrt(h[v]) : h[v]);
     return DNDSMI_OK;
@@ -735,7 +738,7 @@ extern "C" int dndsmi_lusgs_matrix_vec(dndsmi_ctx *c, double alphaDiag, const dn
 }
 
 extern "C" int dndsmi_set_linear_solver(dndsmi_ctx *c, int32_t gmres_code, int32_t n_space, int32_t n_iter) {
-    if (!c || gmres_code < 0 || gmres_code > 2 || n_space < 1 || n_space > kMaxDots - 1 || n_iter < 0)
+    if (!c || gmres_code < 0 || gmres_code > 2 || n_space < 1 || n_space > kMaxKrylov || n_iter < 0)
         return DNDSMI_ERR_INVALID_ARGUMENT;
     c->gmres_code = gmres_code, c->n_gmres_space = n_space, c->n_gmres_iter = n_iter;
     return DNDSMI_OK;
