@@ -130,6 +130,7 @@ struct dndsmi_ctx {
     // cell and the face area; per position the volume
     int32_t *sc_jf = nullptr, *sc_jb = nullptr, *sc_face = nullptr;
     double *sc_n0 = nullptr, *sc_n1 = nullptr, *sc_area = nullptr, *sc_vol = nullptr;
+    double *sc_cf = nullptr, *sc_lam = nullptr; // the solver's coefficients per slot, of the last matrix init
     // mixed precision (allocated on first use): FP32 copy of A^-1 B, FP32
     // correction vectors, FP32 face fluxes
     float *M32 = nullptr;             // A^-1 B, 21 vectors per cell and slot (ab_vec)

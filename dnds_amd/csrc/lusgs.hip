@@ -95,7 +95,8 @@ __global__ __launch_bounds__(kBlock) void k_lusgs_init(int32_t nc, int64_t ldc, 
                                                        const double *__restrict__ sV,
                                                        const double *__restrict__ lambda_face,
                                                        const double *__restrict__ dtau, double dt, double alpha,
-                                                       double *__restrict__ jinv, double *__restrict__ jdiag) {
+                                                       double *__restrict__ jinv, double *__restrict__ jdiag,
+                                                       double *__restrict__ cf, double *__restrict__ lam) {
     const int32_t p = xcd_block() * blockDim.x + threadIdx.x;
     if (p >= nc)
         return;
@@ -106,60 +107,154 @@ __global__ __launch_bounds__(kBlock) void k_lusgs_init(int32_t nc, int64_t ldc, 
         const int32_t f = sf[s * ldc + p];
         if (f < 0)
             continue;
-        fp += (0.5 * alpha) * sS[s * ldc + p] * lambda_face[f] / v;
+        const double S = sS[s * ldc + p], l = lambda_face[f];
+        fp += (0.5 * alpha) * S * l / v;
+        cf[s * ldc + p] = (0.5 * alpha) * S / v;
+        lam[s * ldc + p] = l;
     }
     jdiag[p] = fp + alpha * 0.0; // jacobianCell = fpDivisor I + alphaDiag 0 (source Jacobian)
     jinv[p] = 1.0 / (fp + alpha * 0.0);
 }
 
-// LUSGSMatrixVec (DNDS_FV_EulerEvaluator.cpp:1062-1145), per scan position:
-// Ax_i = D_i x_i - sum_f (alpha/2) S_f / V_i dF(u_j, x_j) over every
-// neighbour (the earlier ones and the later ones), faces in cell2face order
-template <int NF>
-__global__ __launch_bounds__(kBlock) void k_lusgs_matvec(int32_t nc, int64_t ldc, const int32_t *__restrict__ cells,
-                                                         const int32_t *__restrict__ jf,
-                                                         const int32_t *__restrict__ jb,
-                                                         const int32_t *__restrict__ sf,
-                                                         const double *__restrict__ sn0,
-                                                         const double *__restrict__ sn1,
-                                                         const double *__restrict__ sS,
-                                                         const double *__restrict__ sV,
-                                                         const double *__restrict__ lambda_face,
-                                                         const double *__restrict__ jdiag, double gamma, double alpha,
-                                                         const double *__restrict__ u, const double *__restrict__ x,
-                                                         double *__restrict__ Ax) {
-    const int32_t p = xcd_block() * blockDim.x + threadIdx.x;
-    if (p >= nc)
-        return;
-    const int32_t i = cells[p];
-    const double vi = sV[p];
-    double buf[4] = {0, 0, 0, 0};
+// the scan arrays of ensure_lusgs_scan, the diagonal and what the sweeps share
+struct LusgsScan {
+    int64_t ldc;
+    const int32_t *cells, *jf, *jb, *sf;
+    const double *n0, *n1, *area, *vol, *lambda, *jinv, *jdiag;
+    double *cf, *lam; // [slot][ldc] c_f and lambda of the slot's face (k_lusgs_init)
+    double gamma, alpha;
+    int32_t *errw;
+};
+
+// buf -= sum over the slots' neighbours c_f dF(u_j, x_j), c_f = (alpha/2) S_f /
+// V_i, faces in cell2face order; FORWARD: the earlier neighbours, BACKWARD:
+// the later ones.  PRE: c_f and lambda as the last k_lusgs_init stored them by
+// slot (the solver's own sweeps), which saves a division and the load that
+// waits for the face's number; else from lambdaFace and alpha as they are now.
+template <int NF, bool PRE, bool FORWARD, bool BACKWARD>
+__device__ __forceinline__ void lusgs_row(const LusgsScan &sc, int32_t p, const double *__restrict__ u,
+                                          const double *x, double buf[4]) {
+    const double vi = PRE ? 0.0 : sc.vol[p];
 #pragma unroll
     for (int s = 0; s < NF; s++) {
-        const int32_t a = jf[s * ldc + p], b = jb[s * ldc + p];
+        const int64_t q = s * sc.ldc + p;
+        const int32_t a = FORWARD ? sc.jf[q] : -1, b = BACKWARD ? sc.jb[q] : -1;
         const int32_t j = a >= 0 ? a : b;
         if (j < 0)
             continue;
-        const int32_t f = sf[s * ldc + p];
         double uj[4], xj[4], dF[4];
 #pragma unroll
         for (int v = 0; v < 4; v++)
             uj[v] = u[4 * int64_t(j) + v], xj[v] = x[4 * int64_t(j) + v];
-        flux_jacobian_times_du(gamma, uj, sn0[s * ldc + p], sn1[s * ldc + p], xj, lambda_face[f], dF);
-        const double cf = (0.5 * alpha) * sS[s * ldc + p] / vi;
+        const double lam = PRE ? sc.lam[q] : sc.lambda[sc.sf[q]];
+        flux_jacobian_times_du(sc.gamma, uj, sc.n0[q], sc.n1[q], xj, lam, dF);
+        const double cf = PRE ? sc.cf[q] : (0.5 * sc.alpha) * sc.area[q] / vi;
 #pragma unroll
         for (int v = 0; v < 4; v++)
             buf[v] -= cf * dF[v];
     }
-    const double d = jdiag[p];
+}
+
+// LUSGSMatrixVec (DNDS_FV_EulerEvaluator.cpp:1062-1145) per scan position:
+// Ax_i = D_i x_i - sum_f (alpha/2) S_f / V_i dF(u_j, x_j) over every
+// neighbour (the earlier ones and the later ones).  With `first` > 0 also the
+// first colour of the forward sweep on Ax, which has no earlier neighbours:
+// inc = jinv Ax at the scan positions below `first`.
+template <int NF, bool PRE>
+__global__ __launch_bounds__(kBlock) void k_lusgs_matvec(int32_t nc, LusgsScan sc, const double *__restrict__ u,
+                                                         const double *__restrict__ x, double *__restrict__ Ax,
+                                                         int32_t first, double *__restrict__ inc) {
+    const int32_t p = xcd_block() * blockDim.x + threadIdx.x;
+    if (p >= nc)
+        return;
+    const int64_t i = 4 * int64_t(sc.cells[p]);
+    double buf[4] = {0, 0, 0, 0};
+    lusgs_row<NF, PRE, true, true>(sc, p, u, x, buf);
+    const double d = sc.jdiag[p];
+    const double di = p < first ? sc.jinv[p] : 0.0;
+    bool finite = true;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const double a = d * x[i + v] - buf[v];
+        Ax[i + v] = a;
+        if (p < first) {
+            const double o = di * a;
+            finite &= isfinite(o);
+            inc[i + v] = o;
+        }
+    }
+    if (!finite)
+        raise_error(sc.errw, ERR_NAN);
+}
+
+// One colour of an LU-SGS sweep (UpdateLUSGSForward / UpdateLUSGSBackward,
+// DNDS_FV_EulerEvaluator.cpp:1149-1357), scan positions [b, b + n): forward
+//   uIncNew_i = jinv_i (rhs_i - sum_{earlier j} c_f dF(u_j, uInc_j))
+// backward
+//   uIncNew_i += jinv_i (- sum_{later j} c_f dF(u_j, uInc_j)),
+// the normal pointing out of i.  "Earlier" is a lower colour, "later" a higher
+// one.  TURN: the last colour's forward and backward update in one (nothing
+// comes later, so the backward sum is empty).
+template <int NF, bool PRE, bool FORWARD, bool TURN>
+__global__ __launch_bounds__(kBlock) void k_lusgs_sweep(int32_t n, int32_t b, LusgsScan sc,
+                                                        const double *__restrict__ rhs, const double *__restrict__ u,
+                                                        const double *uInc, double *uIncNew) {
+    const int32_t t = xcd_block() * blockDim.x + threadIdx.x;
+    if (t >= n)
+        return;
+    const int32_t p = b + t;
+    const int64_t i = 4 * int64_t(sc.cells[p]);
+    double buf[4];
 #pragma unroll
     for (int v = 0; v < 4; v++)
-        Ax[4 * int64_t(i) + v] = d * x[4 * int64_t(i) + v] - buf[v];
+        buf[v] = FORWARD ? rhs[i + v] : 0.0;
+    lusgs_row<NF, PRE, FORWARD, !FORWARD>(sc, p, u, uInc, buf);
+    const double d = sc.jinv[p];
+    bool finite = true;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        double o = d * buf[v];
+        if (!FORWARD)
+            o = uIncNew[i + v] + o;
+        if (TURN)
+            o = o + d * 0.0;
+        finite &= isfinite(o);
+        uIncNew[i + v] = o;
+    }
+    if (!finite)
+        raise_error(sc.errw, ERR_NAN);
 }
 
 // ------------------------------------------------------- GMRES vectors ----
+// A GMRES iteration is bound by the number of its dependent launches (4 us
+// each, 15 per Krylov vector on a small mesh): of a vector's work the dots are
+// one, the subtraction with the new norm's partials one and the scaling one.
+// Up to kFoldBlocks workgroups each workgroup of the second and third folds
+// the first's and second's partials itself, in the order k_gm_dots_final has;
+// beyond, reading all partials in every workgroup costs more than the two
+// launches.  Per implicit iteration (10 vectors, 2 restarts), us, separate
+// axpy launches before -> fused, not folded -> folded:
+// 1.5k cells 1265 -> - -> 1089, 29k 1576 -> 1265 -> 1187, 68k 1902 -> 1616 ->
+// 1483, 256k (1000 workgroups) 3246 -> 2948 -> 2666, 600k (2344) 8479 -> 6853
+// (launches -> folded), 1M (3907) 11410 -> 11646.
+constexpr int kFoldBlocks = 2048;
+
 // Per-block partial sums of nq dot products w . V_q (V_q = V + q ldv), each
-// cell's 4 products summed in order, then a fixed tree over the block.
+// cell's 4 products summed in order, then a fixed tree over the block of 256:
+// sum() on values of all threads gives it in thread 0.
+__device__ __forceinline__ double block_sum(double a, double *red) {
+    red[threadIdx.x] = a;
+    __syncthreads();
+    for (int st = kBlock / 2; st > 0; st >>= 1) {
+        if (threadIdx.x < st)
+            red[threadIdx.x] += red[threadIdx.x + st];
+        __syncthreads();
+    }
+    const double s = red[0];
+    __syncthreads();
+    return s;
+}
+
 __global__ __launch_bounds__(kBlock) void k_gm_dots(int32_t nc, int32_t nq, const double *__restrict__ w,
                                                     const double *__restrict__ V, int64_t ldv,
                                                     double *__restrict__ part) {
@@ -176,32 +271,31 @@ __global__ __launch_bounds__(kBlock) void k_gm_dots(int32_t nc, int32_t nq, cons
 #pragma unroll
             for (int v = 0; v < 4; v++)
                 a += wi[v] * V[q * ldv + 4 * int64_t(i) + v];
-        red[threadIdx.x] = a;
-        __syncthreads();
-        for (int st = kBlock / 2; st > 0; st >>= 1) {
-            if (threadIdx.x < st)
-                red[threadIdx.x] += red[threadIdx.x + st];
-            __syncthreads();
-        }
+        const double s = block_sum(a, red);
         if (threadIdx.x == 0)
-            part[int64_t(q) * gridDim.x + blockIdx.x] = red[0];
-        __syncthreads();
+            part[int64_t(q) * gridDim.x + blockIdx.x] = s;
     }
 }
 
-// folds the partials of each dot product in a fixed order; out[q * ostride]
-// = the sum, or its square root (norms), in host_out too
+// one wave: the sum of a dot product's partials in a fixed order, in lane 0
+__device__ __forceinline__ double fold_partials(int32_t nblk, const double *__restrict__ part) {
+    const int lane = threadIdx.x & 63;
+    double a = 0.0;
+    for (int32_t b = lane; b < nblk; b += 64)
+        a += part[b];
+    for (int off = 32; off > 0; off >>= 1)
+        a += __shfl_down(a, off, 64);
+    return a;
+}
+
+// folds the partials of each dot product; out[q * ostride] = the sum, or its
+// square root (norms), in host_out too
 __global__ __launch_bounds__(64) void k_gm_dots_final(int32_t nblk, int32_t nq, const double *__restrict__ part,
                                                       int32_t take_sqrt, double *__restrict__ out, int32_t ostride,
                                                       double *host_out) {
-    const int lane = threadIdx.x;
     for (int32_t q = 0; q < nq; q++) {
-        double a = 0.0;
-        for (int32_t b = lane; b < nblk; b += 64)
-            a += part[int64_t(q) * nblk + b];
-        for (int off = 32; off > 0; off >>= 1)
-            a += __shfl_down(a, off, 64);
-        if (lane == 0) {
+        const double a = fold_partials(nblk, part + int64_t(q) * nblk);
+        if (threadIdx.x == 0) {
             const double d = take_sqrt ? sqrt(a) : a;
             out[q * ostride] = d;
             host_out[q * ostride] = d;
@@ -209,98 +303,106 @@ __global__ __launch_bounds__(64) void k_gm_dots_final(int32_t nblk, int32_t nq, 
     }
 }
 
-// y += x * a (ArrayDOFV::addTo, DNDS_DerivedArray.hpp:372-377)
-__global__ __launch_bounds__(kBlock) void k_gm_axpy(int64_t n, double *__restrict__ y, const double *__restrict__ x,
-                                                    double a) {
+// y += x * a (ArrayDOFV::addTo, DNDS_DerivedArray.hpp:372-377) and the block
+// partials of |y|^2
+__global__ __launch_bounds__(kBlock) void k_gm_axpy(int32_t nc, double *__restrict__ y, const double *__restrict__ x,
+                                                    double a, double *__restrict__ part) {
+    __shared__ double red[kBlock];
+    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    double s = 0.0;
+    if (i < nc)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int64_t k = 4 * int64_t(i) + v;
+            const double o = y[k] + x[k] * a;
+            y[k] = o;
+            s += o * o;
+        }
+    s = block_sum(s, red);
+    if (threadIdx.x == 0)
+        part[blockIdx.x] = s;
+}
+
+// v *= a, with a given, or a = 1 / h with h = sqrt of the folded partials
+// (every workgroup folds them: FOLD, nblk <= kFoldBlocks) or read from h_dev
+template <bool FOLD>
+__global__ __launch_bounds__(kBlock) void k_gm_scale(int64_t n, double *__restrict__ v, double a, int32_t nblk,
+                                                     const double *__restrict__ part, const double *__restrict__ h_dev,
+                                                     double *host_out) {
+    __shared__ double h;
+    if (FOLD) {
+        if (threadIdx.x < 64) {
+            const double f = fold_partials(nblk, part);
+            if (threadIdx.x == 0) {
+                h = sqrt(f);
+                if (blockIdx.x == 0)
+                    *host_out = h;
+            }
+        }
+        __syncthreads();
+    }
     const int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (k < n)
-        y[k] += x[k] * a;
+        v[k] *= FOLD ? 1.0 / h : h_dev ? 1.0 / h_dev[0] : a;
 }
 
-// v *= a, with a given, or a = 1 / h[0] read from the device
-__global__ __launch_bounds__(kBlock) void k_gm_scale(int64_t n, double *__restrict__ v, double a,
-                                                     const double *__restrict__ h) {
+// classical Gram-Schmidt subtraction: w += V_i * (-h_i) for i = 0 .. nq-1 in
+// turn, and the block partials of the new |w|^2.  h_i is folded from its
+// partials by every workgroup (FOLD) or read from h_dev[i hstride].
+template <bool FOLD>
+__global__ __launch_bounds__(kBlock) void k_gm_orthogonalize(int32_t nc, int32_t nq, double *__restrict__ w,
+                                                             const double *__restrict__ V, int64_t ldv, int32_t nblk,
+                                                             const double *__restrict__ part,
+                                                             const double *__restrict__ h_dev, int32_t hstride,
+                                                             double *host_out, double *__restrict__ norm_part) {
+    __shared__ double red[kBlock], h[kMaxKrylov];
+    const int wave = threadIdx.x / 64;
+    if (FOLD) {
+        for (int32_t q = wave; q < nq; q += kBlock / 64) {
+            const double f = fold_partials(nblk, part + int64_t(q) * nblk);
+            if ((threadIdx.x & 63) == 0) {
+                h[q] = f;
+                if (blockIdx.x == 0)
+                    host_out[q * hstride] = f;
+            }
+        }
+    } else if (int32_t(threadIdx.x) < nq) {
+        h[threadIdx.x] = h_dev[threadIdx.x * hstride];
+    }
+    __syncthreads();
+    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    double s = 0.0;
+    if (i < nc) {
+        double a[4];
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            a[v] = w[4 * int64_t(i) + v];
+        for (int32_t q = 0; q < nq; q++)
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                a[v] += V[q * ldv + 4 * int64_t(i) + v] * -h[q];
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            w[4 * int64_t(i) + v] = a[v];
+            s += a[v] * a[v];
+        }
+    }
+    s = block_sum(s, red);
+    if (threadIdx.x == 0)
+        norm_part[blockIdx.x] = s;
+}
+
+// x += V_j y_j for j = 0 .. nq-1 in turn, y on the device
+__global__ __launch_bounds__(kBlock) void k_gm_update(int64_t n, int32_t nq, double *__restrict__ x,
+                                                      const double *__restrict__ V, int64_t ldv,
+                                                      const double *__restrict__ y) {
     const int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (k >= n)
         return;
-    const double s = h ? 1.0 / h[0] : a;
-    v[k] *= s;
-}
-
-// classical Gram-Schmidt subtraction: v += V_i * (-h_i) for i = 0 .. nq-1 in
-// turn, h_i = h[i * hstride] on the device; or, with sign +1, x += V_j y_j
-__global__ __launch_bounds__(kBlock) void k_gm_combine(int64_t n, int32_t nq, double *__restrict__ v,
-                                                       const double *__restrict__ V, int64_t ldv,
-                                                       const double *__restrict__ h, int32_t hstride, int32_t negate) {
-    const int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (k >= n)
-        return;
-    double a = v[k];
-    for (int32_t q = 0; q < nq; q++) {
-        const double c = h[q * hstride];
-        a += V[q * ldv + k] * (negate ? -c : c);
-    }
-    v[k] = a;
-}
-
-// One colour of an LU-SGS sweep (UpdateLUSGSForward / UpdateLUSGSBackward,
-// DNDS_FV_EulerEvaluator.cpp:1149-1357), scan positions [b, b + n): forward
-//   uIncNew_i = jinv_i (rhs_i - sum_{earlier j} c_f dF(u_j, uInc_j))
-// backward
-//   uIncNew_i += jinv_i (- sum_{later j} c_f dF(u_j, uInc_j)),
-// c_f = (alpha/2) S_f / V_i, the normal pointing out of i, faces in cell2face
-// order.  "Earlier" is a lower colour, "later" a higher one.
-template <int NF, bool FORWARD>
-__global__ __launch_bounds__(kBlock) void k_lusgs_sweep(int32_t n, int32_t b, int64_t ldc,
-                                                        const int32_t *__restrict__ cells,
-                                                        const int32_t *__restrict__ sj,
-                                                        const int32_t *__restrict__ sf,
-                                                        const double *__restrict__ sn0,
-                                                        const double *__restrict__ sn1,
-                                                        const double *__restrict__ sS,
-                                                        const double *__restrict__ sV,
-                                                        const double *__restrict__ lambda_face,
-                                                        const double *__restrict__ jinv, double gamma, double alpha,
-                                                        const double *__restrict__ rhs, const double *__restrict__ u,
-                                                        const double *uInc, double *uIncNew, int32_t *errw) {
-    const int32_t t = xcd_block() * blockDim.x + threadIdx.x;
-    if (t >= n)
-        return;
-    const int32_t p = b + t, i = cells[p];
-    double buf[4];
-#pragma unroll
-    for (int v = 0; v < 4; v++)
-        buf[v] = FORWARD ? rhs[4 * int64_t(i) + v] : 0.0;
-    const double vi = sV[p];
-#pragma unroll
-    for (int s = 0; s < NF; s++) {
-        const int32_t j = sj[s * ldc + p];
-        if (j < 0)
-            continue;
-        const int32_t f = sf[s * ldc + p];
-        const double n0 = sn0[s * ldc + p], n1 = sn1[s * ldc + p];
-        double uj[4], dj[4], dF[4];
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-            uj[v] = u[4 * int64_t(j) + v], dj[v] = uInc[4 * int64_t(j) + v];
-        flux_jacobian_times_du(gamma, uj, n0, n1, dj, lambda_face[f], dF);
-        const double cf = (0.5 * alpha) * sS[s * ldc + p] / vi;
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-            buf[v] -= cf * dF[v];
-    }
-    const double d = jinv[p];
-    bool finite = true;
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-        double o = d * buf[v];
-        if (!FORWARD)
-            o = uIncNew[4 * int64_t(i) + v] + o;
-        finite &= isfinite(o);
-        uIncNew[4 * int64_t(i) + v] = o;
-    }
-    if (!finite)
-        raise_error(errw, ERR_NAN);
+    double a = x[k];
+    for (int32_t q = 0; q < nq; q++)
+        a += V[q * ldv + k] * y[q];
+    x[k] = a;
 }
 
 // Dual-time right-hand side of ImplicitEulerDualTimeStep::Step
@@ -452,6 +554,8 @@ int ensure_lusgs_scan(dndsmi_ctx *c) {
     DNDSMI_TRY(c->alloc(c->sc_n1, n));
     DNDSMI_TRY(c->alloc(c->sc_area, n));
     DNDSMI_TRY(c->alloc(c->sc_vol, c->ldc));
+    DNDSMI_TRY(c->alloc(c->sc_cf, n));
+    DNDSMI_TRY(c->alloc(c->sc_lam, n));
     const int nc = int(c->nc);
     if (c->nfmax == 3)
         hipLaunchKernelGGL(k_lusgs_scan<3>, dim3(grid_for(nc)), dim3(kBlock), 0, c->stream, nc, c->ldc, c->ldf,
@@ -471,52 +575,67 @@ int launch_lusgs_init(dndsmi_ctx *c, const double *dtau, double dt, double alpha
     const int nc = int(c->nc);
     if (c->nfmax == 3)
         hipLaunchKernelGGL(k_lusgs_init<3>, dim3(grid_for(nc)), dim3(kBlock), 0, c->stream, nc, c->ldc, c->col_cells,
-                           c->sc_face, c->sc_area, c->sc_vol, c->lambda_face, dtau, dt, alpha, c->jinv, c->jdiag);
+                           c->sc_face, c->sc_area, c->sc_vol, c->lambda_face, dtau, dt, alpha, c->jinv, c->jdiag,
+                           c->sc_cf, c->sc_lam);
     else
         hipLaunchKernelGGL(k_lusgs_init<4>, dim3(grid_for(nc)), dim3(kBlock), 0, c->stream, nc, c->ldc, c->col_cells,
-                           c->sc_face, c->sc_area, c->sc_vol, c->lambda_face, dtau, dt, alpha, c->jinv, c->jdiag);
+                           c->sc_face, c->sc_area, c->sc_vol, c->lambda_face, dtau, dt, alpha, c->jinv, c->jdiag,
+                           c->sc_cf, c->sc_lam);
     return c->launch_check("k_lusgs_init");
 }
 
+LusgsScan lusgs_scan(const dndsmi_ctx *c, double alpha) {
+    return {c->ldc,    c->col_cells,   c->sc_jf, c->sc_jb, c->sc_face, c->sc_n0,  c->sc_n1,     c->sc_area,
+            c->sc_vol, c->lambda_face, c->jinv,  c->jdiag, c->sc_cf,   c->sc_lam, c->gas.gamma, alpha,
+            c->errw};
+}
+
+template <bool PRE, bool FORWARD, bool TURN>
+int launch_colour(dndsmi_ctx *c, int32_t col, double alpha, const double *rhs, const double *u, const double *uInc,
+                  double *uIncNew) {
+    const int64_t b = c->col_start[col], n = c->col_start[col + 1] - b;
+    if (n == 0)
+        return DNDSMI_OK;
+    prof_begin(c, DNDSMI_K_LUSGS_SWEEP);
+    hipLaunchKernelGGL((c->nfmax == 3 ? k_lusgs_sweep<3, PRE, FORWARD, TURN> : k_lusgs_sweep<4, PRE, FORWARD, TURN>),
+                       dim3(grid_for(n)), dim3(kBlock), 0, c->stream, int32_t(n), int32_t(b), lusgs_scan(c, alpha),
+                       rhs, u, uInc, uIncNew);
+    prof_end(c);
+    return c->launch_check("k_lusgs_sweep");
+}
+
+// a whole forward or backward sweep, as the entry points have it
 template <bool FORWARD>
 int launch_lusgs_sweep(dndsmi_ctx *c, double alpha, const double *rhs, const double *u, const double *uInc,
                        double *uIncNew) {
     DNDSMI_TRY(ensure_lusgs_scan(c));
-    const int32_t *sj = FORWARD ? c->sc_jf : c->sc_jb;
-    for (int32_t kk = 0; kk < c->n_colour; kk++) {
-        const int32_t col = FORWARD ? kk : c->n_colour - 1 - kk;
-        const int64_t b = c->col_start[col], n = c->col_start[col + 1] - b;
-        if (n == 0)
-            continue;
-        prof_begin(c, DNDSMI_K_LUSGS_SWEEP);
-        if (c->nfmax == 3)
-            hipLaunchKernelGGL((k_lusgs_sweep<3, FORWARD>), dim3(grid_for(n)), dim3(kBlock), 0, c->stream,
-                               int32_t(n), int32_t(b), c->ldc, c->col_cells, sj, c->sc_face, c->sc_n0, c->sc_n1,
-                               c->sc_area, c->sc_vol, c->lambda_face, c->jinv, c->gas.gamma, alpha, rhs, u, uInc,
-                               uIncNew, c->errw);
-        else
-            hipLaunchKernelGGL((k_lusgs_sweep<4, FORWARD>), dim3(grid_for(n)), dim3(kBlock), 0, c->stream,
-                               int32_t(n), int32_t(b), c->ldc, c->col_cells, sj, c->sc_face, c->sc_n0, c->sc_n1,
-                               c->sc_area, c->sc_vol, c->lambda_face, c->jinv, c->gas.gamma, alpha, rhs, u, uInc,
-                               uIncNew, c->errw);
-        prof_end(c);
-        DNDSMI_TRY(c->launch_check("k_lusgs_sweep"));
-    }
+    for (int32_t k = 0; k < c->n_colour; k++)
+        DNDSMI_TRY((launch_colour<false, FORWARD, false>(c, FORWARD ? k : c->n_colour - 1 - k, alpha, rhs, u, uInc,
+                                                         uIncNew)));
     return DNDSMI_OK;
 }
 
-int launch_lusgs_matvec(dndsmi_ctx *c, double alpha, const double *u, const double *x, double *Ax) {
+// the solver's forward then backward sweep in place on x, from forward colour
+// `first` on, with the coefficients of the last launch_lusgs_init
+int launch_lusgs_pair(dndsmi_ctx *c, double alpha, const double *rhs, const double *u, double *x, int32_t first) {
+    const int32_t last = c->n_colour - 1;
+    for (int32_t k = first; k < last; k++)
+        DNDSMI_TRY((launch_colour<true, true, false>(c, k, alpha, rhs, u, x, x)));
+    DNDSMI_TRY((launch_colour<true, true, true>(c, last, alpha, rhs, u, x, x)));
+    for (int32_t k = last - 1; k >= 0; k--)
+        DNDSMI_TRY((launch_colour<true, false, false>(c, k, alpha, rhs, u, x, x)));
+    return DNDSMI_OK;
+}
+
+// Ax, and with inc the first colour of the forward sweep on it
+template <bool PRE>
+int launch_lusgs_matvec(dndsmi_ctx *c, double alpha, const double *u, const double *x, double *Ax,
+                        double *inc = nullptr) {
     DNDSMI_TRY(ensure_lusgs_scan(c));
-    const int nc = int(c->nc);
     prof_begin(c, DNDSMI_K_LUSGS_MATVEC);
-    if (c->nfmax == 3)
-        hipLaunchKernelGGL(k_lusgs_matvec<3>, dim3(grid_for(nc)), dim3(kBlock), 0, c->stream, nc, c->ldc, c->col_cells,
-                           c->sc_jf, c->sc_jb, c->sc_face, c->sc_n0, c->sc_n1, c->sc_area, c->sc_vol, c->lambda_face,
-                           c->jdiag, c->gas.gamma, alpha, u, x, Ax);
-    else
-        hipLaunchKernelGGL(k_lusgs_matvec<4>, dim3(grid_for(nc)), dim3(kBlock), 0, c->stream, nc, c->ldc, c->col_cells,
-                           c->sc_jf, c->sc_jb, c->sc_face, c->sc_n0, c->sc_n1, c->sc_area, c->sc_vol, c->lambda_face,
-                           c->jdiag, c->gas.gamma, alpha, u, x, Ax);
+    hipLaunchKernelGGL((c->nfmax == 3 ? k_lusgs_matvec<3, PRE> : k_lusgs_matvec<4, PRE>), dim3(grid_for(c->nc)),
+                       dim3(kBlock), 0, c->stream, int32_t(c->nc), lusgs_scan(c, alpha), u, x, Ax,
+                       inc ? int32_t(c->col_start[1]) : 0, inc);
     prof_end(c);
     return c->launch_check("k_lusgs_matvec");
 }
@@ -599,39 +718,51 @@ int gmres_solve(dndsmi_ctx *c, double alpha, const double *b, const double *u, d
     const int nc = int(c->nc);
     const unsigned gn = grid_for(n), gc = grid_for(nc);
     double *V = c->gm_v, *Vt = V + int64_t(k + 1) * ldv, *MLb = V + int64_t(k + 2) * ldv;
-    auto FML = [&](const double *in, double *out) -> int {
-        DNDSMI_TRY(launch_lusgs_sweep<true>(c, alpha, in, u, out, out));
-        return launch_lusgs_sweep<false>(c, alpha, in, u, out, out);
+    const bool fold = gc <= kFoldBlocks;
+    // out = ML A in through Vt: with more than one colour the product's launch
+    // does the first one's forward update
+    auto MLA = [&](const double *in, double *out) -> int {
+        const bool merge = c->n_colour > 1;
+        DNDSMI_TRY(launch_lusgs_matvec<true>(c, alpha, u, in, Vt, merge ? out : nullptr));
+        return launch_lusgs_pair(c, alpha, Vt, u, out, merge ? 1 : 0);
     };
-    auto dots = [&](const double *w, const double *Vq, int nq, int take_sqrt, double *out, int ostride, double *host) -> int {
-        hipLaunchKernelGGL(k_gm_dots, dim3(gc), dim3(kBlock), 0, c->stream, nc, nq, w, Vq, ldv, c->gm_part);
+    auto fold_dots = [&](int nq, int take_sqrt, double *out, int ostride, double *host) -> int {
         hipLaunchKernelGGL(k_gm_dots_final, dim3(1), dim3(64), 0, c->stream, int32_t(gc), nq, c->gm_part, take_sqrt,
                            out, ostride, host);
         return c->launch_check("GMRES dot products");
     };
-    DNDSMI_TRY(FML(b, MLb));
+    DNDSMI_TRY(launch_lusgs_pair(c, alpha, b, u, MLb, 0));
     std::vector<double> H(size_t(k + 1) * size_t(k));
     for (int32_t iRestart = 0; iRestart <= c->n_gmres_iter; iRestart++) {
-        DNDSMI_TRY(launch_lusgs_matvec(c, alpha, u, x, Vt));
-        DNDSMI_TRY(FML(Vt, V));
-        hipLaunchKernelGGL(k_gm_axpy, dim3(gn), dim3(kBlock), 0, c->stream, n, V, MLb, -1.0);
-        DNDSMI_TRY(dots(V, V, 1, 1, c->gm_y, 1, &c->host->beta));
+        DNDSMI_TRY(MLA(x, V));
+        hipLaunchKernelGGL(k_gm_axpy, dim3(gc), dim3(kBlock), 0, c->stream, nc, V, MLb, -1.0, c->gm_part);
+        DNDSMI_TRY(fold_dots(1, 1, c->gm_y, 1, &c->host->beta));
         DNDSMI_TRY(c->hip(hipStreamSynchronize(c->stream), "hipStreamSynchronize"));
         const double beta = c->host->beta;
         if (std::fabs(beta) < 1e-200 || iRestart == c->n_gmres_iter)
             break;
-        hipLaunchKernelGGL(k_gm_scale, dim3(gn), dim3(kBlock), 0, c->stream, n, V, -1.0 / beta, nullptr);
+        hipLaunchKernelGGL(k_gm_scale<false>, dim3(gn), dim3(kBlock), 0, c->stream, n, V, -1.0 / beta, 0, nullptr,
+                           nullptr, nullptr);
         for (int j = 0; j < k; j++) {
             double *Vj = V + int64_t(j) * ldv, *Vn = Vj + ldv;
-            DNDSMI_TRY(launch_lusgs_matvec(c, alpha, u, Vj, Vt));
-            DNDSMI_TRY(FML(Vt, Vn));
-            DNDSMI_TRY(dots(Vn, V, j + 1, 0, c->gm_h + j, k, c->host->h + j)); // h(i, j), i <= j
-            hipLaunchKernelGGL(k_gm_combine, dim3(gn), dim3(kBlock), 0, c->stream, n, j + 1, Vn, V, ldv, c->gm_h + j,
-                               k, 1);
-            const int64_t sub = int64_t(j + 1) * k + j; // h(j + 1, j)
-            DNDSMI_TRY(dots(Vn, Vn, 1, 1, c->gm_h + sub, 1, c->host->h + sub));
-            hipLaunchKernelGGL(k_gm_scale, dim3(gn), dim3(kBlock), 0, c->stream, n, Vn, 0.0,
-                               c->gm_h + sub);
+            double *h = c->gm_h + j, *hh = c->host->h + j;                             // h(i, j), i <= j
+            double *hs = h + int64_t(j + 1) * k, *hhs = hh + int64_t(j + 1) * k;       // h(j + 1, j)
+            double *norm_part = c->gm_part + int64_t(k) * gc;
+            DNDSMI_TRY(MLA(Vj, Vn));
+            hipLaunchKernelGGL(k_gm_dots, dim3(gc), dim3(kBlock), 0, c->stream, nc, j + 1, Vn, V, ldv, c->gm_part);
+            if (!fold)
+                DNDSMI_TRY(fold_dots(j + 1, 0, h, k, hh));
+            hipLaunchKernelGGL((fold ? k_gm_orthogonalize<true> : k_gm_orthogonalize<false>), dim3(gc), dim3(kBlock),
+                               0, c->stream, nc, j + 1, Vn, V, ldv, int32_t(gc), c->gm_part, h, k, hh, norm_part);
+            if (!fold) {
+                hipLaunchKernelGGL(k_gm_dots_final, dim3(1), dim3(64), 0, c->stream, int32_t(gc), 1, norm_part, 1, hs,
+                                   1, hhs);
+                hipLaunchKernelGGL(k_gm_scale<false>, dim3(gn), dim3(kBlock), 0, c->stream, n, Vn, 0.0, 0, nullptr,
+                                   hs, nullptr);
+            } else {
+                hipLaunchKernelGGL(k_gm_scale<true>, dim3(gn), dim3(kBlock), 0, c->stream, n, Vn, 0.0, int32_t(gc),
+                                   norm_part, nullptr, hhs);
+            }
             DNDSMI_TRY(c->launch_check("GMRES Arnoldi"));
         }
         DNDSMI_TRY(c->hip(hipStreamSynchronize(c->stream), "hipStreamSynchronize"));
@@ -644,7 +775,7 @@ int gmres_solve(dndsmi_ctx *c, double alpha, const double *b, const double *u, d
         DNDSMI_TRY(c->hip(hipMemcpyAsync(c->gm_y, c->host->y, sizeof(double) * size_t(k), hipMemcpyHostToDevice,
                                          c->stream),
                           "copy"));
-        hipLaunchKernelGGL(k_gm_combine, dim3(gn), dim3(kBlock), 0, c->stream, n, k, x, V, ldv, c->gm_y, 1, 0);
+        hipLaunchKernelGGL(k_gm_update, dim3(gn), dim3(kBlock), 0, c->stream, n, k, x, V, ldv, c->gm_y);
         DNDSMI_TRY(c->launch_check("GMRES update"));
     }
     return DNDSMI_OK;
@@ -656,10 +787,8 @@ int gmres_solve(dndsmi_ctx *c, double alpha, const double *b, const double *u, d
 int fsolve(dndsmi_ctx *c, const double *dtau, double dt, double alpha, const double *rhs, const double *u,
            double *xinc) {
     DNDSMI_TRY(launch_lusgs_init(c, dtau, dt, alpha));
-    if (c->gmres_code == 0 || c->gmres_code == 2) {
-        DNDSMI_TRY(launch_lusgs_sweep<true>(c, alpha, rhs, u, xinc, xinc));
-        DNDSMI_TRY(launch_lusgs_sweep<false>(c, alpha, rhs, u, xinc, xinc));
-    }
+    if (c->gmres_code == 0 || c->gmres_code == 2)
+        DNDSMI_TRY(launch_lusgs_pair(c, alpha, rhs, u, xinc, 0));
     if (c->gmres_code != 0)
         DNDSMI_TRY(gmres_solve(c, alpha, rhs, u, xinc));
     return DNDSMI_OK;
@@ -734,7 +863,7 @@ extern "C" int dndsmi_lusgs_matrix_vec(dndsmi_ctx *c, double alphaDiag, const dn
         c->err = "LUSGSMatrixVec needs a LUSGSMatrixInit first";
         return DNDSMI_ERR_INVALID_ARGUMENT;
     }
-    return launch_lusgs_matvec(c, alphaDiag, u->d, uInc->d, AuInc->d);
+    return launch_lusgs_matvec<false>(c, alphaDiag, u->d, uInc->d, AuInc->d);
 }
 
 extern "C" int dndsmi_set_linear_solver(dndsmi_ctx *c, int32_t gmres_code, int32_t n_space, int32_t n_iter) {

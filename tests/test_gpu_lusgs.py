@@ -207,3 +207,37 @@ def test_gmres_implicit_iterations_match_oracle(code):
                                   scan2cell=ev.LUSGSScanOrder())
     assert rel_err(ou, ol) > 1e-8
     ev.SetLinearSolver(0)
+
+
+@pytest.mark.parametrize("nx,ny,code", [(1, 1, 0), (5, 1, 1), (51, 5, 1), (16, 16, 2), (257, 1, 1), (129, 128, 2),
+                                        (1024, 512, 1), (1025, 512, 1)])
+def test_gmres_vectors_at_block_and_fold_edges(nx, ny, code):
+    """One cell (one colour), cell counts around a workgroup of 256, and the
+    last mesh whose vector kernels fold the dot products themselves (2048
+    workgroups, 524288 cells) with one beyond it; the tolerance is
+    that of the other GMRES comparison, as the dot products' orders differ."""
+    import oracle
+    from dnds_amd import _capi as A
+    from dnds_amd.host import (RIEMANN_VR_SETTING, CompactFacedMeshSerialRW, EulerEvaluator,
+                               ImplicitEulerDualTimeStep, VRFiniteVolume2D, vr_setting)
+    mesh = CompactFacedMeshSerialRW.generate(1, nx, ny, 0.0, nx / 10, 0.0, ny / 10, jitter=0.2, seed=3,
+                                             bc=(A.BC_FARFIELD, A.BC_FARFIELD, A.BC_WALL_EULER, A.BC_FARFIELD))
+    vfv = VRFiniteVolume2D(mesh, vr_setting(**dict(RIEMANN_VR_SETTING, far_weight=1.0)))
+    vfv.Initialization(8)
+    n = mesh.n_cell
+    far = (1.0, 0.5, 0.1, 2.7)
+    rng = np.random.default_rng(31)
+    rho, vx, vy, p = (1 + 0.1 * rng.random(n), 0.5 + 0.1 * rng.random(n), 0.1 * rng.random(n), 1 + 0.1 * rng.random(n))
+    u0 = np.stack([rho, rho * vx, rho * vy, p / 0.4 + 0.5 * rho * (vx * vx + vy * vy)], 1)
+    ev = EulerEvaluator(mesh, vfv, riemannSolverType="HLLC", farFieldStaticValue=far)
+    ev.SetLinearSolver(code, 4, 1)
+    ode = ImplicitEulerDualTimeStep(ev, nInternalRecStep=1, CFL=5.0, nTimeStepInternal=2, rhsThresholdInternal=0.0)
+    u, r, rn = ev.BuildMean().upload(u0), vfv.BuildRec().setConstant(0.0), vfv.BuildRec()
+    ode.Step(u, r, rn, dt=0.1)
+    st = vfv.setting
+    orc = oracle.Oracle(mesh.arrays(), vfv.arrays(), riemann_solver=2, far_field=far, tang_weight=st.tang_weight,
+                        tang_weight_direction=st.tang_weight_direction, gmres_code=code, n_gmres_space=4,
+                        n_gmres_iter=1)
+    ou, _, _ = orc.implicit_euler(u0, np.zeros((n, 36)), 2, 1, 5.0, dt=0.1, threshold=0.0,
+                                  scan2cell=ev.LUSGSScanOrder())
+    assert rel_err(u.download(), ou) <= 1e-9
