@@ -14,11 +14,11 @@
 // cells repeat the cell itself.
 //
 // Training and inference use hand-written kernels on gfx950's matrix cores
-// (v_mfma_f32_16x16x32_bf16: BF16 operands, FP32 accumulation): a GEMM with
-// fused epilogues (bias, GELU, GELU backward) for training, column sums for
-// the bias gradients, the MSE loss and Adam, all FP32 otherwise; and one
-// fused kernel for inference that keeps the three layers' BF16 weights in
-// LDS and the hidden activations on chip.
+// (v_mfma_f32_16x16x32_bf16: BF16 operands, FP32 accumulation), FP32
+// otherwise.  A training step is three launches: the rows' forward and
+// backward pass, the weight and bias gradients' partial sums over the rows,
+// and their sums with Adam.  Inference is one fused kernel that keeps the
+// three layers' BF16 weights in LDS and the hidden activations on chip.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -56,104 +56,326 @@ __device__ inline float gelu_grad(float z) {
     return 0.5f * (1.0f + erff(z * 0.70710678118654752f)) + z * 0.39894228040143268f * expf(-0.5f * z * z);
 }
 
-enum { EPI_STORE = 0, EPI_BIAS = 1, EPI_BIAS_GELU = 2, EPI_GELU_GRAD = 3 };
+__device__ __forceinline__ floatx4 mfma(bf16x8 a, bf16x8 b, floatx4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
 
-// C[M][N] = op(A) op(B) with BF16 operands and FP32 accumulation.
-// A(m, k) = transA ? A[k lda + m] : A[m lda + k]; B(k, n) likewise.
-// 256 threads; a 64 x 64 tile per workgroup, a 32 x 32 quarter per wave as
-// 2 x 2 MFMA 16x16x32 blocks; K in steps of 32 staged through LDS as BF16.
 // Operand layout of v_mfma_f32_16x16x32_bf16: lane l holds A[l % 16][k] and
 // B[k][l % 16] for the eight k = 8 (l / 16) + 0..7 (a product is the same
 // under any assignment of k that A and B share); it receives
 // D[4 (l / 16) + 0..3][l % 16].
 //
-// Split K (EPI_STORE only): block z sums k in [z kchunk, (z + 1) kchunk) and
-// writes its partial product to C + z M ldcm; k_splitk_sum adds the partials
-// in a fixed order.
-template <int EPI>
-__global__ __launch_bounds__(256) void k_gemm(int32_t M, int32_t N, int32_t K, const float *__restrict__ A,
-                                              int64_t lda, int32_t transA, const float *__restrict__ B, int64_t ldb,
-                                              int32_t transB, float *__restrict__ C, int64_t ldcm,
-                                              const float *__restrict__ bias, float *__restrict__ C2,
-                                              const float *__restrict__ Zin, int32_t kchunk) {
-    // As: rows m, k contiguous; Bs: columns n, k contiguous (so that a lane's
-    // eight k are one 16-byte LDS read); rows padded by 8 against bank conflicts
-    __shared__ __attribute__((aligned(16))) unsigned short As[64][32 + 8];
-    __shared__ __attribute__((aligned(16))) unsigned short Bs[64][32 + 8];
-    const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
-    const int64_t m0 = int64_t(blockIdx.x) * 64, n0 = int64_t(blockIdx.y) * 64;
-    const int wm = 32 * (wave / 2), wn = 32 * (wave % 2);
-    const int32_t kbeg = int32_t(blockIdx.z) * kchunk, kend = min(K, kbeg + kchunk);
-    if (EPI == EPI_STORE)
-        C += int64_t(blockIdx.z) * M * ldcm;
+// B fragment of K step `step`: W(k, n) for the lane's n and eight k, zero
+// from k = K on
+template <class F>
+__device__ __forceinline__ bf16x8 weight_fragment(int step, int K, F W) {
+    const int kb = 32 * step + 8 * (int(threadIdx.x % 64) / 16);
+    shortx8 f;
+#pragma unroll
+    for (int e = 0; e < 8; e++)
+        f[e] = kb + e < K ? short(to_bf16(W(kb + e))) : short(0);
+    return __builtin_bit_cast(bf16x8, f);
+}
+
+// The operands of the weight gradients, BF16, transposed: column c's rows
+// contiguous, [column][ld] with ld a multiple of 32 and zeros from the batch's
+// last row on, so that a lane's eight k (rows) are one 16-byte load.
+struct TrainCols {
+    int64_t ld;
+    unsigned short *X, *H1, *H2, *dY, *dZ2, *dZ1; // 64, 128, 128, 64, 128, 128 columns
+};
+constexpr int kColsX = 0, kColsH1 = 64, kColsH2 = 192, kColsdY = 320, kColsdZ2 = 384, kColsdZ1 = 512, kColsAll = 640;
+
+constexpr int kInPad = 64, kOutPad = 48, kLdX = kInPad + 8, kLdH = kHid + 8, kRowWaves = 8;
+
+// Forward and backward pass of the batch, 16 rows per workgroup and turn: row
+// r is row idx[r] (r without idx) of X and T.  Wave w owns columns 16 w .. 16
+// w + 15 of the hidden layers (waves 0 .. 2 the outputs) and holds its columns
+// of the three weight matrices and of the two transposed ones as BF16 operands
+// in registers for all its turns; a layer's output goes through LDS to the
+// next, z1 and z2 stay in registers for the GELU's derivative.  Out come the
+// weight gradients' operands (TrainCols) and the FP32 columns the bias
+// gradients sum; Y where the loss is asked for (else null).
+//
+// The chain of six small products is bound by latency (LDS, barriers, the
+// GELUs); five separate products through memory took 18 + 20 + 18 + 16 + 16
+// us at 4096 rows besides two gathers and the loss gradient.
+__global__ __launch_bounds__(64 * kRowWaves) void k_train_rows(int32_t rows, const int32_t *__restrict__ idx,
+                                                               const float *__restrict__ X,
+                                                               const float *__restrict__ T,
+                                                               const float *__restrict__ P, float scale, TrainCols tc,
+                                                               float *__restrict__ Y, float *__restrict__ dY,
+                                                               float *__restrict__ dZ2, float *__restrict__ dZ1) {
+    __shared__ __attribute__((aligned(16))) unsigned short Xs[16][kLdX], Ds[16][kLdX];
+    __shared__ __attribute__((aligned(16))) unsigned short H1s[16][kLdH], H2s[16][kLdH], Gs[16][kLdH];
+    const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64, lr = lane % 16, lg = lane / 16;
+    const int n = 16 * wave + lr;
+    bf16x8 w1[2], w2[4], w3[4], w3t[2], w2t[4];
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+        w1[s] = weight_fragment(s, kIn, [&](int k) { return P[oW1 + k * kHid + n]; });
+        w3t[s] = weight_fragment(s, kOut, [&](int k) { return P[oW3 + n * kOut + k]; });
+    }
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        w2[s] = weight_fragment(s, kHid, [&](int k) { return P[oW2 + k * kHid + n]; });
+        w2t[s] = weight_fragment(s, kHid, [&](int k) { return P[oW2 + n * kHid + k]; });
+        w3[s] = weight_fragment(s, n < kOut ? kHid : 0, [&](int k) { return P[oW3 + k * kOut + n]; });
+    }
+    const float bias1 = P[ob1 + n], bias2 = P[ob2 + n], bias3 = n < kOut ? P[ob3 + n] : 0.f;
+    const floatx4 zero = floatx4{0.f, 0.f, 0.f, 0.f};
+    const int64_t ntile = tc.ld / 16;
+    for (int64_t tile = blockIdx.x; tile < ntile; tile += gridDim.x) {
+        const int64_t r0 = 16 * tile, rl = r0 + 4 * lg; // the lane's four rows of every result
+        // a fragment of the tile's K step s, and a column's four rows to memory
+        auto frag = [&](const auto &S, int s) {
+            return __builtin_bit_cast(bf16x8, *reinterpret_cast<const shortx8 *>(&S[lr][32 * s + 8 * lg]));
+        };
+        auto to_cols = [&](unsigned short *cols, int c, const unsigned short v[4]) {
+            *reinterpret_cast<ushort4 *>(cols + c * tc.ld + rl) = make_ushort4(v[0], v[1], v[2], v[3]);
+        };
+        float t[4] = {0.f, 0.f, 0.f, 0.f};
+        if (n < kOut)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (rl + j < rows)
+                    t[j] = T[(idx ? idx[rl + j] : rl + j) * int64_t(kOut) + n];
+#pragma unroll
+        for (int q = 0; q < 16 * kInPad / (64 * kRowWaves); q++) {
+            const int e = tid + 64 * kRowWaves * q, r = e / kInPad, k = e % kInPad;
+            float v = 0.f;
+            if (r0 + r < rows && k < kIn)
+                v = X[(idx ? idx[r0 + r] : r0 + r) * int64_t(kIn) + k];
+            Xs[r][k] = to_bf16(v);
+        }
+        __syncthreads();
+        if (wave < kInPad / 16) {
+            unsigned short o[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                o[j] = Xs[4 * lg + j][n];
+            to_cols(tc.X, n, o);
+        }
+        floatx4 z1 = zero, z2 = zero, acc = zero;
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+            z1 = mfma(frag(Xs, s), w1[s], z1);
+        unsigned short o[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            z1[j] = z1[j] + bias1;
+            H1s[4 * lg + j][n] = to_bf16(gelu(z1[j]));
+            o[j] = rl + j < rows ? H1s[4 * lg + j][n] : (unsigned short)(0);
+        }
+        to_cols(tc.H1, n, o);
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+            z2 = mfma(frag(H1s, s), w2[s], z2);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            z2[j] = z2[j] + bias2;
+            H2s[4 * lg + j][n] = to_bf16(gelu(z2[j]));
+            o[j] = rl + j < rows ? H2s[4 * lg + j][n] : (unsigned short)(0);
+        }
+        to_cols(tc.H2, n, o);
+        __syncthreads();
+        // outputs, and the loss's gradient 2 (Y - T) / (rows 36)
+        if (wave < kInPad / 16) {
+            if (wave < kOutPad / 16)
+#pragma unroll
+                for (int s = 0; s < 4; s++)
+                    acc = mfma(frag(H2s, s), w3[s], acc);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const float y = acc[j] + bias3;
+                float d = 0.f;
+                if (n < kOut && rl + j < rows) {
+                    d = scale * (y - t[j]);
+                    dY[(rl + j) * kOut + n] = d;
+                    if (Y)
+                        Y[(rl + j) * kOut + n] = y;
+                }
+                Ds[4 * lg + j][n] = o[j] = to_bf16(d);
+            }
+            to_cols(tc.dY, n, o);
+        }
+        __syncthreads();
+        acc = zero;
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+            acc = mfma(frag(Ds, s), w3t[s], acc);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const float d = rl + j < rows ? acc[j] * gelu_grad(z2[j]) : 0.f;
+            if (rl + j < rows)
+                dZ2[(rl + j) * kHid + n] = d;
+            Gs[4 * lg + j][n] = o[j] = to_bf16(d);
+        }
+        to_cols(tc.dZ2, n, o);
+        __syncthreads();
+        acc = zero;
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+            acc = mfma(frag(Gs, s), w2t[s], acc);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const float d = rl + j < rows ? acc[j] * gelu_grad(z1[j]) : 0.f;
+            if (rl + j < rows)
+                dZ1[(rl + j) * kHid + n] = d;
+            o[j] = to_bf16(d);
+        }
+        to_cols(tc.dZ1, n, o);
+    }
+}
+
+// Partial weight and bias gradients over chunks of the rows.
+//
+// Workgroups of one wave: the first nz * kWTiles take a 32 x 32 tile of one
+// weight matrix's A^T B (A the layer's input, B its output's gradient) over
+// rows [z kchunk, (z + 1) kchunk), 2 x 2 MFMA blocks, K in steps of 32, into
+// part[z] laid out like the parameters; eight steps' operands (16 bytes a
+// lane) are in flight at a time, for the wave waits for nothing else.  The
+// others sum 64 columns over one chunk of rows in order, into bpart[chunk].
+// (Products of 64 x 64 tiles with operands rounded on the way into LDS, one
+// step's at a time, took 40 us each at 4096 rows, the column sums 13.)
+constexpr int kWTiles = 8 + 16 + 8, kBias = 2 * kHid + kOut, kBiasBlocks = 5;
+
+__global__ __launch_bounds__(64) void k_train_grads(int32_t rows, int32_t nz, int32_t kchunk, int32_t bchunk,
+                                                    TrainCols tc, const float *__restrict__ dY,
+                                                    const float *__restrict__ dZ2, const float *__restrict__ dZ1,
+                                                    float *__restrict__ part, float *__restrict__ bpart) {
+    const int lane = threadIdx.x, lr = lane % 16, lg = lane / 16;
+    const int32_t blk = blockIdx.x;
+    if (blk >= nz * kWTiles) {
+        const int32_t z = (blk - nz * kWTiles) / kBiasBlocks, q = (blk - nz * kWTiles) % kBiasBlocks;
+        const int w = q < 4 ? kHid : kOut, c = q < 4 ? 64 * (q % 2) + lane : lane;
+        if (c >= w)
+            return;
+        const float *src = (q < 2 ? dZ1 : q < 4 ? dZ2 : dY) + c;
+        const int32_t r0 = z * bchunk, r1 = min(rows, r0 + bchunk);
+        float sum = 0.f;
+        int32_t r = r0;
+        for (; r + 32 <= r1; r += 32) {
+            float v[32];
+#pragma unroll
+            for (int e = 0; e < 32; e++)
+                v[e] = src[int64_t(r + e) * w];
+#pragma unroll
+            for (int e = 0; e < 32; e++)
+                sum += v[e];
+        }
+        for (; r < r1; r++)
+            sum += src[int64_t(r) * w];
+        bpart[int64_t(z) * kBias + (q < 2 ? 0 : q < 4 ? kHid : 2 * kHid) + c] = sum;
+        return;
+    }
+    const int32_t z = blk / kWTiles, t = blk % kWTiles;
+    // W2: 4 x 4 tiles, W1: 2 x 4 (58 of 64 rows), W3: 4 x 2 (36 of 64 columns)
+    const unsigned short *A, *B;
+    int M, N, m0, n0;
+    int64_t o;
+    if (t < 16)
+        A = tc.H1, B = tc.dZ2, M = kHid, N = kHid, m0 = 32 * (t / 4), n0 = 32 * (t % 4), o = oW2;
+    else if (t < 24)
+        A = tc.X, B = tc.dZ1, M = kIn, N = kHid, m0 = 32 * ((t - 16) / 4), n0 = 32 * (t % 4), o = oW1;
+    else
+        A = tc.H2, B = tc.dY, M = kHid, N = kOut, m0 = 32 * ((t - 24) / 2), n0 = 32 * (t % 2), o = oW3;
+    const int32_t kbeg = z * kchunk, kend = min(rows, kbeg + kchunk);
     floatx4 acc[2][2];
 #pragma unroll
     for (int a = 0; a < 2; a++)
 #pragma unroll
         for (int b = 0; b < 2; b++)
             acc[a][b] = floatx4{0.f, 0.f, 0.f, 0.f};
-    for (int32_t k0 = kbeg; k0 < kend; k0 += 32) {
+    constexpr int kSteps = 8;
+    for (int32_t k0 = kbeg; k0 < kend; k0 += 32 * kSteps) {
+        shortx8 fa[kSteps][2], fb[kSteps][2];
 #pragma unroll
-        for (int q = 0; q < 8; q++) {
-            const int e = tid + 256 * q; // 0 .. 2047
-            {
-                // transA reads A[k lda + m]: consecutive threads take consecutive m
-                const int r = transA ? e % 64 : e / 32, kk = transA ? e / 64 : e % 32;
-                const int64_t m = m0 + r, k = k0 + kk;
-                float v = 0.f;
-                if (m < M && k < kend)
-                    v = transA ? A[k * lda + m] : A[m * lda + k];
-                As[r][kk] = to_bf16(v);
+        for (int s = 0; s < kSteps; s++)
+#pragma unroll
+            for (int a = 0; a < 2; a++) {
+                const int64_t k = k0 + 32 * s + 8 * lg;
+                fa[s][a] = fb[s][a] = shortx8{0, 0, 0, 0, 0, 0, 0, 0};
+                if (k < kend) {
+                    fa[s][a] = *reinterpret_cast<const shortx8 *>(A + (m0 + 16 * a + lr) * tc.ld + k);
+                    fb[s][a] = *reinterpret_cast<const shortx8 *>(B + (n0 + 16 * a + lr) * tc.ld + k);
+                }
             }
-            {
-                const int c = transB ? e / 32 : e % 64, kk = transB ? e % 32 : e / 64;
-                const int64_t n = n0 + c, k = k0 + kk;
-                float v = 0.f;
-                if (n < N && k < kend)
-                    v = transB ? B[n * ldb + k] : B[k * ldb + n];
-                Bs[c][kk] = to_bf16(v);
-            }
-        }
-        __syncthreads();
-        bf16x8 af[2], bfr[2];
-        const int kb = 8 * (lane / 16);
 #pragma unroll
-        for (int a = 0; a < 2; a++)
-            af[a] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const shortx8 *>(&As[wm + 16 * a + lane % 16][kb]));
+        for (int s = 0; s < kSteps; s++)
+            if (k0 + 32 * s < kend)
 #pragma unroll
-        for (int b = 0; b < 2; b++)
-            bfr[b] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const shortx8 *>(&Bs[wn + 16 * b + lane % 16][kb]));
+                for (int a = 0; a < 2; a++)
 #pragma unroll
-        for (int a = 0; a < 2; a++)
-#pragma unroll
-            for (int b = 0; b < 2; b++)
-                acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[a], bfr[b], acc[a][b], 0, 0, 0);
-        __syncthreads();
+                    for (int b = 0; b < 2; b++)
+                        acc[a][b] = mfma(__builtin_bit_cast(bf16x8, fa[s][a]), __builtin_bit_cast(bf16x8, fb[s][b]),
+                                         acc[a][b]);
     }
+    float *C = part + int64_t(z) * kNParam + o;
 #pragma unroll
     for (int a = 0; a < 2; a++)
 #pragma unroll
         for (int b = 0; b < 2; b++)
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const int64_t m = m0 + wm + 16 * a + 4 * (lane / 16) + j;
-                const int64_t n = n0 + wn + 16 * b + lane % 16;
-                if (m >= M || n >= N)
-                    continue;
-                float v = acc[a][b][j];
-                const int64_t o = m * ldcm + n;
-                if (EPI == EPI_STORE) {
-                    C[o] = v;
-                } else if (EPI == EPI_BIAS) {
-                    C[o] = v + bias[n];
-                } else if (EPI == EPI_BIAS_GELU) {
-                    const float z = v + bias[n];
-                    C[o] = z;
-                    C2[o] = gelu(z);
-                } else {
-                    C[o] = v * gelu_grad(Zin[o]);
-                }
+                const int m = m0 + 16 * a + 4 * lg + j, n = n0 + 16 * b + lr;
+                if (m < M && n < N)
+                    C[m * N + n] = acc[a][b][j];
             }
+}
+
+// Adam (Kingma & Ba 2015) with bias correction folded into the step size
+struct AdamStep {
+    float lr_t, b1, b2, eps_t;
+};
+__device__ __forceinline__ void adam_update(int64_t i, float g, const AdamStep &a, float *__restrict__ P,
+                                            float *__restrict__ Mm, float *__restrict__ Vv) {
+    const float m = a.b1 * Mm[i] + (1.f - a.b1) * g;
+    const float v = a.b2 * Vv[i] + (1.f - a.b2) * g * g;
+    Mm[i] = m, Vv[i] = v;
+    P[i] -= a.lr_t * m / (sqrtf(v) + a.eps_t);
+}
+
+// Gradient of every parameter, its partial sums added in order; into G, or
+// (without G) straight into Adam's step
+__global__ __launch_bounds__(256) void k_train_update(int32_t nz, int32_t nb, const float *__restrict__ part,
+                                                      const float *__restrict__ bpart, float *__restrict__ G,
+                                                      AdamStep a, float *__restrict__ P, float *__restrict__ Mm,
+                                                      float *__restrict__ Vv) {
+    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= kNParam)
+        return;
+    const float *src = part + i;
+    int64_t ld = kNParam;
+    int32_t cnt = nz;
+    const bool b1 = i >= ob1 && i < oW2, b2 = i >= ob2 && i < oW3, b3 = i >= ob3;
+    if (b1 || b2 || b3)
+        src = bpart + (b1 ? i - ob1 : b2 ? kHid + i - ob2 : 2 * kHid + i - ob3), ld = kBias, cnt = nb;
+    float acc = 0.f;
+    int32_t z = 0;
+    for (; z + 16 <= cnt; z += 16) {
+        float v[16];
+#pragma unroll
+        for (int e = 0; e < 16; e++)
+            v[e] = src[(z + e) * ld];
+#pragma unroll
+        for (int e = 0; e < 16; e++)
+            acc += v[e];
+    }
+    for (; z < cnt; z++)
+        acc += src[z * ld];
+    if (G)
+        G[i] = acc;
+    else
+        adam_update(i, acc, a, P, Mm, Vv);
+}
+
+__global__ __launch_bounds__(256) void k_adam(int64_t n, float *__restrict__ P, const float *__restrict__ G,
+                                              float *__restrict__ Mm, float *__restrict__ Vv, AdamStep a) {
+    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i < n)
+        adam_update(i, G[i], a, P, Mm, Vv);
 }
 
 // Inference of the whole network, Y = W3^T g(W2^T g(W1^T x + b1) + b2) + b3
@@ -163,10 +385,9 @@ __global__ __launch_bounds__(256) void k_gemm(int32_t M, int32_t N, int32_t K, c
 // the row's features from memory, every hidden layer's output (bias and GELU
 // applied in FP32, then rounded to BF16, as the operand of the next GEMM
 // would be) goes through the wave's own 16 x 128 LDS tile, and only the 36
-// outputs reach memory.  The arithmetic is that of the three k_gemm launches
-// (BF16 operands, FP32 accumulation, FP32 epilogues) without the hidden
-// activations' round trips through HBM.
-constexpr int kInPad = 64, kOutPad = 48, kLdW1 = kInPad + 8, kLdH = kHid + 8, kInferWaves = 16;
+// outputs reach memory.  The arithmetic is that of training's forward pass
+// (BF16 operands, FP32 accumulation, FP32 epilogues).
+constexpr int kLdW1 = kInPad + 8, kInferWaves = 16;
 
 __global__ __launch_bounds__(64 * kInferWaves) void k_mlp_infer(int32_t rows, const float *__restrict__ X,
                                                                   const float *__restrict__ P,
@@ -298,41 +519,14 @@ __global__ __launch_bounds__(64 * kInferWaves) void k_mlp_infer(int32_t rows, co
     }
 }
 
-// C[i] = sum over z of part[z][i], in order
-__global__ __launch_bounds__(256) void k_splitk_sum(int64_t n, int32_t nz, const float *__restrict__ part,
-                                                    float *__restrict__ C) {
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n)
-        return;
-    float acc = 0.f;
-    for (int32_t z = 0; z < nz; z++)
-        acc += part[int64_t(z) * n + i];
-    C[i] = acc;
-}
-
-// partial column sums of X [rows][n] (bias gradients, n <= 256): block z
-// sums rows [z chunk, (z + 1) chunk) in order, one thread per column
-__global__ __launch_bounds__(256) void k_colsum(int32_t rows, int32_t n, int32_t chunk, const float *__restrict__ X,
-                                                float *__restrict__ part) {
-    const int c = threadIdx.x;
-    if (c >= n)
-        return;
-    const int32_t r0 = int32_t(blockIdx.x) * chunk, r1 = min(rows, r0 + chunk);
-    float s = 0.f;
-    for (int32_t r = r0; r < r1; r++)
-        s += X[int64_t(r) * n + c];
-    part[int64_t(blockIdx.x) * n + c] = s;
-}
-
-// MSE loss and its gradient: dY = 2 (Y - T) / (rows * 36); per-block sums of (Y - T)^2
-__global__ __launch_bounds__(256) void k_mse(int64_t n, const float *__restrict__ Y, const float *__restrict__ T,
-                                             float scale, float *__restrict__ dY, float *__restrict__ part) {
+// MSE loss: per-block sums of (Y - T)^2 over the n = rows * 36 outputs
+__global__ __launch_bounds__(256) void k_mse(int64_t n, const int32_t *__restrict__ idx, const float *__restrict__ Y,
+                                             const float *__restrict__ T, float *__restrict__ part) {
     __shared__ float red[256];
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     float e = 0.f;
     if (i < n) {
-        const float d = Y[i] - T[i];
-        dY[i] = scale * d;
+        const float d = Y[i] - T[idx ? idx[i / kOut] * int64_t(kOut) + i % kOut : i];
         e = d * d;
     }
     red[threadIdx.x] = e;
@@ -344,20 +538,6 @@ __global__ __launch_bounds__(256) void k_mse(int64_t n, const float *__restrict_
     }
     if (threadIdx.x == 0)
         part[blockIdx.x] = red[0];
-}
-
-// Adam (Kingma & Ba 2015) with bias correction folded into the step size
-__global__ __launch_bounds__(256) void k_adam(int64_t n, float *__restrict__ P, const float *__restrict__ G,
-                                              float *__restrict__ Mm, float *__restrict__ Vv, float lr_t, float b1,
-                                              float b2, float eps_t) {
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n)
-        return;
-    const float g = G[i];
-    const float m = b1 * Mm[i] + (1.f - b1) * g;
-    const float v = b2 * Vv[i] + (1.f - b2) * g * g;
-    Mm[i] = m, Vv[i] = v;
-    P[i] -= lr_t * m / (sqrtf(v) + eps_t);
 }
 
 // features and scales of cell i: the row goes to `row` (58 floats), the
@@ -465,16 +645,6 @@ __global__ __launch_bounds__(256) void k_unscale(int32_t nc, int64_t ldc, const 
     }
 }
 
-// batch rows by index
-__global__ __launch_bounds__(256) void k_gather_rows(int32_t rows, int32_t width, const int32_t *__restrict__ idx,
-                                                     const float *__restrict__ src, float *__restrict__ dst) {
-    const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (e >= int64_t(rows) * width)
-        return;
-    const int64_t r = e / width, c = e % width;
-    dst[e] = src[int64_t(idx[r]) * width + c];
-}
-
 // du = u - u_prev, then u_prev = u (cell means, [cell][4])
 __global__ __launch_bounds__(256) void k_mean_change(int32_t nc, const double *__restrict__ u,
                                                      double *__restrict__ uprev, double *__restrict__ du) {
@@ -544,14 +714,15 @@ struct dndsmi_warmstart {
     // training set
     float *X = nullptr, *T = nullptr;
     int64_t n_samples = 0, capacity = 0;
-    // per-call work (rows up to max_rows)
-    int64_t max_rows = 0;
-    float *bX = nullptr, *bT = nullptr, *Z1 = nullptr, *H1 = nullptr, *Z2 = nullptr, *H2 = nullptr, *Y = nullptr,
-          *dY = nullptr, *dZ2 = nullptr, *dZ1 = nullptr, *part = nullptr;
-    int32_t *idx = nullptr;
+    // per-call work: Y up to max_rows, the batch's up to max_batch rows
+    int64_t max_rows = 0, max_batch = 0;
+    float *bX = nullptr, *bT = nullptr, *Y = nullptr, *dY = nullptr, *dZ2 = nullptr, *dZ1 = nullptr, *part = nullptr;
+    int32_t *perm = nullptr; // [max_perm] the epoch's order of the samples
+    int64_t max_perm = 0;
+    unsigned short *cols = nullptr; // [kColsAll][max_batch up to a multiple of 32]
     float *fX = nullptr, *fS = nullptr; // features / scales of all cells
     double *dpart = nullptr;
-    float *kpart = nullptr; // split-K partials [64][128][128]
+    float *kpart = nullptr, *bpart = nullptr; // [kMaxSplit][kNParam], [kMaxBiasChunks][kBias] partial sums
     std::mt19937_64 rng;
 
     template <class T>
@@ -578,64 +749,31 @@ int ensure_rows(dndsmi_warmstart *w, int64_t rows) {
         return DNDSMI_OK;
     // growth frees nothing: old buffers stay in the allocation list until destroy
     const int64_t r = std::max<int64_t>(rows, 256);
-    DNDSMI_TRY(w->alloc(w->bX, r * kIn));
-    DNDSMI_TRY(w->alloc(w->bT, r * kOut));
-    DNDSMI_TRY(w->alloc(w->Z1, r * kHid));
-    DNDSMI_TRY(w->alloc(w->H1, r * kHid));
-    DNDSMI_TRY(w->alloc(w->Z2, r * kHid));
-    DNDSMI_TRY(w->alloc(w->H2, r * kHid));
     DNDSMI_TRY(w->alloc(w->Y, r * kOut));
-    DNDSMI_TRY(w->alloc(w->dY, r * kOut));
-    DNDSMI_TRY(w->alloc(w->dZ2, r * kHid));
-    DNDSMI_TRY(w->alloc(w->dZ1, r * kHid));
-    DNDSMI_TRY(w->alloc(w->idx, r));
-    DNDSMI_TRY(w->alloc(w->part, (r * kOut + 255) / 256 + 1));
     w->max_rows = r;
     return DNDSMI_OK;
 }
 
-template <int EPI>
-void gemm(hipStream_t s, int32_t M, int32_t N, int32_t K, const float *A, int64_t lda, int ta, const float *B,
-          int64_t ldb, int tb, float *C, int64_t ldc, const float *bias = nullptr, float *C2 = nullptr,
-          const float *Zin = nullptr) {
-    dim3 grid((M + 63) / 64, (N + 63) / 64);
-    hipLaunchKernelGGL(k_gemm<EPI>, grid, dim3(256), 0, s, M, N, K, A, lda, ta, B, ldb, tb, C, ldc, bias, C2, Zin,
-                       K);
-}
+constexpr int kSplitChunk = 256, kMaxSplit = 64, kMaxBiasChunks = 1024;
 
-constexpr int kSplitChunk = 256, kMaxSplit = 64;
-
-// weight gradients C[M][N] = A^T B over a long K (the batch): split K over
-// up to 64 blocks per tile, then a fixed-order sum (deterministic)
-void gemm_wgrad(hipStream_t s, int32_t M, int32_t N, int32_t K, const float *A, int64_t lda, const float *B,
-                int64_t ldb, float *C, float *part) {
-    const int32_t chunk = std::max<int32_t>(kSplitChunk, (K + kMaxSplit - 1) / kMaxSplit / 16 * 16 + 16);
-    const int32_t nz = (K + chunk - 1) / chunk;
-    dim3 grid((M + 63) / 64, (N + 63) / 64, nz);
-    hipLaunchKernelGGL(k_gemm<EPI_STORE>, grid, dim3(256), 0, s, M, N, K, A, lda, 1, B, ldb, 0, part, int64_t(N),
-                       nullptr, nullptr, nullptr, chunk);
-    const int64_t n = int64_t(M) * N;
-    hipLaunchKernelGGL(k_splitk_sum, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s, n, nz, part, C);
-}
-
-// column sums of X [rows][n] into out (n <= 256, rows >= 1): the rows split
-// into at most 1024 chunks, partial sums per chunk, then added in chunk order
-// (deterministic); part holds the chunks' sums
-void colsum(hipStream_t s, int32_t rows, int32_t n, const float *X, float *out, float *part) {
-    static_assert(1024 * kHid <= kMaxSplit * kHid * kHid, "the chunk sums fit in the split-K partials");
-    const int32_t chunk = std::max<int32_t>(64, (rows + 1023) / 1024);
-    const int32_t nz = (rows + chunk - 1) / chunk;
-    hipLaunchKernelGGL(k_colsum, dim3(unsigned(nz)), dim3(256), 0, s, rows, n, chunk, X, part);
-    hipLaunchKernelGGL(k_splitk_sum, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s, int64_t(n), nz, part, out);
-}
-
-// forward pass of `rows` rows of X into Z1, H1, Z2, H2, Y
-void forward(dndsmi_warmstart *w, const float *X, int32_t rows) {
-    hipStream_t s = w->ctx->stream;
-    const float *P = w->P;
-    gemm<EPI_BIAS_GELU>(s, rows, kHid, kIn, X, kIn, 0, P + oW1, kHid, 0, w->Z1, kHid, P + ob1, w->H1);
-    gemm<EPI_BIAS_GELU>(s, rows, kHid, kHid, w->H1, kHid, 0, P + oW2, kHid, 0, w->Z2, kHid, P + ob2, w->H2);
-    gemm<EPI_BIAS>(s, rows, kOut, kHid, w->H2, kHid, 0, P + oW3, kOut, 0, w->Y, kOut, P + ob3);
+int ensure_batch(dndsmi_warmstart *w, int64_t rows) {
+    DNDSMI_TRY(ensure_rows(w, rows));
+    if (!w->kpart) {
+        DNDSMI_TRY(w->alloc(w->bpart, int64_t(kMaxBiasChunks) * kBias));
+        DNDSMI_TRY(w->alloc(w->kpart, int64_t(kMaxSplit) * kNParam));
+    }
+    if (rows <= w->max_batch)
+        return DNDSMI_OK;
+    const int64_t r = (std::max<int64_t>(rows, 256) + 31) / 32 * 32;
+    DNDSMI_TRY(w->alloc(w->bX, r * kIn));
+    DNDSMI_TRY(w->alloc(w->bT, r * kOut));
+    DNDSMI_TRY(w->alloc(w->dY, r * kOut));
+    DNDSMI_TRY(w->alloc(w->dZ2, r * kHid));
+    DNDSMI_TRY(w->alloc(w->dZ1, r * kHid));
+    DNDSMI_TRY(w->alloc(w->cols, r * kColsAll));
+    DNDSMI_TRY(w->alloc(w->part, (r * kOut + 255) / 256 + 1));
+    w->max_batch = r;
+    return DNDSMI_OK;
 }
 
 // the network's output for `rows` rows of X into Y (fused kernel, inference
@@ -647,30 +785,38 @@ int infer(dndsmi_warmstart *w, const float *X, int32_t rows) {
     return w->ctx->launch_check("k_mlp_infer");
 }
 
-// loss and gradients into G for rows of (X, T); returns the mean squared error
-int loss_grad(dndsmi_warmstart *w, const float *X, const float *T, int32_t rows, double *loss) {
+// loss and gradients of `rows` rows of (X, T), those of idx or the first
+// ones; the gradients go into G, or with `step` into that step of Adam
+int loss_grad(dndsmi_warmstart *w, const float *X, const float *T, const int32_t *idx, int32_t rows, double *loss,
+              const AdamStep *step) {
     hipStream_t s = w->ctx->stream;
-    const float *P = w->P;
-    float *G = w->G;
-    forward(w, X, rows);
-    const int64_t ny = int64_t(rows) * kOut;
-    const unsigned nb = unsigned((ny + 255) / 256);
-    hipLaunchKernelGGL(k_mse, dim3(nb), dim3(256), 0, s, ny, w->Y, T, float(2.0 / double(ny)), w->dY, w->part);
-    // layer 3
-    gemm_wgrad(s, kHid, kOut, rows, w->H2, kHid, w->dY, kOut, G + oW3, w->kpart);
-    colsum(s, rows, kOut, w->dY, G + ob3, w->kpart);
-    gemm<EPI_GELU_GRAD>(s, rows, kHid, kOut, w->dY, kOut, 0, P + oW3, kOut, 1, w->dZ2, kHid, nullptr, nullptr, w->Z2);
-    // layer 2
-    gemm_wgrad(s, kHid, kHid, rows, w->H1, kHid, w->dZ2, kHid, G + oW2, w->kpart);
-    colsum(s, rows, kHid, w->dZ2, G + ob2, w->kpart);
-    gemm<EPI_GELU_GRAD>(s, rows, kHid, kHid, w->dZ2, kHid, 0, P + oW2, kHid, 1, w->dZ1, kHid, nullptr, nullptr, w->Z1);
-    // layer 1
-    gemm_wgrad(s, kIn, kHid, rows, X, kIn, w->dZ1, kHid, G + oW1, w->kpart);
-    colsum(s, rows, kHid, w->dZ1, G + ob1, w->kpart);
-    DNDSMI_TRY(w->ctx->launch_check("warm-start backward"));
+    const int64_t ny = int64_t(rows) * kOut, ld = (int64_t(rows) + 31) / 32 * 32;
+    const TrainCols tc{ld,
+                       w->cols + kColsX * ld,
+                       w->cols + kColsH1 * ld,
+                       w->cols + kColsH2 * ld,
+                       w->cols + kColsdY * ld,
+                       w->cols + kColsdZ2 * ld,
+                       w->cols + kColsdZ1 * ld};
+    const unsigned gr = unsigned(std::min<int64_t>(ld / 16, 512));
+    hipLaunchKernelGGL(k_train_rows, dim3(gr), dim3(64 * kRowWaves), 0, s, rows, idx, X, T, w->P,
+                       float(2.0 / double(ny)), tc, loss ? w->Y : nullptr, w->dY, w->dZ2, w->dZ1);
+    // the rows split into at most kMaxSplit chunks for the weights and
+    // kMaxBiasChunks for the biases
+    const int32_t kchunk = std::max<int32_t>(kSplitChunk, (rows + kMaxSplit - 1) / kMaxSplit / 16 * 16 + 16);
+    const int32_t bchunk = std::max<int32_t>(64, (rows + kMaxBiasChunks - 1) / kMaxBiasChunks);
+    const int32_t nz = (rows + kchunk - 1) / kchunk, nb = (rows + bchunk - 1) / bchunk;
+    hipLaunchKernelGGL(k_train_grads, dim3(unsigned(nz * kWTiles + nb * kBiasBlocks)), dim3(64), 0, s, rows, nz,
+                       kchunk, bchunk, tc, w->dY, w->dZ2, w->dZ1, w->kpart, w->bpart);
+    hipLaunchKernelGGL(k_train_update, dim3(unsigned((kNParam + 255) / 256)), dim3(256), 0, s, nz, nb, w->kpart,
+                       w->bpart, step ? nullptr : w->G, step ? *step : AdamStep{}, w->P, w->Mm, w->Vv);
+    DNDSMI_TRY(w->ctx->launch_check("warm-start training step"));
     if (loss) {
-        std::vector<float> h(nb);
-        DNDSMI_TRY(w->ctx->hip(hipMemcpyAsync(h.data(), w->part, sizeof(float) * nb, hipMemcpyDeviceToHost, s),
+        const unsigned nblk = unsigned((ny + 255) / 256);
+        hipLaunchKernelGGL(k_mse, dim3(nblk), dim3(256), 0, s, ny, idx, w->Y, T, w->part);
+        DNDSMI_TRY(w->ctx->launch_check("k_mse"));
+        std::vector<float> h(nblk);
+        DNDSMI_TRY(w->ctx->hip(hipMemcpyAsync(h.data(), w->part, sizeof(float) * nblk, hipMemcpyDeviceToHost, s),
                                "hipMemcpyAsync"));
         DNDSMI_TRY(w->ctx->hip(hipStreamSynchronize(s), "hipStreamSynchronize"));
         double acc = 0;
@@ -681,14 +827,12 @@ int loss_grad(dndsmi_warmstart *w, const float *X, const float *T, int32_t rows,
     return DNDSMI_OK;
 }
 
-void adam(dndsmi_warmstart *w, double lr) {
+AdamStep adam_step(dndsmi_warmstart *w, double lr) {
     const double b1 = 0.9, b2 = 0.999, eps = 1e-8;
     w->adam_t++;
     const double c1 = 1 - std::pow(b1, double(w->adam_t)), c2 = 1 - std::pow(b2, double(w->adam_t));
     // step lr sqrt(c2) / c1 on m / (sqrt(v) + eps sqrt(c2)), the bias-corrected update
-    hipLaunchKernelGGL(k_adam, dim3(unsigned((kNParam + 255) / 256)), dim3(256), 0, w->ctx->stream, kNParam, w->P,
-                       w->G, w->Mm, w->Vv, float(lr * std::sqrt(c2) / c1), float(b1), float(b2),
-                       float(eps * std::sqrt(c2)));
+    return {float(lr * std::sqrt(c2) / c1), float(b1), float(b2), float(eps * std::sqrt(c2))};
 }
 
 int features(dndsmi_warmstart *w, const double *u) {
@@ -759,7 +903,7 @@ extern "C" int dndsmi_warmstart_create(dndsmi_ctx *c, const dndsmi_mesh_view *me
         if (w->alloc(w->sten, kSten * ldc) || w->alloc(w->mom, 9 * ldc) || w->alloc(w->logsz, ldc) ||
             w->alloc(w->P, kNParam) || w->alloc(w->G, kNParam) || w->alloc(w->Mm, kNParam) ||
             w->alloc(w->Vv, kNParam) || w->alloc(w->X, capacity * kIn) || w->alloc(w->T, capacity * kOut) ||
-            w->alloc(w->dpart, int64_t(grid_for(nc)) + 1) || w->alloc(w->kpart, int64_t(kMaxSplit) * kHid * kHid))
+            w->alloc(w->dpart, int64_t(grid_for(nc)) + 1))
             return fail(DNDSMI_ERR_OUT_OF_MEMORY);
     } catch (...) {
         return fail(DNDSMI_ERR_OUT_OF_MEMORY);
@@ -947,11 +1091,11 @@ extern "C" int dndsmi_warmstart_loss_grad(dndsmi_warmstart *w, const float *X, c
                                           float *grad, double *loss) {
     if (!w || !X || !T || rows < 1)
         return DNDSMI_ERR_INVALID_ARGUMENT;
-    DNDSMI_TRY(ensure_rows(w, rows));
+    DNDSMI_TRY(ensure_batch(w, rows));
     hipStream_t s = w->ctx->stream;
     DNDSMI_TRY(w->ctx->hip(hipMemcpyAsync(w->bX, X, sizeof(float) * rows * kIn, hipMemcpyHostToDevice, s), "copy"));
     DNDSMI_TRY(w->ctx->hip(hipMemcpyAsync(w->bT, T, sizeof(float) * rows * kOut, hipMemcpyHostToDevice, s), "copy"));
-    DNDSMI_TRY(loss_grad(w, w->bX, w->bT, rows, loss));
+    DNDSMI_TRY(loss_grad(w, w->bX, w->bT, nullptr, rows, loss, nullptr));
     if (grad) {
         DNDSMI_TRY(w->ctx->hip(hipMemcpyAsync(grad, w->G, sizeof(float) * kNParam, hipMemcpyDeviceToHost, s), "copy"));
         DNDSMI_TRY(w->ctx->hip(hipStreamSynchronize(s), "hipStreamSynchronize"));
@@ -964,7 +1108,8 @@ extern "C" int dndsmi_warmstart_adam_step(dndsmi_warmstart *w, const float *grad
         return DNDSMI_ERR_INVALID_ARGUMENT;
     DNDSMI_TRY(w->ctx->hip(hipMemcpyAsync(w->G, grad, sizeof(float) * kNParam, hipMemcpyHostToDevice, w->ctx->stream),
                            "copy"));
-    adam(w, lr);
+    hipLaunchKernelGGL(k_adam, dim3(unsigned((kNParam + 255) / 256)), dim3(256), 0, w->ctx->stream, kNParam, w->P,
+                       w->G, w->Mm, w->Vv, adam_step(w, lr));
     return w->ctx->launch_check("k_adam");
 }
 
@@ -1054,9 +1199,12 @@ extern "C" int dndsmi_warmstart_train(dndsmi_warmstart *w, int32_t epochs, int32
         return DNDSMI_ERR_INVALID_ARGUMENT;
     const int64_t n = w->n_samples;
     const int32_t b = int32_t(std::min<int64_t>(batch, n));
-    DNDSMI_TRY(ensure_rows(w, b));
-    int32_t *perm = nullptr;
-    DNDSMI_TRY(w->alloc(perm, n)); // freed with the warm start
+    DNDSMI_TRY(ensure_batch(w, b));
+    if (n > w->max_perm) {
+        DNDSMI_TRY(w->alloc(w->perm, w->capacity));
+        w->max_perm = w->capacity;
+    }
+    int32_t *perm = w->perm;
     std::vector<int32_t> hp(static_cast<size_t>(n));
     std::iota(hp.begin(), hp.end(), 0);
     hipStream_t s = w->ctx->stream;
@@ -1068,16 +1216,12 @@ extern "C" int dndsmi_warmstart_train(dndsmi_warmstart *w, int32_t epochs, int32
         double acc = 0;
         for (int64_t q = 0; q < steps_per_epoch; q++, step++) {
             const int32_t *ix = perm + q * b;
-            hipLaunchKernelGGL(k_gather_rows, dim3(unsigned((int64_t(b) * kIn + 255) / 256)), dim3(256), 0, s, b, kIn,
-                               ix, w->X, w->bX);
-            hipLaunchKernelGGL(k_gather_rows, dim3(unsigned((int64_t(b) * kOut + 255) / 256)), dim3(256), 0, s, b,
-                               kOut, ix, w->T, w->bT);
             double l = 0;
             const bool last = q == steps_per_epoch - 1;
-            DNDSMI_TRY(loss_grad(w, w->bX, w->bT, b, last ? &l : nullptr));
             // cosine decay from lr to lr_final
             const double f = 0.5 * (1 + std::cos(M_PI * double(step) / double(std::max<int64_t>(total, 1))));
-            adam(w, lr_final + (lr - lr_final) * f);
+            const AdamStep as = adam_step(w, lr_final + (lr - lr_final) * f);
+            DNDSMI_TRY(loss_grad(w, w->X, w->T, ix, b, last ? &l : nullptr, &as));
             if (last)
                 acc = l;
         }

@@ -112,3 +112,38 @@ def test_training_gain_over_the_method_without_it():
     assert ev["correction_rel_err"] < 0.9  # the previous reconstruction alone: 1
     for key in ("zero", "learned", "previous", "previous_plus_learned"):
         assert ev[key] < 600, key  # every start reached the tolerance
+
+
+@pytest.mark.parametrize("rows", [1, 15, 17, 33, 257, 8200, 16400, 65600])
+def test_training_step_at_tile_and_chunk_edges(rows):
+    """The training step's kernels at their edges: one row, partial 16-row
+    tiles and 32-row product steps, more tiles than workgroups (8192 rows),
+    chunks that are not multiples of 32 rows (from 16384) and of 64 (from
+    65536).  Tolerances as above: a BF16 operand rounds differently (2^-9)
+    where FP32 and FP64 sums fall on two sides of a tie.  Then one batch of
+    shuffled rows through train(): Adam's first step is lr g / (|g| + eps), the
+    same for every order of the rows wherever |g| is far above eps."""
+    from dnds_amd.host import WarmStart
+    from oracle import mlp_np as M
+    c, ev, _ = _setup()
+    ws = WarmStart(ev, seed=7, capacity=rows)
+    rng = np.random.default_rng(rows)
+    p = (rng.standard_normal(M.N_PARAM) * 0.15).astype(np.float32)
+    X = rng.standard_normal((rows, M.N_IN)).astype(np.float32)
+    T = (rng.standard_normal((rows, M.N_OUT)) * 0.3).astype(np.float32)
+    ws.set_params(p)
+    loss, g = ws.loss_grad(X, T)
+    lr_, gr = M.loss_grad(p.astype(np.float64), X.astype(np.float64), T.astype(np.float64), round_bf16=True)
+    assert abs(loss - lr_) <= 1e-4 * lr_
+    offs = np.cumsum([0] + [int(np.prod(s)) for _, s in M.SHAPES])
+    for (name, _), a, b in zip(M.SHAPES, offs[:-1], offs[1:]):
+        err = np.linalg.norm(g[a:b] - gr[a:b]) / np.linalg.norm(gr[a:b])
+        assert err <= 2e-3, (name, err)
+    ws.add_rows(X, T)
+    hist = ws.train(1, batch=rows, lr=1e-2, lr_final=1e-2)
+    assert abs(hist[0] - loss) <= 1e-5 * loss
+    q = ws.get_params()
+    big = np.abs(g) > 1e-2 * np.abs(g).max()
+    assert big.sum() > 1000
+    step = -1e-2 * g / (np.abs(g) + 1e-8)
+    assert np.abs((q - p) - step)[big].max() <= 1e-3 * 1e-2
