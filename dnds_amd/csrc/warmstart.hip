@@ -65,16 +65,32 @@ __device__ __forceinline__ floatx4 mfma(bf16x8 a, bf16x8 b, floatx4 c) {
 // under any assignment of k that A and B share); it receives
 // D[4 (l / 16) + 0..3][l % 16].
 //
-// B fragment of K step `step`: W(k, n) for the lane's n and eight k, zero
-// from k = K on
-template <class F>
-__device__ __forceinline__ bf16x8 weight_fragment(int step, int K, F W) {
-    const int kb = 32 * step + 8 * (int(threadIdx.x % 64) / 16);
-    shortx8 f;
-#pragma unroll
-    for (int e = 0; e < 8; e++)
-        f[e] = kb + e < K ? short(to_bf16(W(kb + e))) : short(0);
-    return __builtin_bit_cast(bf16x8, f);
+// The weight matrices as training's B operands in BF16: fragment f of wave w
+// (columns 16 w .. 16 w + 15) is 64 lanes x 8 values; zeros where the matrix
+// ends.  Fragments 0-1 are W1's K steps, 2-5 W2's, 6-9 W3's, 10-11 those of
+// W3's transpose, 12-15 those of W2's.  The parameters' update writes them with
+// the parameters: rounded by every workgroup of the rows' pass from strided
+// loads, they were 9 of its 23 us at 4096 rows.
+constexpr int kRowWaves = 8, kFragments = 16, kPacked = kFragments * kRowWaves * 64 * 8;
+__device__ __forceinline__ int packed_at(int f, int k, int n) {
+    return (((f + k / 32) * kRowWaves + n / 16) * 64 + 16 * (k % 32 / 8) + n % 16) * 8 + k % 8;
+}
+__device__ __forceinline__ void pack_parameter(int i, float p, unsigned short *__restrict__ packed) {
+    const unsigned short h = to_bf16(p);
+    if (i < ob1) {
+        packed[packed_at(0, i / kHid, i % kHid)] = h;
+    } else if (i >= oW2 && i < ob2) {
+        const int a = (i - oW2) / kHid, b = (i - oW2) % kHid;
+        packed[packed_at(2, a, b)] = packed[packed_at(12, b, a)] = h;
+    } else if (i >= oW3 && i < ob3) {
+        const int a = (i - oW3) / kOut, b = (i - oW3) % kOut;
+        packed[packed_at(6, a, b)] = packed[packed_at(10, b, a)] = h;
+    }
+}
+__global__ __launch_bounds__(256) void k_pack(const float *__restrict__ P, unsigned short *__restrict__ packed) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < kNParam)
+        pack_parameter(i, P[i], packed);
 }
 
 // The operands of the weight gradients, BF16, transposed: column c's rows
@@ -86,7 +102,7 @@ struct TrainCols {
 };
 constexpr int kColsX = 0, kColsH1 = 64, kColsH2 = 192, kColsdY = 320, kColsdZ2 = 384, kColsdZ1 = 512, kColsAll = 640;
 
-constexpr int kInPad = 64, kOutPad = 48, kLdX = kInPad + 8, kLdH = kHid + 8, kRowWaves = 8;
+constexpr int kInPad = 64, kOutPad = 48, kLdX = kInPad + 8, kLdH = kHid + 8;
 
 // Forward and backward pass of the batch, 16 rows per workgroup and turn: row
 // r is row idx[r] (r without idx) of X and T.  Wave w owns columns 16 w .. 16
@@ -103,7 +119,9 @@ constexpr int kInPad = 64, kOutPad = 48, kLdX = kInPad + 8, kLdH = kHid + 8, kRo
 __global__ __launch_bounds__(64 * kRowWaves) void k_train_rows(int32_t rows, const int32_t *__restrict__ idx,
                                                                const float *__restrict__ X,
                                                                const float *__restrict__ T,
-                                                               const float *__restrict__ P, float scale, TrainCols tc,
+                                                               const float *__restrict__ P,
+                                                               const unsigned short *__restrict__ packed, float scale,
+                                                               TrainCols tc,
                                                                float *__restrict__ Y, float *__restrict__ dY,
                                                                float *__restrict__ dZ2, float *__restrict__ dZ1) {
     __shared__ __attribute__((aligned(16))) unsigned short Xs[16][kLdX], Ds[16][kLdX];
@@ -111,17 +129,16 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_train_rows(int32_t rows, con
     const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64, lr = lane % 16, lg = lane / 16;
     const int n = 16 * wave + lr;
     bf16x8 w1[2], w2[4], w3[4], w3t[2], w2t[4];
+    auto weights = [&](int f) {
+        return __builtin_bit_cast(
+            bf16x8, *reinterpret_cast<const shortx8 *>(packed + ((f * kRowWaves + wave) * 64 + lane) * 8));
+    };
 #pragma unroll
-    for (int s = 0; s < 2; s++) {
-        w1[s] = weight_fragment(s, kIn, [&](int k) { return P[oW1 + k * kHid + n]; });
-        w3t[s] = weight_fragment(s, kOut, [&](int k) { return P[oW3 + n * kOut + k]; });
-    }
+    for (int s = 0; s < 2; s++)
+        w1[s] = weights(s), w3t[s] = weights(10 + s);
 #pragma unroll
-    for (int s = 0; s < 4; s++) {
-        w2[s] = weight_fragment(s, kHid, [&](int k) { return P[oW2 + k * kHid + n]; });
-        w2t[s] = weight_fragment(s, kHid, [&](int k) { return P[oW2 + n * kHid + k]; });
-        w3[s] = weight_fragment(s, n < kOut ? kHid : 0, [&](int k) { return P[oW3 + k * kOut + n]; });
-    }
+    for (int s = 0; s < 4; s++)
+        w2[s] = weights(2 + s), w3[s] = weights(6 + s), w2t[s] = weights(12 + s);
     const float bias1 = P[ob1 + n], bias2 = P[ob2 + n], bias3 = n < kOut ? P[ob3 + n] : 0.f;
     const floatx4 zero = floatx4{0.f, 0.f, 0.f, 0.f};
     const int64_t ntile = tc.ld / 16;
@@ -342,7 +359,7 @@ __device__ __forceinline__ void adam_update(int64_t i, float g, const AdamStep &
 __global__ __launch_bounds__(256) void k_train_update(int32_t nz, int32_t nb, const float *__restrict__ part,
                                                       const float *__restrict__ bpart, float *__restrict__ G,
                                                       AdamStep a, float *__restrict__ P, float *__restrict__ Mm,
-                                                      float *__restrict__ Vv) {
+                                                      float *__restrict__ Vv, unsigned short *__restrict__ packed) {
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= kNParam)
         return;
@@ -365,10 +382,12 @@ __global__ __launch_bounds__(256) void k_train_update(int32_t nz, int32_t nb, co
     }
     for (; z < cnt; z++)
         acc += src[z * ld];
-    if (G)
+    if (G) {
         G[i] = acc;
-    else
+    } else {
         adam_update(i, acc, a, P, Mm, Vv);
+        pack_parameter(int(i), P[i], packed);
+    }
 }
 
 __global__ __launch_bounds__(256) void k_adam(int64_t n, float *__restrict__ P, const float *__restrict__ G,
@@ -719,7 +738,8 @@ struct dndsmi_warmstart {
     float *bX = nullptr, *bT = nullptr, *Y = nullptr, *dY = nullptr, *dZ2 = nullptr, *dZ1 = nullptr, *part = nullptr;
     int32_t *perm = nullptr; // [max_perm] the epoch's order of the samples
     int64_t max_perm = 0;
-    unsigned short *cols = nullptr; // [kColsAll][max_batch up to a multiple of 32]
+    unsigned short *packed = nullptr; // [kPacked] the weights as training's operands
+    unsigned short *cols = nullptr;   // [kColsAll][max_batch up to a multiple of 32]
     float *fX = nullptr, *fS = nullptr; // features / scales of all cells
     double *dpart = nullptr;
     float *kpart = nullptr, *bpart = nullptr; // [kMaxSplit][kNParam], [kMaxBiasChunks][kBias] partial sums
@@ -758,9 +778,13 @@ constexpr int kSplitChunk = 256, kMaxSplit = 64, kMaxBiasChunks = 1024;
 
 int ensure_batch(dndsmi_warmstart *w, int64_t rows) {
     DNDSMI_TRY(ensure_rows(w, rows));
-    if (!w->kpart) {
+    if (!w->packed) {
+        unsigned short *packed = nullptr;
         DNDSMI_TRY(w->alloc(w->bpart, int64_t(kMaxBiasChunks) * kBias));
         DNDSMI_TRY(w->alloc(w->kpart, int64_t(kMaxSplit) * kNParam));
+        DNDSMI_TRY(w->alloc(packed, kPacked));
+        DNDSMI_TRY(w->ctx->upload(packed, std::vector<unsigned short>(kPacked, 0)));
+        w->packed = packed;
     }
     if (rows <= w->max_batch)
         return DNDSMI_OK;
@@ -785,8 +809,15 @@ int infer(dndsmi_warmstart *w, const float *X, int32_t rows) {
     return w->ctx->launch_check("k_mlp_infer");
 }
 
+// the weights as BF16 operands, before the first loss_grad on parameters as
+// they are now
+int pack_weights(dndsmi_warmstart *w) {
+    hipLaunchKernelGGL(k_pack, dim3(unsigned((kNParam + 255) / 256)), dim3(256), 0, w->ctx->stream, w->P, w->packed);
+    return w->ctx->launch_check("k_pack");
+}
+
 // loss and gradients of `rows` rows of (X, T), those of idx or the first
-// ones; the gradients go into G, or with `step` into that step of Adam
+// ones, with the weights last packed; the gradients go into G, or with `step` into that step of Adam
 int loss_grad(dndsmi_warmstart *w, const float *X, const float *T, const int32_t *idx, int32_t rows, double *loss,
               const AdamStep *step) {
     hipStream_t s = w->ctx->stream;
@@ -800,7 +831,7 @@ int loss_grad(dndsmi_warmstart *w, const float *X, const float *T, const int32_t
                        w->cols + kColsdZ1 * ld};
     const unsigned gr = unsigned(std::min<int64_t>(ld / 16, 512));
     hipLaunchKernelGGL(k_train_rows, dim3(gr), dim3(64 * kRowWaves), 0, s, rows, idx, X, T, w->P,
-                       float(2.0 / double(ny)), tc, loss ? w->Y : nullptr, w->dY, w->dZ2, w->dZ1);
+                       w->packed, float(2.0 / double(ny)), tc, loss ? w->Y : nullptr, w->dY, w->dZ2, w->dZ1);
     // the rows split into at most kMaxSplit chunks for the weights and
     // kMaxBiasChunks for the biases
     const int32_t kchunk = std::max<int32_t>(kSplitChunk, (rows + kMaxSplit - 1) / kMaxSplit / 16 * 16 + 16);
@@ -809,7 +840,8 @@ int loss_grad(dndsmi_warmstart *w, const float *X, const float *T, const int32_t
     hipLaunchKernelGGL(k_train_grads, dim3(unsigned(nz * kWTiles + nb * kBiasBlocks)), dim3(64), 0, s, rows, nz,
                        kchunk, bchunk, tc, w->dY, w->dZ2, w->dZ1, w->kpart, w->bpart);
     hipLaunchKernelGGL(k_train_update, dim3(unsigned((kNParam + 255) / 256)), dim3(256), 0, s, nz, nb, w->kpart,
-                       w->bpart, step ? nullptr : w->G, step ? *step : AdamStep{}, w->P, w->Mm, w->Vv);
+                       w->bpart, step ? nullptr : w->G, step ? *step : AdamStep{}, w->P, w->Mm, w->Vv,
+                       w->packed);
     DNDSMI_TRY(w->ctx->launch_check("warm-start training step"));
     if (loss) {
         const unsigned nblk = unsigned((ny + 255) / 256);
@@ -1095,6 +1127,7 @@ extern "C" int dndsmi_warmstart_loss_grad(dndsmi_warmstart *w, const float *X, c
     hipStream_t s = w->ctx->stream;
     DNDSMI_TRY(w->ctx->hip(hipMemcpyAsync(w->bX, X, sizeof(float) * rows * kIn, hipMemcpyHostToDevice, s), "copy"));
     DNDSMI_TRY(w->ctx->hip(hipMemcpyAsync(w->bT, T, sizeof(float) * rows * kOut, hipMemcpyHostToDevice, s), "copy"));
+    DNDSMI_TRY(pack_weights(w));
     DNDSMI_TRY(loss_grad(w, w->bX, w->bT, nullptr, rows, loss, nullptr));
     if (grad) {
         DNDSMI_TRY(w->ctx->hip(hipMemcpyAsync(grad, w->G, sizeof(float) * kNParam, hipMemcpyDeviceToHost, s), "copy"));
@@ -1205,6 +1238,7 @@ extern "C" int dndsmi_warmstart_train(dndsmi_warmstart *w, int32_t epochs, int32
         w->max_perm = w->capacity;
     }
     int32_t *perm = w->perm;
+    DNDSMI_TRY(pack_weights(w));
     std::vector<int32_t> hp(static_cast<size_t>(n));
     std::iota(hp.begin(), hp.end(), 0);
     hipStream_t s = w->ctx->stream;
