@@ -92,6 +92,21 @@ __device__ __forceinline__ T quad_get(T a, int q) { // q: a constant after unrol
     return q == 0 ? quad_bcast<0>(a) : q == 1 ? quad_bcast<1>(a) : q == 2 ? quad_bcast<2>(a) : quad_bcast<3>(a);
 }
 
+// a quad's sum of squares, lane 0's nine in turn, then lane 1's and so on: in
+// the last lane
+__device__ __forceinline__ double quad_norm2(const double d[9]) {
+    double sum = 0.0;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+#pragma unroll
+        for (int r = 0; r < 9; r++)
+            sum += d[r] * d[r];
+        if (q < 3)
+            sum = quad_get(sum, q);
+    }
+    return sum;
+}
+
 // the neighbouring lane's `a` (lanes 2 k and 2 k + 1 exchange)
 __device__ __forceinline__ double pair_swap(double a) {
     const uint64_t w = __builtin_bit_cast(uint64_t, a);
@@ -325,6 +340,12 @@ __global__ __launch_bounds__(kBlock, 3) void k_sor(int32_t n, int32_t base, int6
 // couples the cell to itself (M_if x_i), a Wall face adds b_if (0 - u_i)^T,
 // Wall_Euler / Wall_NoSlip faces add their correction from the old iterate.
 //
+// diff2 (may be null): receives |x_i - new_i|^2 per cell.  A kernel of its own
+// for it read both arrays again (one thread per cell, uncoalesced): 67 us per
+// sweep of dndsmi_reconstruct_to_tolerance on 66 k cells, 47 now, and 425 / 271
+// on 524 k; here
+// the old coefficients come from the caches.
+//
 // RESID (the FP64 step of the mixed-precision sweeps): instead of the new
 // iterate, writes the increment r = J(x) - x rounded to FP32 into r32 (also the
 // start of the FP32 correction sweeps, k_delta32).
@@ -334,7 +355,8 @@ __global__ __launch_bounds__(TILE ? kBlock : 64, 3) void k_jacobi(int32_t nc, in
                                                       const double *__restrict__ M, const double *__restrict__ u,
                                                       const double *__restrict__ x, double *__restrict__ xn,
                                                       double relax, const double *__restrict__ walls, double *corr,
-                                                      int32_t *errw, float *__restrict__ r32, int32_t keep) {
+                                                      int32_t *errw, float *__restrict__ r32, int32_t keep,
+                                                      double *__restrict__ diff2) {
     __shared__ double tile[TILE ? 9 : 1][TILE ? kBlock : 1];
     const int32_t t = xcd_block() * blockDim.x + threadIdx.x, v = t & 3;
     const bool live = (t >> 2) < nc;
@@ -431,6 +453,51 @@ __global__ __launch_bounds__(TILE ? kBlock : 64, 3) void k_jacobi(int32_t nc, in
         } else
             __builtin_nontemporal_store(nw[r], xn + rec_group(i) + (256 * r + lane));
     }
+    if (!RESID && diff2) {
+        double d[9];
+#pragma unroll
+        for (int r = 0; r < 9; r++)
+            d[r] = xo[256 * r + lane] - nw[r];
+        const double sum = quad_norm2(d);
+        if (v == 3)
+            diff2[i] = sum;
+    }
+}
+
+// the increment's squared norm per cell where the sweep does not give it
+__global__ __launch_bounds__(kBlock) void k_rec_diff2(int32_t nc, const double *__restrict__ x,
+                                                      const double *__restrict__ xn, double *__restrict__ diff2) {
+    const int32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    if ((t >> 2) >= nc)
+        return;
+    const int64_t o = rec((t >> 2) & ~15, 0, 0) + (threadIdx.x & 63);
+    double d[9];
+#pragma unroll
+    for (int r = 0; r < 9; r++)
+        d[r] = x[o + 256 * r] - xn[o + 256 * r];
+    const double sum = quad_norm2(d);
+    if ((t & 3) == 3)
+        diff2[t >> 2] = sum;
+}
+
+// sums of the cells' diff2, 256 cells each in a fixed tree, one per wave, into
+// pinned host memory: 16 a workgroup, stored as one run of 128 bytes
+__global__ __launch_bounds__(1024) void k_diff2_sums(int32_t nc, const double *__restrict__ diff2, double *part) {
+    __shared__ double sums[16];
+    const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+    const int64_t i = (int64_t(blockIdx.x) * 16 + wave) * 256 + lane;
+    double e[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+        e[q] = i + 64 * q < nc ? diff2[i + 64 * q] : 0.0;
+    double a = (e[0] + e[2]) + (e[1] + e[3]);
+    for (int off = 32; off > 0; off >>= 1)
+        a += __shfl_down(a, off, 64);
+    if (lane == 0)
+        sums[wave] = a;
+    __syncthreads();
+    if (threadIdx.x < 16)
+        part[int64_t(blockIdx.x) * 16 + threadIdx.x] = sums[threadIdx.x];
 }
 
 // Read-bandwidth probe of the sweep's dominant stream: every cell streams its
@@ -1953,6 +2020,8 @@ extern "C" void dndsmi_ctx_destroy(dndsmi_ctx *c) {
         (void)hipFree(p);
     if (c->host)
         (void)hipHostFree(c->host);
+    if (c->host_sums)
+        (void)hipHostFree(c->host_sums);
     for (hipEvent_t e : c->ev_pool)
         (void)hipEventDestroy(e);
     if (c->own_stream && c->stream)
@@ -2138,12 +2207,16 @@ int step_sweep(dndsmi_ctx *c, const double *u, double *&x, double *&xn, double t
     return DNDSMI_OK;
 }
 
-int launch_jacobi(dndsmi_ctx *c, const double *u, const double *x, double *xn, double t) {
+int launch_jacobi(dndsmi_ctx *c, const double *u, const double *x, double *xn, double t, double *diff2) {
     if (c->sor) {
         // the steps expect the new iterate in xn: start it from x, then update in place
         DNDSMI_TRY(c->hip(hipMemcpyAsync(xn, x, sizeof(double) * 36 * c->ldc, hipMemcpyDeviceToDevice, c->stream),
                           "copy uRec"));
-        return launch_sor(c, u, xn, t);
+        DNDSMI_TRY(launch_sor(c, u, xn, t));
+        if (diff2)
+            hipLaunchKernelGGL(k_rec_diff2, dim3(grid_for(4 * c->nc)), dim3(kBlock), 0, c->stream, int32_t(c->nc), x,
+                               xn, diff2);
+        return c->launch_check("k_rec_diff2");
     }
     const int64_t lanes = 4 * c->nc;
     const int block = sweep_block(lanes);
@@ -2152,9 +2225,26 @@ int launch_jacobi(dndsmi_ctx *c, const double *u, const double *x, double *xn, d
                             : (c->nfmax == 3 ? k_jacobi<3, false, true> : k_jacobi<4, false, true>);
     hipLaunchKernelGGL(kern, dim3(grid_for(lanes, block)), dim3(block), 0, c->stream, int32_t(c->nc),
                        c->ldc, c->nbr, c->sbc, c->M, u, x, xn, c->relax, c->walls, c->wall_corr,
-                       c->errw, nullptr, keep_share(c, kAbVecs, kKeepLargest));
+                       c->errw, nullptr, keep_share(c, kAbVecs, kKeepLargest), diff2);
     prof_end(c);
     return c->launch_check("k_jacobi");
+}
+
+int ensure_increment(dndsmi_ctx *c) {
+    if (!c->rec_diff)
+        DNDSMI_TRY(c->alloc(c->rec_diff, c->ldc));
+    if (!c->host_sums)
+        DNDSMI_TRY(c->hip(hipHostMalloc(&c->host_sums, sizeof(double) * 16 * size_t(grid_for(c->nc, 16 * 256)),
+                                        hipHostMallocCoherent),
+                          "hipHostMalloc"));
+    return DNDSMI_OK;
+}
+
+int launch_increment(dndsmi_ctx *c, const double *u, const double *x, double *xn, double t) {
+    DNDSMI_TRY(launch_jacobi(c, u, x, xn, t, c->rec_diff));
+    hipLaunchKernelGGL(k_diff2_sums, dim3(grid_for(c->nc, 16 * 256)), dim3(1024), 0, c->stream, int32_t(c->nc),
+                       c->rec_diff, c->host_sums);
+    return c->launch_check("k_diff2_sums");
 }
 
 int launch_dt(dndsmi_ctx *c, const double *u, double cfl, double max_dt, double *dt_out) {
@@ -2295,7 +2385,7 @@ int launch_jacobi_mixed(dndsmi_ctx *c, const double *u, double *x, int n_sweeps,
     hipLaunchKernelGGL(first, grid, dim3(block), 0, c->stream, nc,
                        c->ldc, c->nbr, c->sbc, c->M, u, x, nullptr, c->relax, c->walls,
                        c->wall_corr, c->errw, c->r32,
-                       keep_share(c, kAbVecs, kKeepLargestMixed));
+                       keep_share(c, kAbVecs, kKeepLargestMixed), nullptr);
     prof_end(c);
     DNDSMI_TRY(c->launch_check("k_jacobi (residual)"));
     const int32_t keep = keep_share(c, kAb32Vecs, kKeepLargest32);

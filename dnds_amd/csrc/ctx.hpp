@@ -143,6 +143,8 @@ struct dndsmi_ctx {
     double *imp_dtau = nullptr;       // [ldc]
     double *imp_stage = nullptr;      // [3][ldc][4] SDIRK4 stage right-hand sides (first use)
     double *res_part = nullptr;       // [4][grid]
+    double *rec_diff = nullptr;       // [ldc] squared increment of a sweep per cell (launch_increment)
+    double *host_sums = nullptr;      // its sums over 256 cells, pinned
     double *res = nullptr;            // [4]
     // the learned warm start inside the mixed-precision step
     // (dndsmi_ssprk3_set_warm_start): the previous stage's cell means and
@@ -234,7 +236,12 @@ int ws_window_end(dndsmi_ctx *c, double *u, double *x, bool failed);
 int noalloc_scratch_init(dndsmi_ctx *c);
 bool same_ctx(const dndsmi_ctx *c, const dndsmi_array *a, int32_t kind);
 // the explicit path's launches (ctx.hip)
-int launch_jacobi(dndsmi_ctx *c, const double *u, const double *x, double *xn, double t);
+// diff2 (may be null): |x - xn|^2 of every cell
+int launch_jacobi(dndsmi_ctx *c, const double *u, const double *x, double *xn, double t, double *diff2 = nullptr);
+// a sweep from x into xn with the sums of |x - xn|^2 over 256 cells each into
+// c->host_sums; ensure_increment once before
+int ensure_increment(dndsmi_ctx *c);
+int launch_increment(dndsmi_ctx *c, const double *u, const double *x, double *xn, double t);
 // one SOR sweep (SOR_Instead) in place on x, colour by colour
 int launch_sor(dndsmi_ctx *c, const double *u, double *x, double t);
 // one reconstruction sweep of a step: Jacobi into xn, then the two swap; with

@@ -697,28 +697,6 @@ __global__ __launch_bounds__(256) void k_diff2(int64_t n, const double *__restri
         part[2 * blockIdx.x] = red[0][0], part[2 * blockIdx.x + 1] = red[1][0];
 }
 
-// sum over all cells of |x_new - x_old|^2 (per block), for the rec residual
-__global__ __launch_bounds__(256) void k_rec_diff2(int32_t nc, int64_t ldc, const double *__restrict__ a,
-                                                   const double *__restrict__ b, double *__restrict__ part) {
-    __shared__ double red[256];
-    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    double s = 0.0;
-    if (i < nc)
-        for (int k = 0; k < 36; k++) {
-            const double d = a[rec(i, k % 9, k / 9)] - b[rec(i, k % 9, k / 9)];
-            s += d * d;
-        }
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int st = 128; st > 0; st >>= 1) {
-        if (threadIdx.x < st)
-            red[threadIdx.x] += red[threadIdx.x + st];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0)
-        part[blockIdx.x] = red[0];
-}
-
 } // namespace
 
 struct dndsmi_warmstart {
@@ -741,7 +719,6 @@ struct dndsmi_warmstart {
     unsigned short *packed = nullptr; // [kPacked] the weights as training's operands
     unsigned short *cols = nullptr;   // [kColsAll][max_batch up to a multiple of 32]
     float *fX = nullptr, *fS = nullptr; // features / scales of all cells
-    double *dpart = nullptr;
     float *kpart = nullptr, *bpart = nullptr; // [kMaxSplit][kNParam], [kMaxBiasChunks][kBias] partial sums
     std::mt19937_64 rng;
 
@@ -934,8 +911,7 @@ extern "C" int dndsmi_warmstart_create(dndsmi_ctx *c, const dndsmi_mesh_view *me
     try {
         if (w->alloc(w->sten, kSten * ldc) || w->alloc(w->mom, 9 * ldc) || w->alloc(w->logsz, ldc) ||
             w->alloc(w->P, kNParam) || w->alloc(w->G, kNParam) || w->alloc(w->Mm, kNParam) ||
-            w->alloc(w->Vv, kNParam) || w->alloc(w->X, capacity * kIn) || w->alloc(w->T, capacity * kOut) ||
-            w->alloc(w->dpart, int64_t(grid_for(nc)) + 1))
+            w->alloc(w->Vv, kNParam) || w->alloc(w->X, capacity * kIn) || w->alloc(w->T, capacity * kOut))
             return fail(DNDSMI_ERR_OUT_OF_MEMORY);
     } catch (...) {
         return fail(DNDSMI_ERR_OUT_OF_MEMORY);
@@ -1283,29 +1259,17 @@ extern "C" int dndsmi_reconstruct_to_tolerance(dndsmi_ctx *c, const dndsmi_array
     if (!c || !same_ctx(c, u, DNDSMI_ARRAY_DOF) || !same_ctx(c, uRec, DNDSMI_ARRAY_REC) ||
         !same_ctx(c, uRecNewBuf, DNDSMI_ARRAY_REC) || uRec == uRecNewBuf || max_sweeps < 1)
         return DNDSMI_ERR_INVALID_ARGUMENT;
-    const unsigned g = grid_for(c->nc);
-    std::vector<double> part(g);
-    double *dpart = nullptr;
-    if (!c->res_part) { // the implicit path's scratch holds 4 x grid doubles
-        DNDSMI_TRY(c->alloc(c->res_part, 4 * int64_t(g)));
-        DNDSMI_TRY(c->alloc(c->res, 4));
-    }
-    dpart = c->res_part;
+    DNDSMI_TRY(ensure_increment(c));
     double res = 0;
     int32_t k = 0;
     while (k < max_sweeps) {
-        DNDSMI_TRY(launch_jacobi(c, u->d, uRec->d, uRecNewBuf->d, t));
-        hipLaunchKernelGGL(k_rec_diff2, dim3(g), dim3(256), 0, c->stream, int32_t(c->nc), c->ldc, uRec->d,
-                           uRecNewBuf->d, dpart);
-        DNDSMI_TRY(c->launch_check("k_rec_diff2"));
+        DNDSMI_TRY(launch_increment(c, u->d, uRec->d, uRecNewBuf->d, t));
         std::swap(uRec->d, uRecNewBuf->d);
         k++;
-        DNDSMI_TRY(c->hip(hipMemcpyAsync(part.data(), dpart, sizeof(double) * g, hipMemcpyDeviceToHost, c->stream),
-                          "hipMemcpyAsync"));
         DNDSMI_TRY(check_errw(c));
         res = 0;
-        for (double v : part)
-            res += v;
+        for (unsigned b = 0; b < grid_for(c->nc, 256); b++)
+            res += c->host_sums[b];
         res /= double(c->nc);
         if (res < tol)
             break;

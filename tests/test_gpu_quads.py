@@ -71,3 +71,24 @@ def test_more_limited_cells_than_the_grid_holds(procedure):
     orc = _oracle(mesh, vfv, FAR)
     ref, _ = (orc.wbap_v3 if procedure == 3 else orc.wbap_v2)(u, x, if_all=True)
     assert rel_err(dn.download(), ref) <= TOL
+
+
+@pytest.mark.parametrize("nx,ny,sor", [(1, 1, 0), (5, 51, 0), (16, 16, 0), (257, 1, 0), (64, 64, 0), (241, 17, 1),
+                                       (300, 300, 0)])
+def test_sweep_increment_at_sum_edges(nx, ny, sor):
+    """The increment that ReconstructToTolerance returns, (1 / n) sum over
+    cells of |x_new - x_old|^2, from cell counts around a tree of 256 and a
+    workgroup of 16 trees, with both workgroup sizes of the sweep and with
+    SOR: sums of positive terms in FP64, so 1e-12 holds for any order."""
+    from dnds_amd.host import EulerEvaluator
+    mesh, vfv = _case(1, nx, ny, sor=sor)
+    ev = EulerEvaluator(mesh, vfv, riemannSolverType="HLLC", farFieldStaticValue=FAR)
+    u, x = _state(mesh.n_cell, 8)
+    du, dx, dn = ev.BuildMean().upload(u), vfv.BuildRec().upload(x), vfv.BuildRec()
+    before = x
+    for _ in range(2):
+        sweeps, increment = vfv.ReconstructToTolerance(du, dx, dn, 0.0, 1)
+        new = dx.download()
+        ref = ((new - before) ** 2).sum() / mesh.n_cell
+        assert sweeps == 1 and abs(increment - ref) <= 1e-12 * ref
+        before = new
