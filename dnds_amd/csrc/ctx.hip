@@ -812,124 +812,302 @@ __global__ __launch_bounds__(kBlock) void k_fill_from(int32_t n, const double *_
 
 // EvaluateRHS face loop (DNDS_FV_EulerEvaluator.cpp:215-492): left/right
 // states at the three LINE_3 points, Riemann flux, flux-balance fluxes,
-// Gauss sum.  Stores the integrated F, FLfix, FRfix per face.  BOUNDARY
-// selects the boundary-face instance (run over the list of boundary faces);
-// the inner instance skips boundary faces, so neither carries the other's
-// registers.
+// Gauss sum.  Stores the integrated F, FLfix, FRfix per face in its cells'
+// slots.
 //
 // MIXED: the face reconstruction D0 . x runs in FP32 (FP32 bases, FP32
 // accumulation) and the integrated fluxes are stored in FP32; the Riemann
 // solver and the boundary states stay FP64.
-//
-// STRAIGHT (inner faces of a mesh whose face normals are bitwise equal at the
-// three points, as on straight edges): the unit normal, |n| and the
-// flux-balance fluxes are computed at point 0 and reused, which yields the
-// same bits as recomputing them from the same inputs.
 //
 // VIS (muGas > 0, FP64 only): also the gradients of both sides at each point
 // from rows 1, 2 of the DiBj blocks (DNDS_FV_EulerEvaluator.cpp:297-346), the
 // face gradient with the jump term over distGRP = 2 min(V) / A, which walls
 // push to 3e200 (:356-395, USE_DISABLE_DIST_GRP_FIX_AT_WALL), and fluxFace's
 // viscous flux (DNDS_FV_EulerEvaluator.hpp:397-430, 574-577).
-template <bool BOUNDARY, bool MIXED = false, bool STRAIGHT = false, bool VIS = false>
-__global__ __launch_bounds__(kBlock, VIS && !BOUNDARY ? 2 : 1) void k_rhs_face(int32_t n, int64_t ldf, int nfmax,
-                                                     const int32_t *__restrict__ list,
-                                                     const int32_t *__restrict__ f2c,
-                                                     const int32_t *__restrict__ fbc, const double *__restrict__ fxy,
-                                                     const double *__restrict__ cmom,
-                                                     const double *__restrict__ fn, const double *__restrict__ fctr,
-                                                     const double *__restrict__ dlf, const double *__restrict__ u,
-                                                     const double *__restrict__ x, GasParams gp, double t,
-                                                     const uint8_t *__restrict__ fpos,
-                                                     double *__restrict__ fslot, int32_t *errw,
-                                                     float *__restrict__ fslot32,
-                                                     const double *__restrict__ cscale = nullptr,
-                                                     const double *__restrict__ vol = nullptr,
-                                                     const double *__restrict__ farea = nullptr,
-                                                     const double *__restrict__ xalt = nullptr,
-                                                     const uint8_t *__restrict__ limf = nullptr) {
-    static_assert(!(VIS && MIXED), "the viscous terms run in FP64 only");
-    const int32_t tid = xcd_block() * blockDim.x + threadIdx.x;
-    if (tid >= n)
-        return;
-    const int32_t f = BOUNDARY ? list[tid] : tid;
-    const int32_t L = f2c[f], R = f2c[ldf + f];
+struct FaceArgs {
+    int64_t ldf;
+    int32_t nfmax;
+    const int32_t *f2c, *fbc;
+    const double *fxy, *cmom, *fn, *fctr, *dlf, *u, *x;
+    GasParams gp;
+    double t;
+    const uint8_t *fpos;
+    double *fslot;
+    float *fslot32;
+    int32_t *errw;
+    const double *cscale, *vol, *farea; // VIS
+    // the steps' limiter leaves its unlimited cells in x and flags the others
+    const double *xalt;
+    const uint8_t *limf;
+
+    __device__ const double *rec_of(int32_t cell) const { return (limf && limf[cell]) ? xalt : x; }
+};
+
+// reconstructed increments D0 . x of one side's cell at NP of the face's
+// points from point g0 on; the bases D0 (row 0 of the DiBj blocks) are
+// evaluated from the points' scaled coordinates and the cell's moments, in c
+// order as stored bases would be read.  MIXED: the bases are rounded to FP32
+// and the products accumulated in FP32.
+template <int NP, bool MIXED>
+__device__ __forceinline__ void face_increments(const double *xs, const double *cmom, const dbl2 *xy, int32_t cell,
+                                                int sd, int g0, double inc[NP][4]) {
+    double pX[NP][4], pY[NP][4];
+#pragma unroll
+    for (int g = 0; g < NP; g++) {
+        const dbl2 q = __builtin_nontemporal_load(xy + 64 * (sd * 3 + g0 + g));
+        int_powers(q.x, pX[g]);
+        int_powers(q.y, pY[g]);
+    }
+    float acc[NP][4];
+#pragma unroll
+    for (int g = 0; g < NP; g++)
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            inc[g][v] = 0.0, acc[g][v] = 0.f;
+#pragma unroll
+    for (int c = 0; c < 9; c++) {
+        const double m = cmom[blk64(cell, 9) + 64 * c];
+        const dbl2 *xq = reinterpret_cast<const dbl2 *>(xs + rec(cell, c, 0));
+        const dbl2 xa = xq[0], xb = xq[1];
+        const double xc[4] = {xa.x, xa.y, xb.x, xb.y};
+#pragma unroll
+        for (int g = 0; g < NP; g++) {
+            const double d = pX[g][kBX[c + 1]] * pY[g][kBY[c + 1]] - m;
+            if (MIXED) {
+                const float d32 = float(d);
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    acc[g][v] = fmaf(d32, float(xc[v]), acc[g][v]);
+            } else {
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    inc[g][v] += d * xc[v];
+            }
+        }
+    }
+    if (MIXED)
+#pragma unroll
+        for (int g = 0; g < NP; g++)
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                inc[g][v] = double(acc[g][v]);
+}
+
+// the gradient of one side's cell at point g
+__device__ __forceinline__ void face_gradient(const double *xs, const double *cscale, const dbl2 *xy, int32_t cell,
+                                              int sd, int g, double G[2][4]) {
+    const dbl2 q = xy[64 * (sd * 3 + g)];
+    double px[4], py[4];
+    int_powers(q.x, px);
+    int_powers(q.y, py);
+    const dbl2 sc = reinterpret_cast<const dbl2 *>(cscale)[cell];
+    const double isx = 1.0 / sc.x, isy = 1.0 / sc.y; // the rows' scales as reciprocals
+#pragma unroll
+    for (int d = 0; d < 2; d++)
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            G[d][v] = 0.0;
+    // d/dx: bx X^(bx-1) Y^by / sx, d/dy: by X^bx Y^(by-1) / sy
+#pragma unroll
+    for (int c = 0; c < 9; c++) {
+        const int bx = kBX[c + 1], by = kBY[c + 1];
+        const dbl2 *xq = reinterpret_cast<const dbl2 *>(xs + rec(cell, c, 0));
+        const dbl2 xa = xq[0], xb = xq[1];
+        const double xc[4] = {xa.x, xa.y, xb.x, xb.y};
+        if (bx > 0) {
+            const double dx = double(bx) * px[bx - 1] * py[by] * isx;
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                G[0][v] += dx * xc[v];
+        }
+        if (by > 0) {
+            const double dy = double(by) * px[bx] * py[by - 1] * isy;
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                G[1][v] += dy * xc[v];
+        }
+    }
+}
+
+// adds the viscous flux at a point to F, from the gradients of both sides
+// (gR = gL at a boundary face), minVol the smaller volume
+__device__ __forceinline__ void add_viscous_flux(const GasParams &gp, const double gL[2][4], const double gR[2][4],
+                                                 double minVol, double area, int32_t bc, double n0, double n1,
+                                                 const double ULxy[4], const double URxy[4], double F[4]) {
+    double distGRP = minVol / area * 2;
+    distGRP += (bc == BC_WALL_EULER || bc == BC_WALL_NOSLIP) ? 3e200 : 0.0;
+    double GM[2][4], UM[4];
+#pragma unroll
+    for (int d = 0; d < 2; d++) {
+        const double nd = d ? n1 : n0;
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            GM[d][v] = (gR[d][v] + gL[d][v]) * 0.5 + (1.0 / distGRP) * (nd * (URxy[v] - ULxy[v]));
+    }
+#pragma unroll
+    for (int v = 0; v < 4; v++)
+        UM[v] = 0.5 * (ULxy[v] + URxy[v]);
+    const double vm0 = UM[1] / UM[0], vm1 = UM[2] / UM[0];
+    double pM, aM, HM;
+    ideal_gas_thermal(UM[3], UM[0], vm0 * vm0 + vm1 * vm1, gp.gamma, pM, aM, HM);
+    const double muf = sutherland_mu(gp, pM, UM[0]);
+    const double k = gp.cp * (muf - muf) / 0.9 + gp.cp * muf / gp.pr;
+    double vn[4];
+    viscous_flux_n(UM, GM, n0, n1, bc == BC_WALL_NOSLIP, gp.gamma, muf, k, gp.cp, vn);
+#pragma unroll
+    for (int v = 0; v < 4; v++)
+        F[v] += vn[v];
+}
+
+// A quad per face, lane g at point g (the fourth repeats the third's): the
+// flux's long chain of divisions and square roots runs once instead of three
+// times in turn.  A few hundred boundary faces on one lane each were a launch
+// of 15 to 35 us after the inner faces', all of it that chain; as quads in
+// front of the inner faces' workgroups they cost nothing of their own (33 k
+// cells: 16 + 20 us before, 17 now; viscous 27 + 27, 26).  Each lane sums the points in order (the others' values from
+// their lanes) and stores one of the face's four terms.
+template <bool BOUNDARY, bool MIXED, bool VIS>
+__device__ __forceinline__ void face_quad(const FaceArgs &fa, int32_t f) {
+    const int lane = threadIdx.x & 3, g = lane < 3 ? lane : 2;
+    const int32_t L = fa.f2c[f], R = fa.f2c[fa.ldf + f];
     if (!BOUNDARY && R < 0)
         return;
-    double uL[4], uR[4] = {0, 0, 0, 0};
+    double uL[4], uR[4], inc[1][4], ULxy[4], URxy[4], URm[4];
+    const dbl2 *xy = reinterpret_cast<const dbl2 *>(fa.fxy) + blk64(f, 6);
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        uL[k] = fa.u[4 * int64_t(L) + k];
+    const double nx = fa.fn[blk64(f, 6) + 64 * (2 * g)], ny = fa.fn[blk64(f, 6) + 64 * (2 * g + 1)];
+    const double dl = fa.dlf[f];
+    const int32_t bc = BOUNDARY ? fa.fbc[f] : BC_INNER;
+    const int32_t pos = fa.fpos[f];
+    face_increments<1, MIXED>(fa.rec_of(L), fa.cmom, xy, L, 0, g, inc);
+    compress_rec_part(uL, inc[0], ULxy);
+    double n0, n1;
+    normalized(nx, ny, n0, n1);
+    const double nl = sqrt(nx * nx + ny * ny);
+    bool ok = true;
+    if (BOUNDARY) {
+        const double px = fa.fctr[f], py = fa.fctr[fa.ldf + f];
+        ok &= boundary_value(fa.gp, ULxy, n0, n1, px, py, fa.t, bc, URxy);
+        ok &= boundary_value(fa.gp, uL, n0, n1, px, py, fa.t, bc, URm);
+    } else {
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            uR[k] = URm[k] = fa.u[4 * int64_t(R) + k];
+        face_increments<1, MIXED>(fa.rec_of(R), fa.cmom, xy, R, 1, g, inc);
+        compress_rec_part(uR, inc[0], URxy);
+    }
+    double F[4], FL[4], FR[4];
+    ok = ok && balance_fluxes(fa.gp, uL, URm, n0, n1, FL, FR);
+    ok = ok && riemann_face(fa.gp, ULxy, URxy, n0, n1, dl, F);
+    if (VIS) {
+        double gL[2][4], gR[2][4], minVol = fa.vol[L];
+        face_gradient(fa.rec_of(L), fa.cscale, xy, L, 0, g, gL);
+        if (!BOUNDARY) {
+            face_gradient(fa.rec_of(R), fa.cscale, xy, R, 1, g, gR);
+            minVol = fmin(minVol, fa.vol[R]);
+        }
+        add_viscous_flux(fa.gp, gL, BOUNDARY ? gL : gR, minVol, fa.farea[f], bc, n0, n1, ULxy, URxy, F);
+    }
+    if (!ok)
+        raise_error(fa.errw, ERR_NONPOSITIVE);
+    const double w = g == 1 ? kLine3W1 : kLine3W0;
+    double term[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const double a = F[v] * nl, b = FL[v] * nl, c = FR[v] * nl;
+        const double pa = a * w, pb = b * w, pc = c * w;
+        double sa = 0.0, sb = 0.0, sc = 0.0;
+#pragma unroll
+        for (int q = 0; q < 3; q++)
+            sa += quad_get(pa, q), sb += quad_get(pb, q), sc += quad_get(pc, q);
+        // signed as the cells apply them
+        term[v] = lane == 0 ? sa : lane == 1 ? -sb : lane == 2 ? -sa : sc;
+    }
+    if (BOUNDARY && lane > 1)
+        return;
+    const int64_t o = (lane < 2 ? quad64(L, 2 * fa.nfmax, 2 * (pos & 15)) : quad64(R, 2 * fa.nfmax, 2 * (pos >> 4))) +
+                      256 * (lane & 1);
+    if (MIXED) {
+        *reinterpret_cast<flt4 *>(fa.fslot32 + o) = flt4{float(term[0]), float(term[1]), float(term[2]), float(term[3])};
+    } else {
+        dbl2 *p = reinterpret_cast<dbl2 *>(fa.fslot + o);
+        p[0] = dbl2{term[0], term[1]}, p[1] = dbl2{term[2], term[3]};
+    }
+}
+
+// The first nbb workgroups (a multiple of the XCDs) take the nb boundary faces
+// of `list`, the others the n faces' inner ones.
+template <bool MIXED, bool VIS>
+__global__ __launch_bounds__(64) void k_rhs_face_quads(int32_t nb, int32_t nbb, const int32_t *__restrict__ list,
+                                                           int32_t n, FaceArgs fa) {
+    const int32_t b = blockIdx.x;
+    if (b < nbb) {
+        const int32_t q = int32_t(b * blockDim.x + threadIdx.x) >> 2;
+        if (q < nb)
+            face_quad<true, MIXED, VIS>(fa, list[q]);
+    } else {
+        const int32_t f = int32_t(xcd_block(b - nbb, gridDim.x - nbb) * blockDim.x + threadIdx.x) >> 2;
+        if (f < n)
+            face_quad<false, MIXED, VIS>(fa, f);
+    }
+}
+
+// One lane per inner face, for meshes that fill the chip this way; the three
+// points in turn.  Boundary faces as in k_rhs_face_quads.
+//
+// STRAIGHT (a mesh whose face normals are bitwise equal at the three points,
+// as on straight edges): the unit normal, |n| and the flux-balance fluxes are
+// computed at point 0 and reused, which yields the same bits as recomputing
+// them from the same inputs.
+template <bool MIXED, bool STRAIGHT, bool VIS>
+__global__ __launch_bounds__(kBlock, VIS ? 2 : 1) void k_rhs_face(
+    int32_t nb, int32_t nbb, const int32_t *__restrict__ list, FaceArgs fa, int32_t n, int64_t ldf, int nfmax, const int32_t *__restrict__ f2c, const double *__restrict__ fxy,
+    const double *__restrict__ cmom, const double *__restrict__ fn, const double *__restrict__ dlf,
+    const double *__restrict__ u, const double *__restrict__ x, GasParams gp, const uint8_t *__restrict__ fpos,
+    double *__restrict__ fslot, float *__restrict__ fslot32, int32_t *errw, const double *__restrict__ cscale,
+    const double *__restrict__ vol, const double *__restrict__ farea, const double *__restrict__ xalt,
+    const uint8_t *__restrict__ limf) {
+    static_assert(!(VIS && MIXED), "the viscous terms run in FP64 only");
+    const int32_t b = blockIdx.x;
+    if (b < nbb) {
+        const int32_t q = int32_t(b * blockDim.x + threadIdx.x) >> 2;
+        if (q < nb)
+            face_quad<true, MIXED, VIS>(fa, list[q]);
+        return;
+    }
+    const int32_t f = xcd_block(b - nbb, gridDim.x - nbb) * blockDim.x + threadIdx.x;
+    if (f >= n)
+        return;
+    const int32_t L = f2c[f], R = f2c[ldf + f];
+    if (R < 0)
+        return;
+    double uL[4], uR[4];
 #pragma unroll
     for (int k = 0; k < 4; k++)
         uL[k] = u[4 * int64_t(L) + k];
-    // reconstructed increments D0 . x at the 3 points, both sides; the bases
-    // D0 (row 0 of the DiBj blocks) are evaluated from the points' scaled
-    // coordinates and the cell's moments, per side in c order as stored bases
-    // would be read.  MIXED: the bases are rounded to FP32 and the products
-    // accumulated in FP32.
     double incL[3][4], incR[3][4];
-#pragma unroll
-    for (int g = 0; g < 3; g++)
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-            incL[g][v] = 0.0, incR[g][v] = 0.0;
     const dbl2 *xy = reinterpret_cast<const dbl2 *>(fxy) + blk64(f, 6);
 #pragma unroll 1
-    for (int sd = 0; sd < (BOUNDARY ? 1 : 2); sd++) {
-        const int32_t cell = sd ? R : L;
-        // the steps' limiter leaves its unlimited cells in x and flags the others
-        const double *xs = (limf && limf[cell]) ? xalt : x;
-        double pX[3][4], pY[3][4];
-#pragma unroll
-        for (int g = 0; g < 3; g++) {
-            const dbl2 q = __builtin_nontemporal_load(xy + 64 * (sd * 3 + g));
-            int_powers(q.x, pX[g]);
-            int_powers(q.y, pY[g]);
-        }
+    for (int sd = 0; sd < 2; sd++) {
         double inc[3][4];
-        float acc[3][4];
-#pragma unroll
-        for (int g = 0; g < 3; g++)
-#pragma unroll
-            for (int v = 0; v < 4; v++)
-                inc[g][v] = 0.0, acc[g][v] = 0.f;
-#pragma unroll
-        for (int c = 0; c < 9; c++) {
-            const double m = cmom[blk64(cell, 9) + 64 * c];
-            const dbl2 *xq = reinterpret_cast<const dbl2 *>(xs + rec(cell, c, 0));
-            const dbl2 xa = xq[0], xb = xq[1];
-            const double xc[4] = {xa.x, xa.y, xb.x, xb.y};
-#pragma unroll
-            for (int g = 0; g < 3; g++) {
-                const double d = pX[g][kBX[c + 1]] * pY[g][kBY[c + 1]] - m;
-                if (MIXED) {
-                    const float d32 = float(d);
-#pragma unroll
-                    for (int v = 0; v < 4; v++)
-                        acc[g][v] = fmaf(d32, float(xc[v]), acc[g][v]);
-                } else {
-#pragma unroll
-                    for (int v = 0; v < 4; v++)
-                        inc[g][v] += d * xc[v];
-                }
-            }
-        }
+        const int32_t cell = sd ? R : L;
+        face_increments<3, MIXED>((limf && limf[cell]) ? xalt : x, cmom, xy, cell, sd, 0, inc);
 #pragma unroll
         for (int g = 0; g < 3; g++)
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                const double r = MIXED ? double(acc[g][v]) : inc[g][v];
                 if (sd)
-                    incR[g][v] = r;
+                    incR[g][v] = inc[g][v];
                 else
-                    incL[g][v] = r;
+                    incL[g][v] = inc[g][v];
             }
     }
-    if (!BOUNDARY) {
 #pragma unroll
-        for (int k = 0; k < 4; k++)
-            uR[k] = u[4 * int64_t(R) + k];
-    }
+    for (int k = 0; k < 4; k++)
+        uR[k] = u[4 * int64_t(R) + k];
     const double dl = dlf[f];
-    const int32_t bc = BOUNDARY ? fbc[f] : BC_INNER;
     double acc[12];
 #pragma unroll
     for (int k = 0; k < 12; k++)
@@ -938,98 +1116,26 @@ __global__ __launch_bounds__(kBlock, VIS && !BOUNDARY ? 2 : 1) void k_rhs_face(i
     double n0, n1, nl, FL[4], FR[4];
     // the viscous variant keeps its points apart: unrolled, their gradient
     // work would be scheduled together and crowd the registers
-#pragma unroll(VIS && !BOUNDARY ? 1 : 3)
+#pragma unroll(VIS ? 1 : 3)
     for (int g = 0; g < 3; g++) {
-        double ULxy[4], URxy[4], URm[4];
+        double ULxy[4], URxy[4];
         if (!STRAIGHT || g == 0) {
             const double nx = fn[blk64(f, 6) + 64 * (2 * g)], ny = fn[blk64(f, 6) + 64 * (2 * g + 1)];
             normalized(nx, ny, n0, n1);
             nl = sqrt(nx * nx + ny * ny);
         }
         compress_rec_part(uL, incL[g], ULxy);
-        if (!BOUNDARY) {
-            compress_rec_part(uR, incR[g], URxy);
-#pragma unroll
-            for (int k = 0; k < 4; k++)
-                URm[k] = uR[k];
-        } else {
-            const double px = fctr[f], py = fctr[ldf + f];
-            ok &= boundary_value(gp, ULxy, n0, n1, px, py, t, bc, URxy);
-            ok &= boundary_value(gp, uL, n0, n1, px, py, t, bc, URm);
-        }
+        compress_rec_part(uR, incR[g], URxy);
         double F[4];
         if (!STRAIGHT || g == 0)
-            okb = ok && balance_fluxes(gp, uL, URm, n0, n1, FL, FR);
+            okb = ok && balance_fluxes(gp, uL, uR, n0, n1, FL, FR);
         ok &= ok && okb && riemann_face(gp, ULxy, URxy, n0, n1, dl, F);
         if (VIS) {
-            // the gradients of both sides at this point, formed here rather
-            // than kept for all three points
-            auto grad_at = [&](int32_t cell, int sd, double G[2][4]) {
-                const dbl2 q = xy[64 * (sd * 3 + g)];
-                double px[4], py[4];
-                int_powers(q.x, px);
-                int_powers(q.y, py);
-                const dbl2 sc = reinterpret_cast<const dbl2 *>(cscale)[cell];
-                const double isx = 1.0 / sc.x, isy = 1.0 / sc.y; // the rows' scales as reciprocals
-                const double *xs = (limf && limf[cell]) ? xalt : x;
-#pragma unroll
-                for (int d = 0; d < 2; d++)
-#pragma unroll
-                    for (int v = 0; v < 4; v++)
-                        G[d][v] = 0.0;
-                // d/dx: bx X^(bx-1) Y^by / sx, d/dy: by X^bx Y^(by-1) / sy
-#pragma unroll
-                for (int c = 0; c < 9; c++) {
-                    const int bx = kBX[c + 1], by = kBY[c + 1];
-                    const dbl2 *xq = reinterpret_cast<const dbl2 *>(xs + rec(cell, c, 0));
-                    const dbl2 xa = xq[0], xb = xq[1];
-                    const double xc[4] = {xa.x, xa.y, xb.x, xb.y};
-                    if (bx > 0) {
-                        const double dx = double(bx) * px[bx - 1] * py[by] * isx;
-#pragma unroll
-                        for (int v = 0; v < 4; v++)
-                            G[0][v] += dx * xc[v];
-                    }
-                    if (by > 0) {
-                        const double dy = double(by) * px[bx] * py[by - 1] * isy;
-#pragma unroll
-                        for (int v = 0; v < 4; v++)
-                            G[1][v] += dy * xc[v];
-                    }
-                }
-            };
+            // formed here rather than kept for all three points
             double gL[2][4], gR[2][4];
-            grad_at(L, 0, gL);
-            if (!BOUNDARY)
-                grad_at(R, 1, gR);
-            double minVol = vol[L];
-            if (!BOUNDARY)
-                minVol = fmin(minVol, vol[R]);
-            double distGRP = minVol / farea[f] * 2;
-            distGRP += (bc == BC_WALL_EULER || bc == BC_WALL_NOSLIP) ? 3e200 : 0.0;
-            double GM[2][4], UM[4];
-#pragma unroll
-            for (int d = 0; d < 2; d++) {
-                const double nd = d ? n1 : n0;
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const double gr = BOUNDARY ? gL[d][v] : gR[d][v];
-                    GM[d][v] = (gr + gL[d][v]) * 0.5 + (1.0 / distGRP) * (nd * (URxy[v] - ULxy[v]));
-                }
-            }
-#pragma unroll
-            for (int v = 0; v < 4; v++)
-                UM[v] = 0.5 * (ULxy[v] + URxy[v]);
-            const double vm0 = UM[1] / UM[0], vm1 = UM[2] / UM[0];
-            double pM, aM, HM;
-            ideal_gas_thermal(UM[3], UM[0], vm0 * vm0 + vm1 * vm1, gp.gamma, pM, aM, HM);
-            const double muf = sutherland_mu(gp, pM, UM[0]);
-            const double k = gp.cp * (muf - muf) / 0.9 + gp.cp * muf / gp.pr;
-            double vn[4];
-            viscous_flux_n(UM, GM, n0, n1, bc == BC_WALL_NOSLIP, gp.gamma, muf, k, gp.cp, vn);
-#pragma unroll
-            for (int v = 0; v < 4; v++)
-                F[v] += vn[v];
+            face_gradient((limf && limf[L]) ? xalt : x, cscale, xy, L, 0, g, gL);
+            face_gradient((limf && limf[R]) ? xalt : x, cscale, xy, R, 1, g, gR);
+            add_viscous_flux(gp, gL, gR, fmin(vol[L], vol[R]), farea[f], BC_INNER, n0, n1, ULxy, URxy, F);
         }
         const double w = g == 1 ? kLine3W1 : kLine3W0;
 #pragma unroll
@@ -1053,10 +1159,8 @@ __global__ __launch_bounds__(kBlock, VIS && !BOUNDARY ? 2 : 1) void k_rhs_face(i
         };
         put(oL, float(acc[0]), float(acc[1]), float(acc[2]), float(acc[3]));
         put(oL + 256, -float(acc[4]), -float(acc[5]), -float(acc[6]), -float(acc[7]));
-        if (!BOUNDARY) {
-            put(oR, -float(acc[0]), -float(acc[1]), -float(acc[2]), -float(acc[3]));
-            put(oR + 256, float(acc[8]), float(acc[9]), float(acc[10]), float(acc[11]));
-        }
+        put(oR, -float(acc[0]), -float(acc[1]), -float(acc[2]), -float(acc[3]));
+        put(oR + 256, float(acc[8]), float(acc[9]), float(acc[10]), float(acc[11]));
         return;
     }
     // plain stores (with non-temporal ones this kernel ran 19 % slower)
@@ -1066,10 +1170,8 @@ __global__ __launch_bounds__(kBlock, VIS && !BOUNDARY ? 2 : 1) void k_rhs_face(i
     };
     put(oL, acc[0], acc[1], acc[2], acc[3]);
     put(oL + 256, -acc[4], -acc[5], -acc[6], -acc[7]);
-    if (!BOUNDARY) {
-        put(oR, -acc[0], -acc[1], -acc[2], -acc[3]);
-        put(oR + 256, acc[8], acc[9], acc[10], acc[11]);
-    }
+    put(oR, -acc[0], -acc[1], -acc[2], -acc[3]);
+    put(oR + 256, acc[8], acc[9], acc[10], acc[11]);
 }
 
 // EvaluateRHS scatter as a per-cell gather in ascending face order
@@ -2267,37 +2369,41 @@ int launch_dt(dndsmi_ctx *c, const double *u, double cfl, double max_dt, double 
     return c->launch_check("dt kernels");
 }
 
+// Meshes with fewer faces take a quad per face.  EvaluateRHS with EvaluateDt,
+// quads / one lane per face, us: Euler 8 k cells (12 k faces) 43 / 47, 16 k
+// 45 / 49, 33 k (49 k faces) 52 / 49, 131 k 90 / 80; viscous 8 k 45 / 55, 16 k
+// 48 / 56, 33 k 60 / 60, 131 k 116 / 114.
+constexpr int64_t kQuadFaces = 40000;
+
+// the face fluxes into fslot (MIXED: fslot32)
+template <bool MIXED, bool VIS>
+int launch_rhs_faces(dndsmi_ctx *c, const double *u, const double *x, double t, const double *xalt,
+                     const uint8_t *limf) {
+    const int32_t nf = int32_t(c->nf), nb = int32_t(c->n_bface);
+    const FaceArgs fa{c->ldf,   c->nfmax, c->f2c,     c->fbc,  c->fxy,    c->cmom, c->fn,
+                      c->fctr,  c->dlambda_face, u,   x,       c->gas,    t,
+                      c->fpos,  c->fslot, c->fslot32, c->errw, c->cscale, c->vol,  c->farea, xalt, limf};
+    const bool quads = nf < kQuadFaces;
+    const int block = quads ? 64 : kBlock;
+    const unsigned nbb = (grid_for(4 * int64_t(nb), block) + kNumXCD - 1) / kNumXCD * kNumXCD;
+    prof_begin(c, MIXED ? DNDSMI_K_RHS_FACE32 : DNDSMI_K_RHS_FACE);
+    if (quads)
+        hipLaunchKernelGGL((k_rhs_face_quads<MIXED, VIS>), dim3(nbb + grid_for(4 * int64_t(nf), block)), dim3(block), 0,
+                           c->stream, nb, int32_t(nbb), c->bfaces, nf, fa);
+    else
+        hipLaunchKernelGGL((c->straight_faces ? k_rhs_face<MIXED, true, VIS> : k_rhs_face<MIXED, false, VIS>),
+                           dim3(nbb + grid_for(nf, block)), dim3(block), 0, c->stream, nb, int32_t(nbb), c->bfaces, fa,
+                           nf, c->ldf, c->nfmax, c->f2c, c->fxy, c->cmom, c->fn, c->dlambda_face, u, x, c->gas,
+                           c->fpos, c->fslot, c->fslot32, c->errw, c->cscale, c->vol, c->farea, xalt, limf);
+    prof_end(c);
+    return c->launch_check("k_rhs_face");
+}
+
 int launch_rhs(dndsmi_ctx *c, const double *u, const double *x, double t, double *rhs, int stage, double *xs,
                const double *dt, double coefA, double coefB, const double *xalt, const uint8_t *limf) {
-    const int nc = int(c->nc), nf = int(c->nf);
-    prof_begin(c, DNDSMI_K_RHS_FACE);
-    if (c->gas.mu > 0) {
-        hipLaunchKernelGGL((c->straight_faces ? k_rhs_face<false, false, true, true>
-                                              : k_rhs_face<false, false, false, true>),
-                           dim3(grid_for(nf)), dim3(kBlock), 0, c->stream, nf, c->ldf, c->nfmax, c->bfaces, c->f2c,
-                           c->fbc, c->fxy, c->cmom, c->fn, c->fctr, c->dlambda_face, u, x, c->gas, t, c->fpos,
-                           c->fslot, c->errw, nullptr, c->cscale, c->vol, c->farea, xalt, limf);
-    } else {
-        hipLaunchKernelGGL((c->straight_faces ? k_rhs_face<false, false, true> : k_rhs_face<false, false, false>),
-                           dim3(grid_for(nf)), dim3(kBlock), 0, c->stream, nf, c->ldf, c->nfmax, c->bfaces, c->f2c,
-                           c->fbc, c->fxy, c->cmom, c->fn, c->fctr, c->dlambda_face, u, x, c->gas, t, c->fpos,
-                           c->fslot, c->errw, nullptr, nullptr, nullptr, nullptr, xalt, limf);
-    }
-    prof_end(c);
-    if (c->n_bface > 0) {
-        prof_begin(c, DNDSMI_K_RHS_BFACE);
-        if (c->gas.mu > 0)
-            hipLaunchKernelGGL((k_rhs_face<true, false, false, true>), dim3(grid_for(c->n_bface)), dim3(kBlock), 0,
-                               c->stream, int32_t(c->n_bface), c->ldf, c->nfmax, c->bfaces, c->f2c, c->fbc, c->fxy,
-                               c->cmom, c->fn, c->fctr, c->dlambda_face, u, x, c->gas, t, c->fpos, c->fslot, c->errw,
-                               nullptr, c->cscale, c->vol, c->farea, xalt, limf);
-        else
-            hipLaunchKernelGGL(k_rhs_face<true>, dim3(grid_for(c->n_bface)), dim3(kBlock), 0, c->stream,
-                               int32_t(c->n_bface), c->ldf, c->nfmax, c->bfaces, c->f2c, c->fbc, c->fxy, c->cmom, c->fn,
-                               c->fctr, c->dlambda_face, u, x, c->gas, t, c->fpos, c->fslot, c->errw, nullptr,
-                               nullptr, nullptr, nullptr, xalt, limf);
-        prof_end(c);
-    }
+    const int nc = int(c->nc);
+    DNDSMI_TRY((c->gas.mu > 0 ? launch_rhs_faces<false, true> : launch_rhs_faces<false, false>)(c, u, x, t, xalt,
+                                                                                               limf));
     prof_begin(c, DNDSMI_K_RHS_CELL);
     if (c->nfmax == 3)
         hipLaunchKernelGGL(k_rhs_cell<3>, dim3(grid_for(nc)), dim3(kBlock), 0, c->stream, nc, c->ldc, c->gat,
@@ -2408,18 +2514,8 @@ int launch_jacobi_mixed(dndsmi_ctx *c, const double *u, double *x, int n_sweeps,
 
 int launch_rhs_mixed(dndsmi_ctx *c, const double *u, const double *x, double t, double *rhs, int stage, double *xs,
                      const double *dt, double coefA, double coefB, const double *xalt, const uint8_t *limf) {
-    const int nc = int(c->nc), nf = int(c->nf);
-    prof_begin(c, DNDSMI_K_RHS_FACE32);
-    hipLaunchKernelGGL((c->straight_faces ? k_rhs_face<false, true, true> : k_rhs_face<false, true, false>),
-                       dim3(grid_for(nf)), dim3(kBlock), 0, c->stream, nf, c->ldf, c->nfmax, c->bfaces, c->f2c, c->fbc,
-                       c->fxy, c->cmom, c->fn, c->fctr, c->dlambda_face, u, x, c->gas, t, c->fpos, nullptr, c->errw,
-                       c->fslot32, nullptr, nullptr, nullptr, xalt, limf);
-    prof_end(c);
-    if (c->n_bface > 0)
-        hipLaunchKernelGGL((k_rhs_face<true, true>), dim3(grid_for(c->n_bface)), dim3(kBlock), 0, c->stream,
-                           int32_t(c->n_bface), c->ldf, c->nfmax, c->bfaces, c->f2c, c->fbc, c->fxy, c->cmom, c->fn,
-                           c->fctr, c->dlambda_face, u, x, c->gas, t, c->fpos, nullptr, c->errw, c->fslot32,
-                           nullptr, nullptr, nullptr, xalt, limf);
+    const int nc = int(c->nc);
+    DNDSMI_TRY((launch_rhs_faces<true, false>(c, u, x, t, xalt, limf)));
     prof_begin(c, DNDSMI_K_RHS_CELL32);
     if (c->nfmax == 3)
         hipLaunchKernelGGL((k_rhs_cell<3, float>), dim3(grid_for(nc)), dim3(kBlock), 0, c->stream, nc, c->ldc,
@@ -2707,8 +2803,9 @@ extern "C" int64_t dndsmi_kernel_bytes(const dndsmi_ctx *c, int32_t kernel) {
     case DNDSMI_K_DT_CELL: // gather index, lambda + area per slot, volume, dt out
         return c2f * (4 + 16) + nc * (8 + 8);
     case DNDSMI_K_RHS_FACE: // f2c, slot positions, point coordinates, normals, dlambda, 2 x 8 terms out;
-        // x, u and the moments once per cell; viscous: face area, both volumes and cell scales
-        return nif * (8 + 1 + 96 + (c->straight_faces ? 16 : 48) + 8 + 128 + (c->gas.mu > 0 ? 8 + 16 + 32 : 0)) +
+        // x, u and the moments once per cell; viscous: face area, both volumes and cell scales; boundary faces:
+        // index, f2c, slot position, kind, one side's point coordinates, normals, centre, dlambda, 8 terms out
+        return c->n_bface * (4 + 8 + 1 + 4 + 48 + 48 + 16 + 8 + 64 + (c->gas.mu > 0 ? 8 + 8 + 16 : 0)) + nif * (8 + 1 + 96 + (c->straight_faces ? 16 : 48) + 8 + 128 + (c->gas.mu > 0 ? 8 + 16 + 32 : 0)) +
                nc * (36 * 8 + 32 + 72);
     case DNDSMI_K_RHS_CELL: // 8 terms per slot, volume, x read+write, xLast (+ last-slot index for 4 slots)
         return c2f * 64 + nc * (8 + 32 * 3 + (c->nfmax == 4 ? 4 : 0));
@@ -2720,21 +2817,17 @@ extern "C" int64_t dndsmi_kernel_bytes(const dndsmi_ctx *c, int32_t kernel) {
         return c2f * (32 + 4) + nc * (8 + (c->wbap_full_copy ? 36 * 8 * 2 : 1));
     case DNDSMI_K_WBAP_LIM: // depends on the number of limited cells; not a bandwidth kernel
         return 0;
-    case DNDSMI_K_RHS_BFACE: // per boundary face: index, f2c, slot position, kind, one side's point
-        // coordinates, normals, centre, dlambda, 8 terms out, the cell's x, u and moments
-        return c->n_bface * (4 + 8 + 1 + 4 + 48 + 48 + 16 + 8 + 64 + 36 * 8 + 32 + 72 +
-                             (c->gas.mu > 0 ? 8 + 8 + 16 : 0));
-    case DNDSMI_K_LUSGS_MATVEC: // per scan position cell, D, volume, x own in, Ax out; per slot both
-        // neighbour indices, face, normal, area, u and x of the neighbour, lambda
-        return nc * (4 + 8 + 8 + 32 + 32) + c2f * (8 + 4 + 16 + 8 + 32 + 32 + 8);
+    case DNDSMI_K_LUSGS_MATVEC: // per scan position cell, D, x own in, Ax out; per slot both neighbour indices,
+        // normal, c_f, lambda, u and x of the neighbour
+        return nc * (4 + 8 + 32 + 32) + c2f * (8 + 16 + 16 + 32 + 32);
     case DNDSMI_K_LUSGS_SWEEP: // one whole forward (or backward) sweep, all colours together: per scan position
-        // cell, volume, 1/D, rhs (or the increment) in, increment out; per slot the neighbour index, and per used
-        // slot (half of them) face, normal, area, u and the increment of the neighbour, lambda
-        return nc * (4 + 8 + 8 + 32 + 32) + c2f * 4 + c2f / 2 * (4 + 16 + 8 + 32 + 32 + 8);
+        // cell, 1/D, rhs (or the increment) in, increment out; per slot the neighbour index, and per used slot
+        // (half of them) normal, c_f, lambda, u and the increment of the neighbour
+        return nc * (4 + 8 + 32 + 32) + c2f * 4 + c2f / 2 * (16 + 16 + 32 + 32);
     case DNDSMI_K_DELTA32: // FP32 M per slot + slot index; d read + r read + d write (FP32)
         return c2f * (81 * 4 + 4) + nc * (36 * 4 * 3);
     case DNDSMI_K_RHS_FACE32: // as DNDSMI_K_RHS_FACE with 2 x 8 FP32 terms out
-        return nif * (8 + 1 + 96 + (c->straight_faces ? 16 : 48) + 8 + 64) + nc * (36 * 8 + 32 + 72);
+        return c->n_bface * (4 + 8 + 1 + 4 + 48 + 48 + 16 + 8 + 32) + nif * (8 + 1 + 96 + (c->straight_faces ? 16 : 48) + 8 + 64) + nc * (36 * 8 + 32 + 72);
     case DNDSMI_K_RHS_CELL32: // 8 FP32 terms per slot, volume, x read+write, xLast (+ last-slot index)
         return c2f * 32 + nc * (8 + 32 * 3 + (c->nfmax == 4 ? 4 : 0));
     case DNDSMI_K_READ_PROBE: // the sweep's A^-1 B, A^-1 b (45 x 16 B per slot) and slot index, four doubles out

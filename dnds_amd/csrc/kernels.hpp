@@ -48,12 +48,12 @@ __device__ inline double sqr(double x) { return x * x; }
 // a bijection of [0, gridDim.x) for any grid size.
 constexpr int32_t kNumXCD = 8;
 
-__device__ __forceinline__ int32_t xcd_block() {
-    const int32_t n = int32_t(gridDim.x), w = int32_t(blockIdx.x);
+__device__ __forceinline__ int32_t xcd_block(int32_t w, int32_t n) {
     const int32_t x = w % kNumXCD, q = w / kNumXCD;
     const int32_t base = n / kNumXCD, extra = n % kNumXCD; // XCD x < extra runs base + 1 blocks
     return x * base + (x < extra ? x : extra) + q;
 }
+__device__ __forceinline__ int32_t xcd_block() { return xcd_block(int32_t(blockIdx.x), int32_t(gridDim.x)); }
 
 // 16-byte vectors for streaming loads
 typedef double dbl2 __attribute__((ext_vector_type(2)));

@@ -552,17 +552,17 @@ enum {
     DNDSMI_K_WALL_CORR = 1,  /* no launches: the sweeps correct their wall cells themselves */
     DNDSMI_K_DT_FACE = 2,    /* EvaluateDt, face part                         */
     DNDSMI_K_DT_CELL = 3,    /* EvaluateDt, cell part + block minima          */
-    DNDSMI_K_RHS_FACE = 4,   /* EvaluateRHS, inner-face fluxes                */
+    DNDSMI_K_RHS_FACE = 4,   /* EvaluateRHS, face fluxes                      */
     DNDSMI_K_RHS_CELL = 5,   /* EvaluateRHS gather (+ SSP-RK3 stage update)   */
     DNDSMI_K_WBAP_FACE = 6,  /* WBAP smoothness-indicator face terms          */
     DNDSMI_K_WBAP_CELL = 7,  /* WBAP indicator, copy of unlimited cells       */
     DNDSMI_K_WBAP_LIM = 8,   /* WBAP characteristic limiting of flagged cells */
     DNDSMI_K_LUSGS_SWEEP = 9,/* one colour of an LU-SGS forward/backward sweep */
     DNDSMI_K_DELTA32 = 10,   /* mixed precision: FP32 correction sweep       */
-    DNDSMI_K_RHS_FACE32 = 11,/* mixed precision: inner-face fluxes, FP32 reconstruction */
+    DNDSMI_K_RHS_FACE32 = 11,/* mixed precision: face fluxes, FP32 reconstruction */
     DNDSMI_K_RHS_CELL32 = 12,/* mixed precision: FP32 gather + stage update  */
     DNDSMI_K_LUSGS_MATVEC = 13,/* LUSGSMatrixVec (GMRES operator)            */
-    DNDSMI_K_RHS_BFACE = 14, /* EvaluateRHS: boundary-face fluxes (FP64)     */
+    DNDSMI_K_RHS_BFACE = 14, /* no launches: the face kernel takes boundary faces too */
     DNDSMI_K_READ_PROBE = 15,/* read-bandwidth probe of the sweep's A^-1 B stream */
     DNDSMI_K_COUNT = 16
 };

@@ -14,10 +14,10 @@ pytestmark = pytest.mark.gpu
 TOL = 1e-12
 
 
-def _case(kind, nx, ny, sor=0, limiter=0, seed=3):
+def _case(kind, nx, ny, sor=0, limiter=0, seed=3, top=None):
     from dnds_amd import _capi as A
     from dnds_amd.host import RIEMANN_VR_SETTING, CompactFacedMeshSerialRW, VRFiniteVolume2D, vr_setting
-    bcs = (A.BC_FARFIELD, A.BC_WALL_NOSLIP, A.BC_WALL_EULER, A.BC_WALL)
+    bcs = (A.BC_FARFIELD, A.BC_WALL_NOSLIP, A.BC_WALL_EULER, A.BC_WALL if top is None else top)
     mesh = CompactFacedMeshSerialRW.generate(kind, nx, ny, 0.0, 1.0, 0.0, ny / nx, jitter=0.2, seed=seed, bc=bcs)
     vfv = VRFiniteVolume2D(mesh, vr_setting(**dict(RIEMANN_VR_SETTING, far_weight=1.0, jacobi_relax=0.9),
                                             build_limiter_data=limiter, sor_instead=sor))
@@ -92,3 +92,35 @@ def test_sweep_increment_at_sum_edges(nx, ny, sor):
         ref = ((new - before) ** 2).sum() / mesh.n_cell
         assert sweeps == 1 and abs(increment - ref) <= 1e-12 * ref
         before = new
+
+
+@pytest.mark.parametrize("mu", [0.0, 1e-3])
+@pytest.mark.parametrize("kind,nx,ny", [(1, 1, 1), (2, 7, 9), (1, 140, 141), (1, 141, 142), (0, 115, 116),
+                                        (2, 127, 129)])
+def test_rhs_face_quads_and_lanes(kind, nx, ny, mu):
+    """EvaluateRHS on both sides of the face count (40000) where the face
+    fluxes go from a quad per face to a lane per face, with far-field and wall
+    boundaries in the same launch; one mixed step for the FP32 variant
+    (its tolerance: FP32 sweeps and fluxes, as in the mixed-precision tests)."""
+    import oracle
+    from dnds_amd.host import EulerEvaluator, ExplicitSSPRK3LocalDt
+    from dnds_amd import _capi as A
+    mesh, vfv = _case(kind, nx, ny, top=A.BC_FARFIELD)
+    assert (mesh.arrays()["face2cell"].size // 2 < 40000) == \
+        (nx < 115 or (kind, nx) == (1, 140))
+    u, x = _state(mesh.n_cell, 9)
+    x = 0.1 * x
+    ev = EulerEvaluator(mesh, vfv, riemannSolverType="HLLC", farFieldStaticValue=FAR, muGas=mu)
+    st = vfv.setting
+    orc = oracle.Oracle(mesh.arrays(), vfv.arrays(), riemann_solver=2, far_field=FAR, jacobi_relax=st.jacobi_relax,
+                        tang_weight=st.tang_weight, tang_weight_direction=st.tang_weight_direction, mu_gas=mu)
+    du, dx, rhs, dt = ev.BuildMean().upload(u), vfv.BuildRec().upload(x), ev.BuildMean(), ev.BuildScalar()
+    ev.EvaluateDt(dt, du, CFL=0.5, MaxDt=1e100, UseLocaldt=True)
+    ev.EvaluateRHS(rhs, du, dx, 0.1)
+    _, _, _, dlf = orc.evaluate_dt(u, 0.5, use_local_dt=True)
+    assert rel_err(rhs.download(), orc.evaluate_rhs(u, x, dlf, t=0.1)) <= TOL
+    if mu == 0.0:
+        r, rn = vfv.BuildRec().upload(x), vfv.BuildRec()
+        ExplicitSSPRK3LocalDt(ev, nInternalRecStep=2, CFL=0.3, mixedPrecision=True).Step(du, r, rn, 0.0)
+        ru, _, _ = orc.ssprk3_steps(u, x, 1, 2, 0.3)
+        assert rel_err(du.download(), ru) <= 1e-6
