@@ -71,27 +71,6 @@ void prof_end(dndsmi_ctx *c) {
 // the entries around with DPP moves, so no byte is loaded twice.  Every sum
 // runs in the order of a one-lane-per-cell sweep.
 
-// `a` of lane Q of the quad, in all four lanes
-template <int Q>
-__device__ __forceinline__ int quad_bcast32(int a) {
-    return __builtin_amdgcn_mov_dpp(a, Q * 0x55, 0xf, 0xf, true);
-}
-template <int Q>
-__device__ __forceinline__ double quad_bcast(double a) {
-    const uint64_t w = __builtin_bit_cast(uint64_t, a);
-    const uint32_t lo = uint32_t(quad_bcast32<Q>(int(uint32_t(w))));
-    const uint32_t hi = uint32_t(quad_bcast32<Q>(int(uint32_t(w >> 32))));
-    return __builtin_bit_cast(double, uint64_t(lo) | uint64_t(hi) << 32);
-}
-template <int Q>
-__device__ __forceinline__ float quad_bcast(float a) {
-    return __builtin_bit_cast(float, quad_bcast32<Q>(__builtin_bit_cast(int, a)));
-}
-template <typename T>
-__device__ __forceinline__ T quad_get(T a, int q) { // q: a constant after unrolling
-    return q == 0 ? quad_bcast<0>(a) : q == 1 ? quad_bcast<1>(a) : q == 2 ? quad_bcast<2>(a) : quad_bcast<3>(a);
-}
-
 // a quad's sum of squares, lane 0's nine in turn, then lane 1's and so on: in
 // the last lane
 __device__ __forceinline__ double quad_norm2(const double d[9]) {
@@ -773,13 +752,11 @@ __global__ __launch_bounds__(kBlock) void k_dt_cell(int32_t nc, int64_t ldc, con
     }
     red[threadIdx.x] = d;
     __syncthreads();
-    for (int st = kBlock / 2; st > 0; st >>= 1) {
-        if (threadIdx.x < st)
-            red[threadIdx.x] = fmin(red[threadIdx.x], red[threadIdx.x + st]);
-        __syncthreads();
-    }
+    if (threadIdx.x >= 64)
+        return;
+    d = tree256(red, Min());
     if (threadIdx.x == 0)
-        part[blockIdx.x] = red[0];
+        part[blockIdx.x] = d;
 }
 
 __global__ __launch_bounds__(kBlock) void k_min_final(int32_t n, const double *__restrict__ part,
@@ -790,15 +767,13 @@ __global__ __launch_bounds__(kBlock) void k_min_final(int32_t n, const double *_
         d = fmin(d, part[k]);
     red[threadIdx.x] = d;
     __syncthreads();
-    for (int st = kBlock / 2; st > 0; st >>= 1) {
-        if (threadIdx.x < st)
-            red[threadIdx.x] = fmin(red[threadIdx.x], red[threadIdx.x + st]);
-        __syncthreads();
-    }
+    if (threadIdx.x >= 64)
+        return;
+    d = tree256(red, Min());
     if (threadIdx.x == 0) {
-        out[0] = red[0];
-        *host_out = red[0];
-        if (!isfinite(red[0]))
+        out[0] = d;
+        *host_out = d;
+        if (!isfinite(d))
             raise_error(errw, ERR_NAN);
     }
 }
@@ -1255,9 +1230,12 @@ __global__ __launch_bounds__(kBlock) void k_wbap_face(int32_t nf, int64_t ldf, i
                                                       const double *__restrict__ fw,
                                                       const double *__restrict__ fn, const double *__restrict__ u,
                                                       const double *__restrict__ x, double tang_weight, int twd_norm,
-                                                      const uint8_t *__restrict__ wpos, double *__restrict__ wslot) {
+                                                      const uint8_t *__restrict__ wpos, double *__restrict__ wslot,
+                                                      int32_t *__restrict__ lim_count) {
     const int32_t t = xcd_block() * blockDim.x + threadIdx.x, f = t >> 1;
     const bool sd = t & 1;
+    if (t == 0)
+        *lim_count = 0; // k_wbap_ind, the next launch, counts
     if (f >= nf)
         return;
     const int32_t L = f2c[f], R = f2c[ldf + f];
@@ -1678,11 +1656,6 @@ __global__ __launch_bounds__(kBlock, 3) void k_wbap_lim_v2(int64_t ldc, int64_t 
                 xo[rec(i, ls + r, v)] = any ? first * (up + 1.0) / (down + 1.0) : uC[r];
         }
     }
-}
-
-__global__ void k_zero_int2(int32_t *p) {
-    if (threadIdx.x == 0 && blockIdx.x == 0)
-        p[0] = 0;
 }
 
 __global__ __launch_bounds__(kBlock) void k_set(int64_t n, double *__restrict__ p, double v) {
@@ -2427,9 +2400,8 @@ int launch_wbap(dndsmi_ctx *c, const double *u, const double *x, double *xo, dou
     prof_begin(c, DNDSMI_K_WBAP_FACE);
     hipLaunchKernelGGL(k_wbap_face, dim3(grid_for(2 * int64_t(nf))), dim3(kBlock), 0, c->stream, nf, c->ldf,
                        c->nfmax, c->f2c, c->fxy, c->cmom, c->cscale, c->fw, c->fn, u, x, c->tang_weight, c->twd_norm, c->wpos,
-                       c->wslot);
+                       c->wslot, c->lim_count);
     prof_end(c);
-    hipLaunchKernelGGL(k_zero_int2, dim3(1), dim3(64), 0, c->stream, c->lim_count);
     prof_begin(c, DNDSMI_K_WBAP_CELL);
     if (c->nfmax == 3)
         hipLaunchKernelGGL(k_wbap_ind<3>, dim3(grid_for(nc)), dim3(kBlock), 0, c->stream, nc, c->ldc, c->nbr,

@@ -55,6 +55,49 @@ __device__ __forceinline__ int32_t xcd_block(int32_t w, int32_t n) {
 }
 __device__ __forceinline__ int32_t xcd_block() { return xcd_block(int32_t(blockIdx.x), int32_t(gridDim.x)); }
 
+// The fold of 256 values in LDS, pairs at distance 128, 64, ... 1, by one wave:
+// the result in its lane 0.  (In place with a barrier per level, by the whole
+// workgroup, each fold was 8 barriers.)
+template <class Op>
+__device__ __forceinline__ double tree256(const double *red, Op op) {
+    const int lane = threadIdx.x & 63;
+    double a = op(op(red[lane], red[lane + 128]), op(red[lane + 64], red[lane + 192]));
+    for (int off = 32; off > 0; off >>= 1)
+        a = op(a, __shfl_down(a, off, 64));
+    return a;
+}
+struct Add {
+    __device__ double operator()(double a, double b) const { return a + b; }
+};
+struct Max {
+    __device__ double operator()(double a, double b) const { return fmax(a, b); }
+};
+struct Min {
+    __device__ double operator()(double a, double b) const { return fmin(a, b); }
+};
+
+// Four neighbouring lanes (a quad) share a cell or face in many kernels:
+// `a` of lane Q of the quad, in all four lanes
+template <int Q>
+__device__ __forceinline__ int quad_bcast32(int a) {
+    return __builtin_amdgcn_mov_dpp(a, Q * 0x55, 0xf, 0xf, true);
+}
+template <int Q>
+__device__ __forceinline__ double quad_bcast(double a) {
+    const uint64_t w = __builtin_bit_cast(uint64_t, a);
+    const uint32_t lo = uint32_t(quad_bcast32<Q>(int(uint32_t(w))));
+    const uint32_t hi = uint32_t(quad_bcast32<Q>(int(uint32_t(w >> 32))));
+    return __builtin_bit_cast(double, uint64_t(lo) | uint64_t(hi) << 32);
+}
+template <int Q>
+__device__ __forceinline__ float quad_bcast(float a) {
+    return __builtin_bit_cast(float, quad_bcast32<Q>(__builtin_bit_cast(int, a)));
+}
+template <typename T>
+__device__ __forceinline__ T quad_get(T a, int q) { // q: a constant after unrolling
+    return q == 0 ? quad_bcast<0>(a) : q == 1 ? quad_bcast<1>(a) : q == 2 ? quad_bcast<2>(a) : quad_bcast<3>(a);
+}
+
 // 16-byte vectors for streaming loads
 typedef double dbl2 __attribute__((ext_vector_type(2)));
 typedef float flt4 __attribute__((ext_vector_type(4)));

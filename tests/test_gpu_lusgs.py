@@ -211,7 +211,7 @@ def test_gmres_implicit_iterations_match_oracle(code):
 
 @pytest.mark.parametrize("nx,ny,code", [(1, 1, 0), (5, 1, 1), (51, 5, 1), (16, 16, 2), (257, 1, 1), (129, 128, 2),
                                         (1024, 512, 1), (1025, 512, 1)])
-def test_gmres_vectors_at_block_and_fold_edges(nx, ny, code):
+def test_gmres_vectors_at_block_and_fold_edges(nx, ny, code, n_space=4):
     """One cell (one colour), cell counts around a workgroup of 256, and the
     last mesh whose vector kernels fold the dot products themselves (2048
     workgroups, 524288 cells) with one beyond it; the tolerance is
@@ -230,14 +230,21 @@ def test_gmres_vectors_at_block_and_fold_edges(nx, ny, code):
     rho, vx, vy, p = (1 + 0.1 * rng.random(n), 0.5 + 0.1 * rng.random(n), 0.1 * rng.random(n), 1 + 0.1 * rng.random(n))
     u0 = np.stack([rho, rho * vx, rho * vy, p / 0.4 + 0.5 * rho * (vx * vx + vy * vy)], 1)
     ev = EulerEvaluator(mesh, vfv, riemannSolverType="HLLC", farFieldStaticValue=far)
-    ev.SetLinearSolver(code, 4, 1)
+    ev.SetLinearSolver(code, n_space, 1)
     ode = ImplicitEulerDualTimeStep(ev, nInternalRecStep=1, CFL=5.0, nTimeStepInternal=2, rhsThresholdInternal=0.0)
     u, r, rn = ev.BuildMean().upload(u0), vfv.BuildRec().setConstant(0.0), vfv.BuildRec()
     ode.Step(u, r, rn, dt=0.1)
     st = vfv.setting
     orc = oracle.Oracle(mesh.arrays(), vfv.arrays(), riemann_solver=2, far_field=far, tang_weight=st.tang_weight,
-                        tang_weight_direction=st.tang_weight_direction, gmres_code=code, n_gmres_space=4,
+                        tang_weight_direction=st.tang_weight_direction, gmres_code=code, n_gmres_space=n_space,
                         n_gmres_iter=1)
     ou, _, _ = orc.implicit_euler(u0, np.zeros((n, 36)), 2, 1, 5.0, dt=0.1, threshold=0.0,
                                   scan2cell=ev.LUSGSScanOrder())
     assert rel_err(u.download(), ou) <= 1e-9
+
+
+@pytest.mark.parametrize("n_space", [16, 17])
+def test_gmres_more_vectors_than_one_batch_of_dots(n_space):
+    """The dot products are folded 16 at a time: the last subspace of one
+    batch and the first of two."""
+    test_gmres_vectors_at_block_and_fold_edges(40, 30, 1, n_space)
