@@ -126,33 +126,53 @@ struct LusgsScan {
     int32_t *errw;
 };
 
-// buf -= sum over the slots' neighbours c_f dF(u_j, x_j), c_f = (alpha/2) S_f /
-// V_i, faces in cell2face order; FORWARD: the earlier neighbours, BACKWARD:
-// the later ones.  PRE: c_f and lambda as the last k_lusgs_init stored them by
-// slot (the solver's own sweeps), which saves a division and the load that
-// waits for the face's number; else from lambdaFace and alpha as they are now.
+// A quad takes a scan position, lane s its slot s: `buf` of lane v is variable
+// v's, and
+//   buf -= sum over the slots' neighbours c_f dF(u_j, x_j), c_f = (alpha/2) S_f
+//          / V_i,
+// faces in cell2face order; FORWARD: the earlier neighbours, BACKWARD: the
+// later ones.  A slot without one contributes a zero, which changes no bit.
+// PRE: c_f and lambda as the last k_lusgs_init stored them by slot (the
+// solver's own sweeps), which saves a division and the load that waits for the
+// face's number; else from lambdaFace and alpha as they are now.
+//
+// A colour of a small mesh is bound by this chain of loads and divisions; with
+// one lane per position it ran slot after slot.  Implicit iteration with GMRES,
+// us: 1.5 k cells 1012 -> 852, 3.2 k 1040 -> 866, 30 k 883 -> 762, 120 k 1436 ->
+// 1326; without GMRES 120 k 231 -> 227, 500 k 792 -> 786.
 template <int NF, bool PRE, bool FORWARD, bool BACKWARD>
-__device__ __forceinline__ void lusgs_row(const LusgsScan &sc, int32_t p, const double *__restrict__ u,
-                                          const double *x, double buf[4]) {
-    const double vi = PRE ? 0.0 : sc.vol[p];
-#pragma unroll
-    for (int s = 0; s < NF; s++) {
-        const int64_t q = s * sc.ldc + p;
-        const int32_t a = FORWARD ? sc.jf[q] : -1, b = BACKWARD ? sc.jb[q] : -1;
-        const int32_t j = a >= 0 ? a : b;
-        if (j < 0)
-            continue;
-        double uj[4], xj[4], dF[4];
+__device__ __forceinline__ double lusgs_row(const LusgsScan &sc, int32_t p, const double *__restrict__ u,
+                                            const double *x, double buf) {
+    const int s = threadIdx.x & 3;
+    const int64_t q = s * sc.ldc + p;
+    int32_t j = -1;
+    if (s < NF) {
+        j = FORWARD ? sc.jf[q] : -1;
+        if (BACKWARD && j < 0)
+            j = sc.jb[q];
+    }
+    double term[4] = {0, 0, 0, 0};
+    if (j >= 0) {
+        double uj[4], xj[4];
 #pragma unroll
         for (int v = 0; v < 4; v++)
             uj[v] = u[4 * int64_t(j) + v], xj[v] = x[4 * int64_t(j) + v];
         const double lam = PRE ? sc.lam[q] : sc.lambda[sc.sf[q]];
-        flux_jacobian_times_du(sc.gamma, uj, sc.n0[q], sc.n1[q], xj, lam, dF);
-        const double cf = PRE ? sc.cf[q] : (0.5 * sc.alpha) * sc.area[q] / vi;
+        flux_jacobian_times_du(sc.gamma, uj, sc.n0[q], sc.n1[q], xj, lam, term);
+        const double cf = PRE ? sc.cf[q] : (0.5 * sc.alpha) * sc.area[q] / sc.vol[p];
 #pragma unroll
         for (int v = 0; v < 4; v++)
-            buf[v] -= cf * dF[v];
+            term[v] *= cf;
     }
+#pragma unroll
+    for (int k = 0; k < NF; k++) {
+        double t[4];
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            t[v] = quad_get(term[v], k);
+        buf -= s == 0 ? t[0] : s == 1 ? t[1] : s == 2 ? t[2] : t[3];
+    }
+    return buf;
 }
 
 // LUSGSMatrixVec (DNDS_FV_EulerEvaluator.cpp:1062-1145) per scan position:
@@ -164,27 +184,19 @@ template <int NF, bool PRE>
 __global__ __launch_bounds__(kBlock) void k_lusgs_matvec(int32_t nc, LusgsScan sc, const double *__restrict__ u,
                                                          const double *__restrict__ x, double *__restrict__ Ax,
                                                          int32_t first, double *__restrict__ inc) {
-    const int32_t p = xcd_block() * blockDim.x + threadIdx.x;
+    const int32_t t = xcd_block() * blockDim.x + threadIdx.x, p = t >> 2;
     if (p >= nc)
         return;
-    const int64_t i = 4 * int64_t(sc.cells[p]);
-    double buf[4] = {0, 0, 0, 0};
-    lusgs_row<NF, PRE, true, true>(sc, p, u, x, buf);
-    const double d = sc.jdiag[p];
-    const double di = p < first ? sc.jinv[p] : 0.0;
-    bool finite = true;
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-        const double a = d * x[i + v] - buf[v];
-        Ax[i + v] = a;
-        if (p < first) {
-            const double o = di * a;
-            finite &= isfinite(o);
-            inc[i + v] = o;
-        }
+    const int64_t k = 4 * int64_t(sc.cells[p]) + (t & 3);
+    const double buf = lusgs_row<NF, PRE, true, true>(sc, p, u, x, 0.0);
+    const double a = sc.jdiag[p] * x[k] - buf;
+    Ax[k] = a;
+    if (p < first) {
+        const double o = sc.jinv[p] * a;
+        if (!isfinite(o))
+            raise_error(sc.errw, ERR_NAN);
+        inc[k] = o;
     }
-    if (!finite)
-        raise_error(sc.errw, ERR_NAN);
 }
 
 // One colour of an LU-SGS sweep (UpdateLUSGSForward / UpdateLUSGSBackward,
@@ -200,29 +212,19 @@ __global__ __launch_bounds__(kBlock) void k_lusgs_sweep(int32_t n, int32_t b, Lu
                                                         const double *__restrict__ rhs, const double *__restrict__ u,
                                                         const double *uInc, double *uIncNew) {
     const int32_t t = xcd_block() * blockDim.x + threadIdx.x;
-    if (t >= n)
+    if ((t >> 2) >= n)
         return;
-    const int32_t p = b + t;
-    const int64_t i = 4 * int64_t(sc.cells[p]);
-    double buf[4];
-#pragma unroll
-    for (int v = 0; v < 4; v++)
-        buf[v] = FORWARD ? rhs[i + v] : 0.0;
-    lusgs_row<NF, PRE, FORWARD, !FORWARD>(sc, p, u, uInc, buf);
+    const int32_t p = b + (t >> 2);
+    const int64_t k = 4 * int64_t(sc.cells[p]) + (t & 3);
     const double d = sc.jinv[p];
-    bool finite = true;
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-        double o = d * buf[v];
-        if (!FORWARD)
-            o = uIncNew[i + v] + o;
-        if (TURN)
-            o = o + d * 0.0;
-        finite &= isfinite(o);
-        uIncNew[i + v] = o;
-    }
-    if (!finite)
+    double o = d * lusgs_row<NF, PRE, FORWARD, !FORWARD>(sc, p, u, uInc, FORWARD ? rhs[k] : 0.0);
+    if (!FORWARD)
+        o = uIncNew[k] + o;
+    if (TURN)
+        o = o + d * 0.0;
+    if (!isfinite(o))
         raise_error(sc.errw, ERR_NAN);
+    uIncNew[k] = o;
 }
 
 // ------------------------------------------------------- GMRES vectors ----
@@ -582,6 +584,9 @@ int launch_lusgs_init(dndsmi_ctx *c, const double *dtau, double dt, double alpha
     return c->launch_check("k_lusgs_init");
 }
 
+// a wave per workgroup: the sweeps of small meshes spread over all CUs
+constexpr int kSweepBlock = 64;
+
 LusgsScan lusgs_scan(const dndsmi_ctx *c, double alpha) {
     return {c->ldc,    c->col_cells,   c->sc_jf, c->sc_jb, c->sc_face, c->sc_n0,  c->sc_n1,     c->sc_area,
             c->sc_vol, c->lambda_face, c->jinv,  c->jdiag, c->sc_cf,   c->sc_lam, c->gas.gamma, alpha,
@@ -596,8 +601,8 @@ int launch_colour(dndsmi_ctx *c, int32_t col, double alpha, const double *rhs, c
         return DNDSMI_OK;
     prof_begin(c, DNDSMI_K_LUSGS_SWEEP);
     hipLaunchKernelGGL((c->nfmax == 3 ? k_lusgs_sweep<3, PRE, FORWARD, TURN> : k_lusgs_sweep<4, PRE, FORWARD, TURN>),
-                       dim3(grid_for(n)), dim3(kBlock), 0, c->stream, int32_t(n), int32_t(b), lusgs_scan(c, alpha),
-                       rhs, u, uInc, uIncNew);
+                       dim3(grid_for(4 * n, kSweepBlock)), dim3(kSweepBlock), 0, c->stream, int32_t(n), int32_t(b),
+                       lusgs_scan(c, alpha), rhs, u, uInc, uIncNew);
     prof_end(c);
     return c->launch_check("k_lusgs_sweep");
 }
@@ -631,8 +636,9 @@ int launch_lusgs_matvec(dndsmi_ctx *c, double alpha, const double *u, const doub
                         double *inc = nullptr) {
     DNDSMI_TRY(ensure_lusgs_scan(c));
     prof_begin(c, DNDSMI_K_LUSGS_MATVEC);
-    hipLaunchKernelGGL((c->nfmax == 3 ? k_lusgs_matvec<3, PRE> : k_lusgs_matvec<4, PRE>), dim3(grid_for(c->nc)),
-                       dim3(kBlock), 0, c->stream, int32_t(c->nc), lusgs_scan(c, alpha), u, x, Ax,
+    hipLaunchKernelGGL((c->nfmax == 3 ? k_lusgs_matvec<3, PRE> : k_lusgs_matvec<4, PRE>),
+                       dim3(grid_for(4 * c->nc, kSweepBlock)), dim3(kSweepBlock), 0, c->stream, int32_t(c->nc),
+                       lusgs_scan(c, alpha), u, x, Ax,
                        inc ? int32_t(c->col_start[1]) : 0, inc);
     prof_end(c);
     return c->launch_check("k_lusgs_matvec");
