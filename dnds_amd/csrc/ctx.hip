@@ -130,6 +130,14 @@ struct AbPart {
             last = rs.get<dbl2, true>(cl * 16, 256 * (kAbVecs - 1));
         }
     }
+    // the same for lanes of one wave at different slots, ordinary loads
+    __device__ __forceinline__ void load_each(const double *__restrict__ M, int s, int32_t i, int64_t ldc, int v) {
+        const dbl2 *p = reinterpret_cast<const dbl2 *>(M) + ab_group(s, i, ldc, kAbVecs);
+#pragma unroll
+        for (int k = 0; k < kAbVecs / 4; k++)
+            w[k] = p[64 * k + 4 * (i & 15) + v];
+        last = p[16 * (kAbVecs - 1) + (i & 15)];
+    }
     // entry d = 10 r + c: A^-1 B (c < 9) or A^-1 b (c = 9) of row r
     __device__ __forceinline__ double get(int d) const {
         const int p = d / 2;
@@ -328,19 +336,17 @@ __global__ __launch_bounds__(kBlock, 3) void k_sor(int32_t n, int32_t base, int6
 // RESID (the FP64 step of the mixed-precision sweeps): instead of the new
 // iterate, writes the increment r = J(x) - x rounded to FP32 into r32 (also the
 // start of the FP32 correction sweeps, k_delta32).
-template <int NF, bool RESID, bool TILE>
-__global__ __launch_bounds__(TILE ? kBlock : 64, 3) void k_jacobi(int32_t nc, int64_t ldc, const int32_t *__restrict__ nbr,
+template <int NF, bool RESID>
+__global__ __launch_bounds__(kBlock, 3) void k_jacobi(int32_t nc, int64_t ldc, const int32_t *__restrict__ nbr,
                                                       const int32_t *__restrict__ sbc,
                                                       const double *__restrict__ M, const double *__restrict__ u,
                                                       const double *__restrict__ x, double *__restrict__ xn,
                                                       double relax, const double *__restrict__ walls, double *corr,
                                                       int32_t *errw, float *__restrict__ r32, int32_t keep,
                                                       double *__restrict__ diff2) {
-    __shared__ double tile[TILE ? 9 : 1][TILE ? kBlock : 1];
+    __shared__ double tile[9][kBlock];
     const int32_t t = xcd_block() * blockDim.x + threadIdx.x, v = t & 3;
     const bool live = (t >> 2) < nc;
-    if (!TILE && !live)
-        return;
     const int32_t i = live ? t >> 2 : nc - 1;
     const uint32_t lane = threadIdx.x & 63;
     const double *xo = x + rec((t >> 2) & ~15, 0, 0);
@@ -374,14 +380,12 @@ __global__ __launch_bounds__(TILE ? kBlock : 64, 3) void k_jacobi(int32_t nc, in
 #pragma unroll
     for (int r = 0; r < 9; r++) {
         nw[r] = xo[256 * r + lane];
-        if (TILE)
-            tile[r][threadIdx.x] = nw[r];
+        tile[r][threadIdx.x] = nw[r];
         nw[r] = (1 - relax) * nw[r];
     }
     AbPart ab;
     ab.load(M, 0, i, ldc, v, keep);
-    if (TILE)
-        __syncthreads();
+    __syncthreads();
     const int32_t i0 = (t - int32_t(threadIdx.x)) >> 2;
 #pragma unroll
     for (int s = 0; s < NF; s++) {
@@ -393,7 +397,7 @@ __global__ __launch_bounds__(TILE ? kBlock : 64, 3) void k_jacobi(int32_t nc, in
         const double uj = u[4 * int64_t(j) + v];
         double xj[9];
         const uint32_t jl = uint32_t(j - i0);
-        if (TILE && jl < kBlock / 4) {
+        if (jl < kBlock / 4) {
 #pragma unroll
             for (int c = 0; c < 9; c++)
                 xj[c] = tile[c][4 * jl + v];
@@ -419,7 +423,7 @@ __global__ __launch_bounds__(TILE ? kBlock : 64, 3) void k_jacobi(int32_t nc, in
             raise_error(errw, ERR_BC);
         }
     }
-    if (TILE && !live)
+    if (!live)
         return;
     // the new iterate streams out with non-temporal stores: written once and
     // read by the next launch, it would only displace the neighbours'
@@ -437,6 +441,91 @@ __global__ __launch_bounds__(TILE ? kBlock : 64, 3) void k_jacobi(int32_t nc, in
 #pragma unroll
         for (int r = 0; r < 9; r++)
             d[r] = xo[256 * r + lane] - nw[r];
+        const double sum = quad_norm2(d);
+        if (v == 3)
+            diff2[i] = sum;
+    }
+}
+
+// The sweep of a small mesh: 16 lanes per cell, a quad per slot.  Small sweeps
+// are bound by one cell's chain of loads and sums, which k_jacobi runs slot
+// after slot (and a corner cell's two walls one after the other, 4 us each);
+// here the slots' terms form side by side and the first quad adds them in the
+// slots' order.  An absent slot adds -0, which changes no bit.
+template <int NF, bool RESID>
+__global__ __launch_bounds__(64) void k_jacobi_wide(int32_t nc, int64_t ldc, const int32_t *__restrict__ nbr,
+                                                    const int32_t *__restrict__ sbc, const double *__restrict__ M,
+                                                    const double *__restrict__ u, const double *__restrict__ x,
+                                                    double *__restrict__ xn, double relax,
+                                                    const double *__restrict__ walls, int32_t *errw,
+                                                    float *__restrict__ r32, double *__restrict__ diff2) {
+    const int32_t t = xcd_block() * 64 + threadIdx.x, i = t >> 4;
+    const int s = (t >> 2) & 3, v = t & 3;
+    if (i >= nc)
+        return;
+    const int32_t jn = s < NF ? nbr[s * ldc + i] : -2;
+    double term[9], own[9];
+#pragma unroll
+    for (int r = 0; r < 9; r++)
+        term[r] = -0.0;
+    const double ui = u[4 * int64_t(i) + v];
+    if (s == 0 || is_wall_slot(jn))
+#pragma unroll
+        for (int r = 0; r < 9; r++)
+            own[r] = x[rec(i, r, v)];
+    if (is_wall_slot(jn)) {
+        wall_correction(jn, own, ui, v, walls, relax, errw, term);
+    } else if (jn != -2) {
+        AbPart ab;
+        ab.load_each(M, s, i, ldc, v);
+        const int32_t j = jn < 0 ? i : jn;
+        const double uj = u[4 * int64_t(j) + v];
+        double xj[9];
+#pragma unroll
+        for (int c = 0; c < 9; c++)
+            xj[c] = x[rec(j, c, v)];
+        const int32_t bc = jn == -1 ? sbc[s * ldc + i] : BC_INNER;
+        if (jn >= 0 || is_far(bc)) {
+            const double bmul = jn < 0 ? 0.0 : 1.0, du = bmul * (uj - ui);
+#pragma unroll
+            for (int r = 0; r < 9; r++) {
+                double tt = 0.0;
+#pragma unroll
+                for (int c = 0; c < 9; c++)
+                    tt += ab.get(10 * r + c) * xj[c];
+                const double b = bmul * ab.get(10 * r + 9);
+                term[r] = relax * (tt + du * b);
+            }
+        } else if (bc == BC_WALL) {
+#pragma unroll
+            for (int r = 0; r < 9; r++)
+                term[r] = relax * ((0.0 - ui) * ab.get(10 * r + 9));
+        } else {
+            raise_error(errw, ERR_BC);
+        }
+    }
+    double nw[9];
+#pragma unroll
+    for (int r = 0; r < 9; r++) {
+        nw[r] = (1 - relax) * own[r];
+#pragma unroll
+        for (int q = 0; q < NF; q++)
+            nw[r] += row_ahead(term[r], q);
+    }
+    if (s > 0)
+        return;
+#pragma unroll
+    for (int r = 0; r < 9; r++) {
+        if (RESID)
+            r32[rec(i, r, v)] = float(nw[r] - own[r]);
+        else
+            xn[rec(i, r, v)] = nw[r];
+    }
+    if (!RESID && diff2) {
+        double d[9];
+#pragma unroll
+        for (int r = 0; r < 9; r++)
+            d[r] = own[r] - nw[r];
         const double sum = quad_norm2(d);
         if (v == 3)
             diff2[i] = sum;
@@ -1406,23 +1495,6 @@ __global__ __launch_bounds__(kBlock) void k_wbap_ind(int32_t nc, int64_t ldc, co
 // and 487 -> 22.  With every cell limited (262 088 triangles) V2 keeps its
 // time (536, 525 us) and V3 goes from 1577 to 430.
 
-// `a` of the lane 4 q further on in the row
-template <typename T>
-__device__ __forceinline__ T row_ahead(T a, int q) { // q: a constant after unrolling
-    auto get = [&](uint32_t w) -> uint32_t {
-        return q == 0   ? w
-               : q == 1 ? uint32_t(__builtin_amdgcn_mov_dpp(int(w), 0x104, 0xf, 0xf, true))
-               : q == 2 ? uint32_t(__builtin_amdgcn_mov_dpp(int(w), 0x108, 0xf, 0xf, true))
-                        : uint32_t(__builtin_amdgcn_mov_dpp(int(w), 0x10c, 0xf, 0xf, true));
-    };
-    if constexpr (sizeof(T) == 4) {
-        return __builtin_bit_cast(T, get(__builtin_bit_cast(uint32_t, a)));
-    } else {
-        const uint64_t w = __builtin_bit_cast(uint64_t, a);
-        return __builtin_bit_cast(T, uint64_t(get(uint32_t(w))) | uint64_t(get(uint32_t(w >> 32))) << 32);
-    }
-}
-
 constexpr int kSecEntries = 82; // 81 and a pad, per face and side
 constexpr unsigned kLimBlocks = 8192; // workgroups that walk the list (131 072 cells at once)
 
@@ -2246,6 +2318,13 @@ constexpr int64_t kKeepLargest = 900000000, kKeepLargest32 = 600000000;
 // the FP64 sweep of a mixed-precision stage shares the cache with the FP32 ones
 constexpr int64_t kKeepLargestMixed = 450000000;
 
+// A sweep takes 16 lanes per cell (k_jacobi_wide) while its whole stream stays
+// in the Infinity Cache.  us, four lanes per cell / 16: FP64 triangles 1.8 k
+// cells 8.9 / 7.2, 8 k 10.0 / 10.1, 33 k 20.0 / 20.1, 66 k 35.3 / 31.7, 80 k
+// (173 MB) 40.4 / 36.8, 97 k (209 MB) 46.2 / 48.9, 180 k 76.6 / 104; mixed
+// cells with walls 0.9 k 17.0 / 10.2, 9.5 k 20.8 / 18.3, 39 k 42.6 / 36.0.
+bool wide_sweep(const dndsmi_ctx *c) { return keep_share(c, kAbVecs, kKeepLargest) == 64; }
+
 // Workgroup size of a sweep over `lanes` lanes.  Waves are independent; small
 // sweeps take one wave per workgroup, so that their waves spread over all CUs.
 int sweep_block(int64_t lanes) { return lanes < 300000 ? 64 : kBlock; }
@@ -2293,14 +2372,18 @@ int launch_jacobi(dndsmi_ctx *c, const double *u, const double *x, double *xn, d
                                xn, diff2);
         return c->launch_check("k_rec_diff2");
     }
-    const int64_t lanes = 4 * c->nc;
-    const int block = sweep_block(lanes);
+    if (wide_sweep(c)) {
+        prof_begin(c, DNDSMI_K_JACOBI);
+        hipLaunchKernelGGL((c->nfmax == 3 ? k_jacobi_wide<3, false> : k_jacobi_wide<4, false>),
+                           dim3(grid_for(16 * c->nc, 64)), dim3(64), 0, c->stream, int32_t(c->nc), c->ldc, c->nbr,
+                           c->sbc, c->M, u, x, xn, c->relax, c->walls, c->errw, nullptr, diff2);
+        prof_end(c);
+        return c->launch_check("k_jacobi_wide");
+    }
     prof_begin(c, DNDSMI_K_JACOBI);
-    auto kern = block == 64 ? (c->nfmax == 3 ? k_jacobi<3, false, false> : k_jacobi<4, false, false>)
-                            : (c->nfmax == 3 ? k_jacobi<3, false, true> : k_jacobi<4, false, true>);
-    hipLaunchKernelGGL(kern, dim3(grid_for(lanes, block)), dim3(block), 0, c->stream, int32_t(c->nc),
-                       c->ldc, c->nbr, c->sbc, c->M, u, x, xn, c->relax, c->walls, c->wall_corr,
-                       c->errw, nullptr, keep_share(c, kAbVecs, kKeepLargest), diff2);
+    hipLaunchKernelGGL((c->nfmax == 3 ? k_jacobi<3, false> : k_jacobi<4, false>), dim3(grid_for(4 * c->nc)),
+                       dim3(kBlock), 0, c->stream, int32_t(c->nc), c->ldc, c->nbr, c->sbc, c->M, u, x, xn, c->relax,
+                       c->walls, c->wall_corr, c->errw, nullptr, keep_share(c, kAbVecs, kKeepLargest), diff2);
     prof_end(c);
     return c->launch_check("k_jacobi");
 }
@@ -2458,12 +2541,15 @@ int launch_jacobi_mixed(dndsmi_ctx *c, const double *u, double *x, int n_sweeps,
     const int block = sweep_block(lanes), nc = int(c->nc);
     const dim3 grid(grid_for(lanes, block));
     prof_begin(c, DNDSMI_K_JACOBI);
-    auto first = block == 64 ? (c->nfmax == 3 ? k_jacobi<3, true, false> : k_jacobi<4, true, false>)
-                             : (c->nfmax == 3 ? k_jacobi<3, true, true> : k_jacobi<4, true, true>);
-    hipLaunchKernelGGL(first, grid, dim3(block), 0, c->stream, nc,
-                       c->ldc, c->nbr, c->sbc, c->M, u, x, nullptr, c->relax, c->walls,
-                       c->wall_corr, c->errw, c->r32,
-                       keep_share(c, kAbVecs, kKeepLargestMixed), nullptr);
+    if (wide_sweep(c)) {
+        hipLaunchKernelGGL((c->nfmax == 3 ? k_jacobi_wide<3, true> : k_jacobi_wide<4, true>),
+                           dim3(grid_for(16 * c->nc, 64)), dim3(64), 0, c->stream, nc, c->ldc, c->nbr, c->sbc, c->M, u,
+                           x, nullptr, c->relax, c->walls, c->errw, c->r32, nullptr);
+    } else {
+        hipLaunchKernelGGL((c->nfmax == 3 ? k_jacobi<3, true> : k_jacobi<4, true>), dim3(grid_for(lanes)), dim3(kBlock),
+                           0, c->stream, nc, c->ldc, c->nbr, c->sbc, c->M, u, x, nullptr, c->relax, c->walls,
+                           c->wall_corr, c->errw, c->r32, keep_share(c, kAbVecs, kKeepLargestMixed), nullptr);
+    }
     prof_end(c);
     DNDSMI_TRY(c->launch_check("k_jacobi (residual)"));
     const int32_t keep = keep_share(c, kAb32Vecs, kKeepLargest32);

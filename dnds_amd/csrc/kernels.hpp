@@ -98,6 +98,23 @@ __device__ __forceinline__ T quad_get(T a, int q) { // q: a constant after unrol
     return q == 0 ? quad_bcast<0>(a) : q == 1 ? quad_bcast<1>(a) : q == 2 ? quad_bcast<2>(a) : quad_bcast<3>(a);
 }
 
+// `a` of the lane 4 q further on in the row
+template <typename T>
+__device__ __forceinline__ T row_ahead(T a, int q) { // q: a constant after unrolling
+    auto get = [&](uint32_t w) -> uint32_t {
+        return q == 0   ? w
+               : q == 1 ? uint32_t(__builtin_amdgcn_mov_dpp(int(w), 0x104, 0xf, 0xf, true))
+               : q == 2 ? uint32_t(__builtin_amdgcn_mov_dpp(int(w), 0x108, 0xf, 0xf, true))
+                        : uint32_t(__builtin_amdgcn_mov_dpp(int(w), 0x10c, 0xf, 0xf, true));
+    };
+    if constexpr (sizeof(T) == 4) {
+        return __builtin_bit_cast(T, get(__builtin_bit_cast(uint32_t, a)));
+    } else {
+        const uint64_t w = __builtin_bit_cast(uint64_t, a);
+        return __builtin_bit_cast(T, uint64_t(get(uint32_t(w))) | uint64_t(get(uint32_t(w >> 32))) << 32);
+    }
+}
+
 // 16-byte vectors for streaming loads
 typedef double dbl2 __attribute__((ext_vector_type(2)));
 typedef float flt4 __attribute__((ext_vector_type(4)));

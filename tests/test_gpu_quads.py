@@ -124,3 +124,28 @@ def test_rhs_face_quads_and_lanes(kind, nx, ny, mu):
         ExplicitSSPRK3LocalDt(ev, nInternalRecStep=2, CFL=0.3, mixedPrecision=True).Step(du, r, rn, 0.0)
         ru, _, _ = orc.ssprk3_steps(u, x, 1, 2, 0.3)
         assert rel_err(du.download(), ru) <= 1e-6
+
+
+@pytest.mark.parametrize("n", [240, 243])
+def test_sweeps_on_both_sides_of_the_wide_one(n):
+    """The last mesh whose sweep takes 16 lanes per cell (168 MB of A^-1 B) and
+    one beyond it, with walls of every kind and the increment; then one
+    mixed-precision step on far field and walls (tolerances as in its tests)."""
+    from dnds_amd import _capi as A
+    from dnds_amd.host import EulerEvaluator, ExplicitSSPRK3LocalDt
+    mesh, vfv = _case(1, n, n)
+    assert (4 * mesh.n_cell * 720 <= 168e6) == (n == 240)
+    ev = EulerEvaluator(mesh, vfv, riemannSolverType="HLLC", farFieldStaticValue=FAR)
+    u, x = _state(mesh.n_cell, 5)
+    du, dx, dn = ev.BuildMean().upload(u), vfv.BuildRec().upload(x), vfv.BuildRec()
+    _, increment = vfv.ReconstructToTolerance(du, dx, dn, 0.0, 1)
+    ref = _oracle(mesh, vfv, FAR).jacobi_step(u, x)
+    assert rel_err(dx.download(), ref) <= TOL
+    expect = ((ref - x) ** 2).sum() / mesh.n_cell
+    assert abs(increment - expect) <= 1e-11 * expect
+    mesh, vfv = _case(1, n, n, top=A.BC_FARFIELD)
+    ev = EulerEvaluator(mesh, vfv, riemannSolverType="HLLC", farFieldStaticValue=FAR)
+    du, dx, dn = ev.BuildMean().upload(u), vfv.BuildRec().upload(0.1 * x), vfv.BuildRec()
+    ExplicitSSPRK3LocalDt(ev, nInternalRecStep=2, CFL=0.3, mixedPrecision=True).Step(du, dx, dn, 0.0)
+    ru, rr, _ = _oracle(mesh, vfv, FAR).ssprk3_steps(u, 0.1 * x, 1, 2, 0.3)
+    assert rel_err(du.download(), ru) <= 1e-6 and rel_err(dx.download(), rr) <= 1e-5
