@@ -330,8 +330,7 @@ __global__ __launch_bounds__(kBlock, 3) void k_sor(int32_t n, int32_t base, int6
 // diff2 (may be null): receives |x_i - new_i|^2 per cell.  A kernel of its own
 // for it read both arrays again (one thread per cell, uncoalesced): 67 us per
 // sweep of dndsmi_reconstruct_to_tolerance on 66 k cells, 47 now, and 425 / 271
-// on 524 k; here
-// the old coefficients come from the caches.
+// on 524 k; here the old coefficients come from the caches.
 //
 // RESID (the FP64 step of the mixed-precision sweeps): instead of the new
 // iterate, writes the increment r = J(x) - x rounded to FP32 into r32 (also the
@@ -2332,8 +2331,11 @@ constexpr int64_t kKeepLargestMixed = 450000000;
 // cells with walls 0.9 k 17.0 / 10.2, 9.5 k 20.8 / 18.3, 39 k 42.6 / 36.0.
 bool wide_sweep(const dndsmi_ctx *c) { return keep_share(c, kAbVecs, kKeepLargest) == 64; }
 
-// Workgroup size of a sweep over `lanes` lanes.  Waves are independent; small
-// sweeps take one wave per workgroup, so that their waves spread over all CUs.
+// Workgroup size of an SOR pass or FP32 sweep over `lanes` lanes.  Waves are
+// independent; small sweeps take one wave per workgroup, so that their waves
+// spread over all CUs.  FP32 sweep, us, 64 / 256 threads: 1.8 k cells 7.4 / 8.4,
+// 8 k 7.8 / 8.2, 33 k 12.2 / 12.1, 80 k 23.4 / 23.4, 146 k 39.1 / 38.3, 259 k
+// 67.0 / 65.1; SOR colour of 1.8 k cells 8.5 / 9.2, of 131 k 22.9 / 23.6.
 int sweep_block(int64_t lanes) { return lanes < 300000 ? 64 : kBlock; }
 
 // SOR_Instead: colour by colour in place on x (forward; with
