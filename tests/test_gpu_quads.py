@@ -4,6 +4,10 @@ counts around a group, a wave and a workgroup's worth of cells, the counts
 where the workgroup size changes, and more limited cells than the limiter's
 grid holds at once.  All of it is FP64 in the oracle's operation order, so the
 tolerance is that of the other FP64 parity tests."""
+# The Jacobi sweeps below run with 16 lanes per cell (k_jacobi_wide: A^-1 B up
+# to 168 MB, here 58333 quads), the two largest and the mixed mesh with
+# four (k_jacobi); a sweep's 256-thread workgroups, the FP32 sweep's and SOR's,
+# are in test_gpu_sweep_variants.py.
 import numpy as np
 import pytest
 
