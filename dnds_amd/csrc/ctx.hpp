@@ -31,8 +31,8 @@ struct dndsmi_ctx {
     std::string err;
     int64_t nc = 0, nf = 0, ldc = 0, ldf = 0;
     // device numbering of the mesh's cells and faces (host arrays keep the
-    // mesh numbering)
-    std::vector<int32_t> c2d, f2d;
+    // mesh numbering), and the mesh cell of a device cell
+    std::vector<int32_t> c2d, f2d, d2c;
     int nfmax = 3;
     GasParams gas{};
     double relax = 1.0;
