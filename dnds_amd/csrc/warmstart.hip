@@ -622,16 +622,25 @@ __global__ __launch_bounds__(256) void k_features(int32_t nc, int64_t ldc, const
 }
 
 // targets: converged rec coefficients x (k = r + 9 v) divided by
-// s_v, rows of 36 formed in LDS and written contiguously
+// s_v, rows of 36 formed in LDS and written contiguously; x is read, and in
+// k_unscale written, in whole 32-byte elements (predict on 1 M cells, value by
+// value -> now: 589 -> 574 us)
 __global__ __launch_bounds__(256) void k_targets(int32_t nc, int64_t ldc, const double *__restrict__ x,
                                                  const float *__restrict__ S, float *__restrict__ T) {
     __shared__ float tile[256][kOut + 1];
     const int64_t i0 = int64_t(blockIdx.x) * 256;
     const int32_t i = int32_t(i0) + int32_t(threadIdx.x);
     if (i < nc) {
+        const floatx4 sv = reinterpret_cast<const floatx4 *>(S)[i];
 #pragma unroll
-        for (int k = 0; k < kOut; k++)
-            tile[threadIdx.x][k] = float(x[rec(i, k % 9, k / 9)] / double(S[4 * int64_t(i) + k / 9]));
+        for (int r = 0; r < 9; r++) {
+            const dbl2 *xq = reinterpret_cast<const dbl2 *>(x + rec(i, r, 0));
+            const dbl2 a = xq[0], b = xq[1];
+            const double e[4] = {a.x, a.y, b.x, b.y};
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                tile[threadIdx.x][r + 9 * v] = float(e[v] / double(sv[v]));
+        }
     }
     __syncthreads();
     const int64_t nrow = min(int64_t(256), int64_t(nc) - i0);
@@ -654,13 +663,19 @@ __global__ __launch_bounds__(256) void k_unscale(int32_t nc, int64_t ldc, const 
     const int32_t i = int32_t(i0) + int32_t(threadIdx.x);
     if (i >= nc)
         return;
+    const floatx4 sv = reinterpret_cast<const floatx4 *>(S)[i];
 #pragma unroll
-    for (int k = 0; k < kOut; k++) {
-        const double v = double(tile[threadIdx.x][k]) * double(S[4 * int64_t(i) + k / 9]);
-        if (ADD)
-            x[rec(i, k % 9, k / 9)] += v;
-        else
-            x[rec(i, k % 9, k / 9)] = v;
+    for (int r = 0; r < 9; r++) {
+        dbl2 *xq = reinterpret_cast<dbl2 *>(x + rec(i, r, 0));
+        double e[4];
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            e[v] = double(tile[threadIdx.x][r + 9 * v]) * double(sv[v]);
+        if (ADD) {
+            const dbl2 a = xq[0], b = xq[1];
+            e[0] = a.x + e[0], e[1] = a.y + e[1], e[2] = b.x + e[2], e[3] = b.y + e[3];
+        }
+        xq[0] = dbl2{e[0], e[1]}, xq[1] = dbl2{e[2], e[3]};
     }
 }
 
