@@ -88,8 +88,9 @@ __global__ __launch_bounds__(kBlock) void k_lusgs_scan(int32_t nc, int64_t ldc, 
 
 // LUSGSMatrixInit (DNDS_FV_EulerEvaluator.cpp:995-1047), jacobianCode 0, zero
 // source Jacobian, per scan position:
-// jinv = 1 / (1/dTau_i + 1/dt + sum_f (alpha/2) S_f lambda_f / V_i)
-template <int NF>
+// jinv = 1 / (1/dTau_i + 1/dt + sum_f (alpha/2) S_f lambda_f / V_i); KEEP: c_f
+// and lambda by slot too
+template <int NF, bool KEEP>
 __global__ __launch_bounds__(kBlock) void k_lusgs_init(int32_t nc, int64_t ldc, const int32_t *__restrict__ cells,
                                                        const int32_t *__restrict__ sf, const double *__restrict__ sS,
                                                        const double *__restrict__ sV,
@@ -109,8 +110,10 @@ __global__ __launch_bounds__(kBlock) void k_lusgs_init(int32_t nc, int64_t ldc, 
             continue;
         const double S = sS[s * ldc + p], l = lambda_face[f];
         fp += (0.5 * alpha) * S * l / v;
-        cf[s * ldc + p] = (0.5 * alpha) * S / v;
-        lam[s * ldc + p] = l;
+        if (KEEP) {
+            cf[s * ldc + p] = (0.5 * alpha) * S / v;
+            lam[s * ldc + p] = l;
+        }
     }
     jdiag[p] = fp + alpha * 0.0; // jacobianCell = fpDivisor I + alphaDiag 0 (source Jacobian)
     jinv[p] = 1.0 / (fp + alpha * 0.0);
@@ -554,8 +557,6 @@ int ensure_lusgs_scan(dndsmi_ctx *c) {
     DNDSMI_TRY(c->alloc(c->sc_n1, n));
     DNDSMI_TRY(c->alloc(c->sc_area, n));
     DNDSMI_TRY(c->alloc(c->sc_vol, c->ldc));
-    DNDSMI_TRY(c->alloc(c->sc_cf, n));
-    DNDSMI_TRY(c->alloc(c->sc_lam, n));
     const int nc = int(c->nc);
     if (c->nfmax == 3)
         hipLaunchKernelGGL(k_lusgs_scan<3>, dim3(grid_for(nc)), dim3(kBlock), 0, c->stream, nc, c->ldc, c->ldf,
@@ -568,19 +569,22 @@ int ensure_lusgs_scan(dndsmi_ctx *c) {
     return c->launch_check("k_lusgs_scan");
 }
 
-int launch_lusgs_init(dndsmi_ctx *c, const double *dtau, double dt, double alpha) {
+// keep: also c_f and lambda by slot, for the solver's own sweeps (LUSGSMatrixInit
+// as an entry point has no use for them: 19.0 us with their stores on 550 k
+// cells, 16.5 without)
+int launch_lusgs_init(dndsmi_ctx *c, const double *dtau, double dt, double alpha, bool keep) {
     DNDSMI_TRY(ensure_lusgs_scan(c));
     if (!c->jdiag)
         DNDSMI_TRY(c->alloc(c->jdiag, c->ldc));
+    if (keep && !c->sc_cf)
+        DNDSMI_TRY(c->alloc(c->sc_cf, int64_t(c->nfmax) * c->ldc));
+    if (keep && !c->sc_lam)
+        DNDSMI_TRY(c->alloc(c->sc_lam, int64_t(c->nfmax) * c->ldc));
     const int nc = int(c->nc);
-    if (c->nfmax == 3)
-        hipLaunchKernelGGL(k_lusgs_init<3>, dim3(grid_for(nc)), dim3(kBlock), 0, c->stream, nc, c->ldc, c->col_cells,
-                           c->sc_face, c->sc_area, c->sc_vol, c->lambda_face, dtau, dt, alpha, c->jinv, c->jdiag,
-                           c->sc_cf, c->sc_lam);
-    else
-        hipLaunchKernelGGL(k_lusgs_init<4>, dim3(grid_for(nc)), dim3(kBlock), 0, c->stream, nc, c->ldc, c->col_cells,
-                           c->sc_face, c->sc_area, c->sc_vol, c->lambda_face, dtau, dt, alpha, c->jinv, c->jdiag,
-                           c->sc_cf, c->sc_lam);
+    auto kern = c->nfmax == 3 ? (keep ? k_lusgs_init<3, true> : k_lusgs_init<3, false>)
+                              : (keep ? k_lusgs_init<4, true> : k_lusgs_init<4, false>);
+    hipLaunchKernelGGL(kern, dim3(grid_for(nc)), dim3(kBlock), 0, c->stream, nc, c->ldc, c->col_cells, c->sc_face,
+                       c->sc_area, c->sc_vol, c->lambda_face, dtau, dt, alpha, c->jinv, c->jdiag, c->sc_cf, c->sc_lam);
     return c->launch_check("k_lusgs_init");
 }
 
@@ -790,7 +794,7 @@ int gmres_solve(dndsmi_ctx *c, double alpha, const double *b, const double *u, d
 // GMRES as c->gmres_code says (DNDS_FV_EulerSolver.hpp:852-975)
 int fsolve(dndsmi_ctx *c, const double *dtau, double dt, double alpha, const double *rhs, const double *u,
            double *xinc) {
-    DNDSMI_TRY(launch_lusgs_init(c, dtau, dt, alpha));
+    DNDSMI_TRY(launch_lusgs_init(c, dtau, dt, alpha, true));
     if (c->gmres_code == 0 || c->gmres_code == 2)
         DNDSMI_TRY(launch_lusgs_pair(c, alpha, rhs, u, xinc, 0));
     if (c->gmres_code != 0)
@@ -837,7 +841,7 @@ extern "C" int dndsmi_lusgs_matrix_init(dndsmi_ctx *c, const dndsmi_array *dTau,
         c->err = "LUSGSMatrixInit: only jacobianCode 0 (the analytic diagonal) is implemented";
         return DNDSMI_ERR_UNSUPPORTED;
     }
-    return launch_lusgs_init(c, dTau->d, dt, alphaDiag);
+    return launch_lusgs_init(c, dTau->d, dt, alphaDiag, false);
 }
 
 extern "C" int dndsmi_update_lusgs_forward(dndsmi_ctx *c, double alphaDiag, const dndsmi_array *rhs,

@@ -248,3 +248,26 @@ def test_gmres_more_vectors_than_one_batch_of_dots(n_space):
     """The dot products are folded 16 at a time: the last subspace of one
     batch and the first of two."""
     test_gmres_vectors_at_block_and_fold_edges(40, 30, 1, n_space)
+
+
+def test_matrix_init_leaves_the_solvers_coefficients_out():
+    """LUSGSMatrixInit as an entry point stores no coefficients by slot: only
+    the implicit steps' own sweeps read those (two doubles per cell and slot),
+    and a program that drives the sweeps itself does not hold them.  The
+    implicit steps besides hold right-hand side, increment and time step (nine
+    doubles per cell) and the residual's partials."""
+    from dnds_amd.host import ImplicitEulerDualTimeStep
+    mesh, vfv, ev, _ = build(1, "farfield")
+    ldc, nf = (mesh.n_cell + 63) // 64 * 64, 4
+    u0, _ = random_state(mesh.n_cell, 3, amp=0.1)
+    u, r, rn = ev.BuildMean().upload(u0), vfv.BuildRec().setConstant(0.0), vfv.BuildRec()
+    dtau, rhs, inc = ev.BuildScalar(), ev.BuildMean(), ev.BuildMean().setConstant(0.0)
+    ev.EvaluateDt(dtau, u, 5.0, 1e100, True)
+    ev.EvaluateRHS(rhs, u, r, 0.0)
+    ev.LUSGSMatrixInit(dtau, 0.1, 1.0)
+    ev.UpdateLUSGSForward(1.0, rhs, u, inc, inc)
+    ev.UpdateLUSGSBackward(1.0, rhs, u, inc, inc)
+    before = ev.device.device_bytes()
+    ImplicitEulerDualTimeStep(ev, nInternalRecStep=1, CFL=5.0, nTimeStepInternal=2,
+                              rhsThresholdInternal=0.0).Step(u, r, rn, dt=0.1)
+    assert ev.device.device_bytes() - before >= 8 * ldc * (9 + 2 * nf)
