@@ -1498,36 +1498,26 @@ __global__ __launch_bounds__(kBlock) void k_wbap_ind(int32_t nc, int64_t ldc, co
 // what a cell reads of them is contiguous.
 //
 // Measured against one lane per cell, a Mach-3 shock on 24 727 mixed cells:
-// V2 (three launches) 138 -> 23 us, V3 349 -> 13; on 393 734 cells 201 -> 35
-// and 487 -> 22.  With every cell limited (262 088 triangles) V2 keeps its
-// time (536, 525 us) and V3 goes from 1577 to 430.
+// V2 (three launches) 140 -> 21 us, V3 354 -> 13; on 393 734 cells 198 -> 32
+// and 490 -> 21.  With every cell limited (262 088 triangles) 528 -> 417 and
+// 1562 -> 411, on 810 000 quads the whole call 1940 -> 1773 and 6707 -> 1656.
+// There the divisions bound it, so that a quad shares them (quad_char_rows):
+// with whole matrices formed in every lane V2 took 525 and 2088.
 
 constexpr int kSecEntries = 82; // 81 and a pad, per face and side
 constexpr unsigned kLimBlocks = 8192; // workgroups that walk the list (131 072 cells at once)
-
-// row v of a 4 x 4 matrix
-__device__ __forceinline__ void matrix_row(const double M[16], int v, double row[4]) {
-#pragma unroll
-    for (int b = 0; b < 4; b++)
-        row[b] = v == 0 ? M[b] : v == 1 ? M[4 + b] : v == 2 ? M[8 + b] : M[12 + b];
-}
 
 // a lane's row of the face's eigenvector matrices for neighbour j of cell i
 // through face f, and the side of i
 __device__ __forceinline__ bool face_char_rows(double gamma, const double *__restrict__ u, int32_t i, int32_t j,
                                                int32_t f, int side, int64_t ldf, const double *__restrict__ fnc, int v,
                                                double ml[4], double mr[4]) {
-    double un0, un1;
-    stable_normalized(fnc[f], fnc[ldf + f], un0, un1);
     const double *uLp = u + 4 * int64_t(side ? j : i), *uRp = u + 4 * int64_t(side ? i : j);
-    double UL[4], UR[4], ML[16], MR[16];
+    double UL[4], UR[4];
 #pragma unroll
     for (int k = 0; k < 4; k++)
         UL[k] = uLp[k], UR[k] = uRp[k];
-    const bool ok = char_matrices(gamma, UL, UR, un0, un1, ML, MR);
-    matrix_row(ML, v, ml);
-    matrix_row(MR, v, mr);
-    return ok;
+    return quad_char_rows(gamma, UL, UR, fnc[f], fnc[ldf + f], v, ml, mr);
 }
 
 // sum over the quad's lanes b of row[b] a_b, in order

@@ -769,50 +769,63 @@ __device__ inline double ff_self(const FFParams &p, const double d[10]) {
     return c;
 }
 
-// fML / fMR (DNDS_FV_EulerSolver.hpp:749-795): left / right eigenvector
-// matrices at the mean of UL and UR in the face frame, mapped back to the
-// global frame.  ML, MR row-major 4x4.
-__device__ inline bool char_matrices(double gamma, const double UL[4], const double UR[4], double n0, double n1,
-                                     double ML[16], double MR[16]) {
-    double UC[4];
+// stable_normalized by the four lanes of a quad together (v: the lane's place),
+// the x quotients in its even lanes, the y ones in its odd
+__device__ __forceinline__ void quad_stable_normalized(double x, double y, int v, double &ox, double &oy) {
+    const double w = fmax(fabs(x), fabs(y)), c = v & 1 ? y : x;
+    const double zc = c / w;
+    const double zx = quad_bcast<0>(zc), zy = quad_bcast<1>(zc);
+    const double z = zx * zx + zy * zy;
+    if (z > 0) {
+        const double o = (c / sqrt(z)) / w;
+        ox = quad_bcast<0>(o), oy = quad_bcast<1>(o);
+    } else
+        ox = x, oy = y;
+}
+
+// Rows v of fML / fMR (DNDS_FV_EulerSolver.hpp:749-795), the left / right
+// eigenvector matrices at the mean of UL and UR in the face frame, mapped back
+// to the global frame, by the four lanes of a quad together.  The quotients by
+// one divisor are taken by a lane each and passed around: with every lane
+// dividing 15 times for whole matrices, the limiter was bound by that where
+// all cells are limited.
+__device__ __forceinline__ bool quad_char_rows(double gamma, const double UL[4], const double UR[4], double nx,
+                                               double ny, int v, double ml[4], double mr[4]) {
+    double n0, n1, UC[4];
+    quad_stable_normalized(nx, ny, v, n0, n1);
+#pragma unroll
     for (int k = 0; k < 4; k++)
-        UC[k] = (UL[k] + UR[k]) * 0.5;
+        UC[k] = (UL[k] + UR[k]) * 0.5, ml[k] = mr[k] = 0.0;
     const double r1 = n0 * UC[1] + n1 * UC[2];
     const double r2 = (-n1) * UC[1] + n0 * UC[2];
-    UC[1] = r1, UC[2] = r2;
     if (!(UC[0] > 0))
         return false;
-    const double v0 = UC[1] / UC[0], v1 = UC[2] / UC[0];
+    const double vq = (v & 1 ? r2 : r1) / UC[0];
+    const double v0 = quad_bcast<0>(vq), v1 = quad_bcast<1>(vq);
     const double vsqr = v0 * v0 + v1 * v1;
-    double asqr, p, H;
-    ideal_gas_thermal(UC[3], UC[0], vsqr, gamma, p, asqr, H);
+    const double p = (gamma - 1) * (UC[3] - UC[0] * 0.5 * vsqr);
+    const double tq = (v & 1 ? UC[3] + p : gamma * p) / UC[0];
+    const double asqr = quad_bcast<0>(tq), H = quad_bcast<1>(tq);
     if (!(asqr >= 0))
         return false;
-    const double a = sqrt(asqr);
-    const double gb = gamma - 1;
-    double L[16];
-    L[0] = H + a / gb * (v0 - a), L[1] = -v0 - a / gb, L[2] = -v1, L[3] = 1;
-    L[4] = -2 * H + 4 / gb * (a * a), L[5] = v0 * 2, L[6] = v1 * 2, L[7] = -2;
-    L[8] = v1 * (-2 * (a * a) / gb), L[9] = 0, L[10] = 2 * (a * a) / gb, L[11] = 0;
-    L[12] = H - a / gb * (v0 + a), L[13] = -v0 + a / gb, L[14] = -v1, L[15] = 1;
-    const double sc = gb / (2 * a * a);
-    for (int k = 0; k < 16; k++)
+    const double a = sqrt(asqr), gb = gamma - 1;
+    const double gq = (v == 0 ? a : v == 1 ? 4.0 : v == 2 ? 2 * (a * a) : gb) / (v == 3 ? 2 * a * a : gb);
+    const double agb = quad_bcast<0>(gq), fgb = quad_bcast<1>(gq), tgb = quad_bcast<2>(gq), sc = quad_bcast<3>(gq);
+    double L[4];
+    L[0] = v == 0 ? H + agb * (v0 - a) : v == 1 ? -2 * H + fgb * (a * a) : v == 2 ? v1 * -tgb : H - agb * (v0 + a);
+    L[1] = v == 0 ? -v0 - agb : v == 1 ? v0 * 2 : v == 2 ? 0.0 : -v0 + agb;
+    L[2] = v == 1 ? v1 * 2 : v == 2 ? tgb : -v1;
+    L[3] = v == 1 ? -2.0 : v == 2 ? 0.0 : 1.0;
+#pragma unroll
+    for (int k = 0; k < 4; k++)
         L[k] *= sc;
-    for (int r = 0; r < 4; r++) {
-        const double c1 = L[4 * r + 1] * n0 + L[4 * r + 2] * (-n1);
-        const double c2 = L[4 * r + 1] * n1 + L[4 * r + 2] * n0;
-        ML[4 * r] = L[4 * r], ML[4 * r + 1] = c1, ML[4 * r + 2] = c2, ML[4 * r + 3] = L[4 * r + 3];
-    }
-    double R[16];
-    R[0] = 1, R[1] = 1, R[2] = 0, R[3] = 1;
-    R[4] = v0 - a, R[5] = v0, R[6] = 0, R[7] = v0 + a;
-    R[8] = v1, R[9] = v1, R[10] = 1, R[11] = v1;
-    R[12] = H - v0 * a, R[13] = 0.5 * vsqr, R[14] = v1, R[15] = H + v0 * a;
-    for (int c = 0; c < 4; c++) {
-        const double a1 = n0 * R[4 + c] + (-n1) * R[8 + c];
-        const double a2 = n1 * R[4 + c] + n0 * R[8 + c];
-        MR[c] = R[c], MR[4 + c] = a1, MR[8 + c] = a2, MR[12 + c] = R[12 + c];
-    }
+    ml[0] = L[0], ml[1] = L[1] * n0 + L[2] * (-n1), ml[2] = L[1] * n1 + L[2] * n0, ml[3] = L[3];
+    const double m0 = v == 1 ? n0 : n1, m1 = v == 1 ? -n1 : n0; // lanes 1, 2: the momentum rows turned back
+    const double R1[4] = {v0 - a, v0, 0.0, v0 + a}, R2[4] = {v1, v1, 1.0, v1};
+    const double R0[4] = {1.0, 1.0, 0.0, 1.0}, R3[4] = {H - v0 * a, 0.5 * vsqr, v1, H + v0 * a};
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+        mr[c] = v == 0 ? R0[c] : v == 3 ? R3[c] : m0 * R1[c] + m1 * R2[c];
     return true;
 }
 
