@@ -235,13 +235,22 @@ __global__ __launch_bounds__(kBlock) void k_lusgs_sweep(int32_t n, int32_t b, Lu
 // each, 15 per Krylov vector on a small mesh): of a vector's work the dots are
 // one, the subtraction with the new norm's partials one and the scaling one.
 // Up to kFoldBlocks workgroups each workgroup of the second and third folds
-// the first's and second's partials itself, in the order k_gm_dots_final has;
-// beyond, reading all partials in every workgroup costs more than the two
-// launches.  Per implicit iteration (10 vectors, 2 restarts), us, separate
-// axpy launches before -> fused, not folded -> folded:
-// 1.5k cells 1265 -> - -> 1089, 29k 1576 -> 1265 -> 1187, 68k 1902 -> 1616 ->
-// 1483, 256k (1000 workgroups) 3246 -> 2948 -> 2666, 600k (2344) 8479 -> 6853
-// (launches -> folded), 1M (3907) 11410 -> 11646.
+// the first's and second's partials itself, in the order k_gm_dots_final has.
+// Those are the workgroups that the chip holds at once (8 of 256 threads on
+// each of 256 CUs); of more, the later ones fold all partials once again in
+// their turn.  Per implicit iteration (2 restarts), us, two launches for the
+// sums / folded:
+//   workgroups    5 vectors      10 (the default)      30
+//      500        862 /  816     1531 /  1322      5923 /  4362
+//     1020       1410 / 1329     2562 /  2242     10424 /  7661
+//     2048       2448 / 2381     4677 /  4222     20700 / 15805
+//     2100       2537 / 2580     4939 /  4772     22002 / 19455
+//     2343       2839 / 2912     5503 /  5440     24046 / 21813
+//     2700       3293 / 3422     6359 /  6322     27923 / 25012
+//     3100       3826 / 4076     7292 /  7502     32748 / 29851
+//     3905       4909 / 5217     9266 /  9528     42585 / 37790
+// Below the line folding wins with every number of vectors, beyond it by its
+// 10 vectors it is even and then behind; only long subspaces would still gain.
 constexpr int kFoldBlocks = 2048;
 
 // the sum of a workgroup's 256 values, in thread 0
@@ -571,7 +580,7 @@ int ensure_lusgs_scan(dndsmi_ctx *c) {
 
 // keep: also c_f and lambda by slot, for the solver's own sweeps (LUSGSMatrixInit
 // as an entry point has no use for them: 19.0 us with their stores on 550 k
-// cells, 16.5 without)
+// cells, 14.1 without)
 int launch_lusgs_init(dndsmi_ctx *c, const double *dtau, double dt, double alpha, bool keep) {
     DNDSMI_TRY(ensure_lusgs_scan(c));
     if (!c->jdiag)
