@@ -145,7 +145,6 @@ struct dndsmi_ctx {
     double *res_part = nullptr;       // [4][grid]
     double *rec_diff = nullptr;       // [ldc] squared increment of a sweep per cell (launch_increment)
     double *host_sums = nullptr;      // its sums over 256 cells, pinned
-    double *res = nullptr;            // [4]
     // the learned warm start inside the mixed-precision step
     // (dndsmi_ssprk3_set_warm_start): the previous stage's cell means and
     // their change [ldc][4], the plain shadow run of a check window

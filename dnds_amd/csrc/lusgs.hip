@@ -306,8 +306,8 @@ __device__ __forceinline__ double fold_partials(int32_t nblk, const double *__re
     return a;
 }
 
-// folds the partials of each dot product; out[q * ostride] = the sum, or its
-// square root (norms), in host_out too
+// folds the partials of each dot product; host_out[q * ostride] = the sum, or
+// its square root (norms), and where a kernel reads it out[q * ostride] too
 __global__ __launch_bounds__(64) void k_gm_dots_final(int32_t nblk, int32_t nq, const double *__restrict__ part,
                                                       int32_t take_sqrt, double *__restrict__ out, int32_t ostride,
                                                       double *host_out) {
@@ -315,7 +315,8 @@ __global__ __launch_bounds__(64) void k_gm_dots_final(int32_t nblk, int32_t nq, 
         const double a = fold_partials(nblk, part + int64_t(q) * nblk);
         if (threadIdx.x == 0) {
             const double d = take_sqrt ? sqrt(a) : a;
-            out[q * ostride] = d;
+            if (out)
+                out[q * ostride] = d;
             host_out[q * ostride] = d;
         }
     }
@@ -480,7 +481,7 @@ __global__ __launch_bounds__(kBlock) void k_residual(int32_t nc, const double *_
 
 // one wavefront per variable folds the block partials in a fixed order
 __global__ __launch_bounds__(kBlock) void k_residual_final(int32_t nblk, int32_t P, const double *__restrict__ part,
-                                                           double *__restrict__ res, double *host_res) {
+                                                           double *host_res) {
     const int v = threadIdx.x / 64, lane = threadIdx.x % 64;
     if (v >= 4)
         return;
@@ -491,10 +492,8 @@ __global__ __launch_bounds__(kBlock) void k_residual_final(int32_t nblk, int32_t
         const double o = __shfl_down(a, off, 64);
         a = P >= 3 ? fmax(a, o) : a + o;
     }
-    if (lane == 0) {
-        res[v] = a;
+    if (lane == 0)
         host_res[v] = a;
-    }
 }
 
 // fdtau's division by alphaDiag (DNDS_FV_EulerSolver.hpp:846-847)
@@ -551,7 +550,6 @@ int ensure_implicit_scratch(dndsmi_ctx *c) {
     DNDSMI_TRY(c->alloc(c->imp_xinc, 4 * c->ldc));
     DNDSMI_TRY(c->alloc(c->imp_dtau, c->ldc));
     DNDSMI_TRY(c->alloc(c->res_part, 4 * int64_t(grid_for(c->nc))));
-    DNDSMI_TRY(c->alloc(c->res, 4));
     return DNDSMI_OK;
 }
 
@@ -753,7 +751,7 @@ int gmres_solve(dndsmi_ctx *c, double alpha, const double *b, const double *u, d
     for (int32_t iRestart = 0; iRestart <= c->n_gmres_iter; iRestart++) {
         DNDSMI_TRY(MLA(x, V));
         hipLaunchKernelGGL(k_gm_axpy, dim3(gc), dim3(kBlock), 0, c->stream, nc, V, MLb, -1.0, c->gm_part);
-        DNDSMI_TRY(fold_dots(1, 1, c->gm_y, 1, &c->host->beta));
+        DNDSMI_TRY(fold_dots(1, 1, nullptr, 1, &c->host->beta));
         DNDSMI_TRY(c->hip(hipStreamSynchronize(c->stream), "hipStreamSynchronize"));
         const double beta = c->host->beta;
         if (std::fabs(beta) < 1e-200 || iRestart == c->n_gmres_iter)
@@ -811,14 +809,13 @@ int fsolve(dndsmi_ctx *c, const double *dtau, double dt, double alpha, const dou
     return DNDSMI_OK;
 }
 
-// residual into c->res (device) and then into host res[4]; x += r first when x
-// part: [4][grid_for(nc)] block partials, res_dev: [4]; both written before read
-int residual(dndsmi_ctx *c, const double *r, double *x, int32_t P, int32_t vol_wise, double *res_host, double *part,
-             double *res_dev) {
+// residual into the context's host words and then into res_host[4]; x += r
+// first when x.  part: [4][grid_for(nc)] block partials, written before read
+int residual(dndsmi_ctx *c, const double *r, double *x, int32_t P, int32_t vol_wise, double *res_host, double *part) {
     const unsigned g = grid_for(c->nc);
     hipLaunchKernelGGL(k_residual, dim3(g), dim3(kBlock), 0, c->stream, int32_t(c->nc), r, x, c->vol, P, vol_wise,
                        part);
-    hipLaunchKernelGGL(k_residual_final, dim3(1), dim3(kBlock), 0, c->stream, int32_t(g), P, part, res_dev,
+    hipLaunchKernelGGL(k_residual_final, dim3(1), dim3(kBlock), 0, c->stream, int32_t(g), P, part,
                        c->host->res);
     DNDSMI_TRY(c->launch_check("residual kernels"));
     DNDSMI_TRY(check_errw(c));
@@ -895,15 +892,16 @@ extern "C" int dndsmi_evaluate_residual(dndsmi_ctx *c, const dndsmi_array *rhs, 
     if (!c || !same_ctx(c, rhs, DNDSMI_ARRAY_DOF) || !res || P < 1)
         return DNDSMI_ERR_INVALID_ARGUMENT;
     DNDSMI_TRY(ensure_implicit_scratch(c));
-    return residual(c, rhs->d, nullptr, P, volWise, res, c->res_part, c->res);
+    return residual(c, rhs->d, nullptr, P, volWise, res, c->res_part);
 }
 
 // ---- the allocation-free residual ---------------------------------------
 //
 // dndsmi_evaluate_residual_noalloc computes what dndsmi_evaluate_residual
-// does, with the same kernels, but keeps the block partials and the four
-// results in `scratch`, a static array of the library on each GPU, instead
-// of the context's lazily allocated buffers.  Host code must not pass
+// does, with the same kernels, but keeps the block partials in `scratch`, a
+// static array of the library on each GPU, instead of the context's lazily
+// allocated buffer (the four results go to the context's host words, as
+// there).  Host code must not pass
 // `scratch` itself to a kernel (on the host the name is only a stand-in);
 // its device address is looked up once per device and kept in
 // g_scratch_dev.  Every k_residual block writes its partials before
@@ -911,7 +909,7 @@ extern "C" int dndsmi_evaluate_residual(dndsmi_ctx *c, const dndsmi_array *rhs, 
 // All calls on one GPU share the array: calls that overlap in time on one
 // GPU (from other streams or host threads) race.
 constexpr int64_t kNoAllocMaxBlocks = 65536; // n_cell <= 65536 * 256 = 16,777,216
-constexpr int64_t kNoAllocScratch = 4 * kNoAllocMaxBlocks + 4;
+constexpr int64_t kNoAllocScratch = 4 * kNoAllocMaxBlocks;
 static __device__ __align__(256) double scratch[kNoAllocScratch];
 
 namespace {
@@ -955,8 +953,7 @@ extern "C" int dndsmi_evaluate_residual_noalloc(dndsmi_ctx *c, const dndsmi_arra
         c->err = "dndsmi_evaluate_residual_noalloc: the static scratch was not looked up";
         return DNDSMI_ERR_HIP;
     }
-    double *part = c->noalloc_scratch;
-    return residual(c, rhs->d, nullptr, P, volWise, res, part, part + 4 * kNoAllocMaxBlocks);
+    return residual(c, rhs->d, nullptr, P, volWise, res, c->noalloc_scratch);
 }
 
 extern "C" int dndsmi_implicit_euler_step(dndsmi_ctx *c, dndsmi_array *u, dndsmi_array *uRec, dndsmi_array *uRecNew,
@@ -995,7 +992,7 @@ extern "C" int dndsmi_implicit_euler_step(dndsmi_ctx *c, dndsmi_array *u, dndsmi
         DNDSMI_TRY(fsolve(c, c->imp_dtau, dt, alpha, c->imp_rhs, u->d, c->imp_xinc));
         // x += xinc, fstop on the L1 norm of xinc
         double res[4];
-        DNDSMI_TRY(residual(c, c->imp_xinc, u->d, 1, 0, res, c->res_part, c->res));
+        DNDSMI_TRY(residual(c, c->imp_xinc, u->d, 1, 0, res, c->res_part));
         if (res_hist)
             for (int v = 0; v < 4; v++)
                 res_hist[4 * (iter - 1) + v] = res[v];
@@ -1111,7 +1108,7 @@ extern "C" int dndsmi_sdirk4_step(dndsmi_ctx *c, dndsmi_array *u, dndsmi_array *
             DNDSMI_TRY(c->launch_check("k_sdirk_rhs"));
             DNDSMI_TRY(fsolve(c, c->imp_dtau, dt, aii, c->imp_rhs, u->d, c->imp_xinc));
             double res[4];
-            DNDSMI_TRY(residual(c, c->imp_xinc, u->d, 1, 0, res, c->res_part, c->res));
+            DNDSMI_TRY(residual(c, c->imp_xinc, u->d, 1, 0, res, c->res_part));
             if (res_hist)
                 for (int v = 0; v < 4; v++)
                     res_hist[(int64_t(ib) * max_iter + (iter - 1)) * 4 + v] = res[v];
@@ -1238,7 +1235,7 @@ extern "C" int dndsmi_bdf_step(dndsmi_bdf *b, dndsmi_array *u, dndsmi_array *uRe
         // fsolve with alphaDiag = alpha0
         DNDSMI_TRY(fsolve(c, c->imp_dtau, dt, alpha0, c->imp_rhs, u->d, c->imp_xinc));
         double res[4];
-        DNDSMI_TRY(residual(c, c->imp_xinc, u->d, 1, 0, res, c->res_part, c->res));
+        DNDSMI_TRY(residual(c, c->imp_xinc, u->d, 1, 0, res, c->res_part));
         if (res_hist)
             for (int v = 0; v < 4; v++)
                 res_hist[4 * (iter - 1) + v] = res[v];
