@@ -365,8 +365,8 @@ def main():
         if pp:
             probe = {"launches": pp["launches"], "avg_ms": pp["avg_ms"], "bytes": pp["bytes"], "gbs": pp["gbs"],
                      "frac_of_peak": pp["gbs"] / HBM_PEAK_GBS,
-                     "what": "16-byte non-temporal loads of the sweep's A^-1 B pairs, as the sweep issues them, "
-                             "one double written per cell"}
+                     "what": "the sweep's 16-byte loads of A^-1 B and A^-1 b in the sweep's layout, as the sweep "
+                             "issues them, four doubles written per cell"}
             log(f"read probe: {pp['gbs']:.0f} GB/s ({pp['gbs'] / HBM_PEAK_GBS:.2f} of peak)")
     mixed = None
     if args.mixed:

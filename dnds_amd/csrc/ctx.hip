@@ -569,12 +569,15 @@ __global__ __launch_bounds__(1024) void k_diff2_sums(int32_t nc, const double *_
 }
 
 // Read-bandwidth probe of the sweep's dominant stream: every cell streams its
-// slots' A^-1 B, A^-1 b exactly as k_jacobi does (16-byte non-temporal loads,
-// the same slots skipped) with none of the sweep's gathers, and writes one
-// double per lane.  Its rate is the ceiling of the sweep's streaming part.
+// slots' A^-1 B, A^-1 b with k_jacobi's loads (four lanes per cell, 16 bytes
+// each, the same share of the stream kept in the Infinity Cache, the same slots
+// skipped) and none of the sweep's gathers, and writes one double per lane.
+// Its rate is the ceiling of the sweep's streaming part in this layout; it says
+// nothing about another one.
 template <int NF>
 __global__ __launch_bounds__(kBlock) void k_read_probe(int32_t nc, int64_t ldc, const int32_t *__restrict__ nbr,
-                                                       const double *__restrict__ M, double *__restrict__ out) {
+                                                       const double *__restrict__ M, double *__restrict__ out,
+                                                       int32_t keep) {
     const int32_t t = xcd_block() * blockDim.x + threadIdx.x, i = t >> 2, v = t & 3;
     if (i >= nc)
         return;
@@ -584,7 +587,7 @@ __global__ __launch_bounds__(kBlock) void k_read_probe(int32_t nc, int64_t ldc, 
         if (nbr[s * ldc + i] == -2)
             continue;
         AbPart ab;
-        ab.load(M, s, i, ldc, v, 0);
+        ab.load(M, s, i, ldc, v, keep);
 #pragma unroll
         for (int k = 0; k < kAbVecs / 4; k++)
             a += ab.w[k].x + ab.w[k].y;
@@ -2847,7 +2850,8 @@ extern "C" int dndsmi_read_probe(dndsmi_ctx *c, int32_t reps) {
     for (int k = 0; k < reps; k++) {
         prof_begin(c, DNDSMI_K_READ_PROBE);
         hipLaunchKernelGGL((c->nfmax == 3 ? k_read_probe<3> : k_read_probe<4>), dim3(grid_for(4 * c->nc)),
-                           dim3(kBlock), 0, c->stream, int32_t(c->nc), c->ldc, c->nbr, c->M, c->probe_out);
+                           dim3(kBlock), 0, c->stream, int32_t(c->nc), c->ldc, c->nbr, c->M, c->probe_out,
+                           keep_share(c, kAbVecs, kKeepLargest));
         prof_end(c);
         DNDSMI_TRY(c->launch_check("k_read_probe"));
     }

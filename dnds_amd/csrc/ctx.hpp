@@ -156,7 +156,7 @@ struct dndsmi_ctx {
     int32_t ws_check_steps = 1, ws_recheck = 0, ws_win_left = 0, ws_since_check = 0;
     double ws_tol = 0.0, ws_last_dev = -1.0;
     int64_t ws_stats[3] = {0, 0, 0}; // stages corrected, windows passed, windows failed (fallbacks)
-    double *probe_out = nullptr; // [ldc] output of the read-bandwidth probe (first use)
+    double *probe_out = nullptr; // [ldc][4] output of the read-bandwidth probe (first use)
     // device address of this GPU's static scratch of the allocation-free
     // residual (set at context creation; never freed: it is not an allocation)
     double *noalloc_scratch = nullptr;

@@ -578,9 +578,10 @@ int dndsmi_profile_query(dndsmi_ctx *ctx, int32_t kernel, int64_t *count, double
 int64_t dndsmi_kernel_bytes(const dndsmi_ctx *ctx, int32_t kernel);
 
 /* No counterpart in the reference (measurement): reps launches of a kernel
- * that streams the sweep's A^-1 B pairs exactly as the Jacobi sweep does,
- * without its gathers (DNDSMI_K_READ_PROBE in the profile): the read
- * bandwidth the sweep's streaming part can reach on this device. */
+ * that streams A^-1 B and A^-1 b with the loads and the layout of the Jacobi
+ * sweep, without its gathers (DNDSMI_K_READ_PROBE in the profile): the read
+ * bandwidth the sweep's streaming part can reach on this device in this
+ * layout. */
 int dndsmi_read_probe(dndsmi_ctx *ctx, int32_t reps);
 
 #ifdef __cplusplus
