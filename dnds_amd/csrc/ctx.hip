@@ -1,9 +1,11 @@
 // Device context, arrays and the FP64 kernels of the hot path (gfx950).
 //
 // The context holds the mesh and the VR setup in device memory, repacked from
-// the reference layouts into structure-of-arrays streams so that a wavefront
-// of 64 cells (or faces) reads each matrix element as one contiguous 512-byte
-// segment.  All kernels are launched on the context's stream.
+// the reference layouts into those of kernels.hpp: the sweep matrices in groups
+// of 16 cells as a wave of four lanes per cell loads them (ab_vec), coefficients
+// in blocks of 64 cells with the four variables side by side (rec), the other
+// arrays of several values per cell or face in blocks of 64 (blk64, quad64).
+// All kernels are launched on the context's stream.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -328,10 +330,10 @@ __global__ __launch_bounds__(kBlock, 3) void k_sor(int32_t n, int32_t base, int6
 // couples the cell to itself (M_if x_i), a Wall face adds b_if (0 - u_i)^T,
 // Wall_Euler / Wall_NoSlip faces add their correction from the old iterate.
 //
-// diff2 (may be null): receives |x_i - new_i|^2 per cell.  A kernel of its own
-// for it read both arrays again (one thread per cell, uncoalesced): 67 us per
-// sweep of dndsmi_reconstruct_to_tolerance on 66 k cells, 47 now, and 425 / 271
-// on 524 k; here the old coefficients come from the caches.
+// diff2 (may be null): receives |x_i - new_i|^2 per cell; the old coefficients
+// come from the caches.  With a kernel of its own that reads both arrays again
+// (k_rec_diff2) a sweep of dndsmi_reconstruct_to_tolerance takes 49.5 us on 66 k
+// cells, 43.5 this way, and 300 / 268 on 524 k.
 //
 // RESID (the FP64 step of the mixed-precision sweeps): instead of the new
 // iterate, writes the increment r = J(x) - x rounded to FP32 into r32 (also the
