@@ -2572,12 +2572,12 @@ int ensure_mixed(dndsmi_ctx *c) {
     if (c->M32)
         return DNDSMI_OK;
     const int64_t nm = int64_t(c->nfmax) * kAb32Vecs * 4 * c->ldc;
-    DNDSMI_TRY(c->alloc(c->M32, nm));
-    DNDSMI_TRY(c->alloc(c->r32, 36 * c->ldc));
-    DNDSMI_TRY(c->alloc(c->dA32, 36 * c->ldc));
-    DNDSMI_TRY(c->alloc(c->dB32, 36 * c->ldc));
-    DNDSMI_TRY(c->alloc(c->fslot32, int64_t(c->nfmax) * 8 * c->ldc));
-    DNDSMI_TRY(c->alloc(c->wcorr32, kRec * c->n_wall));
+    DNDSMI_TRY(c->ensure(c->r32, 36 * c->ldc));
+    DNDSMI_TRY(c->ensure(c->dA32, 36 * c->ldc));
+    DNDSMI_TRY(c->ensure(c->dB32, 36 * c->ldc));
+    DNDSMI_TRY(c->ensure(c->fslot32, int64_t(c->nfmax) * 8 * c->ldc));
+    DNDSMI_TRY(c->ensure(c->wcorr32, kRec * c->n_wall));
+    DNDSMI_TRY(c->alloc(c->M32, nm)); // the last: all are there where it is
     hipLaunchKernelGGL(k_m_to_f32, dim3(grid_for(nm / 4)), dim3(kBlock), 0, c->stream, int32_t(c->nfmax), c->ldc,
                        c->M, c->M32);
     DNDSMI_TRY(c->launch_check("k_m_to_f32"));

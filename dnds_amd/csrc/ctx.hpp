@@ -182,6 +182,13 @@ struct dndsmi_ctx {
         p = static_cast<T *>(q);
         return DNDSMI_OK;
     }
+    // an array that a call takes on first use.  Where several belong together,
+    // each is asked for by itself on every call: after a call that ran out of
+    // memory half-way the next one goes on where it stopped.
+    template <class T>
+    int ensure(T *&p, int64_t n) {
+        return p ? int(DNDSMI_OK) : alloc(p, n);
+    }
     int hip(hipError_t e, const char *what) {
         if (e != hipSuccess) {
             err = std::string(what) + ": " + hipGetErrorString(e);

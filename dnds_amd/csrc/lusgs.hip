@@ -544,26 +544,23 @@ __global__ __launch_bounds__(kBlock) void k_fill_scalar(int32_t n, const double 
 }
 
 int ensure_implicit_scratch(dndsmi_ctx *c) {
-    if (c->imp_rhs)
-        return DNDSMI_OK;
-    DNDSMI_TRY(c->alloc(c->imp_rhs, 4 * c->ldc));
-    DNDSMI_TRY(c->alloc(c->imp_xinc, 4 * c->ldc));
-    DNDSMI_TRY(c->alloc(c->imp_dtau, c->ldc));
-    DNDSMI_TRY(c->alloc(c->res_part, 4 * int64_t(grid_for(c->nc))));
-    return DNDSMI_OK;
+    DNDSMI_TRY(c->ensure(c->imp_rhs, 4 * c->ldc));
+    DNDSMI_TRY(c->ensure(c->imp_xinc, 4 * c->ldc));
+    DNDSMI_TRY(c->ensure(c->imp_dtau, c->ldc));
+    return c->ensure(c->res_part, 4 * int64_t(grid_for(c->nc)));
 }
 
 int ensure_lusgs_scan(dndsmi_ctx *c) {
-    if (c->sc_jf)
+    if (c->sc_vol)
         return DNDSMI_OK;
     const int64_t n = int64_t(c->nfmax) * c->ldc;
-    DNDSMI_TRY(c->alloc(c->sc_jf, n));
-    DNDSMI_TRY(c->alloc(c->sc_jb, n));
-    DNDSMI_TRY(c->alloc(c->sc_face, n));
-    DNDSMI_TRY(c->alloc(c->sc_n0, n));
-    DNDSMI_TRY(c->alloc(c->sc_n1, n));
-    DNDSMI_TRY(c->alloc(c->sc_area, n));
-    DNDSMI_TRY(c->alloc(c->sc_vol, c->ldc));
+    DNDSMI_TRY(c->ensure(c->sc_jf, n));
+    DNDSMI_TRY(c->ensure(c->sc_jb, n));
+    DNDSMI_TRY(c->ensure(c->sc_face, n));
+    DNDSMI_TRY(c->ensure(c->sc_n0, n));
+    DNDSMI_TRY(c->ensure(c->sc_n1, n));
+    DNDSMI_TRY(c->ensure(c->sc_area, n));
+    DNDSMI_TRY(c->alloc(c->sc_vol, c->ldc)); // the last: all are there where it is
     const int nc = int(c->nc);
     if (c->nfmax == 3)
         hipLaunchKernelGGL(k_lusgs_scan<3>, dim3(grid_for(nc)), dim3(kBlock), 0, c->stream, nc, c->ldc, c->ldf,
@@ -581,12 +578,11 @@ int ensure_lusgs_scan(dndsmi_ctx *c) {
 // cells, 14.1 without)
 int launch_lusgs_init(dndsmi_ctx *c, const double *dtau, double dt, double alpha, bool keep) {
     DNDSMI_TRY(ensure_lusgs_scan(c));
-    if (!c->jdiag)
-        DNDSMI_TRY(c->alloc(c->jdiag, c->ldc));
-    if (keep && !c->sc_cf)
-        DNDSMI_TRY(c->alloc(c->sc_cf, int64_t(c->nfmax) * c->ldc));
-    if (keep && !c->sc_lam)
-        DNDSMI_TRY(c->alloc(c->sc_lam, int64_t(c->nfmax) * c->ldc));
+    if (keep) {
+        DNDSMI_TRY(c->ensure(c->sc_cf, int64_t(c->nfmax) * c->ldc));
+        DNDSMI_TRY(c->ensure(c->sc_lam, int64_t(c->nfmax) * c->ldc));
+    }
+    DNDSMI_TRY(c->ensure(c->jdiag, c->ldc));
     const int nc = int(c->nc);
     auto kern = c->nfmax == 3 ? (keep ? k_lusgs_init<3, true> : k_lusgs_init<3, false>)
                               : (keep ? k_lusgs_init<4, true> : k_lusgs_init<4, false>);
@@ -715,6 +711,7 @@ int ensure_gmres(dndsmi_ctx *c) {
         }
     };
     release(c->gm_v), release(c->gm_h), release(c->gm_part), release(c->gm_y);
+    c->gm_alloc_space = 0;
     DNDSMI_TRY(c->alloc(c->gm_v, int64_t(k + 3) * 4 * c->ldc));
     DNDSMI_TRY(c->alloc(c->gm_h, int64_t(k + 1) * k));
     DNDSMI_TRY(c->alloc(c->gm_part, int64_t(k + 1) * grid_for(c->nc)));

@@ -860,10 +860,10 @@ AdamStep adam_step(dndsmi_warmstart *w, double lr) {
 }
 
 int features(dndsmi_warmstart *w, const double *u) {
-    if (!w->fX) {
-        DNDSMI_TRY(w->alloc(w->fX, w->nc * kIn));
+    if (!w->fS)
         DNDSMI_TRY(w->alloc(w->fS, w->nc * 4));
-    }
+    if (!w->fX)
+        DNDSMI_TRY(w->alloc(w->fX, w->nc * kIn));
     hipLaunchKernelGGL(k_features, dim3(grid_for(w->nc)), dim3(256), 0, w->ctx->stream, int32_t(w->nc), w->ldc,
                        w->sten, u, w->mom, w->logsz, w->fX, w->fS);
     return w->ctx->launch_check("k_features");
@@ -987,10 +987,8 @@ namespace dndsmi_host {
 
 int ws_stage_begin(dndsmi_ctx *c, const double *u, double *x, bool use) {
     dndsmi_warmstart *w = c->step_ws;
-    if (!c->ws_uprev) {
-        DNDSMI_TRY(c->alloc(c->ws_uprev, 4 * c->ldc));
-        DNDSMI_TRY(c->alloc(c->ws_du, 4 * c->ldc));
-    }
+    DNDSMI_TRY(c->ensure(c->ws_uprev, 4 * c->ldc));
+    DNDSMI_TRY(c->ensure(c->ws_du, 4 * c->ldc));
     if (!c->ws_have_prev) {
         DNDSMI_TRY(c->hip(hipMemcpyAsync(c->ws_uprev, u, sizeof(double) * 4 * c->nc, hipMemcpyDeviceToDevice,
                                          c->stream),
@@ -1014,11 +1012,9 @@ int ws_stage_begin(dndsmi_ctx *c, const double *u, double *x, bool use) {
 }
 
 int ws_window_begin(dndsmi_ctx *c, const double *u, const double *x) {
-    if (!c->ws_sh_u) {
-        DNDSMI_TRY(c->alloc(c->ws_sh_u, 4 * c->ldc));
-        DNDSMI_TRY(c->alloc(c->ws_sh_x, 36 * c->ldc));
-        DNDSMI_TRY(c->alloc(c->ws_part, 2 * int64_t(grid_for(36 * c->ldc)) + 2));
-    }
+    DNDSMI_TRY(c->ensure(c->ws_sh_u, 4 * c->ldc));
+    DNDSMI_TRY(c->ensure(c->ws_sh_x, 36 * c->ldc));
+    DNDSMI_TRY(c->ensure(c->ws_part, 2 * int64_t(grid_for(36 * c->ldc)) + 2));
     DNDSMI_TRY(c->hip(hipMemcpyAsync(c->ws_sh_u, u, sizeof(double) * 4 * c->ldc, hipMemcpyDeviceToDevice, c->stream),
                       "copy u to the shadow"));
     return c->hip(hipMemcpyAsync(c->ws_sh_x, x, sizeof(double) * 36 * c->ldc, hipMemcpyDeviceToDevice, c->stream),
