@@ -274,8 +274,8 @@ def main():
                     help="after the timed steps, N device copies of one rec array (a plain copy of known size "
                          "for scaling profiler byte counters), timed (0 = skip)")
     ap.add_argument("--read-probe", type=int, default=10,
-                    help="after the timed steps, N launches of a kernel that streams the sweep's A^-1 B pairs as the "
-                         "sweep does, without its gathers: the read ceiling of the sweep's streaming part (0 = skip)")
+                    help="after the timed steps, N launches of a kernel that streams A^-1 B and A^-1 b as the sweep "
+                         "does, without its gathers: the read ceiling of its streaming part in its layout (0 = skip)")
     ap.add_argument("--mixed", type=int, default=1,
                     help="also run the mixed-precision arm (FP32 correction sweeps + FP64 refinement) over the same "
                          "steps from the same initial state")
@@ -509,8 +509,14 @@ def main():
             lib.dndsmi_profile_query(ev.device.ctx, k, C.byref(cnt), C.byref(tot))
             if cnt.value:
                 b = int(lib.dndsmi_kernel_bytes(ev.device.ctx, k))
-                if name == "k_lusgs_sweep":  # bytes are per whole sweep (one launch per colour)
-                    sweeps = cnt.value // max(ev.LUSGSColouring()[1], 1)
+                if name == "k_lusgs_sweep":
+                    # bytes are per whole sweep.  Sweeps come in pairs, forward and backward: one for LU-SGS by
+                    # itself, one for GMRES' right-hand side and one per product.  (A launch is a colour, but the
+                    # last colour of a pair takes both directions at once and a product the first forward one.)
+                    mv, mv_ms = C.c_int64(), C.c_double()
+                    lib.dndsmi_profile_query(ev.device.ctx, A.KERNEL_NAMES.index("k_lusgs_matvec"), C.byref(mv),
+                                             C.byref(mv_ms))
+                    sweeps = 2 * (len(hist) * ((args.gmres != 1) + (args.gmres != 0)) + mv.value)
                     iprof[name] = dict(launches=cnt.value, sweeps=sweeps, ms_per_sweep=tot.value / sweeps, bytes=b,
                                        gbs=b * sweeps / (tot.value * 1e-3) / 1e9)
                 else:
