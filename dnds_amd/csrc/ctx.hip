@@ -2214,6 +2214,7 @@ extern "C" int dndsmi_array_create(dndsmi_ctx *c, int32_t kind, dndsmi_array **o
     a->elems = kind == DNDSMI_ARRAY_DOF ? 4 * c->ldc : (kind == DNDSMI_ARRAY_REC ? 36 * c->ldc : c->ldc);
     void *p = nullptr;
     if (hipMalloc(&p, sizeof(double) * a->elems) != hipSuccess) {
+        (void)hipGetLastError();
         delete a;
         c->err = "hipMalloc of an array failed";
         return DNDSMI_ERR_OUT_OF_MEMORY;

@@ -174,6 +174,7 @@ struct dndsmi_ctx {
         void *q = nullptr;
         hipError_t e = hipMalloc(&q, b);
         if (e != hipSuccess) {
+            (void)hipGetLastError(); // reported here, not again by the next launch_check
             err = std::string("hipMalloc: ") + hipGetErrorString(e);
             return DNDSMI_ERR_OUT_OF_MEMORY;
         }
@@ -191,6 +192,7 @@ struct dndsmi_ctx {
     }
     int hip(hipError_t e, const char *what) {
         if (e != hipSuccess) {
+            (void)hipGetLastError();
             err = std::string(what) + ": " + hipGetErrorString(e);
             return DNDSMI_ERR_HIP;
         }

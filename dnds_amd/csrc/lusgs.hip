@@ -1162,6 +1162,7 @@ extern "C" int dndsmi_bdf_create(dndsmi_ctx *c, int32_t k, dndsmi_bdf **out) {
     if (k > 1) {
         void *q = nullptr;
         if (hipMalloc(&q, sizeof(double) * 4 * size_t(c->ldc) * size_t(k - 1)) != hipSuccess) {
+            (void)hipGetLastError();
             delete b;
             c->err = "hipMalloc failed for the BDF history";
             return DNDSMI_ERR_OUT_OF_MEMORY;

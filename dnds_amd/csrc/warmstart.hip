@@ -741,6 +741,7 @@ struct dndsmi_warmstart {
     int alloc(T *&p, int64_t n) {
         void *q = nullptr;
         if (hipMalloc(&q, sizeof(T) * size_t(std::max<int64_t>(n, 1))) != hipSuccess) {
+            (void)hipGetLastError();
             ctx->err = "hipMalloc failed (warm start)";
             return DNDSMI_ERR_OUT_OF_MEMORY;
         }

@@ -23,3 +23,22 @@ def test_upload_download_round_trip(kind, nx, ny, sor):
         # the same rows again
         a.setConstant(3.0).upload(h[::-1].copy())
         assert np.array_equal(a.download(), h[::-1])
+
+
+def test_a_failed_allocation_is_reported_once():
+    """A warm start for 10^10 training rows (2.3 TB) is refused; the calls
+    after it are not."""
+    from conftest import rel_err
+    from dnds_amd import _capi as A
+    from dnds_amd.host import DNDSError, EulerEvaluator, WarmStart
+    from test_gpu_quads import TOL, _oracle, _state
+    mesh, vfv = _case(1, 12, 9)
+    ev = EulerEvaluator(mesh, vfv, riemannSolverType="HLLC", farFieldStaticValue=FAR)
+    u, x = _state(mesh.n_cell, 4)
+    du, dx, dn = ev.BuildMean().upload(u), vfv.BuildRec().upload(x), vfv.BuildRec()
+    with pytest.raises(DNDSError) as e:
+        WarmStart(ev, capacity=10**10)
+    assert e.value.code == A.ERR_OUT_OF_MEMORY
+    vfv.ReconstructionJacobiStep(du, dx, dn, 0.0)
+    assert rel_err(dx.download(), _oracle(mesh, vfv, FAR).jacobi_step(u, x)) <= TOL
+    ev.device.sync()
